@@ -94,9 +94,6 @@ inline XcdMap choose_xcd_map(uint32_t n_col_tiles, uint32_t n_token_tiles, uint3
     return best;
 }
 
-constexpr int GATHER_WAVES = 8;
-constexpr int GATHER_THREADS = GATHER_WAVES * 64;
-
 // The tanh form of GELU, 0.5 y (1 + tanh u) with u = sqrt(2/pi) (y + 0.044715 y^3), evaluated as
 // y * sigmoid(2u) = y / (1 + exp(-2u)): no cancellation of 1 + tanh u for negative y, exp overflow gives
 // y / inf = -0, and one v_exp_f32 plus one v_rcp_f32 (1 ulp each) keep it within 1e-6 relative.

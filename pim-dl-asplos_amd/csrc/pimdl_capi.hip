@@ -399,6 +399,21 @@ static void retile_lut(const T* lut, T* tiled, const AmmGeom& g, uint32_t row_el
             }
 }
 
+// canonical [CB][C][M] -> [M_pad/16][CB_pad/16][C_tile rows][16 codebooks][16 columns], zero padded (the byte adder)
+static void retile_lut_rows(const int8_t* lut, int8_t* tiled, const AmmGeom& g)
+{
+    const size_t slice = (size_t)g.C_tile * 256, chunk = (g.CB_pad / 16) * slice;  // bytes
+    for (uint32_t f0 = 0; f0 < g.M; f0 += 64)  // a cache line of every row at a time, written to four chunks
+        for (uint32_t cb0 = 0; cb0 < g.CB; cb0 += 16)
+            for (uint32_t c = 0; c < g.C; ++c)
+                for (uint32_t cb = cb0; cb < g.CB && cb < cb0 + 16; ++cb) {
+                    const int8_t* src = lut + ((size_t)cb * g.C + c) * g.M;
+                    int8_t* dst = tiled + (cb0 / 16) * slice + (size_t)c * 256 + (cb - cb0) * 16;
+                    for (uint32_t f = f0; f < g.M && f < f0 + 64; f += 16)
+                        memcpy(dst + (f / 16) * chunk, src + f, f + 16 <= g.M ? 16 : g.M - f);
+                }
+}
+
 // canonical [CB][C][M] -> [M_pad/col_block][CB_pad][col_block][16], zero padded (C <= 16);
 // C_tile 8 (C <= 8): [M_pad/col_block][CB_pad/2][col_block][2][8], codebooks 2k and 2k+1 side by side
 static void retile_lut_onehot(const int8_t* lut, int8_t* tiled, const AmmGeom& g)
@@ -554,7 +569,8 @@ int pimdl_amm_set_tuning(pimdl_amm* a, const pimdl_amm_tuning* t)
     Ctx* ctx = a->ctx;
     if (!t) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_set_tuning: null argument");
     const uint32_t kind = a->g.gather_kind == 0 ? PIMDL_GATHER_ROWS : a->g.gather_kind == 1 ? PIMDL_GATHER_ONEHOT : PIMDL_GATHER_SPARSE;
-    if ((t->col_block && t->col_block != a->g.col_block) || (t->gather_kernel && t->gather_kernel != kind))
+    if ((t->col_block && t->col_block != a->g.col_block) ||
+        (t->gather_kernel && t->gather_kernel != kind && !(a->g.auto_rows && t->gather_kernel == PIMDL_GATHER_SPARSE)))
         return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_set_tuning: col_block and gather_kernel fix the resident table; "
                                                  "create the operator with them (pimdl_amm_create_with)");
     std::string why;
@@ -630,7 +646,7 @@ int pimdl_amm_create_with(pimdl_ctx* ctx, const pimdl_amm_desc* desc, const floa
         return set_error(ctx, PIMDL_ERR_NOMEM, "pimdl_amm_create: host staging of %zu bytes failed", a->lut_bytes);
     }
     if (i8 && g.gather_kind != 0) retile_lut_onehot(reinterpret_cast<const int8_t*>(lut), reinterpret_cast<int8_t*>(tiled.data()), g);
-    else if (i8) retile_lut(reinterpret_cast<const int8_t*>(lut), reinterpret_cast<int8_t*>(tiled.data()), g, row_elems);
+    else if (i8) retile_lut_rows(reinterpret_cast<const int8_t*>(lut), reinterpret_cast<int8_t*>(tiled.data()), g);
     else if (grouped) {
         std::vector<float> wide;
         try {
@@ -773,13 +789,13 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
     if (!rc) rc = launch_ccs_prep(ctx, g, grp->d_centroids);
     if (!rc) rc = ensure(ctx, &ctx->d_idx, &ctx->idx_bytes, idx_buffer_bytes(g, max_n), "hipMalloc(index scratch)");
     // one gather launch for all members?
-    bool same = first->desc.lut_dtype == PIMDL_LUT_I8 && !first->grouped && first->g.gather_kind != 0 &&
+    bool same = first->desc.lut_dtype == PIMDL_LUT_I8 && !first->grouped && (first->g.gather_kind != 0 || first->g.auto_rows) &&
                 first->g.M % first->g.col_block == 0;
     const float lbt0 = first->desc.bias_mode == PIMDL_BIAS_TIMES_CB ? first->desc.lut_bias * (float)first->g.CB : first->desc.lut_bias;
     for (uint32_t i = 1; i < count && same; ++i) {
         const Amm* a = amms[i];
         const float lbt = a->desc.bias_mode == PIMDL_BIAS_TIMES_CB ? a->desc.lut_bias * (float)a->g.CB : a->desc.lut_bias;
-        same = a->desc.lut_dtype == PIMDL_LUT_I8 && !a->grouped && a->g.gather_kind == first->g.gather_kind && a->g.M == first->g.M &&
+        same = a->desc.lut_dtype == PIMDL_LUT_I8 && !a->grouped && a->g.gather_kind == first->g.gather_kind && a->g.auto_rows == first->g.auto_rows && a->g.M == first->g.M &&
                a->g.q == first->g.q && a->g.C_tile == first->g.C_tile && a->g.CB_pad == first->g.CB_pad &&
                a->lut_bytes == first->lut_bytes && a->desc.activation == first->desc.activation && lbt == lbt0;
     }

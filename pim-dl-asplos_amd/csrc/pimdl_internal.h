@@ -15,16 +15,15 @@ namespace pimdl {
 //
 // Index rows   [N][idx_row_bytes] bytes; IDX_BITS = 4 (C <= 16, codebook 2k in the low nibble
 //              of byte k) or 8.  Codebooks are padded to a multiple of 32 with index 0.
-//              idx_tiled (operators served by the one-hot gather): the same bytes stored as
+//              idx_tiled (int8 tables): the same bytes stored as
 //              [N/64][idx_row_bytes/4][64 tokens][4 bytes], so that the 32-bit index words one
 //              wave needs for one codebook slice (64 tokens x 1 word) are 256 contiguous bytes;
 //              the buffer covers N rounded up to 64 tokens.
-// int8 LUT     gather_kind 0: tiled [M_pad / col_block][CB_pad][C_tile][col_block] bytes
-//              (col_block = 16*Q); gather_kind 1: [M_pad / col_block][CB_pad][col_block][16] bytes
-//              (the 16 centroid entries of a column are contiguous).  Either way one (column block,
-//              codebook range) slice is contiguous, so staging it into LDS is a flat copy.  Padded
-//              codebooks / centroid rows / columns hold zeros.
-// fp32 LUT     tiled the same way with col_block floats per row.
+// int8 LUT     gather_kind 0: [M_pad / 16][CB_pad / 16][C_tile][16 codebooks][16 columns] bytes; gather_kind 1:
+//              [M_pad / col_block][CB_pad][col_block][16] bytes (the 16 centroid entries of a column are
+//              contiguous).  Either way one (columns, codebook range) slice is contiguous, so staging it
+//              into LDS is a flat copy.  Padded codebooks / centroid rows / columns hold zeros.
+// fp32 LUT     tiled [M_pad / col_block][CB_pad][C_tile][col_block] floats.
 // ---------------------------------------------------------------------------------------------
 struct AmmGeom {
     uint32_t K, v, CB, CB_pad, C, C_tile, M, M_pad;
@@ -32,14 +31,15 @@ struct AmmGeom {
     uint32_t idx_tiled;     // layout of the packed index buffer, see above
     uint32_t lut_chunked;   // fp32 table of 32 centroids: [column block][codebook][8-byte chunk][row][2 floats]
     // gather kernel
-    uint32_t gather_kind;   // 0: byte-adder rows kernel, 1: one-hot matrix-core kernel (int8, C <= 16),
+    uint32_t gather_kind;   // int8 tables: 0: byte adder, 1: one-hot matrix-core kernel (int8, C <= 16),
                             // 2: one-hot on the sparse matrix instruction (int8, C <= 32: a codebook of 17..32
                             //    centroids is two of 16 side by side; table laid out as for 1, with the columns
                             //    of a tile permuted by sparse_tile_column)
+    uint32_t auto_rows;     // 17..32 centroids, kind 0 by the library's own choice (the caller named no gather setting)
     uint32_t q;             // 16-byte chunks per LUT row in LDS
-    uint32_t col_block;     // columns per workgroup (int8: 16*q, fp32: 4*q)
-    uint32_t row_pitch;     // bytes between LUT rows in LDS (16*q + 16: bank-conflict-free b128 gathers)
-    uint32_t gq;            // int8: codebooks per lane group per slice; slice = 4*gq codebooks
+    uint32_t col_block;     // columns per workgroup (int8: 16*q -- the byte adder picks its own at launch --, fp32: 4*q)
+    uint32_t row_pitch;     // bytes between LUT rows in LDS
+    uint32_t gq;            // int8: codebooks per lane group per slice
     uint32_t cb_per_slice;
     uint32_t gather_threads, tokens_per_wg, gather_lds_bytes;
     // ccs kernel
@@ -180,6 +180,10 @@ int launch_diag_mfma_error(Ctx* ctx, uint32_t trials, bool crafted, float* max_e
 // the sparse one-hot gather (gather_sp_kernel.hip)
 int launch_gather_sparse(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc_or_null,
                          uint32_t n, float scale, float lut_bias_term);
+// the byte adder (gather_rows_kernel.hip)
+int launch_gather_rows(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc_or_null, uint32_t n,
+                       float scale, float lut_bias_term);
+uint32_t rows_lds_bytes(uint32_t c_tile, uint32_t q);
 uint32_t sparse_tile_column(uint32_t tn, uint32_t s);  // column of a tile stored at position s of the tile
 uint32_t sparse_lds_bytes(uint32_t tn, bool wide);
 // codebooks of 16 centroids in the table of the sparse one-hot gather: a codebook of 17..32 centroids is two

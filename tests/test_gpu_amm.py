@@ -573,3 +573,27 @@ def test_random_shapes_against_the_oracle(ctx, case):
         want = oracle.gather_i8_grouped(want_idx, lut, scales, bias, group, threads=THREADS)
         assert np.array_equal(amm.run(x).view(np.uint32), want.view(np.uint32))
     amm.close()
+
+
+@pytest.mark.parametrize("N,CB,C,M", [
+    (1, 1, 17, 1),          # one token, one codebook of a 16-codebook slice, one column of a 16-column chunk
+    (63, 15, 33, 15), (65, 17, 64, 17), (129, 33, 65, 33),   # edges of token blocks, slices, rows, chunks
+    (1025, 16, 32, 130),    # one token past an item, an odd number of chunks
+    (2500, 48, 24, 1040), (2500, 48, 50, 1040), (2500, 32, 100, 530), (2500, 32, 250, 530),  # several item sizes
+    (40000, 16, 32, 1040), (40000, 16, 64, 1040), (40000, 16, 128, 1040), (40000, 16, 256, 530),  # the widest waves
+])
+def test_byte_adder_edges(ctx, N, CB, C, M):
+    """17 centroids and more through the byte adder: every index, accumulator and output bit of the oracle."""
+    check_i8(ctx, 4200 + C + N, N, 4 * CB, 4, C, M, lut_bias=0.5, bias_mode=1)
+
+
+def test_byte_adder_item_sizes(ctx):
+    """The launch rule's ends: a batch that fills the chip takes eight token groups per wave, a small one a single group."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    x, cent, lut, bias = make_case(5, 40000, 64, 4, 64, 1040)
+    amm = ctx.amm(cent, lut, np.float32(0.01), bias, max_n=40000)
+    for n, groups in ((40000, 8), (70, 1)):
+        amm.run_debug(x[:n])  # the whole batch in one launch (run cuts host buffers into chunks)
+        assert amm.last_gather_kernel().split(", ")[3] == str(groups), amm.last_gather_kernel()
+    amm.close()
