@@ -1,0 +1,358 @@
+// LUT gather-accumulate for launches of few tokens (gfx950): the codebooks are what is dealt out.
+//
+// Same operator as the other gather kernels (inference-engine/src/dpu/pim_lut_kernel.c:97-2296, row-major
+// statement inference-engine/test/test_amm.cpp:164-175, epilogue inference-engine/src/host/pim_lut_host.cpp:190-203):
+//     acc[n][f] = sum over cb of lut[cb][idx[n][cb]][f]
+// on the tables of the large kernels, whatever their layout.  Those kernels give an item of 128 tokens or more and 16 to
+// 96 columns to a workgroup, which goes through all codebooks slice by slice; a launch with fewer items than CUs
+// then takes the time of that chain -- copy, barrier, operands, 32 codebooks further -- however few its tokens are.
+#include "gather_common.h"
+
+namespace pimdl {
+namespace {
+
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+
+// An int8 launch: a workgroup takes 16 columns of 16 * TM tokens, its NW waves deal out the K-steps of the matrix
+// instruction, every operand comes straight from memory (nothing is shared between waves, so nothing is staged), and the
+// waves' int32 sums meet in LDS once, at the end.  All loads of a wave are in flight together: a launch is one
+// round trip for the indices and the table, not one per slice.  What bounds it: up to 16 tokens the launch itself and
+// that round trip (3.0 us at 768 -> 3072, 4.5 at 3072 -> 768, whose 9.4 MB of table 48 CUs read; before 8.1 / 19.8);
+// beyond, the table entries that every 64 tokens read again and the operands made from index bytes (7.5 us at N = 64).
+constexpr int FEW_UNROLL = 4;       // K-steps of a wave whose loads are in flight together
+// floats between a wave's registers in the exchange: the reads below meet in no bank
+constexpr int FEW_PITCH_ONEHOT = 80, FEW_PITCH_ROWS = 68;
+constexpr int few_lds_bytes(int nw, int tm, int pitch) { return nw * tm * 4 * pitch * 4; }
+
+enum FewTable { FEW_SPARSE, FEW_PAIRED, FEW_ROWS };
+
+struct FewArgs {
+    const uint8_t* idx;
+    const int8_t* lut;
+    float* out;
+    int32_t* acc_out;
+    uint32_t N, M;
+    uint32_t groups;        // 16-column groups of the table
+    uint32_t steps;         // K-steps
+    uint32_t tile_groups;   // one-hot tables: 16-column groups per column tile; rows: 1
+    uint32_t c_tile;        // rows: rows per codebook in the table
+    uint32_t idx_row_bytes;
+    uint32_t op_groups;     // operators side by side: 16-column groups of each (0: one operator)
+};
+
+// Column of position s of a tile of one-hot tables (sparse_tile_column on the device)
+__device__ __forceinline__ uint32_t few_column(uint32_t tn, uint32_t c, uint32_t j)
+{
+    const uint32_t n4 = tn / 4 * 4, n2 = n4 + (tn % 4) / 2 * 2;
+    if (c < n4) return 16 * (c / 4 * 4) + 4 * j + c % 4;
+    if (c < n2) return 16 * n4 + 2 * j + (c - n4);
+    return 16 * c + j;
+}
+
+// One workgroup per (16 columns, 16 * TM tokens).  Operands of a K-step, lane l = 16 g + j:
+//   FEW_SPARSE  the sparse one-hot product (8 codebooks of 16): lane (g, token j) turns byte g of index word s into value
+//               bytes and positions, lane (g, column j) reads the table entries of codebooks g and g + 4
+//   FEW_PAIRED  the same instruction on the paired table (up to 8 centroids): an entry's 16 slots are two codebooks of
+//               8, whose one-hots fall into different groups of four, so a K-step covers 16 codebooks
+//   FEW_ROWS    the byte adder: lane (g, token j) reads its 16 columns of codebook 4 s + g, the constant operand
+//               A[i][16 g + b] = (b == i) adds them
+template <FewTable T, int TM, int NW>
+__global__ __launch_bounds__(NW * 64) void gather_few_kernel(FewArgs a, Epilogue ep)
+{
+    constexpr int PITCH = T == FEW_ROWS ? FEW_PITCH_ROWS : FEW_PITCH_ONEHOT;
+    extern __shared__ __attribute__((aligned(16))) int part[];  // [wave][4 TM registers][PITCH]
+    const uint32_t lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t col_group = blockIdx.x % a.groups, tok0 = blockIdx.x / a.groups * (16 * TM);
+    const uint32_t tile = col_group / a.tile_groups, c = col_group % a.tile_groups;
+    const uint32_t op = a.op_groups ? col_group / a.op_groups : 0u;
+    const uint32_t wn = 16 * a.tile_groups;
+    // 64-token block of the tiled index buffer (16 TM tokens lie in one block), this operator's words
+    const uint8_t* ix = a.idx + (size_t)op * ep.op_idx_stride + (size_t)(tok0 / 64) * a.idx_row_bytes * 64 + ((tok0 & 63) + j) * 4;
+
+    v4i acc[TM];
+#pragma unroll
+    for (int t = 0; t < TM; ++t) acc[t] = (v4i){0, 0, 0, 0};
+
+    if constexpr (T != FEW_ROWS) {
+        // entry e of column j: ((tile * entries + e) * wn + 16 c + j) * 16 bytes; a K-step is 8 entries
+        const int8_t* tab = a.lut + (((size_t)tile * a.steps * 8 + g) * wn + 16 * c + j) * 16;
+        ix += T == FEW_SPARSE ? g : (g >> 1) * 256 + (g & 1) * 2;
+        for (uint32_t s0 = wave; s0 < a.steps; s0 += NW * FEW_UNROLL) {
+            v4i lo[FEW_UNROLL], hi[FEW_UNROLL];
+            uint32_t raw[FEW_UNROLL][TM];
+#pragma unroll
+            for (int u = 0; u < FEW_UNROLL; ++u) {
+                const uint32_t s = s0 + u * NW;
+                if (s < a.steps) {  // uniform
+                    const int8_t* p = tab + (size_t)s * 8 * wn * 16;
+                    lo[u] = *reinterpret_cast<const v4i*>(p);
+                    hi[u] = *reinterpret_cast<const v4i*>(p + (size_t)4 * wn * 16);
+#pragma unroll
+                    for (int t = 0; t < TM; ++t) {
+                        if constexpr (T == FEW_SPARSE) raw[u][t] = ix[(size_t)s * 256 + t * 64];
+                        else raw[u][t] = *reinterpret_cast<const uint16_t*>(ix + (size_t)s * 512 + t * 64);
+                    }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < FEW_UNROLL; ++u) {
+                if (s0 + u * NW >= a.steps) break;  // uniform
+                const v8i bb = {lo[u][0], lo[u][1], lo[u][2], lo[u][3], hi[u][0], hi[u][1], hi[u][2], hi[u][3]};
+#pragma unroll
+                for (int t = 0; t < TM; ++t) {
+                    const uint32_t r = raw[u][t];
+                    // centroid k of an entry: value 1 in the first slot of group k / 4, position k % 4
+                    auto pos = [](uint32_t k) { return (k & 3u) << (4 * ((k >> 2) & 3u)); };
+                    v4i aa;
+                    uint32_t pw;
+                    if constexpr (T == FEW_SPARSE) {
+                        const uint64_t v0 = 1ull << ((r & 0x0Cu) << 2), v1 = 1ull << ((r >> 2) & 0x30u);
+                        aa = (v4i){(int)(uint32_t)v0, (int)(uint32_t)(v0 >> 32), (int)(uint32_t)v1, (int)(uint32_t)(v1 >> 32)};
+                        pw = pos(r & 15) | pos(r >> 4) << 16;
+                    } else {
+                        // four centroids of 8, a nibble each: codebooks 2e, 2e + 1 in the low and high half of entry e
+                        auto val = [&](int n) { return (int)(1u << ((r >> (4 * n) & 4u) << 2)); };
+                        aa = (v4i){val(0), val(1), val(2), val(3)};
+                        pw = pos(r & 7) | pos(r >> 4 & 7) << 8 | pos(r >> 8 & 7) << 16 | pos(r >> 12 & 7) << 24;
+                    }
+                    acc[t] = __builtin_amdgcn_smfmac_i32_16x16x128_i8(aa, bb, acc[t], (int)pw, 0, 0);
+                }
+            }
+        }
+    } else {
+        // codebook cb, row r: (((chunk * (CB_pad / 16) + cb / 16) * c_tile + r) * 16 + cb % 16) * 16 bytes
+        const int8_t* tab = a.lut + (size_t)col_group * (a.steps / 4) * a.c_tile * 256 + g * 16;
+        v4i one = (v4i){0, 0, 0, 0};  // byte j of lane (g, j)
+#pragma unroll
+        for (int w = 0; w < 4; ++w) one[w] = j / 4 == (uint32_t)w ? 1 << (8 * (j % 4)) : 0;
+        ix += g;
+        for (uint32_t s0 = wave; s0 < a.steps; s0 += NW * FEW_UNROLL) {
+            uint32_t raw[FEW_UNROLL][TM];
+            v4i row[FEW_UNROLL][TM];
+#pragma unroll
+            for (int u = 0; u < FEW_UNROLL; ++u)
+                if (s0 + u * NW < a.steps) {
+#pragma unroll
+                    for (int t = 0; t < TM; ++t)  // (index bytes of tokens past the batch were never written)
+                        raw[u][t] = tok0 + 16 * t + j < a.N ? ix[(size_t)(s0 + u * NW) * 256 + t * 64] : 0u;
+                }
+#pragma unroll
+            for (int u = 0; u < FEW_UNROLL; ++u) {
+                const uint32_t s = s0 + u * NW;
+                if (s < a.steps) {
+                    const int8_t* p = tab + (size_t)(s / 4) * a.c_tile * 256 + (s % 4) * 64;
+#pragma unroll
+                    for (int t = 0; t < TM; ++t) row[u][t] = *reinterpret_cast<const v4i*>(p + (size_t)raw[u][t] * 256);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < FEW_UNROLL; ++u) {
+                if (s0 + u * NW >= a.steps) break;
+#pragma unroll
+                for (int t = 0; t < TM; ++t) acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(one, row[u][t], acc[t], 0, 0, 0);
+            }
+        }
+    }
+
+    // lane (g, j) holds: one-hot forms tokens 4 g + r of column position j, byte adder columns 4 g + r of token j
+#pragma unroll
+    for (int t = 0; t < TM; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[((size_t)wave * TM * 4 + t * 4 + r) * PITCH + lane] = acc[t][r];
+    __syncthreads();
+    for (uint32_t o = threadIdx.x; o < TM * 256; o += NW * 64) {
+        const uint32_t x = o % 16, tok = o / 16;  // column position, token of the item
+        const uint32_t reg = tok / 16 * 4 + (T == FEW_ROWS ? x % 4 : tok % 4);
+        const uint32_t src = T == FEW_ROWS ? x / 4 * 16 + tok % 16 : (tok % 16) / 4 * 16 + x;
+        int32_t sum = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sum += part[((size_t)w * TM * 4 + reg) * PITCH + src];
+        const uint32_t n = tok0 + tok;
+        const uint32_t f = T == FEW_SPARSE ? tile * wn + few_column(a.tile_groups, c, x) : 16 * col_group + x;
+        if (n >= a.N || f >= a.M) continue;
+        Epilogue epl = ep;
+        if (a.op_groups) epl.scale = ep.op_scales[op];
+        const float b = ep.bias ? ep.bias[f] : 0.0f;
+        a.out[(size_t)n * a.M + f] = ep.act == PIMDL_ACT_GELU_TANH ? dequant<true>(sum, epl, b) : dequant<false>(sum, epl, b);
+        if (a.acc_out) a.acc_out[(size_t)n * a.M + f] = sum;
+    }
+}
+
+template <FewTable T, int TM, int NW>
+int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
+{
+    constexpr int LDS = few_lds_bytes(NW, TM, T == FEW_ROWS ? FEW_PITCH_ROWS : FEW_PITCH_ONEHOT);
+    auto kern = gather_few_kernel<T, TM, NW>;
+    if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_few)")) return rc;
+    // (the name says which of the large kernels it stands in for)
+    static const char* const names[] = {"gather_sparse_few_kernel", "gather_onehot_few_kernel", "gather_i8_few_kernel"};
+    snprintf(a.last_gather, sizeof(a.last_gather), "%s<%d, %d>", names[T], TM, NW);
+    a.note_launch(0, LDS, 16 * TM, NW * 64);
+    hipLaunchKernelGGL(kern, dim3(f.groups * ((f.N + 16 * TM - 1) / (16 * TM))), dim3(NW * 64), LDS, ctx->stream, f, ep);
+    return hip_check(ctx, hipGetLastError(), "gather_few_kernel launch");
+}
+
+// tokens of an item, by what the launch has: 16, 32 or 64
+constexpr uint32_t few_item(uint32_t n) { return n <= 16 ? 16 : n <= 32 ? 32 : 64; }
+
+// Sixteen waves while every workgroup has a CU to itself, eight (two workgroups share a CU) beyond: us at 3072 -> 768,
+// 16 centroids, sixteen / eight waves: N = 64 7.5 / 8.4 (48 workgroups), N = 512 14.1 / 13.1 (384 workgroups).
+template <FewTable T>
+int launch_few(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
+{
+    const uint32_t item = few_item(f.N);
+    const bool deep = f.groups * ((f.N + item - 1) / item) <= (uint32_t)ctx->prop.multiProcessorCount;
+    if (item == 16) return deep ? launch_few_as<T, 1, 16>(ctx, a, f, ep) : launch_few_as<T, 1, 8>(ctx, a, f, ep);
+    if (item == 32) return deep ? launch_few_as<T, 2, 16>(ctx, a, f, ep) : launch_few_as<T, 2, 8>(ctx, a, f, ep);
+    return deep ? launch_few_as<T, 4, 16>(ctx, a, f, ep) : launch_few_as<T, 4, 8>(ctx, a, f, ep);
+}
+
+// fp32 tables (and int8 ones with a scale per group of codebooks, resident as floats): a lane is one column of one
+// token and adds its entries in ascending codebook order -- the order, and so the bits, of gather_f32_kernel -- with the
+// loads of two times 32 codebooks in flight.  The table is read where it lies: every entry that is added is fetched, and
+// nothing else.
+template <int FB, int IDX_BITS, bool GROUPED>
+__global__ __launch_bounds__(64) void gather_f32_few_kernel(const uint8_t* __restrict__ idx, const float* __restrict__ lut,
+                                                            float* __restrict__ out, uint32_t N, uint32_t M, uint32_t CB_pad,
+                                                            uint32_t idx_row_bytes, const float* __restrict__ bias,
+                                                            const float* __restrict__ scales, uint32_t CB, uint32_t group,
+                                                            uint32_t act, uint32_t colblocks, uint32_t c_tile, uint32_t chunked)
+{
+    constexpr int TOK = 64 / FB, WORDS = IDX_BITS;  // tokens per wave; index words of 32 codebooks
+    const uint32_t colblk = blockIdx.x % colblocks, e = threadIdx.x % FB;
+    const uint32_t tok = blockIdx.x / colblocks * TOK + threadIdx.x / FB, f = colblk * FB + e;
+    const uint32_t* ix = reinterpret_cast<const uint32_t*>(idx + (size_t)(tok < N ? tok : N - 1) * idx_row_bytes);
+    // entry of row r: plain [row][FB], chunked (see gather_f32_kernel) [FB / 2][row][2]
+    const uint32_t row = chunked ? 2 : FB;
+    const float* tab = lut + (size_t)colblk * CB_pad * c_tile * FB + (chunked ? e / 2 * c_tile * 2 + e % 2 : e);
+    const uint32_t per_cb = c_tile * FB, batches = CB_pad / 32;
+
+    uint32_t w[WORDS];
+    float v[2][32];
+    auto load_ix = [&](uint32_t b) {
+#pragma unroll
+        for (int i = 0; i < WORDS; ++i) w[i] = ix[(b < batches ? b : batches - 1) * WORDS + i];
+    };
+    auto fetch = [&](uint32_t b, float (&dst)[32]) {
+        const float* p = tab + (size_t)b * 32 * per_cb;
+#pragma unroll
+        for (int k = 0; k < 32; ++k) {
+            constexpr int PER = 32 / IDX_BITS;
+            dst[k] = p[k * per_cb + (w[k / PER] >> (k % PER * IDX_BITS) & ((1u << IDX_BITS) - 1)) * row];
+        }
+    };
+    float acc = 0.0f, tot = 0.0f;
+    uint32_t cb = 0, in_group = 0, gi = 0;
+    auto add = [&](const float (&src)[32]) {
+#pragma unroll
+        for (int k = 0; k < 32; ++k) {
+            acc = __fadd_rn(acc, src[k]);
+            if constexpr (GROUPED) {
+                // codebooks past CB are padding (zero rows) and belong to no group
+                if (cb < CB && (++in_group == group || cb + 1 == CB)) {
+                    tot = __fadd_rn(tot, __fmul_rn(acc, scales[gi++]));
+                    acc = 0.0f;
+                    in_group = 0;
+                }
+                ++cb;
+            }
+        }
+    };
+    load_ix(0);
+    fetch(0, v[0]);
+    load_ix(1);
+    for (uint32_t b = 0; b < batches; b += 2) {
+        if (b + 1 < batches) fetch(b + 1, v[1]);
+        load_ix(b + 2);
+        add(v[0]);
+        if (b + 1 < batches) {
+            if (b + 2 < batches) fetch(b + 2, v[0]);
+            load_ix(b + 3);
+            add(v[1]);
+        }
+    }
+    if (tok < N && f < M) out[(size_t)tok * M + f] = activate(__fadd_rn(GROUPED ? tot : acc, bias ? bias[f] : 0.0f), act);
+}
+
+template <int FB, int IDX_BITS, bool GROUPED>
+int launch_f32_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, uint32_t n)
+{
+    const AmmGeom& g = a.g;
+    const uint32_t colblocks = g.M_pad / FB, tok = 64 / FB;
+    snprintf(a.last_gather, sizeof(a.last_gather), "gather_f32_few_kernel<%d, %d, %s>", FB, IDX_BITS, GROUPED ? "true" : "false");
+    a.note_launch(0, 0, tok, 64);
+    hipLaunchKernelGGL((gather_f32_few_kernel<FB, IDX_BITS, GROUPED>), dim3(colblocks * ((n + tok - 1) / tok)), dim3(64), 0, ctx->stream,
+                       d_idx, reinterpret_cast<const float*>(a.d_lut), d_out, n, g.M, g.CB_pad, g.idx_row_bytes, a.d_bias,
+                       a.d_scales, g.CB, a.desc.scale_group, a.desc.activation, colblocks, g.C_tile, g.lut_chunked);
+    return hip_check(ctx, hipGetLastError(), "gather_f32_few_kernel launch");
+}
+
+}  // namespace
+
+// Whether these kernels are the shorter launch.  The large kernels' time is flat while their items do not fill the chip
+// (us, large / few): one-hot tables 768 -> 3072 8.1 / 3.0 at N = 1, 8.7 / 4.1 at 64, 9.1 / 9.7 at 300; 3072 -> 768
+// 19.8 / 4.5 at 1, 20.2 / 7.7 at 150, 19.8 / 13.1 at 512, 20.3 / 18.2 at 1024; 8 centroids 3072 -> 768 15.4 / 5.9 at 64,
+// 15.6 / 10.0 at 512: up to two workgroups of this launch per CU.
+// The byte adder and the floats read every gathered piece from the caches on its own, which costs in proportion to
+// tokens x codebooks x columns; against that stands the large kernels' chain of slices.  Byte adder, 3072 -> 768,
+// 32 centroids: 17.6 / 4.4 at N = 1, 17.7 / 7.9 at 13, 17.8 / 27.4 at 64; 1000 -> 1001, 200 centroids: 18.9 / 5.8 at 13,
+// 24.1 / 40.8 at 300.  Floats, 16 centroids, 3072 -> 768: 59.9 / 13.3 at 1, 60.2 / 26.1 at 150, 61 / 43 at 300, 61 / 68
+// at 512; 768 -> 3072: 18.1 / 4.7 at 1, 18.4 / 11.9 at 64, 19.0 / 24.8 at 150.  The two estimates are fits to these.
+bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
+{
+    const AmmGeom& g = a.g;
+    if (g.tune_token_item || g.tune_cb_per_slice || g.tune_xcd_col_split) return false;  // settings of the large kernels
+    const uint64_t cus = ctx->prop.multiProcessorCount, item = few_item(n), wgs = (n + item - 1) / item * (g.M_pad / 16);
+    const double pieces = (double)n * g.CB_pad * (g.M_pad / 16);  // of 16 columns
+    if (a.desc.lut_dtype == PIMDL_LUT_F32 || a.grouped) {
+        const bool bounds = a.grouped && !a.prescaled;  // a scale to apply at the end of every group
+        const double piece = g.lut_chunked || g.q != 4 ? 32e-6 : 4e-6;
+        return 2.7 + g.CB_pad * (bounds ? 0.062 : 0.0137) + pieces * piece < 4.0 + g.CB_pad * (bounds ? 0.14 : 0.07);
+    }
+    if (g.gather_kind == 0)
+        return g.idx_bits == 8 && 2.6 + pieces * (g.C_tile <= 32 ? 0.5e-3 : 1e-3) / (double)(wgs < cus ? wgs : cus) <
+                                      3.3 + (g.CB + 15) / 16 * (0.2 + 0.003 * g.C_tile);
+    if (g.gather_kind == 2 ? g.C_tile == 32 : g.C_tile != 8) return false;  // tables only a tuning asks for
+    return wgs <= 2 * cus;
+}
+
+int launch_gather_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc, uint32_t n, float scale,
+                      float lut_bias_term)
+{
+    const AmmGeom& g = a.g;
+    if (a.desc.lut_dtype == PIMDL_LUT_F32 || a.grouped) {
+        if (a.grouped && !a.prescaled) {
+            if (g.idx_bits == 4) return launch_f32_few<16, 4, true>(ctx, a, d_idx, d_out, n);
+            if (g.q == 4) return launch_f32_few<16, 8, true>(ctx, a, d_idx, d_out, n);
+            return launch_f32_few<8, 8, true>(ctx, a, d_idx, d_out, n);
+        }
+        if (g.idx_bits == 4) return launch_f32_few<16, 4, false>(ctx, a, d_idx, d_out, n);
+        if (g.q == 4) return launch_f32_few<16, 8, false>(ctx, a, d_idx, d_out, n);
+        return launch_f32_few<8, 8, false>(ctx, a, d_idx, d_out, n);
+    }
+    Epilogue ep;
+    ep.scale = scale;
+    ep.lut_bias_term = lut_bias_term;
+    ep.bias = a.d_bias;
+    ep.act = a.desc.activation;
+    ep.op_scales = a.d_op_scales;
+    ep.op_col_tiles = a.op_col_tiles;
+    ep.op_idx_stride = a.op_idx_stride;
+    FewArgs f = {d_idx, reinterpret_cast<const int8_t*>(a.d_lut), d_out, d_acc, n, g.M, g.M_pad / 16, 0, g.q, g.C_tile,
+                 g.idx_row_bytes, a.op_col_tiles * g.q};
+    if (g.gather_kind == 2) {
+        f.steps = g.CB_pad / 8;
+        return launch_few<FEW_SPARSE>(ctx, a, f, ep);
+    }
+    if (g.gather_kind == 1) {
+        f.steps = g.CB_pad / 16;
+        return launch_few<FEW_PAIRED>(ctx, a, f, ep);
+    }
+    f.steps = g.CB_pad / 4;
+    f.tile_groups = 1;
+    return launch_few<FEW_ROWS>(ctx, a, f, ep);
+}
+
+}  // namespace pimdl

@@ -1000,6 +1000,7 @@ int launch_gather(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, in
         ep.op_scales = a.d_op_scales;
         ep.op_col_tiles = a.op_col_tiles;
         ep.op_idx_stride = a.op_idx_stride;
+        if (gather_few_wanted(ctx, a, n)) return launch_gather_few(ctx, a, d_idx, d_out, d_acc, n, ep.scale, ep.lut_bias_term);
         if (g.gather_kind == 2) return launch_gather_sparse(ctx, a, d_idx, d_out, d_acc, n, ep.scale, ep.lut_bias_term);
         if (g.gather_kind == 1) {
             if (g.C_tile == 8) {
@@ -1018,6 +1019,7 @@ int launch_gather(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, in
         }
         return launch_gather_rows(ctx, a, d_idx, d_out, d_acc, n, ep.scale, ep.lut_bias_term);
     } else {
+        if (gather_few_wanted(ctx, a, n)) return launch_gather_few(ctx, a, d_idx, d_out, nullptr, n, 0.0f, 0.0f);
         switch (g.C_tile) {
             case 8: return launch_f32<8, 4, 32, 4>(ctx, a, d_idx, d_out, n);
             case 16: return launch_f32<16, 4, 16, 4>(ctx, a, d_idx, d_out, n);

@@ -183,6 +183,10 @@ int launch_gather_sparse(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_
 // the byte adder (gather_rows_kernel.hip)
 int launch_gather_rows(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc_or_null, uint32_t n,
                        float scale, float lut_bias_term);
+// launches of few tokens (gather_few_kernel.hip)
+bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n);
+int launch_gather_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc_or_null, uint32_t n,
+                      float scale, float lut_bias_term);
 uint32_t rows_lds_bytes(uint32_t c_tile, uint32_t q);
 uint32_t sparse_tile_column(uint32_t tn, uint32_t s);  // column of a tile stored at position s of the tile
 uint32_t sparse_lds_bytes(uint32_t tn, bool wide);

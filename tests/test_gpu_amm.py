@@ -597,3 +597,59 @@ def test_byte_adder_item_sizes(ctx):
         amm.run_debug(x[:n])  # the whole batch in one launch (run cuts host buffers into chunks)
         assert amm.last_gather_kernel().split(", ")[3] == str(groups), amm.last_gather_kernel()
     amm.close()
+
+
+FEW_SHAPES = [
+    # N, CB, v, C, M, lut, scale_group: launches of few tokens, whose codebooks are dealt out to waves
+    (1, 192, 4, 16, 3072, "i8", 0),     # one token
+    (16, 40, 2, 9, 100, "i8", 0),       # the last of 16-token items; padded codebooks; a ragged column tile
+    (17, 33, 4, 16, 49, "i8", 0),       # 32-token items; ragged columns of a second tile
+    (33, 768, 4, 16, 768, "i8", 0),     # 64-token items, more K-steps per wave than are in flight together
+    (300, 96, 4, 12, 1001, "i8", 0),    # eight waves: more items than CUs
+    (5, 70, 4, 8, 100, "i8", 0),        # paired codebooks
+    (300, 192, 4, 5, 768, "i8", 0),
+    (1, 256, 4, 64, 1001, "i8", 0),     # byte adder
+    (13, 768, 2, 17, 768, "i8", 0),
+    (3, 50, 8, 256, 70, "i8", 0),
+    (1, 192, 4, 16, 770, "f32", 0),     # floats: rows of 16, in 8-byte pieces (32 centroids), rows of 8
+    (67, 768, 4, 8, 96, "f32", 0),
+    (5, 96, 4, 32, 50, "f32", 0),
+    (9, 64, 4, 130, 33, "f32", 0),
+    (7, 192, 4, 16, 100, "i8", 1),      # a scale per codebook, and per 5 with a ragged last group
+    (3, 193, 4, 16, 100, "i8", 5),
+    (3, 64, 4, 20, 40, "i8", 7),
+]
+
+
+@pytest.mark.parametrize("N,CB,v,C,M,lut,group", FEW_SHAPES)
+def test_launches_of_few_tokens(ctx, N, CB, v, C, M, lut, group):
+    """Bit for bit the oracle's indices and output, with the guard rows behind the output untouched, and the kernel
+    that takes them is the one for few tokens."""
+    x, cent, table, bias = make_case(6100 + N + C, N, CB * v, v, C, M, lut)
+    scales = None if lut == "f32" else np.float32(0.0123)
+    if group:
+        scales = np.random.default_rng(N).uniform(0.001, 0.02, (CB + group - 1) // group).astype(np.float32)
+    amm = ctx.amm(cent, table, scales, bias, max_n=N, scale_group=group)
+    out, idx, acc = amm.run_debug(x, want_acc=lut == "i8" and not group)
+    want_idx = oracle.index_calculation(x, cent, v, threads=THREADS)
+    assert np.array_equal(idx, want_idx)
+    if lut == "f32":
+        want = oracle.gather_f32(want_idx, table, bias, threads=THREADS)
+    elif group:
+        want = oracle.gather_i8_grouped(want_idx, table, scales, bias, group, threads=THREADS)
+    else:
+        want_acc = oracle.gather_i8(want_idx, table, threads=THREADS)
+        assert np.array_equal(acc, want_acc)
+        want = oracle.dequant(want_acc, bias, CB, 0.0123, 0.0, 0, threads=THREADS)
+    assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
+    if not kernel_switches():
+        assert "_few_" in amm.last_gather_kernel(), amm.last_gather_kernel()
+    import torch
+    guarded = torch.full((N + 3, M), -5.0, device="cuda")
+    xd = torch.from_numpy(x).cuda()
+    torch.cuda.synchronize()
+    amm.run_ptr(xd.data_ptr(), N, guarded.data_ptr())
+    ctx.synchronize()
+    got = guarded.cpu().numpy()
+    assert np.array_equal(got[:N].view(np.uint32), want.view(np.uint32)) and (got[N:] == -5.0).all()
+    amm.close()
