@@ -1138,6 +1138,81 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
 
 // Generic sub-vector length (any v): one lane per (token, codebook), operands straight from
 // global memory.  Correct for every shape; only used where no specialisation exists.
+// Few tokens, more than 32 centroids: a wave takes one codebook and goes through its tokens, lane l holds centroids
+// l, l + 64, ... in registers and computes their distances in the reference's own order of operations.  The wave's
+// smallest distance is the scan's result if every other one is larger by more than the hysteresis -- the scan takes it when
+// it comes to it, whatever it holds, and nothing after it -- which one ballot tells; else (near ties, NaN, infinities)
+// the scan reads the distances lane by lane.
+// A lane per token (ccs_kernel) leaves all but N lanes of a wave idle and goes through the centroids one after the
+// other: 20.9 us at one token, 256 codebooks, 64 centroids, where this takes 4.7.  Bound by the launch and one round trip
+// at a few tokens, by the vector ALU (3 v R operations and a reduction over the wave per pair) from about 50 on.
+template <int V, int R>  // R: centroids per lane
+__global__ __launch_bounds__(CCS_THREADS) void ccs_few_kernel(const float* __restrict__ x, const float* __restrict__ cent,
+                                                              uint8_t* __restrict__ idx, uint32_t N, uint32_t K, uint32_t CB,
+                                                              uint32_t CB_pad, uint32_t C, uint32_t idx_row_bytes, int idx_tiled,
+                                                              uint32_t tokens_per_wave)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(blockIdx.x * (CCS_THREADS / 64) + (threadIdx.x >> 6));
+    const uint32_t cb = w % CB_pad, tok0 = w / CB_pad * tokens_per_wave;
+    const uint32_t tok1 = tok0 + tokens_per_wave < N ? tok0 + tokens_per_wave : N;
+    if (cb >= CB) {  // padding: index 0
+        for (uint32_t tok = tok0 + lane; tok < tok1; tok += 64) idx[idx_offset(tok, cb, idx_row_bytes, idx_tiled)] = 0;
+        return;
+    }
+    float c[R][V];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint32_t k = lane + 64 * r;
+        const float* cp = cent + ((size_t)cb * C + (k < C ? k : 0)) * V;
+#pragma unroll
+        for (int t = 0; t < V; ++t) c[r][t] = cp[t];
+    }
+    for (uint32_t tok = tok0; tok < tok1; ++tok) {
+        const float* xs = x + (size_t)tok * K + (size_t)cb * V;
+        float d[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) d[r] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < V; ++t) {
+            const float xt = xs[t];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const float diff = __fsub_rn(xt, c[r][t]);
+                d[r] = __fadd_rn(d[r], __fmul_rn(diff, diff));
+            }
+        }
+        float m = __builtin_inff();
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (lane + 64 * r >= C) d[r] = __builtin_inff();
+            m = fminf(m, d[r]);
+        }
+#pragma unroll
+        for (int s = 1; s < 64; s *= 2) m = fminf(m, __shfl_xor(m, s));
+        uint32_t found = 0, near = 0;  // near: centroids that the scan may prefer to one another (the nearest among them)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint64_t b = __ballot(!(__fsub_rn(d[r], m) > 1e-6f));
+            near += __builtin_popcountll(b);
+            if (b) found = 64 * r + __builtin_ctzll(b);
+        }
+        if (near != 1) {
+            float best = 0.0f;
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                for (uint32_t k = 0; k < 64 && 64 * r + k < C; ++k) {
+                    const float dk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(d[r]), k));
+                    if ((r == 0 && k == 0) || __fsub_rn(best, dk) > 1e-6f) {
+                        best = dk;
+                        found = 64 * r + k;
+                    }
+                }
+        }
+        if (lane == 0) idx[idx_offset(tok, cb, idx_row_bytes, idx_tiled)] = (uint8_t)found;
+    }
+}
+
 template <int IDX_BITS>
 __global__ __launch_bounds__(256) void ccs_generic_kernel(const float* __restrict__ x,
                                                          const float* __restrict__ cent,
@@ -1341,6 +1416,20 @@ int launch_ccs_bf16(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     return launch_ccs_bf16_tt<V, WIDE, 128>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
 }
 
+template <int V>
+int launch_ccs_few(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent, uint8_t* d_idx, uint32_t n)
+{
+    constexpr uint32_t WAVES = CCS_THREADS / 64;
+    // up to eight waves per SIMD, then more tokens per wave (the centroids are loaded once for them)
+    const uint64_t waves = 32ull * ctx->prop.multiProcessorCount, pairs = (uint64_t)n * g.CB_pad;
+    const uint32_t per = (uint32_t)((pairs + waves - 1) / waves), chunks = (n + per - 1) / per;
+    auto kern = g.C <= 64 ? ccs_few_kernel<V, 1> : g.C <= 128 ? ccs_few_kernel<V, 2> : ccs_few_kernel<V, 4>;
+    // (CB_pad is a multiple of the waves of a workgroup)
+    hipLaunchKernelGGL(kern, dim3(chunks * (g.CB_pad / WAVES)), dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent, d_idx, n, g.K, g.CB,
+                       g.CB_pad, g.C, g.idx_row_bytes, (int)g.idx_tiled, per);
+    return hip_check(ctx, hipGetLastError(), "ccs_few_kernel launch");
+}
+
 template <int IDX_BITS>
 int launch_ccs_bits(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent, uint8_t* d_idx, uint32_t n,
                     uint32_t x_cols)
@@ -1372,6 +1461,20 @@ int launch_ccs_bits(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
             case 2: return launch_ccs_mfma<2>(ctx, g, d_x, d_cent, d_idx, n);
             case 4: return launch_ccs_mfma<4>(ctx, g, d_x, d_cent, d_idx, n);
             case 8: return launch_ccs_mfma<8>(ctx, g, d_x, d_cent, d_idx, n);
+            default: break;
+        }
+    }
+    // Few (token, codebook) pairs: a wave per pair.  The lane-per-token kernel takes about 0.3 us per centroid however few
+    // the tokens are, the wave-per-pair one about 4 us + 6 ps per pair and centroid (us, v = 4: 64 centroids, 256
+    // codebooks N = 64 21.3 / 9.2, N = 128 24.5 / 16.4, N = 256 24.4 / 30.4; 128 centroids N = 128 38.7 / 27.9,
+    // N = 256 39.1 / 53.1; 200 centroids N = 128 60 / 42, N = 256 70 / 81).
+    if (IDX_BITS == 8 && g.C > 32 && !g.tune_search && !exact && (double)n * g.CB * 6e-6 + 4.0 / g.C < 0.25) {
+        switch (g.v) {
+            case 2: return launch_ccs_few<2>(ctx, g, d_x, d_cent, d_idx, n);
+            case 4: return launch_ccs_few<4>(ctx, g, d_x, d_cent, d_idx, n);
+            case 8: return launch_ccs_few<8>(ctx, g, d_x, d_cent, d_idx, n);
+            case 16: return launch_ccs_few<16>(ctx, g, d_x, d_cent, d_idx, n);
+            case 32: return launch_ccs_few<32>(ctx, g, d_x, d_cent, d_idx, n);
             default: break;
         }
     }

@@ -653,3 +653,26 @@ def test_launches_of_few_tokens(ctx, N, CB, v, C, M, lut, group):
     got = guarded.cpu().numpy()
     assert np.array_equal(got[:N].view(np.uint32), want.view(np.uint32)) and (got[N:] == -5.0).all()
     amm.close()
+
+
+@pytest.mark.parametrize("N,v,C", [(1, 4, 64), (5, 2, 33), (40, 8, 65), (3, 16, 128), (2, 32, 200), (70, 4, 256)])
+def test_search_of_few_tokens_with_many_centroids(ctx, N, v, C):
+    """A wave per (token, codebook) pair: near ties within the hysteresis in either order, repeated and zero centroids,
+    NaN and infinities, codebooks that are no multiple of a workgroup's."""
+    CB, M = 37, 20
+    x, cent, lut, bias = make_case(7100 + N + C, N, CB * v, v, C, M)
+    cent[1, :] = 0.0
+    cent[2, C - 1] = cent[2, 0]
+    cent[3] = cent[3, 7] + np.linspace(2e-7, 0, C, dtype=np.float32)[:, None]   # a chain of steps below the hysteresis
+    cent[4] = cent[4, 7] + np.linspace(3e-4, 0, C, dtype=np.float32)[:, None]   # ... and around it
+    cent[5, C // 2] = np.nan
+    cent[6, 0] = np.inf
+    x[:, 3 * v:5 * v] = np.tile(np.concatenate([cent[3, 7], cent[4, 7]]), (N, 1))
+    x[0, 7 * v] = np.nan
+    x[0, 8 * v] = np.inf
+    x[0, 9 * v] = 1e30
+    amm = ctx.amm(cent, lut, np.float32(0.01), bias, max_n=N)
+    _, idx, _ = amm.run_debug(x)
+    want = oracle.index_calculation(x, cent, v, threads=THREADS)
+    assert np.array_equal(idx, want), np.argwhere(idx != want)[:8]
+    amm.close()
