@@ -95,6 +95,19 @@ inline size_t ccs_bf16_floats(const AmmGeom& g)
     return ccs_has_bf16(g) ? ccs_bf16_units(g) * ccs_bf16_nm(g.v) * 64 * 4 + ccs_bf16_units(g) * 2 * 16 : 0;
 }
 
+// more than 32 centroids, or sub-vectors of 16 or 32 dimensions: the matrix search over groups of 32 centroids
+// (ccs_many_kernel).  Its operands stand where the bf16 ones of the shapes above would.
+inline bool ccs_has_many(const AmmGeom& g)
+{
+    return g.v == 16 || g.v == 32 || (g.C > 32 && (g.v == 2 || g.v == 4 || g.v == 8));
+}
+inline size_t ccs_many_groups(const AmmGeom& g) { return (size_t)g.CB * ((g.C + 31) / 32); }
+constexpr uint32_t ccs_many_nm(uint32_t v) { return v == 2 ? 1 : v == 4 ? 2 : 3 * (v / 8); }  // matrix instructions per group
+inline size_t ccs_many_floats(const AmmGeom& g)
+{
+    return ccs_has_many(g) ? ccs_many_groups(g) * (ccs_many_nm(g.v) * 64 * 4 + 32) : 0;
+}
+
 template <int N, typename F>
 __device__ __forceinline__ void static_for(F&& f)
 {
@@ -1136,15 +1149,400 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
     }
 }
 
-// Generic sub-vector length (any v): one lane per (token, codebook), operands straight from
-// global memory.  Correct for every shape; only used where no specialisation exists.
+// =============================================================================================
+// The matrix search for more than 32 centroids (v = 2, 4, 8) and for v = 16 and 32: one wave takes one codebook at a time
+// for 32 * TG tokens and goes through its centroids 32 by 32.  Scores, tags, tournament, margin test and exact replay are
+// those of the bf16 search above; a group's winner meets the smallest and second smallest so far.
+// Operands of a group: lane (row i, half kh) supplies dims DL kh .. DL kh + DL - 1 (DL = v / 2) of centroid 32 grp + 16 h + r
+// (row i = (r & 3) + 8 (r >> 2) + 4 h, so that result register r of lane (token, h) is that centroid's score).  A register
+// holds a piece of dims d and d + 1; per two such pairs three instructions:
+//   [H0 M0 H1 M1] x [CH CH CH CH], the same x [CM CM CM CM], [H0 L0 H1 L1] x [CL CH CL CH]      (v >= 8)
+//   [H M H M] x [CH CH CM CM], [H L H L] x [CL CH 0 0]                                         (v = 4)
+//   [(xh|xh) (xm|xm) (xh|xl) 0] x [(ch|cm) (ch|cm) (cl|ch) 0]                                   (v = 2)
+// The activations' pieces are made once per token and codebook, whatever the number of centroids.
+// Bound by the vector ALU: 16 tags, 20 operations of the tournament and 5 of the merge per 32 x 32 scores.
+// A lane per token and a scalar operand per centroid (ccs_kernel) spent v + 4 operations at half rate per score and
+// replayed 64 tokens for each near tie (us at N = 8192, before / now: v = 4, 64 centroids, K = 768 43 / 21, K = 3072 141 / 70; 128
+// centroids, K = 1024 97 / 42; 256 204 / 76; v = 16, K = 1024, 64 centroids 54 / 13; v = 32, K = 1280, 64 centroids 118 / 22,
+// K = 2048, 128 centroids 244 / 37, K = 1024, 16 centroids 24 / 9.3; N = 128: 21 / 8, 39 / 12, 22 / 7, 102 / 8).
+//   aux  [CB][groups][NM][64 lanes] uint4, then cn [CB][groups][2 h][16] |c|^2 (3e38 past the last centroid)
+// =============================================================================================
+template <uint32_t V>
+__global__ void ccs_prep_many_kernel(const float* __restrict__ cent, uint4* __restrict__ aux, float* __restrict__ cn32, uint32_t C)
+{
+    constexpr uint32_t DL = V / 2, NM = ccs_many_nm(V);
+    const uint32_t cb = blockIdx.x, grp = blockIdx.y, groups = gridDim.y, lane = threadIdx.x;
+    const uint32_t i = lane & 31, kh = lane >> 5, h = (i >> 2) & 1, r = (i & 3) + 4 * (i >> 3);
+    const uint32_t cid = 32 * grp + 16 * h + r;
+    const bool real = cid < C;
+    const float* cp = cent + ((size_t)cb * C + (real ? cid : 0)) * V;
+    uint32_t pc[DL][3];  // bf16 pieces of -2c
+#pragma unroll
+    for (uint32_t d = 0; d < DL; ++d) {
+        const float a = real ? -2.0f * cp[DL * kh + d] : 0.0f;
+        const uint32_t au = __float_as_uint(a);
+        const float r1 = __fsub_rn(a, __uint_as_float(au & 0xffff0000u));
+        const uint32_t r1u = __float_as_uint(r1);
+        const float r2 = __fsub_rn(r1, __uint_as_float(r1u & 0xffff0000u));
+        pc[d][0] = au >> 16;
+        pc[d][1] = r1u >> 16;
+        pc[d][2] = __float_as_uint(r2) >> 16;
+    }
+    uint4* dst = aux + ((size_t)cb * groups + grp) * NM * 64 + lane;
+    if constexpr (DL == 1) {
+        const uint32_t hm = pc[0][0] | pc[0][1] << 16, lh = pc[0][2] | pc[0][0] << 16;
+        dst[0] = make_uint4(hm, hm, lh, 0);
+    } else {
+        auto pair = [&](uint32_t d, uint32_t t) { return pc[d][t] | pc[d + 1][t] << 16; };
+        if constexpr (DL == 2) {
+            dst[0] = make_uint4(pair(0, 0), pair(0, 0), pair(0, 1), pair(0, 1));
+            dst[64] = make_uint4(pair(0, 2), pair(0, 0), 0, 0);
+        } else {
+#pragma unroll
+            for (uint32_t q = 0; q < DL / 4; ++q) {
+                const uint32_t a = 4 * q, b = 4 * q + 2;
+                dst[(3 * q + 0) * 64] = make_uint4(pair(a, 0), pair(a, 0), pair(b, 0), pair(b, 0));
+                dst[(3 * q + 1) * 64] = make_uint4(pair(a, 1), pair(a, 1), pair(b, 1), pair(b, 1));
+                dst[(3 * q + 2) * 64] = make_uint4(pair(a, 2), pair(a, 0), pair(b, 2), pair(b, 0));
+            }
+        }
+    }
+    if (kh == 0) {
+        float cn = 3e38f;
+        if (real) {
+            cn = 0.0f;
+#pragma unroll
+            for (uint32_t t = 0; t < V; ++t) cn = fmaf(cp[t], cp[t], cn);
+        }
+        cn32[((size_t)cb * groups + grp) * 32 + 16 * h + r] = cn;
+    }
+}
+
+// The reference's result for one sub-vector, by the whole wave: lane l computes the distances to centroids l, l + 64, ... in
+// the reference's own order of operations.  The smallest one is the scan's result if every other is larger by more than
+// the hysteresis (the scan takes it when it comes to it, whatever it holds, and nothing after it), which one ballot tells;
+// else (near ties, NaN, infinities) the scan reads the distances lane by lane.
+// c(r, t): dimension t of centroid lane + 64 r (of any centroid past the last)
+template <int V, int R, class X, class Cent>
+__device__ __forceinline__ uint32_t wave_scan(const X& xs, uint32_t C, uint32_t lane, const Cent& c)
+{
+    float d[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) d[r] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < V; ++t) {
+        const float xt = xs[t];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float diff = __fsub_rn(xt, c(r, t));
+            d[r] = __fadd_rn(d[r], __fmul_rn(diff, diff));
+        }
+    }
+    float m = __builtin_inff();
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (lane + 64 * r >= C) d[r] = __builtin_inff();
+        m = fminf(m, d[r]);
+    }
+#pragma unroll
+    for (int s = 1; s < 64; s *= 2) m = fminf(m, __shfl_xor(m, s));
+    uint32_t found = 0, near = 0;  // near: centroids that the scan may prefer to one another (the nearest among them)
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint64_t b = __ballot(!(__fsub_rn(d[r], m) > 1e-6f));
+        near += __builtin_popcountll(b);
+        if (b) found = 64 * r + __builtin_ctzll(b);
+    }
+    if (near != 1) {
+        float best = 0.0f;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            for (uint32_t k = 0; k < 64 && 64 * r + k < C; ++k) {
+                const float dk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(d[r]), k));
+                if ((r == 0 && k == 0) || __fsub_rn(best, dk) > 1e-6f) {
+                    best = dk;
+                    found = 64 * r + k;
+                }
+            }
+    }
+    return found;
+}
+
+template <int V>
+struct CcsManyShape {
+    // 32-token groups per tile: one for each half of the wave to replay.  (Four halve the operand loads and were within 9 % of
+    // two at N = 8192, and half as fast again at small batches.)
+    static constexpr int TG = 2, TT = 32 * TG;               // ... tokens
+    static constexpr int P = V >= 16 ? 1 : 16 / V;           // codebooks per wave
+    static constexpr int CBW = 4 * P;                        // codebooks per workgroup (CB_pad is a multiple of it)
+    static constexpr int TF = CBW * V, PITCH = TF + 4;       // floats of a token in the tile, in LDS
+};
+
+template <int V, int IDX_BITS>
+__global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* __restrict__ x, const float* __restrict__ cent,
+                                                                  const uint4* __restrict__ aux, const float* __restrict__ cn32,
+                                                                  const float* __restrict__ cnmax, uint8_t* __restrict__ idx,
+                                                                  uint32_t N, uint32_t K, uint32_t CB, uint32_t C,
+                                                                  uint32_t idx_row_bytes, int idx_tiled, int vec_ok, uint32_t tiles_cb)
+{
+    using S = CcsManyShape<V>;
+    constexpr int TG = S::TG, TT = S::TT, P = S::P, CBW = S::CBW, TF = S::TF, PITCH = S::PITCH;
+    constexpr int DL = V / 2, NM = (int)ccs_many_nm(V);
+    constexpr int NB = V == 2 ? 1 : V <= 8 ? 2 : V / 4;  // activation operands of a token group
+    __shared__ __attribute__((aligned(16))) float tile[TT * PITCH];
+    __shared__ __attribute__((aligned(16))) uint8_t ist[TT * CBW];
+    const uint32_t lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t tcb = blockIdx.x % tiles_cb, tok0 = blockIdx.x / tiles_cb * TT;
+    const uint32_t groups = (C + 31) / 32;
+
+    {
+        constexpr int F4 = TF / 4, ROWS = CCS_THREADS / F4, PASSES = TT / ROWS;
+        static_assert(CCS_THREADS % F4 == 0 && TT % ROWS == 0, "tile shape");
+        const uint32_t fq = threadIdx.x % F4, fr = threadIdx.x / F4, col0 = tcb * TF, col = col0 + 4 * fq;
+        float4 pf[PASSES];
+        if (vec_ok && col0 + TF <= K) {  // workgroup-uniform: the whole tile inside the row, 16-byte aligned
+#pragma unroll
+            for (int i = 0; i < PASSES; ++i) {
+                uint32_t tok = tok0 + fr + i * ROWS;
+                tok = tok < N ? tok : N - 1;  // rows past N repeat the last token; never stored
+                pf[i] = *reinterpret_cast<const float4*>(x + (size_t)tok * K + col);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < PASSES; ++i) {
+                uint32_t tok = tok0 + fr + i * ROWS;
+                tok = tok < N ? tok : N - 1;
+                const float* src = x + (size_t)tok * K + col;
+                pf[i].x = (col + 0 < K) ? src[0] : 0.0f;
+                pf[i].y = (col + 1 < K) ? src[1] : 0.0f;
+                pf[i].z = (col + 2 < K) ? src[2] : 0.0f;
+                pf[i].w = (col + 3 < K) ? src[3] : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < PASSES; ++i) *reinterpret_cast<float4*>(&tile[(fr + i * ROWS) * PITCH + 4 * fq]) = pf[i];
+    }
+    __syncthreads();
+
+#pragma nounroll
+    for (int p = 0; p < P; ++p) {
+        const uint32_t cbl = wave * P + p, cb = tcb * CBW + cbl;
+        if (cb >= CB) {  // padding: index 0
+#pragma unroll
+            for (int tg = 0; tg < TG; ++tg) ist[(32 * tg + j) * CBW + cbl] = 0;
+            continue;
+        }
+        // pieces of the lane's activations, x = xh + xm + xl exactly, and |x|^2
+        v4u bop[TG][NB];
+        float mag[TG];
+        const float cmax = cnmax[cb];
+#pragma unroll
+        for (int tg = 0; tg < TG; ++tg) {
+            const float* src = tile + (32 * tg + j) * PITCH + cbl * V + DL * h;
+            float xs[DL];
+            if constexpr (DL == 1) xs[0] = src[0];
+            else if constexpr (DL == 2) {
+                const float2 t2 = *reinterpret_cast<const float2*>(src);
+                xs[0] = t2.x;
+                xs[1] = t2.y;
+            } else {
+#pragma unroll
+                for (int q = 0; q < DL / 4; ++q) {
+                    const float4 t4 = *reinterpret_cast<const float4*>(src + 4 * q);
+                    xs[4 * q] = t4.x;
+                    xs[4 * q + 1] = t4.y;
+                    xs[4 * q + 2] = t4.z;
+                    xs[4 * q + 3] = t4.w;
+                }
+            }
+            uint32_t u0[DL], u1[DL], u2[DL];
+            float sq = 0.0f;
+#pragma unroll
+            for (int d = 0; d < DL; ++d) {
+                u0[d] = __float_as_uint(xs[d]);
+                const float r1 = xs[d] - __uint_as_float(u0[d] & 0xffff0000u);
+                u1[d] = __float_as_uint(r1);
+                u2[d] = __float_as_uint(r1 - __uint_as_float(u1[d] & 0xffff0000u));
+                sq = d == 0 ? xs[d] * xs[d] : fmaf(xs[d], xs[d], sq);
+            }
+            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(sq), __float_as_uint(sq), false, false);
+            mag[tg] = __uint_as_float(sw[0]) + __uint_as_float(sw[1]) + cmax;
+            // __builtin_amdgcn_perm(p, q, 0x07060302) = (bf16 of q | bf16 of p << 16)
+            auto both = [](uint32_t q, uint32_t p) { return __builtin_amdgcn_perm(p, q, 0x07060302u); };
+            if constexpr (DL == 1) {
+                bop[tg][0] = v4u{both(u0[0], u0[0]), both(u1[0], u1[0]), both(u0[0], u2[0]), 0};
+            } else if constexpr (DL == 2) {
+                const uint32_t H = both(u0[0], u0[1]), M = both(u1[0], u1[1]), L = both(u2[0], u2[1]);
+                bop[tg][0] = v4u{H, M, H, M};
+                bop[tg][1] = v4u{H, L, H, L};
+            } else {
+#pragma unroll
+                for (int q = 0; q < DL / 4; ++q) {
+                    const int a = 4 * q, b = 4 * q + 2;
+                    const uint32_t H0 = both(u0[a], u0[a + 1]), H1 = both(u0[b], u0[b + 1]);
+                    bop[tg][2 * q] = v4u{H0, both(u1[a], u1[a + 1]), H1, both(u1[b], u1[b + 1])};
+                    bop[tg][2 * q + 1] = v4u{H0, both(u2[a], u2[a + 1]), H1, both(u2[b], u2[b + 1])};
+                }
+            }
+        }
+        // smallest and second smallest tagged score of the lane's half of every group so far, the group of the smallest
+        float m1[TG], m2[TG];
+        uint32_t grp[TG];
+#pragma unroll
+        for (int tg = 0; tg < TG; ++tg) {
+            m1[tg] = m2[tg] = 3.2e38f;
+            grp[tg] = 0;
+        }
+        const uint4* ap = aux + (size_t)cb * groups * NM * 64 + lane;
+        const float* cnp = cn32 + (size_t)cb * groups * 32 + 16 * h;
+        uint4 aq[NM], an[NM];
+        float4 cn[4], cnn[4];
+        auto load = [&](uint32_t g) {
+#pragma unroll
+            for (int m = 0; m < NM; ++m) an[m] = ap[((size_t)g * NM + m) * 64];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) cnn[q] = *reinterpret_cast<const float4*>(cnp + g * 32 + 4 * q);
+        };
+        load(0);
+#pragma nounroll
+        for (uint32_t g = 0; g < groups; ++g) {
+#pragma unroll
+            for (int m = 0; m < NM; ++m) aq[m] = an[m];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) cn[q] = cnn[q];
+            load(g + 1 < groups ? g + 1 : g);
+            floatx16 start;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                start[4 * q] = cn[q].x;
+                start[4 * q + 1] = cn[q].y;
+                start[4 * q + 2] = cn[q].z;
+                start[4 * q + 3] = cn[q].w;
+            }
+#pragma unroll
+            for (int tg = 0; tg < TG; ++tg) {
+                floatx16 acc = start;
+#pragma unroll
+                for (int m = 0; m < NM; ++m) {
+                    const int b = V <= 4 ? m : 2 * (m / 3) + (m % 3 == 2);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, aq[m]), __builtin_bit_cast(bf16x8, bop[tg][b]), acc, 0, 0, 0);
+                }
+                float key[16];
+#pragma unroll
+                for (int r = 0; r < 16; ++r) key[r] = __uint_as_float((__float_as_uint(acc[r]) & ~15u) | (uint32_t)r);
+                float lo[5], md[5];
+#pragma unroll
+                for (int i = 0; i < 5; ++i) {
+                    lo[i] = vmin3(key[3 * i], key[3 * i + 1], key[3 * i + 2]);
+                    md[i] = __builtin_amdgcn_fmed3f(key[3 * i], key[3 * i + 1], key[3 * i + 2]);
+                }
+                const float a1 = vmin3(lo[0], lo[1], lo[2]), a2 = __builtin_amdgcn_fmed3f(lo[0], lo[1], lo[2]);
+                const float b1 = vmin3(lo[3], lo[4], key[15]), b2 = __builtin_amdgcn_fmed3f(lo[3], lo[4], key[15]);
+                const float g1 = vmin(a1, b1);
+                const float g2 = vmin3(vmin3(md[0], md[1], md[2]), vmin3(md[3], md[4], vmax(a1, b1)), vmin(a2, b2));
+                grp[tg] = g1 < m1[tg] ? g : grp[tg];
+                m2[tg] = vmin3(vmax(m1[tg], g1), m2[tg], g2);
+                m1[tg] = vmin(m1[tg], g1);
+            }
+        }
+        uint32_t fail = 0, found = 0;  // found: one byte per token group
+#pragma unroll
+        for (int tg = 0; tg < TG; ++tg) {
+            // lanes l and l ^ 32 hold the two halves of every group: both merge them.  Equal tagged minima give
+            // second == smallest, which fails the margin test.
+            const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m1[tg]), __float_as_uint(m1[tg]), false, false);
+            const auto s2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m2[tg]), __float_as_uint(m2[tg]), false, false);
+            const auto sg = __builtin_amdgcn_permlane32_swap(grp[tg], grp[tg], false, false);
+            const float lo1 = __uint_as_float(s1[0]), hi1 = __uint_as_float(s1[1]);
+            const float best = vmin(lo1, hi1), second = vmin3(vmax(lo1, hi1), __uint_as_float(s2[0]), __uint_as_float(s2[1]));
+            const bool up = hi1 < lo1;
+            found |= ((__float_as_uint(best) & 15u) + (up ? 16u : 0u) + 32u * (up ? sg[1] : sg[0])) << (8 * tg);
+            // 2 * [ (v+1)u (|c|^2) + 16u (omitted products) + 2.02 (6v + NM + 1) u (that many additions, each within u of a
+            //       partial sum below 2.02 mag) + 2(v+2)u (the reference's own chain) ], and the tags
+            constexpr float A2 = 2.0f * ((V + 1) + 16.0f + 2.02f * (6 * V + NM + 1) + 2 * (V + 2)) * 5.9604645e-8f;
+            constexpr float B2 = 2.0f * 16.0f * 2.3841858e-7f;  // 2 * 2^(4-22)
+            const float thr = fmaf(A2, mag[tg], fmaf(B2, fabsf(second), 1.001e-6f));
+            // NaN anywhere makes a compare false, which counts as "not safe"
+            const bool safe = ((second - best) > thr) && (mag[tg] < 1e36f);
+            fail |= (safe ? 0u : 1u) << tg;
+        }
+        // ---- exact replay of the tokens that failed the margin test (rare) ----
+        if (__builtin_amdgcn_ballot_w64(fail != 0) != 0) {
+            const float* cp = cent + (size_t)cb * C * V;
+#pragma unroll
+            for (int q = 0; q < TG / 2; ++q) {  // token groups 2 q and 2 q + 1: a half of the wave each
+                auto set = [&](uint32_t k) { found = (found & ~(255u << (8 * (2 * q + h)))) | k << (8 * (2 * q + h)); };
+                const bool mine = (fail >> (2 * q + h)) & 1u;
+                uint64_t mask = __builtin_amdgcn_ballot_w64(mine);
+                if (mask == 0) continue;
+                const uint32_t row = 64 * q + lane;  // the lane's token in the tile
+                if (__builtin_popcountll(mask) <= 8) {  // one token at a time, by the whole wave
+                    while (mask) {
+                        const uint32_t l = (uint32_t)__builtin_ctzll(mask);
+                        mask &= mask - 1;
+                        const float* xo = tile + (64 * q + l) * PITCH + cbl * V;
+                        auto c1 = [&](int r, int t) {
+                            const uint32_t k = lane + 64 * r;
+                            return cp[(size_t)(k < C ? k : 0) * V + t];
+                        };
+                        const uint32_t b = C <= 64 ? wave_scan<V, 1>(xo, C, lane, c1) : C <= 128 ? wave_scan<V, 2>(xo, C, lane, c1) : wave_scan<V, 4>(xo, C, lane, c1);
+                        if (lane == l) set(b);
+                    }
+                } else if (mine) {  // ties everywhere (repeated centroids): every lane scans for its token
+                    const float* xo = tile + row * PITCH + cbl * V;
+                    float xr[V];
+#pragma unroll
+                    for (int t = 0; t < V; ++t) xr[t] = xo[t];
+                    float best = 0.0f;
+                    uint32_t k = 0;
+                    // several centroids per trip: their (uniform) rows are fetched together
+                    constexpr uint32_t UN = V >= 32 ? 2 : V == 16 ? 4 : 8;
+#pragma nounroll
+                    for (uint32_t c0 = 0; c0 < C; c0 += UN) {
+                        float row[UN][V];
+#pragma unroll
+                        for (uint32_t u = 0; u < UN; ++u)
+#pragma unroll
+                            for (int t = 0; t < V; ++t) row[u][t] = cp[(size_t)(c0 + u < C ? c0 + u : C - 1) * V + t];
+#pragma unroll
+                        for (uint32_t u = 0; u < UN; ++u) {
+                            float d = 0.0f;
+#pragma unroll
+                            for (int t = 0; t < V; ++t) {
+                                const float diff = __fsub_rn(xr[t], row[u][t]);
+                                d = __fadd_rn(d, __fmul_rn(diff, diff));
+                            }
+                            const bool take = c0 + u < C && ((c0 + u == 0) || (__fsub_rn(best, d) > 1e-6f));
+                            best = take ? d : best;
+                            k = take ? c0 + u : k;
+                        }
+                    }
+                    set(k);
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < TG / 2; ++q) ist[(64 * q + lane) * CBW + cbl] = (uint8_t)(found >> (8 * (2 * q + h)));
+    }
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < (uint32_t)(TT * P); e += CCS_THREADS) {  // four codebooks of a token
+        const uint32_t t = e % TT, w = e / TT, tok = tok0 + t;
+        if (tok >= N) continue;
+        const uint32_t b = *reinterpret_cast<const uint32_t*>(&ist[t * CBW + 4 * w]);
+        const uint32_t cb0 = tcb * CBW + 4 * w;
+        if constexpr (IDX_BITS == 8)
+            *reinterpret_cast<uint32_t*>(idx + idx_offset(tok, cb0, idx_row_bytes, idx_tiled)) = b;
+        else
+            *reinterpret_cast<uint16_t*>(idx + idx_offset(tok, cb0 / 2, idx_row_bytes, idx_tiled)) =
+                (uint16_t)((b & 15u) | (b >> 4 & 0xF0u) | (b >> 8 & 0xF00u) | (b >> 12 & 0xF000u));
+    }
+}
+
 // Few tokens, more than 32 centroids: a wave takes one codebook and goes through its tokens, lane l holds centroids
-// l, l + 64, ... in registers and computes their distances in the reference's own order of operations.  The wave's
-// smallest distance is the scan's result if every other one is larger by more than the hysteresis -- the scan takes it when
-// it comes to it, whatever it holds, and nothing after it -- which one ballot tells; else (near ties, NaN, infinities)
-// the scan reads the distances lane by lane.
+// l, l + 64, ... in registers (wave_scan).
 // A lane per token (ccs_kernel) leaves all but N lanes of a wave idle and goes through the centroids one after the
-// other: 20.9 us at one token, 256 codebooks, 64 centroids, where this takes 4.7.  Bound by the launch and one round trip
+// other: 14.7 us at one token, 192 codebooks, 64 centroids, where this takes 3 and the matrix search 7.  Bound by the launch and one round trip
 // at a few tokens, by the vector ALU (3 v R operations and a reduction over the wave per pair) from about 50 on.
 template <int V, int R>  // R: centroids per lane
 __global__ __launch_bounds__(CCS_THREADS) void ccs_few_kernel(const float* __restrict__ x, const float* __restrict__ cent,
@@ -1170,49 +1568,13 @@ __global__ __launch_bounds__(CCS_THREADS) void ccs_few_kernel(const float* __res
     }
     for (uint32_t tok = tok0; tok < tok1; ++tok) {
         const float* xs = x + (size_t)tok * K + (size_t)cb * V;
-        float d[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) d[r] = 0.0f;
-#pragma unroll
-        for (int t = 0; t < V; ++t) {
-            const float xt = xs[t];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const float diff = __fsub_rn(xt, c[r][t]);
-                d[r] = __fadd_rn(d[r], __fmul_rn(diff, diff));
-            }
-        }
-        float m = __builtin_inff();
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (lane + 64 * r >= C) d[r] = __builtin_inff();
-            m = fminf(m, d[r]);
-        }
-#pragma unroll
-        for (int s = 1; s < 64; s *= 2) m = fminf(m, __shfl_xor(m, s));
-        uint32_t found = 0, near = 0;  // near: centroids that the scan may prefer to one another (the nearest among them)
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const uint64_t b = __ballot(!(__fsub_rn(d[r], m) > 1e-6f));
-            near += __builtin_popcountll(b);
-            if (b) found = 64 * r + __builtin_ctzll(b);
-        }
-        if (near != 1) {
-            float best = 0.0f;
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                for (uint32_t k = 0; k < 64 && 64 * r + k < C; ++k) {
-                    const float dk = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(d[r]), k));
-                    if ((r == 0 && k == 0) || __fsub_rn(best, dk) > 1e-6f) {
-                        best = dk;
-                        found = 64 * r + k;
-                    }
-                }
-        }
+        const uint32_t found = wave_scan<V, R>(xs, C, lane, [&](int r, int t) { return c[r][t]; });
         if (lane == 0) idx[idx_offset(tok, cb, idx_row_bytes, idx_tiled)] = (uint8_t)found;
     }
 }
 
+// Generic sub-vector length (any v): one lane per (token, codebook), operands straight from
+// global memory.  Correct for every shape; only used where no specialisation exists.
 template <int IDX_BITS>
 __global__ __launch_bounds__(256) void ccs_generic_kernel(const float* __restrict__ x,
                                                          const float* __restrict__ cent,
@@ -1416,6 +1778,23 @@ int launch_ccs_bf16(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     return launch_ccs_bf16_tt<V, WIDE, 128>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
 }
 
+template <int V, int IDX_BITS>
+int launch_ccs_many(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent, uint8_t* d_idx, uint32_t n)
+{
+    using S = CcsManyShape<V>;
+    const uint32_t tiles_cb = g.CB_pad / S::CBW;  // CB_pad is a multiple of 32
+    const uint64_t total = (uint64_t)((n + S::TT - 1) / S::TT) * tiles_cb;
+    if (total > 0x7FFFFFFFull) return set_error(ctx, PIMDL_ERR_INVALID, "ccs: too many tiles");
+    const int vec_ok = (g.K % 4 == 0) && ((reinterpret_cast<uintptr_t>(d_x) & 15) == 0);
+    const float* cnmax = d_cent + (size_t)g.CB * g.C * g.v + ccs_aux_floats(g);
+    const float* many = d_cent + ccs_bf16_offset(g);
+    const float* cn32 = many + ccs_many_groups(g) * ccs_many_nm(V) * 64 * 4;
+    hipLaunchKernelGGL((ccs_many_kernel<V, IDX_BITS>), dim3((uint32_t)total), dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent,
+                       reinterpret_cast<const uint4*>(many), cn32, cnmax, d_idx, n, g.K, g.CB, g.C, g.idx_row_bytes,
+                       (int)g.idx_tiled, vec_ok, tiles_cb);
+    return hip_check(ctx, hipGetLastError(), "ccs_many_kernel launch");
+}
+
 template <int V>
 int launch_ccs_few(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent, uint8_t* d_idx, uint32_t n)
 {
@@ -1464,11 +1843,15 @@ int launch_ccs_bits(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
             default: break;
         }
     }
-    // Few (token, codebook) pairs: a wave per pair.  The lane-per-token kernel takes about 0.3 us per centroid however few
-    // the tokens are, the wave-per-pair one about 4 us + 6 ps per pair and centroid (us, v = 4: 64 centroids, 256
-    // codebooks N = 64 21.3 / 9.2, N = 128 24.5 / 16.4, N = 256 24.4 / 30.4; 128 centroids N = 128 38.7 / 27.9,
-    // N = 256 39.1 / 53.1; 200 centroids N = 128 60 / 42, N = 256 70 / 81).
-    if (IDX_BITS == 8 && g.C > 32 && !g.tune_search && !exact && (double)n * g.CB * 6e-6 + 4.0 / g.C < 0.25) {
+    // Few (token, codebook) pairs and more than 32 centroids: a wave per pair takes about 2.2 us + 0.12 ns per pair (2 ns at
+    // v = 32, whose rows of 128 bytes a lane each fetches for itself), the matrix search 4 us + 0.42 us for every 32
+    // centroids of every codebook of a wave, until it has filled the chip (us, pair / matrix: v = 4, 64 centroids, 192
+    // codebooks N = 1 3.1 / 7.3, N = 128 4.6 / 8.0, N = 512 11.8 / 8.0; 256 centroids, 256 codebooks N = 128 7.1 / 19.8,
+    // N = 512 24.7 / 20.0; v = 16, 64 centroids, 64 codebooks N = 512 6.4 / 7.4, N = 2048 16.4 / 7.5; v = 32, 64 centroids,
+    // 40 codebooks N = 37 4.8 / 6.9, N = 128 9.3 / 6.9).
+    const double groups = (double)((g.C + 31) / 32) * (g.v >= 16 ? 1 : 16 / g.v);
+    if (IDX_BITS == 8 && g.C > 32 && !g.tune_search && !exact && !f32 &&
+        (double)n * g.CB * (g.v == 32 ? 1.9e-3 : 0.12e-3) < 1.8 + 0.42 * groups) {
         switch (g.v) {
             case 2: return launch_ccs_few<2>(ctx, g, d_x, d_cent, d_idx, n);
             case 4: return launch_ccs_few<4>(ctx, g, d_x, d_cent, d_idx, n);
@@ -1477,6 +1860,17 @@ int launch_ccs_bits(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
             case 32: return launch_ccs_few<32>(ctx, g, d_x, d_cent, d_idx, n);
             default: break;
         }
+    }
+    if (ccs_has_many(g) && !g.tune_search && !exact && !f32) {
+        if constexpr (IDX_BITS == 8) {
+            switch (g.v) {
+                case 2: return launch_ccs_many<2, 8>(ctx, g, d_x, d_cent, d_idx, n);
+                case 4: return launch_ccs_many<4, 8>(ctx, g, d_x, d_cent, d_idx, n);
+                case 8: return launch_ccs_many<8, 8>(ctx, g, d_x, d_cent, d_idx, n);
+            }
+        }
+        return g.v == 16 ? launch_ccs_many<16, IDX_BITS>(ctx, g, d_x, d_cent, d_idx, n)
+                         : launch_ccs_many<32, IDX_BITS>(ctx, g, d_x, d_cent, d_idx, n);
     }
     switch (g.v) {
         case 2: return launch_ccs_t<2, IDX_BITS>(ctx, g, d_x, d_cent, d_idx, n);
@@ -1631,7 +2025,7 @@ bool ccs_exact_only()
 
 size_t ccs_centroid_bytes(const AmmGeom& g)
 {
-    return (ccs_bf16_offset(g) + ccs_bf16_floats(g)) * sizeof(float);
+    return (ccs_bf16_offset(g) + ccs_bf16_floats(g) + ccs_many_floats(g)) * sizeof(float);
 }
 
 int launch_ccs_prep(Ctx* ctx, const AmmGeom& g, float* d_cent)
@@ -1646,6 +2040,14 @@ int launch_ccs_prep(Ctx* ctx, const AmmGeom& g, float* d_cent)
     hipLaunchKernelGGL(ccs_prep_mfma_kernel, dim3(g.CB_pad / 2), dim3(64), 0, ctx->stream, d_cent, cnmax, aux_a,
                        aux_a + (size_t)(g.CB_pad / 2) * (g.v + 1) * 64, g.CB, g.C, g.v);
     rc = hip_check(ctx, hipGetLastError(), "ccs_prep_mfma_kernel launch");
+    if (!rc && ccs_has_many(g)) {
+        float* many = d_cent + ccs_bf16_offset(g);
+        float* cn32 = many + ccs_many_groups(g) * ccs_many_nm(g.v) * 64 * 4;
+        auto prep = g.v == 2 ? ccs_prep_many_kernel<2> : g.v == 4 ? ccs_prep_many_kernel<4> : g.v == 8 ? ccs_prep_many_kernel<8>
+                  : g.v == 16 ? ccs_prep_many_kernel<16> : ccs_prep_many_kernel<32>;
+        hipLaunchKernelGGL(prep, dim3(g.CB, (g.C + 31) / 32), dim3(64), 0, ctx->stream, d_cent, reinterpret_cast<uint4*>(many), cn32, g.C);
+        rc = hip_check(ctx, hipGetLastError(), "ccs_prep_many_kernel launch");
+    }
     if (rc || !ccs_has_bf16(g)) return rc;
     float* bf = d_cent + ccs_bf16_offset(g);
     uint4* aux_b = reinterpret_cast<uint4*>(bf);

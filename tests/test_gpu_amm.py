@@ -676,3 +676,30 @@ def test_search_of_few_tokens_with_many_centroids(ctx, N, v, C):
     want = oracle.index_calculation(x, cent, v, threads=THREADS)
     assert np.array_equal(idx, want), np.argwhere(idx != want)[:8]
     amm.close()
+
+
+@pytest.mark.parametrize("N,v,C,lut", [(1170, 2, 33, "i8"), (1201, 4, 64, "i8"), (3600, 4, 256, "i8"), (2000, 8, 100, "f32"), (705, 16, 65, "i8"),
+                                       (200, 32, 200, "i8"), (1, 16, 8, "i8"), (65, 32, 32, "i8"), (129, 16, 16, "i8"), (63, 32, 3, "f32"),
+                                       (64, 16, 32, "f32")])
+def test_matrix_search_over_groups_of_centroids(ctx, N, v, C, lut):
+    """More than 32 centroids, and sub-vectors of 16 and 32: ragged tiles and groups, padded codebooks, both index
+    layouts; single near ties (replayed by the whole wave) and codebooks in which every token ties (lane by lane);
+    NaN, infinities, magnitudes from 1e-20 to 1e20."""
+    CB, M = 37, 20
+    x, cent, table, bias = make_case(8100 + N + C, N, CB * v, v, C, M, lut)
+    cent[1] = 0.0                                   # every token ties
+    cent[2, C - 1] = cent[2, 0]                     # those nearest to the repeated centroid do
+    cent[3, C // 2] = np.nan
+    cent[4, 0] = np.inf
+    cent[5] = cent[5, :1] + np.linspace(3e-4, 0, C, dtype=np.float32)[:, None]   # steps around the hysteresis
+    x[N // 2, 2 * v:3 * v] = cent[2, 0]
+    x[0, 5 * v:6 * v] = cent[5, 0]
+    x[N - 1, 6 * v] = np.nan
+    x[N // 3, 7 * v] = -np.inf
+    x[N - 1, 8 * v:] *= np.float32(1e20)
+    x[N // 4] *= np.float32(1e-20)
+    amm = ctx.amm(cent, table, None if lut == "f32" else np.float32(0.01), bias, max_n=N)
+    _, idx, _ = amm.run_debug(x, want_acc=False)
+    want = oracle.index_calculation(x, cent, v, threads=THREADS)
+    assert np.array_equal(idx, want), (int((idx != want).sum()), np.argwhere(idx != want)[:8])
+    amm.close()
