@@ -218,15 +218,15 @@ __global__ __launch_bounds__(64) void gather_f32_few_kernel(const uint8_t* __res
                                                             float* __restrict__ out, uint32_t N, uint32_t M, uint32_t CB_pad,
                                                             uint32_t idx_row_bytes, const float* __restrict__ bias,
                                                             const float* __restrict__ scales, uint32_t CB, uint32_t group,
-                                                            uint32_t act, uint32_t colblocks, uint32_t c_tile, uint32_t chunked)
+                                                            uint32_t act, uint32_t colblocks, uint32_t c_tile, uint32_t piece)
 {
     constexpr int TOK = 64 / FB, WORDS = IDX_BITS;  // tokens per wave; index words of 32 codebooks
     const uint32_t colblk = blockIdx.x % colblocks, e = threadIdx.x % FB;
     const uint32_t tok = blockIdx.x / colblocks * TOK + threadIdx.x / FB, f = colblk * FB + e;
     const uint32_t* ix = reinterpret_cast<const uint32_t*>(idx + (size_t)(tok < N ? tok : N - 1) * idx_row_bytes);
-    // entry of row r: plain [row][FB], chunked (see gather_f32_kernel) [FB / 2][row][2]
-    const uint32_t row = chunked ? 2 : FB;
-    const float* tab = lut + (size_t)colblk * CB_pad * c_tile * FB + (chunked ? e / 2 * c_tile * 2 + e % 2 : e);
+    // entry of row r: [row][FB], or [FB / piece][row][piece]
+    const uint32_t row = piece ? piece : FB;
+    const float* tab = lut + (size_t)colblk * CB_pad * c_tile * FB + (piece ? e / piece * c_tile * piece + e % piece : e);
     const uint32_t per_cb = c_tile * FB, batches = CB_pad / 32;
 
     uint32_t w[WORDS];
@@ -285,7 +285,7 @@ int launch_f32_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, u
     a.note_launch(0, 0, tok, 64);
     hipLaunchKernelGGL((gather_f32_few_kernel<FB, IDX_BITS, GROUPED>), dim3(colblocks * ((n + tok - 1) / tok)), dim3(64), 0, ctx->stream,
                        d_idx, reinterpret_cast<const float*>(a.d_lut), d_out, n, g.M, g.CB_pad, g.idx_row_bytes, a.d_bias,
-                       a.d_scales, g.CB, a.desc.scale_group, a.desc.activation, colblocks, g.C_tile, g.lut_chunked);
+                       a.d_scales, g.CB, a.desc.scale_group, a.desc.activation, colblocks, g.C_tile, g.lut_chunk);
     return hip_check(ctx, hipGetLastError(), "gather_f32_few_kernel launch");
 }
 
@@ -298,8 +298,10 @@ int launch_f32_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, u
 // The byte adder and the floats read every gathered piece from the caches on its own, which costs in proportion to
 // tokens x codebooks x columns; against that stands the large kernels' chain of slices.  Byte adder, 3072 -> 768,
 // 32 centroids: 17.6 / 4.4 at N = 1, 17.7 / 7.9 at 13, 17.8 / 27.4 at 64; 1000 -> 1001, 200 centroids: 18.9 / 5.8 at 13,
-// 24.1 / 40.8 at 300.  Floats, 16 centroids, 3072 -> 768: 59.9 / 13.3 at 1, 60.2 / 26.1 at 150, 61 / 43 at 300, 61 / 68
-// at 512; 768 -> 3072: 18.1 / 4.7 at 1, 18.4 / 11.9 at 64, 19.0 / 24.8 at 150.  The two estimates are fits to these.
+// 24.1 / 40.8 at 300.  Floats, 16 centroids (the large kernel with 64-token workgroups): 3072 -> 768 23.7 / 14.4 at 1,
+// 24.0 / 19.6 at 13, 25.5 / 28.7 at 64; 768 -> 3072 8.6 / 5.2 at 1, 8.4 / 9.3 at 13; 32 centroids 3072 -> 768 44 / 33 at 1,
+// 47 / 71 at 64; 200 centroids (whole rows) 1000 -> 1001 49 / 5.3 at 1, 51 / 32 at 64, 56 / 73 at 150; a scale per 5
+// codebooks 19.8 / 18.7 at 1, 19.7 / 22.6 at 13.  The estimates are fits to these.
 bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
 {
     const AmmGeom& g = a.g;
@@ -308,7 +310,8 @@ bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
     const double pieces = (double)n * g.CB_pad * (g.M_pad / 16);  // of 16 columns
     if (a.desc.lut_dtype == PIMDL_LUT_F32 || a.grouped) {
         const bool bounds = a.grouped && !a.prescaled;  // a scale to apply at the end of every group
-        const double piece = g.lut_chunked || g.q != 4 ? 32e-6 : 4e-6;
+        if (g.lut_chunk) return pieces * (g.lut_chunk == 2 ? 18e-6 : 7.5e-6) < (bounds ? 1.0 : 1.4 + 0.0103 * g.CB_pad);
+        const double piece = g.q != 4 ? 32e-6 : 4e-6;
         return 2.7 + g.CB_pad * (bounds ? 0.062 : 0.0137) + pieces * piece < 4.0 + g.CB_pad * (bounds ? 0.14 : 0.07);
     }
     if (g.gather_kind == 0)

@@ -501,8 +501,8 @@ int launch_onehot(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, in
 }
 
 // ---------------------------------------------------------------------------------------------
-// fp32 LUT: out[n][f] = (sum over cb ascending, fp32) lut[cb][idx][f] + bias[f]
-// One lane = one token; a workgroup = 256 tokens x 4*Q columns; slices of GS codebooks in LDS.
+// fp32 LUT, more than 32 centroids (up to 32: gather_f32_kernel.hip): out[n][f] = (sum over cb ascending, fp32)
+// lut[cb][idx][f] + bias[f].  One lane = one token; a workgroup = 256 tokens x 4*Q columns; slices of GS codebooks in LDS.
 //
 // GROUPED (int8 table with one scale per `group` consecutive codebooks; not in the reference): the
 // table holds the int8 entries converted to fp32, so the sum inside a group is an exact integer
@@ -524,13 +524,7 @@ __global__ __launch_bounds__(GF_THREADS) void gather_f32_kernel(const uint8_t* _
                                                                uint32_t n_token_tiles, uint32_t by_xcd)
 {
     constexpr int FB = 4 * Q;             // columns per row
-    // 32 rows of 16-byte pieces cover the 64 banks twice: two lanes of a ds_read_b128 pass that want
-    // different rows 16 apart collide (measured 1.7x the conflict-free time).  8-byte pieces of 32 rows
-    // cover the banks exactly once, and a ds_read_b64 takes half the time of a b128: the table for 32
-    // centroids is therefore kept as [codebook][8-byte chunk][row], read with twice as many b64 reads
-    // and no conflicts (the same layout in HBM, so that staging stays a flat copy).
-    constexpr bool CHUNKED = f32_lut_chunked(C_T, Q);
-    constexpr int PITCH = CHUNKED ? 16 * Q : 16 * Q + 16;    // bytes
+    constexpr int PITCH = 16 * Q + 16;    // bytes
     constexpr int CB_BYTES = C_T * PITCH;
     constexpr int SLICE_LDS = GS * CB_BYTES;
     constexpr int SLICE_UNITS = GS * C_T * Q;
@@ -589,7 +583,7 @@ __global__ __launch_bounds__(GF_THREADS) void gather_f32_kernel(const uint8_t* _
         {                                                                                           \
             const uint32_t unit_ = threadIdx.x + u * GF_THREADS;                                    \
             if (SLICE_UNITS % GF_THREADS == 0 || unit_ < SLICE_UNITS)                               \
-                *reinterpret_cast<uint4*>(dst_ + (CHUNKED ? unit_ * 16 : (unit_ / Q) * PITCH + (unit_ % Q) * 16)) = stage[u]; \
+                *reinterpret_cast<uint4*>(dst_ + (unit_ / Q) * PITCH + (unit_ % Q) * 16) = stage[u]; \
         }                                                                                           \
     }
     PIMDL_FETCH_SLICE(0)
@@ -621,27 +615,14 @@ __global__ __launch_bounds__(GF_THREADS) void gather_f32_kernel(const uint8_t* _
                 for (int t = 0; t < TPL; ++t) {
                     const uint32_t r = word[t] & ((1u << IDX_BITS) - 1);
                     word[t] >>= IDX_BITS;
-                    if constexpr (CHUNKED) {
-                        const unsigned char* row = cbbase + r * 8;
+                    const unsigned char* row = cbbase + r * PITCH;
 #pragma unroll
-                        for (int c = 0; c < 2 * Q; ++c) {
-                            // volatile: keeps the compiler from pairing two chunks into one ds_read2_b64, whose
-                            // halves (256 bytes apart) would meet in the same banks
-                            typedef float v2f __attribute__((ext_vector_type(2)));
-                            const v2f vv = *(const volatile __attribute__((address_space(3))) v2f*)(row + c * (C_T * 8));
-                            acc[t][2 * c + 0] = __fadd_rn(acc[t][2 * c + 0], vv[0]);
-                            acc[t][2 * c + 1] = __fadd_rn(acc[t][2 * c + 1], vv[1]);
-                        }
-                    } else {
-                        const unsigned char* row = cbbase + r * PITCH;
-#pragma unroll
-                        for (int c = 0; c < Q; ++c) {
-                            const float4 vv = *reinterpret_cast<const float4*>(row + c * 16);
-                            acc[t][4 * c + 0] = __fadd_rn(acc[t][4 * c + 0], vv.x);
-                            acc[t][4 * c + 1] = __fadd_rn(acc[t][4 * c + 1], vv.y);
-                            acc[t][4 * c + 2] = __fadd_rn(acc[t][4 * c + 2], vv.z);
-                            acc[t][4 * c + 3] = __fadd_rn(acc[t][4 * c + 3], vv.w);
-                        }
+                    for (int c = 0; c < Q; ++c) {
+                        const float4 vv = *reinterpret_cast<const float4*>(row + c * 16);
+                        acc[t][4 * c + 0] = __fadd_rn(acc[t][4 * c + 0], vv.x);
+                        acc[t][4 * c + 1] = __fadd_rn(acc[t][4 * c + 1], vv.y);
+                        acc[t][4 * c + 2] = __fadd_rn(acc[t][4 * c + 2], vv.z);
+                        acc[t][4 * c + 3] = __fadd_rn(acc[t][4 * c + 3], vv.w);
                     }
                 }
                 cbbase += CB_BYTES;
@@ -698,7 +679,7 @@ __global__ __launch_bounds__(GF_THREADS) void gather_f32_kernel(const uint8_t* _
 template <int C_T, int Q, int GS, int IDX_BITS, bool GROUPED, int TPL>
 int launch_f32_impl(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, uint32_t n)
 {
-    constexpr int LDS = 2 * GS * C_T * (f32_lut_chunked(C_T, Q) ? 16 * Q : 16 * Q + 16);
+    constexpr int LDS = 2 * GS * C_T * (16 * Q + 16);
     auto kern = gather_f32_kernel<C_T, Q, GS, IDX_BITS, GROUPED, TPL>;
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_f32)")) return rc;
     const uint32_t n_token_tiles = (n + GF_THREADS * TPL - 1) / (GF_THREADS * TPL), colblocks = a.g.M_pad / (4 * Q);
@@ -719,7 +700,7 @@ int f32_wgs_per_cu()
 {
     static int cached = 0;
     if (cached == 0) {
-        constexpr int LDS = 2 * GS * C_T * (f32_lut_chunked(C_T, Q) ? 16 * Q : 16 * Q + 16);
+        constexpr int LDS = 2 * GS * C_T * (16 * Q + 16);
         int q = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, gather_f32_kernel<C_T, Q, GS, IDX_BITS, GROUPED, TPL>, GF_THREADS,
                                                          LDS) != hipSuccess || q < 1) {
@@ -761,11 +742,8 @@ int launch_f32(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, uint3
 
 }  // namespace
 
-// Tiling choices of the fp32 gather per centroid count: rows of 4 * Q floats, slices of GS codebooks.
+// Tiling choices of gather_f32_kernel per centroid count: rows of 4 * Q floats, slices of GS codebooks.
 //   C_T   (Q, GS) -> slice bytes
-//   8     (4, 32) 20 KB
-//   16    (4, 16) 20 KB
-//   32    (4, 8)  20 KB
 //   64    (4, 8)  40 KB
 //   128   (2, 8)  48 KB
 //   256   (2, 4)  48 KB
@@ -966,14 +944,14 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
         g->tokens_per_wg = g->gather_threads;
     } else {
         g->gq = 0;
-        g->cb_per_slice = ct == 8 ? 32 : ct == 16 ? 16 : ct <= 128 ? 8 : 4;
+        g->cb_per_slice = ct <= 16 ? 16 : ct <= 128 ? 8 : 4;
         g->col_block = 4 * g->q;
         g->gather_threads = GF_THREADS;
         g->tokens_per_wg = GF_THREADS;
     }
-    g->lut_chunked = !i8 && f32_lut_chunked((int)ct, (int)g->q);
-    g->row_pitch = g->lut_chunked ? 16 * g->q : 16 * (g->q | 1);
-    g->gather_lds_bytes = 2 * g->cb_per_slice * ct * g->row_pitch;
+    g->lut_chunk = i8 ? 0 : f32_lut_chunk(ct);
+    g->row_pitch = g->lut_chunk ? 4 * g->lut_chunk : 16 * (g->q | 1);
+    g->gather_lds_bytes = g->lut_chunk ? f32_rows_lds_bytes(ct) : 2 * g->cb_per_slice * ct * g->row_pitch;
     g->M_pad = (M + g->col_block - 1) / g->col_block * g->col_block;
     if (i8) {
         g->row_pitch = 256;
@@ -1020,10 +998,8 @@ int launch_gather(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, in
         return launch_gather_rows(ctx, a, d_idx, d_out, d_acc, n, ep.scale, ep.lut_bias_term);
     } else {
         if (gather_few_wanted(ctx, a, n)) return launch_gather_few(ctx, a, d_idx, d_out, nullptr, n, 0.0f, 0.0f);
+        if (g.C_tile <= 32) return launch_gather_f32_rows(ctx, a, d_idx, d_out, n);
         switch (g.C_tile) {
-            case 8: return launch_f32<8, 4, 32, 4>(ctx, a, d_idx, d_out, n);
-            case 16: return launch_f32<16, 4, 16, 4>(ctx, a, d_idx, d_out, n);
-            case 32: return launch_f32<32, 4, 8, 8>(ctx, a, d_idx, d_out, n);
             case 64: return launch_f32<64, 4, 8, 8>(ctx, a, d_idx, d_out, n);
             case 128: return launch_f32<128, 2, 8, 8>(ctx, a, d_idx, d_out, n);
             case 256: return launch_f32<256, 2, 4, 8>(ctx, a, d_idx, d_out, n);

@@ -23,13 +23,14 @@ namespace pimdl {
 //              [M_pad / col_block][CB_pad][col_block][16] bytes (the 16 centroid entries of a column are
 //              contiguous).  Either way one (columns, codebook range) slice is contiguous, so staging it
 //              into LDS is a flat copy.  Padded codebooks / centroid rows / columns hold zeros.
-// fp32 LUT     tiled [M_pad / col_block][CB_pad][C_tile][col_block] floats.
+// fp32 LUT     tiled [M_pad / col_block][CB_pad][C_tile][col_block] floats, rows in pieces where lut_chunk says so.
 // ---------------------------------------------------------------------------------------------
 struct AmmGeom {
     uint32_t K, v, CB, CB_pad, C, C_tile, M, M_pad;
     uint32_t idx_bits, idx_row_bytes;
     uint32_t idx_tiled;     // layout of the packed index buffer, see above
-    uint32_t lut_chunked;   // fp32 table of 32 centroids: [column block][codebook][8-byte chunk][row][2 floats]
+    uint32_t lut_chunk;     // fp32 table of up to 32 centroids: [column block][codebook][chunk][row][lut_chunk floats], chunks of
+                            // 4 floats, or 2 with 32 rows (either way the rows of a chunk are all LDS banks at most once)
     // gather kernel
     uint32_t gather_kind;   // int8 tables: 0: byte adder, 1: one-hot matrix-core kernel (int8, C <= 16),
                             // 2: one-hot on the sparse matrix instruction (int8, C <= 32: a codebook of 17..32
@@ -48,8 +49,8 @@ struct AmmGeom {
     uint32_t tune_search, tune_search_tile, tune_token_item, tune_cb_per_slice, tune_xcd_col_split;
 };
 
-// fp32 tables whose rows are read in 8-byte chunks (see gather_f32_kernel)
-constexpr bool f32_lut_chunked(int c_tile, int q) { return c_tile == 32 && q == 4; }
+// floats of the pieces in which the rows of an fp32 table are kept (0: whole rows)
+constexpr uint32_t f32_lut_chunk(uint32_t c_tile) { return c_tile == 32 ? 2 : c_tile <= 16 ? 4 : 0; }
 
 // bytes of a packed index buffer for n tokens
 inline size_t idx_buffer_bytes(const AmmGeom& g, uint32_t n)
@@ -180,6 +181,9 @@ int launch_diag_mfma_error(Ctx* ctx, uint32_t trials, bool crafted, float* max_e
 // the sparse one-hot gather (gather_sp_kernel.hip)
 int launch_gather_sparse(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc_or_null,
                          uint32_t n, float scale, float lut_bias_term);
+// fp32 tables of up to 32 centroids (gather_f32_kernel.hip)
+int launch_gather_f32_rows(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, uint32_t n);
+uint32_t f32_rows_lds_bytes(uint32_t c_tile);
 // the byte adder (gather_rows_kernel.hip)
 int launch_gather_rows(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc_or_null, uint32_t n,
                        float scale, float lut_bias_term);

@@ -703,3 +703,25 @@ def test_matrix_search_over_groups_of_centroids(ctx, N, v, C, lut):
     want = oracle.index_calculation(x, cent, v, threads=THREADS)
     assert np.array_equal(idx, want), (int((idx != want).sum()), np.argwhere(idx != want)[:8])
     amm.close()
+
+
+@pytest.mark.parametrize("N,CB,v,C,M,group", [
+    (63, 32, 4, 16, 4096, 0), (500, 33, 4, 16, 500, 0), (65, 64, 2, 8, 2031, 0), (900, 96, 4, 17, 770, 0),  # 64-token workgroups
+    (257, 40, 4, 16, 4100, 0), (8200, 32, 4, 7, 800, 0), (5000, 65, 4, 32, 1001, 0),                       # 256-token ones
+    (600, 70, 4, 12, 100, 1), (300, 70, 4, 16, 4096, 9), (520, 41, 4, 30, 3000, 3), (900, 41, 4, 8, 64, 6)])
+def test_float_tables_in_pieces(ctx, N, CB, v, C, M, group):
+    """fp32 tables and scales per group of codebooks up to 32 centroids: the additions are made in ascending codebook
+    order whatever the kernel, so the output is the oracle's to the bit; the last tokens and ragged columns included."""
+    x, cent, table, bias = make_case(9100 + N + C, N, CB * v, v, C, M, "i8" if group else "f32")
+    scales = np.random.default_rng(N).uniform(0.001, 0.02, (CB + group - 1) // group).astype(np.float32) if group else None
+    amm = ctx.amm(cent, table, scales, bias, max_n=N, scale_group=group)
+    out, idx, _ = amm.run_debug(x, want_acc=False)
+    rows = np.unique(np.concatenate([np.arange(0, min(N, 70)), np.arange(max(0, N - 70), N),
+                                     np.random.default_rng(1).choice(N, size=min(N, 100), replace=False)]))
+    want_idx = oracle.index_calculation(x[rows], cent, v, threads=THREADS)
+    assert np.array_equal(idx[rows], want_idx)
+    want = (oracle.gather_i8_grouped(want_idx, table, scales, bias, group, threads=THREADS) if group
+            else oracle.gather_f32(want_idx, table, bias, threads=THREADS))
+    assert np.array_equal(out[rows].view(np.uint32), want.view(np.uint32))
+    assert "_f32_rows_" in amm.last_gather_kernel(), amm.last_gather_kernel()
+    amm.close()
