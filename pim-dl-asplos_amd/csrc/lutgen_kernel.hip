@@ -7,7 +7,9 @@
 //
 // One wave computes a 16-centroid x 64-column tile of one codebook with v_mfma_f32_16x16x4_f32
 // (K = 4 matches sub_vec_len 4 in one step; other v loop/zero-pad).  The work is tiny
-// (2*C*K*M flop) and the kernel is bound by reading W and writing the LUT once.
+// (2*C*K*M flop) and the kernel is bound by reading W and writing the LUT once.  Every workgroup leaves the largest
+// magnitude it has written beside the table, and the workgroups of the quantisation reduce those (a pass of its own over the
+// table, with an atomic per wave, took 57 us of the 93 at 768 -> 3072, 16 centroids; now 15 + LUTGEN_US).
 #include "pimdl_internal.h"
 
 namespace pimdl {
@@ -19,23 +21,33 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 constexpr int LG_WAVES = 4;
 constexpr int LG_FT = 4;  // 16-column tiles per wave
 
+// largest value of a workgroup of four waves, in thread 0 (m >= 0; NaN is passed over)
+__device__ __forceinline__ float block_max(float m)
+{
+    __shared__ float part[4];
+    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+    __syncthreads();
+    return fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+}
+
+// part [codebook][workgroups of a codebook]: the largest magnitude each workgroup wrote (here and below)
 __global__ __launch_bounds__(LG_WAVES * 64) void lutgen_f32_kernel(const float* __restrict__ cent,
                                                                   const float* __restrict__ W,
-                                                                  float* __restrict__ lut, uint32_t CB,
-                                                                  uint32_t C, uint32_t v, uint32_t M)
+                                                                  float* __restrict__ lut, float* __restrict__ part,
+                                                                  uint32_t CB, uint32_t C, uint32_t v, uint32_t M)
 {
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t j = lane & 15, k = lane >> 4;
     const uint32_t cb = blockIdx.z;
     const uint32_t c0 = blockIdx.y * 16;
     const uint32_t f0 = (blockIdx.x * LG_WAVES + wave) * (16 * LG_FT);
-    if (f0 >= M) return;  // whole wave
 
     v4f acc[LG_FT];
 #pragma unroll
     for (int t = 0; t < LG_FT; ++t) acc[t] = (v4f){0.f, 0.f, 0.f, 0.f};
 
-    for (uint32_t t0 = 0; t0 < v; t0 += 4) {
+    for (uint32_t t0 = 0; t0 < v && f0 < M; t0 += 4) {
         const uint32_t t = t0 + k;
         // A[i = centroid c0 + j][k = t]
         float a = 0.0f;
@@ -49,6 +61,7 @@ __global__ __launch_bounds__(LG_WAVES * 64) void lutgen_f32_kernel(const float* 
         }
     }
     // D[i = 4*k + r][j]: centroid c0 + 4k + r, column f0 + ft*16 + j
+    float m = 0.0f;
 #pragma unroll
     for (int ft = 0; ft < LG_FT; ++ft) {
         const uint32_t f = f0 + ft * 16 + j;
@@ -56,9 +69,14 @@ __global__ __launch_bounds__(LG_WAVES * 64) void lutgen_f32_kernel(const float* 
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const uint32_t c = c0 + 4 * k + r;
-            if (c < C) lut[((size_t)cb * C + c) * M + f] = acc[ft][r];
+            if (c < C) {
+                lut[((size_t)cb * C + c) * M + f] = acc[ft][r];
+                m = fmaxf(m, fabsf(acc[ft][r]));
+            }
         }
     }
+    m = block_max(m);
+    if (threadIdx.x == 0) part[((size_t)cb * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = m;
 }
 
 // The same product with the v terms of every entry added in ascending order, each multiplication and each
@@ -67,47 +85,58 @@ __global__ __launch_bounds__(LG_WAVES * 64) void lutgen_f32_kernel(const float* 
 // form is "the" reference result; this one makes a converter's output reproducible bit for bit by scalar code.
 // One thread = one output column of one codebook, all C centroids: W is read once, the LUT written once.
 __global__ __launch_bounds__(256) void lutgen_ordered_kernel(const float* __restrict__ cent, const float* __restrict__ W,
-                                                           float* __restrict__ lut, uint32_t C, uint32_t v, uint32_t M)
+                                                           float* __restrict__ lut, float* __restrict__ part, uint32_t C,
+                                                           uint32_t v, uint32_t M)
 {
     const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x, cb = blockIdx.y;
-    if (f >= M) return;
     const float* w = W + (size_t)cb * v * M + f;
-    for (uint32_t c = 0; c < C; ++c) {
+    float m = 0.0f;
+    for (uint32_t c = 0; c < C && f < M; ++c) {
         const float* a = cent + ((size_t)cb * C + c) * v;
         float acc = 0.0f;
         for (uint32_t t = 0; t < v; ++t) acc = __fadd_rn(acc, __fmul_rn(a[t], w[(size_t)t * M]));
         lut[((size_t)cb * C + c) * M + f] = acc;
+        m = fmaxf(m, fabsf(acc));
     }
+    m = block_max(m);
+    if (threadIdx.x == 0) part[(size_t)cb * gridDim.x + blockIdx.x] = m;
 }
 
-// max |x| per scale group; non-negative floats order like their bit patterns
-__global__ void absmax_kernel(const float* __restrict__ lut, uint32_t* __restrict__ absmax_bits,
-                              uint64_t group_elems, uint64_t total)
+__device__ __forceinline__ int8_t quantise(float x, float scale)
 {
-    const uint64_t grp = blockIdx.y;
-    const uint64_t beg = grp * group_elems;
-    const uint64_t end = beg + group_elems < total ? beg + group_elems : total;
-    float m = 0.0f;
-    for (uint64_t i = beg + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < end;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        m = fmaxf(m, fabsf(lut[i]));
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-    if ((threadIdx.x & 63) == 0) atomicMax(&absmax_bits[grp], __float_as_uint(m));
-}
-
-__global__ void quant_kernel(const float* __restrict__ lut, int8_t* __restrict__ q,
-                             const uint32_t* __restrict__ absmax_bits, float* __restrict__ scales,
-                             uint64_t group_elems, uint64_t total)
-{
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= total) return;
-    const uint64_t grp = i / group_elems;
-    float scale = __fdiv_rn(__uint_as_float(absmax_bits[grp]), 127.0f);
-    if (!(scale > 0.0f)) scale = 1.0f;  // all-zero group: any scale represents it
-    if (i % group_elems == 0) scales[grp] = scale;
-    float t = __fdiv_rn(lut[i], scale);
+    float t = __fdiv_rn(x, scale);
     t = fminf(fmaxf(t, -128.0f), 127.0f);
-    q[i] = (int8_t)rintf(t);  // round half to even
+    return (int8_t)rintf(t);  // round half to even
+}
+
+// Workgroup (x, g): a share of group g's entries.  Every workgroup reduces the group's magnitudes for itself (a few KB
+// from L2).  group_cbs codebooks per group, parts workgroups per codebook in `part`.
+__global__ __launch_bounds__(256) void quant_kernel(const float* __restrict__ lut, int8_t* __restrict__ q, const float* __restrict__ part,
+                                                    float* __restrict__ scales, uint32_t group_cbs, uint32_t parts, uint32_t CB,
+                                                    uint64_t cb_elems)
+{
+    const uint32_t grp = blockIdx.y, cb0 = grp * group_cbs, cb1 = cb0 + group_cbs < CB ? cb0 + group_cbs : CB;
+    float m = 0.0f;
+    for (uint64_t i = (uint64_t)cb0 * parts + threadIdx.x; i < (uint64_t)cb1 * parts; i += 256) m = fmaxf(m, part[i]);
+    float scale = __fdiv_rn(block_max(m), 127.0f);
+    if (!(scale > 0.0f)) scale = 1.0f;  // all-zero group: any scale represents it
+    if (blockIdx.x == 0 && threadIdx.x == 0) scales[grp] = scale;
+    const uint64_t beg = cb0 * cb_elems, end = cb1 * cb_elems;
+    const uint64_t step = (uint64_t)gridDim.x * 256, first = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    uint64_t done = beg;
+    if (beg % 4 == 0) {  // four entries per thread; the last ones of a ragged group below
+        done = beg + (end - beg) / 4 * 4;
+        for (uint64_t i = beg + 4 * first; i < done; i += 4 * step) {
+            const float4 x = *reinterpret_cast<const float4*>(lut + i);
+            char4 o;
+            o.x = quantise(x.x, scale);
+            o.y = quantise(x.y, scale);
+            o.z = quantise(x.z, scale);
+            o.w = quantise(x.w, scale);
+            *reinterpret_cast<char4*>(q + i) = o;
+        }
+    }
+    for (uint64_t i = done + first; i < end; i += step) q[i] = quantise(lut[i], scale);
 }
 
 // ---- diagnostics: a plain copy (HBM) and a ds_read_b128 loop (LDS) ------------------------------
@@ -141,44 +170,34 @@ __global__ __launch_bounds__(1024) void lds_read_kernel(int* __restrict__ sink, 
 
 }  // namespace
 
-int launch_lutgen_f32(Ctx* ctx, const float* d_cent, const float* d_w, float* d_lut, uint32_t CB, uint32_t C,
+// workgroups per codebook, each of which leaves its largest magnitude
+uint32_t lutgen_parts(uint32_t C, uint32_t M, bool ordered)
+{
+    return ordered ? (M + 255) / 256 : (M + LG_WAVES * 16 * LG_FT - 1) / (LG_WAVES * 16 * LG_FT) * ((C + 15) / 16);
+}
+
+int launch_lutgen_f32(Ctx* ctx, const float* d_cent, const float* d_w, float* d_lut, float* d_part, uint32_t CB, uint32_t C,
                       uint32_t v, uint32_t M, bool ordered)
 {
     if (ordered) {
-        hipLaunchKernelGGL(lutgen_ordered_kernel, dim3((M + 255) / 256, CB), dim3(256), 0, ctx->stream, d_cent, d_w, d_lut, C, v, M);
+        hipLaunchKernelGGL(lutgen_ordered_kernel, dim3((M + 255) / 256, CB), dim3(256), 0, ctx->stream, d_cent, d_w, d_lut, d_part, C, v, M);
         return hip_check(ctx, hipGetLastError(), "lutgen_ordered_kernel launch");
     }
     dim3 grid((M + LG_WAVES * 16 * LG_FT - 1) / (LG_WAVES * 16 * LG_FT), (C + 15) / 16, CB);
-    hipLaunchKernelGGL(lutgen_f32_kernel, grid, dim3(LG_WAVES * 64), 0, ctx->stream, d_cent, d_w, d_lut, CB, C, v, M);
+    hipLaunchKernelGGL(lutgen_f32_kernel, grid, dim3(LG_WAVES * 64), 0, ctx->stream, d_cent, d_w, d_lut, d_part, CB, C, v, M);
     return hip_check(ctx, hipGetLastError(), "lutgen_f32_kernel launch");
 }
 
-int launch_lut_quant(Ctx* ctx, const float* d_lut, int8_t* d_q, float* d_scales, uint32_t CB, uint32_t C,
-                     uint32_t M, uint32_t scale_group)
+int launch_lut_quant(Ctx* ctx, const float* d_lut, const float* d_part, uint32_t parts, int8_t* d_q, float* d_scales, uint32_t CB,
+                     uint32_t C, uint32_t M, uint32_t scale_group)
 {
-    const uint64_t total = (uint64_t)CB * C * M;
-    const uint32_t ngroups = scale_group ? (CB + scale_group - 1) / scale_group : 1;
-    const uint64_t group_elems = scale_group ? (uint64_t)scale_group * C * M : total;
-    uint32_t* d_bits = nullptr;
-    int rc = hip_check(ctx, hipMalloc(&d_bits, sizeof(uint32_t) * ngroups), "hipMalloc(absmax)");
-    if (rc) return rc;
-    rc = hip_check(ctx, hipMemsetAsync(d_bits, 0, sizeof(uint32_t) * ngroups, ctx->stream), "hipMemsetAsync(absmax)");
-    if (!rc) {
-        uint64_t bx = (group_elems + 256 * 16 - 1) / (256 * 16);
-        if (bx > 1024) bx = 1024;
-        if (bx < 1) bx = 1;
-        hipLaunchKernelGGL(absmax_kernel, dim3((uint32_t)bx, ngroups), dim3(256), 0, ctx->stream, d_lut, d_bits,
-                           group_elems, total);
-        rc = hip_check(ctx, hipGetLastError(), "absmax_kernel launch");
-    }
-    if (!rc) {
-        hipLaunchKernelGGL(quant_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, ctx->stream, d_lut, d_q,
-                           d_bits, d_scales, group_elems, total);
-        rc = hip_check(ctx, hipGetLastError(), "quant_kernel launch");
-    }
-    if (!rc) rc = hip_check(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize(quant)");
-    (void)hipFree(d_bits);
-    return rc;
+    const uint32_t cbs = scale_group && scale_group < CB ? scale_group : CB, ngroups = (CB + cbs - 1) / cbs;
+    const uint64_t cb_elems = (uint64_t)C * M;
+    uint64_t bx = (cbs * cb_elems + 256 * 16 - 1) / (256 * 16);
+    if (bx > 2048) bx = 2048;
+    hipLaunchKernelGGL(quant_kernel, dim3((uint32_t)bx, ngroups), dim3(256), 0, ctx->stream, d_lut, d_q, d_part, d_scales, cbs, parts,
+                       CB, cb_elems);
+    return hip_check(ctx, hipGetLastError(), "quant_kernel launch");
 }
 
 int launch_diag(Ctx* ctx, uint64_t bytes, float* copy_gbps, float* lds_gbps)

@@ -368,6 +368,69 @@ static int run_piped(Ctx* ctx, uint32_t K, uint32_t M, const float* in, bool in_
     return PIMDL_OK;
 }
 
+// One host buffer to device memory and back through the ring's pinned slots, 2 MiB at a time, so that the host's copy of one
+// piece overlaps the transfer of another (a pageable transfer of the runtime's takes about 25 GB/s, this the link's 57).
+// Ordered against the context's stream.  ring_to_device returns once `src` has been read, ring_to_host once `dst` is
+// complete.  Small buffers, and pointers the CPU cannot read, take the runtime's copy.
+constexpr size_t RING_PIECE = 2u << 20;
+
+static int ring_to_device(Ctx* ctx, void* dst, const void* src, size_t bytes)
+{
+    if (bytes < RING_PIECE / 4 || is_device_ptr(src))
+        return hip_check(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream), "H2D");
+    HostPipe* hp;
+    int rc = pipe_get(ctx, &hp);
+    if (rc) return rc;
+    rc = pipe_reserve(ctx, hp, RING_PIECE, 0);
+    // the destination is free once what the context's stream has queued is done
+    if (!rc) rc = hip_check(ctx, hipEventRecord(ctx->ev[0], ctx->stream), "hipEventRecord");
+    if (!rc) rc = hip_check(ctx, hipStreamWaitEvent(hp->s_in, ctx->ev[0], 0), "hipStreamWaitEvent");
+    int s = 0;
+    for (size_t at = 0; at < bytes && !rc; at += RING_PIECE, s = (s + 1) % HostPipe::SLOTS) {
+        const size_t len = std::min(RING_PIECE, bytes - at);
+        if (hp->used_in[s] && (rc = hip_check(ctx, hipEventSynchronize(hp->ev_in[s]), "hipEventSynchronize(staging in)"))) break;
+        parallel_copy(hp->pin_in[s], static_cast<const char*>(src) + at, len);
+        if ((rc = hip_check(ctx, hipMemcpyAsync(static_cast<char*>(dst) + at, hp->pin_in[s], len, hipMemcpyHostToDevice, hp->s_in), "H2D piece"))) break;
+        if ((rc = hip_check(ctx, hipEventRecord(hp->ev_in[s], hp->s_in), "hipEventRecord"))) break;
+        hp->used_in[s] = true;
+        if (at + len == bytes) rc = hip_check(ctx, hipStreamWaitEvent(ctx->stream, hp->ev_in[s], 0), "hipStreamWaitEvent");
+    }
+    if (rc) (void)hipStreamSynchronize(hp->s_in);
+    return rc;
+}
+
+static int ring_to_host(Ctx* ctx, void* dst, const void* src, size_t bytes)
+{
+    if (bytes < RING_PIECE / 4 || is_device_ptr(dst)) {
+        const int r = hip_check(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream), "D2H");
+        return r ? r : hip_check(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    }
+    HostPipe* hp;
+    int rc = pipe_get(ctx, &hp);
+    if (rc) return rc;
+    if ((rc = pipe_reserve(ctx, hp, 0, RING_PIECE))) return rc;
+    rc = hip_check(ctx, hipEventRecord(ctx->ev[0], ctx->stream), "hipEventRecord");
+    if (!rc) rc = hip_check(ctx, hipStreamWaitEvent(hp->s_out, ctx->ev[0], 0), "hipStreamWaitEvent");
+    const size_t pieces = (bytes + RING_PIECE - 1) / RING_PIECE;
+    constexpr size_t LAG = HostPipe::SLOTS;
+    for (size_t p = 0; p < pieces + LAG && !rc; ++p) {
+        if (p >= LAG) {  // piece p - LAG is copied out before its slot is used again
+            const size_t r = p - LAG, at = r * RING_PIECE;
+            if (r >= pieces) break;
+            if ((rc = hip_check(ctx, hipEventSynchronize(hp->ev_out[r % LAG]), "hipEventSynchronize(staging out)"))) break;
+            parallel_copy(static_cast<char*>(dst) + at, hp->pin_out[r % LAG], std::min(RING_PIECE, bytes - at));
+        }
+        if (p < pieces) {
+            const size_t at = p * RING_PIECE, s = p % LAG;
+            if ((rc = hip_check(ctx, hipMemcpyAsync(hp->pin_out[s], static_cast<const char*>(src) + at, std::min(RING_PIECE, bytes - at), hipMemcpyDeviceToHost, hp->s_out), "D2H piece"))) break;
+            if ((rc = hip_check(ctx, hipEventRecord(hp->ev_out[s], hp->s_out), "hipEventRecord"))) break;
+            hp->used_out[s] = true;
+        }
+    }
+    if (rc) (void)hipStreamSynchronize(hp->s_out);
+    return rc;
+}
+
 static int check_run_args(Amm* amm, const void* a, const void* b, uint32_t n)
 {
     if (!amm) return PIMDL_ERR_INVALID;
@@ -489,6 +552,7 @@ int pimdl_init(int device, pimdl_ctx** out)
     ctx->d_acc = nullptr; ctx->acc_bytes = 0;
     ctx->d_idx16 = nullptr; ctx->idx16_bytes = 0;
     ctx->d_tmp = nullptr; ctx->tmp_bytes = 0;
+    ctx->d_lutgen = nullptr; ctx->lutgen_bytes = 0;
     ctx->d_cent = nullptr; ctx->cent_bytes = 0;
     ctx->d_static_scratch = nullptr;
     ctx->pipe = nullptr;
@@ -525,6 +589,7 @@ int pimdl_destroy(pimdl_ctx* ctx)
     (void)hipFree(ctx->d_acc);
     (void)hipFree(ctx->d_idx16);
     (void)hipFree(ctx->d_tmp);
+    (void)hipFree(ctx->d_lutgen);
     (void)hipFree(ctx->d_cent);
     for (void* p : ctx->retired) (void)hipFree(p);
     for (auto& ev : ctx->ev)
@@ -1211,32 +1276,45 @@ int pimdl_lutgen_mode(pimdl_ctx* ctx, const float* centroids, const float* weigh
     if (CB > 65535) return set_error(ctx, PIMDL_ERR_UNSUPPORTED, "pimdl_lutgen: more than 65535 codebooks");
     int rc = activate(ctx);
     if (rc) return rc;
+    const bool ordered = mode == PIMDL_LUTGEN_ORDERED, i8 = lut_dtype == PIMDL_LUT_I8;
     const size_t cent_bytes = (size_t)CB * C * v * 4, w_bytes = (size_t)CB * v * M * 4, lut_elems = (size_t)CB * C * M;
-    const uint32_t ngroups = scale_group ? (CB + scale_group - 1) / scale_group : 1;
-    float *d_cent = nullptr, *d_w = nullptr, *d_lut = nullptr, *d_scales = nullptr;
-    int8_t* d_q = nullptr;
-    rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&d_cent), cent_bytes), "hipMalloc(lutgen centroids)");
-    if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&d_w), w_bytes), "hipMalloc(lutgen weight)");
-    if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&d_lut), lut_elems * 4), "hipMalloc(lutgen lut)");
-    if (!rc) rc = hip_check(ctx, hipMemcpyAsync(d_cent, centroids, cent_bytes, hipMemcpyHostToDevice, ctx->stream), "H2D centroids");
-    if (!rc) rc = hip_check(ctx, hipMemcpyAsync(d_w, weight, w_bytes, hipMemcpyHostToDevice, ctx->stream), "H2D weight");
-    if (!rc) rc = launch_lutgen_f32(ctx, d_cent, d_w, d_lut, CB, C, v, M, mode == PIMDL_LUTGEN_ORDERED);
-    if (!rc && lut_dtype == PIMDL_LUT_F32) {
-        rc = hip_check(ctx, hipMemcpyAsync(lut_out, d_lut, lut_elems * 4, hipMemcpyDeviceToHost, ctx->stream), "D2H lut");
-    } else if (!rc) {
-        rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&d_q), lut_elems), "hipMalloc(lutgen q)");
-        if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&d_scales), sizeof(float) * ngroups), "hipMalloc(lutgen scales)");
-        if (!rc) rc = launch_lut_quant(ctx, d_lut, d_q, d_scales, CB, C, M, scale_group);
-        if (!rc) rc = hip_check(ctx, hipMemcpyAsync(lut_out, d_q, lut_elems, hipMemcpyDeviceToHost, ctx->stream), "D2H lut");
+    const uint32_t ngroups = scale_group ? (CB + scale_group - 1) / scale_group : 1, parts = lutgen_parts(C, M, ordered);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) (void)hipGetLastError();
+    if (cap != hipStreamCaptureStatusNone) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_lutgen: the stream is being captured; the call copies from and to host memory");
+    // One block of device memory for the call: centroids, weight, fp32 table, magnitudes, int8 table, scales.  Up to 256 MiB
+    // the context keeps it (an allocation and a release cost as much as the kernels); larger ones are given back.
+    auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+    const size_t o_w = up(cent_bytes), o_lut = o_w + up(w_bytes), o_part = o_lut + up(lut_elems * 4),
+                 o_q = o_part + up((size_t)CB * parts * 4), o_scales = o_q + (i8 ? up(lut_elems) : 0), need = o_scales + up((size_t)ngroups * 4);
+    const bool kept = need <= (256u << 20);
+    char* dev = ctx->d_lutgen;
+    if (!kept || ctx->lutgen_bytes < need) {
+        if (kept) {  // (calls are synchronous: nothing uses the smaller one any more)
+            (void)hipFree(ctx->d_lutgen);
+            ctx->d_lutgen = nullptr;
+            ctx->lutgen_bytes = 0;
+        }
+        if ((rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&dev), need), "hipMalloc(lutgen)"))) return rc;
+        if (kept) {
+            ctx->d_lutgen = dev;
+            ctx->lutgen_bytes = need;
+        }
+    }
+    float *d_cent = reinterpret_cast<float*>(dev), *d_w = reinterpret_cast<float*>(dev + o_w), *d_lut = reinterpret_cast<float*>(dev + o_lut),
+          *d_part = reinterpret_cast<float*>(dev + o_part), *d_scales = reinterpret_cast<float*>(dev + o_scales);
+    int8_t* d_q = reinterpret_cast<int8_t*>(dev + o_q);
+    rc = hip_check(ctx, hipMemcpyAsync(d_cent, centroids, cent_bytes, hipMemcpyHostToDevice, ctx->stream), "H2D centroids");
+    if (!rc) rc = ring_to_device(ctx, d_w, weight, w_bytes);
+    if (!rc) rc = launch_lutgen_f32(ctx, d_cent, d_w, d_lut, d_part, CB, C, v, M, ordered);
+    if (!rc && i8) {
+        rc = launch_lut_quant(ctx, d_lut, d_part, parts, d_q, d_scales, CB, C, M, scale_group);
         if (!rc) rc = hip_check(ctx, hipMemcpyAsync(scales_out, d_scales, sizeof(float) * ngroups, hipMemcpyDeviceToHost, ctx->stream), "D2H scales");
     }
+    if (!rc) rc = ring_to_host(ctx, lut_out, i8 ? static_cast<void*>(d_q) : d_lut, lut_elems * (i8 ? 1 : 4));
     if (!rc) rc = hip_check(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     else (void)hipStreamSynchronize(ctx->stream);
-    (void)hipFree(d_cent);
-    (void)hipFree(d_w);
-    (void)hipFree(d_lut);
-    (void)hipFree(d_q);
-    (void)hipFree(d_scales);
+    if (!kept) (void)hipFree(dev);
     return rc;
 }
 

@@ -137,6 +137,8 @@ struct Ctx {
     size_t idx16_bytes;
     float* d_tmp;        // row-major output before re-tiling
     size_t tmp_bytes;
+    char* d_lutgen;      // device memory of pimdl_lutgen calls (at most 256 MiB)
+    size_t lutgen_bytes;
     float* d_cent;       // centroids of a context-level pimdl_index_calculation call
     size_t cent_bytes;
     hipEvent_t ev[4];
@@ -167,10 +169,12 @@ int launch_pack_idx(Ctx* ctx, const AmmGeom& g, const uint16_t* d_idx16, uint8_t
                     uint32_t n_stile, uint32_t cb_mtile);
 int launch_retile_output(Ctx* ctx, const float* d_rowmajor, float* d_tiled, uint32_t n, uint32_t M,
                          uint32_t n_stile, uint32_t f_stile, uint32_t f_mtile);
-int launch_lutgen_f32(Ctx* ctx, const float* d_cent, const float* d_w, float* d_lut, uint32_t CB,
-                      uint32_t C, uint32_t v, uint32_t M, bool ordered = false);
-int launch_lut_quant(Ctx* ctx, const float* d_lut, int8_t* d_q, float* d_scales, uint32_t CB, uint32_t C,
-                     uint32_t M, uint32_t scale_group);
+// part: [CB][lutgen_parts()] floats, the largest magnitude that each workgroup wrote
+uint32_t lutgen_parts(uint32_t C, uint32_t M, bool ordered);
+int launch_lutgen_f32(Ctx* ctx, const float* d_cent, const float* d_w, float* d_lut, float* d_part, uint32_t CB,
+                      uint32_t C, uint32_t v, uint32_t M, bool ordered);
+int launch_lut_quant(Ctx* ctx, const float* d_lut, const float* d_part, uint32_t parts, int8_t* d_q, float* d_scales,
+                     uint32_t CB, uint32_t C, uint32_t M, uint32_t scale_group);
 int launch_layer_norm(Ctx* ctx, const float* d_x, const float* d_w, const float* d_b, const float* d_residual,
                       float* d_out, uint32_t n, uint32_t d, float eps);
 int launch_attention_hd64(Ctx* ctx, const float* d_q, const float* d_k, const float* d_v, float* d_out, uint32_t batch,

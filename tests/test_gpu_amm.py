@@ -725,3 +725,27 @@ def test_float_tables_in_pieces(ctx, N, CB, v, C, M, group):
     assert np.array_equal(out[rows].view(np.uint32), want.view(np.uint32))
     assert "_f32_rows_" in amm.last_gather_kernel(), amm.last_gather_kernel()
     amm.close()
+
+
+@pytest.mark.parametrize("CB,v,C,M,group", [(48, 4, 16, 1001, 0), (7, 3, 17, 333, 2), (96, 4, 16, 1024, 1), (3, 8, 5, 6, 0), (64, 4, 64, 1537, 5)])
+@pytest.mark.parametrize("ordered", [False, True])
+def test_lutgen_quantisation_of_any_group(ctx, CB, v, C, M, group, ordered):
+    """The int8 table and the scales are those of the fp32 table of the same call form to the bit: magnitudes per workgroup,
+    entries four at a time and one by one (group boundaries that are no multiple of four), pieces through the pinned
+    ring and small buffers, an all-zero group."""
+    rng = np.random.default_rng(CB + M)
+    cent = rng.standard_normal((CB, C, v)).astype(np.float32)
+    weight = (rng.standard_normal((CB * v, M)) * 0.02).astype(np.float32)
+    cbs = group or CB
+    if group:
+        cent[cbs:2 * cbs] = 0.0
+    full, _ = ctx.lutgen(cent, weight, lut_dtype=pimdl.LUT_F32, ordered=ordered)
+    if ordered:
+        assert np.array_equal(full.view(np.uint32), oracle.lutgen_f32(cent, weight, threads=THREADS).view(np.uint32))
+    table, scales = ctx.lutgen(cent, weight, scale_group=group, ordered=ordered)
+    for g in range((CB + cbs - 1) // cbs):
+        part = full[g * cbs:(g + 1) * cbs]
+        s = np.abs(part).max() / np.float32(127)
+        s = s if s > 0 else np.float32(1)
+        assert scales[g] == s
+        assert np.array_equal(table[g * cbs:(g + 1) * cbs], np.rint(np.clip(part / s, -128, 127)).astype(np.int8))
