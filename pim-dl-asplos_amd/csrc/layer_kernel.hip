@@ -15,11 +15,47 @@ namespace pimdl {
 
 namespace {
 
+// The value of lane ^ OFF (for OFF < 8: of a lane that holds the same value, given that the steps above were done before,
+// which leave values that repeat every 2 * OFF lanes), without the LDS crossbar's round trip: half-wave and row swaps, then
+// rotations within a row of 16 and a quad.
+template <int OFF>
+__device__ __forceinline__ void xor_pair(uint32_t v, uint32_t& a, uint32_t& b)
+{
+    if constexpr (OFF >= 16) {  // a: the lower halves (rows) in both places, b: the upper ones
+        auto r = [&] {
+            if constexpr (OFF == 32) return __builtin_amdgcn_permlane32_swap(v, v, false, false);
+            else return __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        }();
+        a = r[0];
+        b = r[1];
+    } else {
+        constexpr int ctrl = OFF == 8 ? 0x128 : OFF == 4 ? 0x124 : OFF == 2 ? 0x4E : 0xB1;  // row_ror:8, row_ror:4, quad_perm
+        a = v;
+        b = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
+    }
+}
+
+template <int OFF>
+__device__ __forceinline__ double add_pair(double v)
+{
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    uint32_t alo, blo, ahi, bhi;
+    xor_pair<OFF>((uint32_t)u, alo, blo);
+    xor_pair<OFF>((uint32_t)(u >> 32), ahi, bhi);
+    return __longlong_as_double((long long)((uint64_t)ahi << 32 | alo)) + __longlong_as_double((long long)((uint64_t)bhi << 32 | blo));
+}
+
+// Butterfly over the 64 lanes, 32 lanes apart first: the same additions, and so the same bits, as with __shfl_xor, whose
+// twelve trips through the LDS crossbar per sum stood in the wave's only chain (us in a layer: d = 768, n = 4096
+// 8.1 -> 7.65, with the registers of a row cut to its 768 columns; d = 1024, n = 8192 17.5 -> 16.8).
 __device__ __forceinline__ double wave_sum(double v)
 {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off);
-    return v;
+    v = add_pair<32>(v);
+    v = add_pair<16>(v);
+    v = add_pair<8>(v);
+    v = add_pair<4>(v);
+    v = add_pair<2>(v);
+    return add_pair<1>(v);
 }
 
 // one wave per row
@@ -307,7 +343,10 @@ int launch_layer_norm(Ctx* ctx, const float* d_x, const float* d_w, const float*
                           reinterpret_cast<uintptr_t>(d_b) | reinterpret_cast<uintptr_t>(d_residual) |
                           reinterpret_cast<uintptr_t>(d_out);
     if (d % 4 == 0 && (all & 15) == 0 && d <= 64 * 4 * 8) {
-        if (d <= 64 * 4 * 4)
+        if (d <= 64 * 4 * 3)
+            hipLaunchKernelGGL(layer_norm_vec_kernel<3>, dim3((n + 3) / 4), dim3(256), 0, ctx->stream, d_x, d_w, d_b,
+                               d_residual, d_out, n, d, eps);
+        else if (d <= 64 * 4 * 4)
             hipLaunchKernelGGL(layer_norm_vec_kernel<4>, dim3((n + 3) / 4), dim3(256), 0, ctx->stream, d_x, d_w, d_b,
                                d_residual, d_out, n, d, eps);
         else

@@ -58,6 +58,36 @@ def test_layer_norm_matches_the_reference_statement(ctx, n, d):
     assert np.array_equal(ctx.layer_norm(c, w, b), np.broadcast_to(b, (2, d)))
 
 
+@pytest.mark.parametrize("d", [4, 70, 252, 256, 764, 768, 772, 1024, 1028, 2048, 2052])
+def test_layer_norm_is_a_64_lane_butterfly_to_the_bit(ctx, d):
+    """Lane by lane in ascending order, four columns at a time where the row allows it, then over the lanes, 32 apart first."""
+    rng = np.random.default_rng(d)
+    n = 67
+    x = (rng.standard_normal((n, d)) * np.exp(rng.uniform(-8, 8, (n, 1)))).astype(np.float32)
+    w, b = rng.standard_normal((2, d)).astype(np.float32)
+    r = rng.standard_normal((n, d)).astype(np.float32)
+    width = 4 if d % 4 == 0 and d <= 2048 else 1
+    cols = -(-d // (64 * width)) * 64 * width
+
+    def lane_sum(values):
+        full = np.zeros((n, cols))
+        full[:, :d] = values
+        per_lane = full.reshape(n, -1, 64, width).transpose(0, 2, 1, 3).reshape(n, 64, -1)
+        s = np.zeros((n, 64))
+        for i in range(per_lane.shape[2]):
+            s = s + per_lane[:, :, i]
+        for off in (32, 16, 8, 4, 2, 1):
+            s = s + s[:, np.arange(64) ^ off]
+        return s[:, :1]
+
+    centred = x - (lane_sum(x) / d).astype(np.float32)
+    variance = (lane_sum(centred * centred) / d).astype(np.float32)
+    scale = np.float32(1) / np.sqrt(variance + np.float32(1e-6))
+    want = centred * scale * w + b
+    assert np.array_equal(ctx.layer_norm(x, w, b), want)
+    assert np.array_equal(ctx.layer_norm(x, w, b, residual=r), r + want)
+
+
 def gelu_tanh64(f):
     f = f.astype(np.float64)
     return 0.5 * f * (1 + np.tanh(math.sqrt(2 / math.pi) * (f + 0.044715 * f ** 3)))
