@@ -301,6 +301,7 @@ static int run_piped(Ctx* ctx, uint32_t K, uint32_t M, const float* in, bool in_
     if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) (void)hipGetLastError();
     if (cap != hipStreamCaptureStatusNone)
         return set_error(ctx, PIMDL_ERR_INVALID, "host buffers cannot be staged while the stream is being captured: pass device pointers");
+    std::lock_guard<std::mutex> lock(ctx->host_mutex);
     HostPipe* hp;
     int rc = pipe_get(ctx, &hp);
     if (rc) return rc;
@@ -383,8 +384,8 @@ static int ring_to_device(Ctx* ctx, void* dst, const void* src, size_t bytes)
     if (rc) return rc;
     rc = pipe_reserve(ctx, hp, RING_PIECE, 0);
     // the destination is free once what the context's stream has queued is done
-    if (!rc) rc = hip_check(ctx, hipEventRecord(ctx->ev[0], ctx->stream), "hipEventRecord");
-    if (!rc) rc = hip_check(ctx, hipStreamWaitEvent(hp->s_in, ctx->ev[0], 0), "hipStreamWaitEvent");
+    if (!rc) rc = hip_check(ctx, hipEventRecord(ctx->ev[2], ctx->stream), "hipEventRecord");
+    if (!rc) rc = hip_check(ctx, hipStreamWaitEvent(hp->s_in, ctx->ev[2], 0), "hipStreamWaitEvent");
     int s = 0;
     for (size_t at = 0; at < bytes && !rc; at += RING_PIECE, s = (s + 1) % HostPipe::SLOTS) {
         const size_t len = std::min(RING_PIECE, bytes - at);
@@ -409,8 +410,8 @@ static int ring_to_host(Ctx* ctx, void* dst, const void* src, size_t bytes)
     int rc = pipe_get(ctx, &hp);
     if (rc) return rc;
     if ((rc = pipe_reserve(ctx, hp, 0, RING_PIECE))) return rc;
-    rc = hip_check(ctx, hipEventRecord(ctx->ev[0], ctx->stream), "hipEventRecord");
-    if (!rc) rc = hip_check(ctx, hipStreamWaitEvent(hp->s_out, ctx->ev[0], 0), "hipStreamWaitEvent");
+    rc = hip_check(ctx, hipEventRecord(ctx->ev[2], ctx->stream), "hipEventRecord");
+    if (!rc) rc = hip_check(ctx, hipStreamWaitEvent(hp->s_out, ctx->ev[2], 0), "hipStreamWaitEvent");
     const size_t pieces = (bytes + RING_PIECE - 1) / RING_PIECE;
     constexpr size_t LAG = HostPipe::SLOTS;
     for (size_t p = 0; p < pieces + LAG && !rc; ++p) {
@@ -1288,6 +1289,7 @@ int pimdl_lutgen_mode(pimdl_ctx* ctx, const float* centroids, const float* weigh
     const size_t o_w = up(cent_bytes), o_lut = o_w + up(w_bytes), o_part = o_lut + up(lut_elems * 4),
                  o_q = o_part + up((size_t)CB * parts * 4), o_scales = o_q + (i8 ? up(lut_elems) : 0), need = o_scales + up((size_t)ngroups * 4);
     const bool kept = need <= (256u << 20);
+    std::lock_guard<std::mutex> lock(ctx->host_mutex);
     char* dev = ctx->d_lutgen;
     if (!kept || ctx->lutgen_bytes < need) {
         if (kept) {  // (calls are synchronous: nothing uses the smaller one any more)

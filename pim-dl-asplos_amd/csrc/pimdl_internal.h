@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -143,6 +144,7 @@ struct Ctx {
     size_t cent_bytes;
     hipEvent_t ev[4];
     HostPipe* pipe;      // created by the first call that hands over a host buffer
+    std::mutex host_mutex;  // held by a call while it uses `pipe` or d_lutgen: table construction may run beside another thread's calls
 };
 
 int set_error(Ctx* ctx, int code, const char* fmt, ...);

@@ -123,3 +123,38 @@ def test_fp32_lut_export(ctx):
     want = oracle.lutgen_f32(t["encoder.layer.0.intermediate.dense.centroids.weight"].reshape(4, 8, 4),
                              t["encoder.layer.0.intermediate.dense.weight"])
     np.testing.assert_allclose(lut.reshape(4, 8, 64), want, rtol=1e-5, atol=1e-7)
+
+
+def test_lutgen_beside_other_threads_of_one_context(ctx):
+    """Table construction in two threads while a third runs an operator on host buffers: each result is that of a lone call."""
+    import threading
+    rng = np.random.default_rng(77)
+    jobs = []
+    for CB, C, v, M in [(96, 16, 4, 2048), (64, 16, 8, 1537)]:
+        cent = rng.standard_normal((CB, C, v)).astype(np.float32)
+        weight = (rng.standard_normal((CB * v, M)) * 0.02).astype(np.float32)
+        jobs.append((cent, weight, *ctx.lutgen(cent, weight)))
+    cent, _, table, scales = jobs[0]
+    amm = ctx.amm(cent, table, scales[0], np.zeros(2048, np.float32), max_n=1500)
+    x = rng.standard_normal((1500, 384)).astype(np.float32)
+    out = amm.run(x).copy()
+    wrong = []
+
+    def construct(cent, weight, table, scales):
+        for _ in range(6):
+            got, s = ctx.lutgen(cent, weight)
+            if not (np.array_equal(got, table) and np.array_equal(s, scales)):
+                wrong.append("table")
+
+    def gather():
+        for _ in range(6):
+            if not np.array_equal(amm.run(x), out):
+                wrong.append("output")
+
+    threads = [threading.Thread(target=construct, args=j) for j in jobs] + [threading.Thread(target=gather)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not wrong and not any(t.is_alive() for t in threads)
+    amm.close()
