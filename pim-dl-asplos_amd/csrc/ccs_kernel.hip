@@ -1544,6 +1544,9 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
 // A lane per token (ccs_kernel) leaves all but N lanes of a wave idle and goes through the centroids one after the
 // other: 14.7 us at one token, 192 codebooks, 64 centroids, where this takes 3 and the matrix search 7.  Bound by the launch and one round trip
 // at a few tokens, by the vector ALU (3 v R operations and a reduction over the wave per pair) from about 50 on.
+// Waves are dealt over the real codebooks; a codebook's waves also write the zeros of its share of the padding.  (Dealt over the
+// padded codebooks, most waves did nothing else: one codebook, v = 2, 256 centroids, N = 5000 11.5 us, N = 20000 50, N = 50000 103;
+// now 3, 6.2 and, on the matrix search, 8.0.)
 template <int V, int R>  // R: centroids per lane
 __global__ __launch_bounds__(CCS_THREADS) void ccs_few_kernel(const float* __restrict__ x, const float* __restrict__ cent,
                                                               uint8_t* __restrict__ idx, uint32_t N, uint32_t K, uint32_t CB,
@@ -1552,12 +1555,13 @@ __global__ __launch_bounds__(CCS_THREADS) void ccs_few_kernel(const float* __res
 {
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t w = __builtin_amdgcn_readfirstlane(blockIdx.x * (CCS_THREADS / 64) + (threadIdx.x >> 6));
-    const uint32_t cb = w % CB_pad, tok0 = w / CB_pad * tokens_per_wave;
+    const uint32_t cb = w % CB, tok0 = w / CB * tokens_per_wave;
+    if (tok0 >= N) return;  // whole wave, past the last chunk of tokens
     const uint32_t tok1 = tok0 + tokens_per_wave < N ? tok0 + tokens_per_wave : N;
-    if (cb >= CB) {  // padding: index 0
-        for (uint32_t tok = tok0 + lane; tok < tok1; tok += 64) idx[idx_offset(tok, cb, idx_row_bytes, idx_tiled)] = 0;
-        return;
-    }
+    // padding codebooks CB + cb, 2 CB + cb, ...: index 0 (a byte per lane)
+    const uint32_t pads = (CB_pad - cb - 1) / CB;
+    for (uint32_t e = lane; e < pads * (tok1 - tok0); e += 64)
+        idx[idx_offset(tok0 + e / pads, CB + cb + e % pads * CB, idx_row_bytes, idx_tiled)] = 0;
     float c[R][V];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -1800,11 +1804,10 @@ int launch_ccs_few(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_
 {
     constexpr uint32_t WAVES = CCS_THREADS / 64;
     // up to eight waves per SIMD, then more tokens per wave (the centroids are loaded once for them)
-    const uint64_t waves = 32ull * ctx->prop.multiProcessorCount, pairs = (uint64_t)n * g.CB_pad;
+    const uint64_t waves = 32ull * ctx->prop.multiProcessorCount, pairs = (uint64_t)n * g.CB;
     const uint32_t per = (uint32_t)((pairs + waves - 1) / waves), chunks = (n + per - 1) / per;
     auto kern = g.C <= 64 ? ccs_few_kernel<V, 1> : g.C <= 128 ? ccs_few_kernel<V, 2> : ccs_few_kernel<V, 4>;
-    // (CB_pad is a multiple of the waves of a workgroup)
-    hipLaunchKernelGGL(kern, dim3(chunks * (g.CB_pad / WAVES)), dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent, d_idx, n, g.K, g.CB,
+    hipLaunchKernelGGL(kern, dim3((chunks * g.CB + WAVES - 1) / WAVES), dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent, d_idx, n, g.K, g.CB,
                        g.CB_pad, g.C, g.idx_row_bytes, (int)g.idx_tiled, per);
     return hip_check(ctx, hipGetLastError(), "ccs_few_kernel launch");
 }
@@ -1848,10 +1851,13 @@ int launch_ccs_bits(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     // centroids of every codebook of a wave, until it has filled the chip (us, pair / matrix: v = 4, 64 centroids, 192
     // codebooks N = 1 3.1 / 7.3, N = 128 4.6 / 8.0, N = 512 11.8 / 8.0; 256 centroids, 256 codebooks N = 128 7.1 / 19.8,
     // N = 512 24.7 / 20.0; v = 16, 64 centroids, 64 codebooks N = 512 6.4 / 7.4, N = 2048 16.4 / 7.5; v = 32, 64 centroids,
-    // 40 codebooks N = 37 4.8 / 6.9, N = 128 9.3 / 6.9).
-    const double groups = (double)((g.C + 31) / 32) * (g.v >= 16 ? 1 : 16 / g.v);
+    // 40 codebooks N = 37 4.8 / 6.9, N = 128 9.3 / 6.9).  With fewer codebooks than a wave of the matrix search takes that
+    // wave has less to do (v = 2, 256 centroids, one codebook N = 1000 2.5 / 6.7, N = 50000 10.6 / 8.1; v = 4, 64 centroids, one
+    // codebook N = 5000 3.1 / 3.7, N = 20000 5.0 / 4.4; v = 8, 128 centroids, two codebooks N = 20000 8.3 / 13.4).
+    const uint32_t wave_cbs = g.v >= 16 ? 1 : 16 / g.v, real_cbs = g.CB < wave_cbs ? g.CB : wave_cbs;
+    const double groups = (double)((g.C + 31) / 32) * real_cbs;
     if (IDX_BITS == 8 && g.C > 32 && !g.tune_search && !exact && !f32 &&
-        (double)n * g.CB * (g.v == 32 ? 1.9e-3 : 0.12e-3) < 1.8 + 0.42 * groups) {
+        (double)n * g.CB * (g.v == 32 ? 1.9e-3 : 0.12e-3) < 0.6 + 1.2 * real_cbs / wave_cbs + 0.42 * groups) {
         switch (g.v) {
             case 2: return launch_ccs_few<2>(ctx, g, d_x, d_cent, d_idx, n);
             case 4: return launch_ccs_few<4>(ctx, g, d_x, d_cent, d_idx, n);

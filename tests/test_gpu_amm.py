@@ -749,3 +749,40 @@ def test_lutgen_quantisation_of_any_group(ctx, CB, v, C, M, group, ordered):
         s = s if s > 0 else np.float32(1)
         assert scales[g] == s
         assert np.array_equal(table[g * cbs:(g + 1) * cbs], np.rint(np.clip(part / s, -128, 127)).astype(np.int8))
+
+
+@pytest.mark.parametrize("N,CB,v,C,lut", [(9000, 1, 2, 256, "f32"), (5000, 2, 8, 100, "f32"), (700, 31, 4, 65, "i8"), (900, 33, 2, 130, "f32"),
+                                          (300, 33, 16, 64, "i8"), (8200, 1, 4, 200, "i8"), (3, 70, 2, 40, "f32")])
+def test_search_of_few_pairs_writes_the_padding_too(ctx, N, CB, v, C, lut):
+    """A wave per (token, codebook) pair, several tokens per wave: the indices are the oracle's, and those of the padded codebooks are
+    zero (a float table would add whatever lies behind its rows)."""
+    x, cent, table, bias = make_case(8800 + N + CB, N, CB * v, v, C, 20, lut)
+    amm = ctx.amm(cent, table, None if lut == "f32" else np.float32(0.01), bias, max_n=N)
+    other = ctx.amm(cent[::-1], table, None if lut == "f32" else np.float32(0.01), bias, max_n=N)
+    other.run_debug(x + np.float32(1), want_acc=False)   # leaves other indices in the context's scratch
+    out, idx, _ = amm.run_debug(x, want_acc=False)
+    want_idx = oracle.index_calculation(x, cent, v, threads=THREADS)
+    assert np.array_equal(idx, want_idx)
+    want = (oracle.gather_f32(want_idx, table, bias, threads=THREADS) if lut == "f32"
+            else oracle.dequant(oracle.gather_i8(want_idx, table, threads=THREADS), bias, CB, 0.01, 0.0, 0, threads=THREADS))
+    assert np.array_equal(out.view(np.uint32), want.view(np.uint32))
+    amm.close()
+    other.close()
+
+
+@pytest.mark.parametrize("v,C", [(2, 64), (2, 256), (8, 128)])
+def test_search_of_one_codebook_takes_no_longer_than_that_of_eight(ctx, v, C):
+    """The search's launch rule prices what its waves do: a codebook among 31 padded ones is one codebook."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    import torch
+    for N in (20000, 50000):
+        us = []
+        for CB in (1, 8):
+            _, cent, table, bias = make_case(CB, 1, CB * v, v, C, 16)
+            amm = ctx.amm(cent, table, np.float32(0.01), bias, max_n=N)
+            x, y = torch.randn(N, CB * v, device="cuda"), torch.empty(N, 16, device="cuda")
+            torch.cuda.synchronize()
+            us.append(min(amm.profile(x.data_ptr(), N, y.data_ptr(), warmup=5, iters=20)["ccs_ms"] for _ in range(5)) * 1e3)
+            amm.close()
+        assert us[0] < 1.2 * us[1] + 1, (N, us)
