@@ -771,9 +771,8 @@ bool gather_dense_only()
 
 bool apply_runtime_tuning(AmmGeom* g, const pimdl_amm_tuning& t, std::string* why)
 {
-    // (auto_rows: the settings of the sparse kernel are accepted where the library would have been free to take it)
-    const bool matrix_core = g->gather_kind != 0 || g->auto_rows;
-    const bool sparse = g->gather_kind == 2 || g->auto_rows;
+    const bool matrix_core = g->gather_kind != 0;
+    const bool sparse = g->gather_kind == 2;
     const bool eight_waves = t.token_item == 512 && sparse && g->C_tile != 32;  // one workgroup of eight waves per CU
     if (t.token_item && (!matrix_core || (t.token_item != 128 && t.token_item != 256 && !eight_waves))) {
         *why = "token_item must be 128 or 256 (512 for the sparse kernel up to 16 centroids), and only the matrix-core gathers (int8, up to 32 centroids) have it";

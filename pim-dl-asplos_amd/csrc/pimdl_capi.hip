@@ -484,6 +484,17 @@ static void retile_lut_rows(const int8_t* lut, int8_t* tiled, const AmmGeom& g)
                 }
 }
 
+// ... and back
+static void untile_lut_rows(const int8_t* tiled, int8_t* lut, const AmmGeom& g)
+{
+    const size_t slice = (size_t)g.C_tile * 256, chunk = (g.CB_pad / 16) * slice;  // bytes
+    for (uint32_t f = 0; f < g.M; f += 16)
+        for (uint32_t cb = 0; cb < g.CB; ++cb)
+            for (uint32_t c = 0; c < g.C; ++c)
+                memcpy(lut + ((size_t)cb * g.C + c) * g.M + f, tiled + f / 16 * chunk + cb / 16 * slice + (size_t)c * 256 + cb % 16 * 16,
+                       f + 16 <= g.M ? 16 : g.M - f);
+}
+
 // canonical [CB][C][M] -> [M_pad/col_block][CB_pad][col_block][16], zero padded (C <= 16);
 // C_tile 8 (C <= 8): [M_pad/col_block][CB_pad/2][col_block][2][8], codebooks 2k and 2k+1 side by side
 static void retile_lut_onehot(const int8_t* lut, int8_t* tiled, const AmmGeom& g)
@@ -526,6 +537,70 @@ struct pimdl_amm_group {
     bool has_merged;
     Amm merged;
 };
+
+static uint32_t kernel_of(const AmmGeom& g)
+{
+    return g.gather_kind == 0 ? PIMDL_GATHER_ROWS : g.gather_kind == 1 ? PIMDL_GATHER_ONEHOT : PIMDL_GATHER_SPARSE;
+}
+
+static size_t table_bytes(const Amm& a, const AmmGeom& g)
+{
+    return (size_t)g.M_pad * g.CB_pad * g.C_tile * (a.desc.lut_dtype == PIMDL_LUT_I8 && !a.grouped ? 1 : 4);
+}
+
+// An operator's geometry with gather kernel `kind`.  Only one that the library gave to the byte adder by its own choice
+// (auto_rows) has a second one, the sparse kernel's.
+static int geometry_as(const Amm* a, uint32_t kind, AmmGeom* g)
+{
+    *g = a->g;
+    if (a->g.gather_kind == kind) return PIMDL_OK;
+    if (!a->g.auto_rows) return set_error(a->ctx, PIMDL_ERR_INVALID, "the operator's table has one layout");
+    pimdl_amm_tuning t;
+    memset(&t, 0, sizeof(t));
+    if (kind != 0) t.gather_kernel = PIMDL_GATHER_SPARSE;
+    std::string why;
+    memset(g, 0, sizeof(*g));
+    if (!plan_geometry(a->desc, a->ctx->prop.multiProcessorCount, g, &why, &t)) return set_error(a->ctx, PIMDL_ERR_INVALID, "%s", why.c_str());
+    g->auto_rows = 1;
+    return PIMDL_OK;
+}
+
+// The operator's table as geometry_as(kind) = g has it.  The second one is laid out from the first when it is first asked for and
+// kept until the operator is destroyed: graphs captured before hold the other's address.
+static int table_as(Amm* a, const AmmGeom& g, void** table)
+{
+    Ctx* ctx = a->ctx;
+    *table = a->g.gather_kind == g.gather_kind ? a->d_lut : a->d_lut_other;
+    if (*table) return PIMDL_OK;
+    // (what the operator has is the byte adder's, which it was created with)
+    int rc = activate(ctx);
+    if (rc) return rc;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) (void)hipGetLastError();
+    if (cap != hipStreamCaptureStatusNone)
+        return set_error(ctx, PIMDL_ERR_INVALID, "the stream is being captured, and the table has to be laid out for another gather kernel: "
+                                                 "name its settings once outside the capture first");
+    const size_t bytes = table_bytes(*a, g);
+    std::vector<int8_t> have, canonical, want;
+    try {
+        have.resize(a->lut_bytes);
+        canonical.resize((size_t)g.CB * g.C * g.M);
+        want.assign(bytes, 0);
+        if ((rc = hip_check(ctx, hipMemcpy(have.data(), a->d_lut, a->lut_bytes, hipMemcpyDeviceToHost), "D2H lut"))) return rc;
+        untile_lut_rows(have.data(), canonical.data(), a->g);
+        retile_lut_onehot(canonical.data(), want.data(), g);
+    } catch (...) {
+        return set_error(ctx, PIMDL_ERR_NOMEM, "host staging of a table of %zu bytes failed", bytes);
+    }
+    void* fresh = nullptr;
+    if ((rc = hip_check(ctx, hipMalloc(&fresh, bytes), "hipMalloc(lut)"))) return rc;
+    if ((rc = hip_check(ctx, hipMemcpy(fresh, want.data(), bytes, hipMemcpyHostToDevice), "H2D lut"))) {
+        (void)hipFree(fresh);
+        return rc;
+    }
+    *table = a->d_lut_other = fresh;
+    return PIMDL_OK;
+}
 
 extern "C" {
 
@@ -640,15 +715,24 @@ int pimdl_amm_set_tuning(pimdl_amm* a, const pimdl_amm_tuning* t)
     if (!a) return PIMDL_ERR_INVALID;
     Ctx* ctx = a->ctx;
     if (!t) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_set_tuning: null argument");
-    const uint32_t kind = a->g.gather_kind == 0 ? PIMDL_GATHER_ROWS : a->g.gather_kind == 1 ? PIMDL_GATHER_ONEHOT : PIMDL_GATHER_SPARSE;
-    if ((t->col_block && t->col_block != a->g.col_block) ||
-        (t->gather_kernel && t->gather_kernel != kind && !(a->g.auto_rows && t->gather_kernel == PIMDL_GATHER_SPARSE)))
+    AmmGeom g = a->g;
+    if (g.auto_rows) {
+        // the choice that pimdl_amm_create_with makes of these settings
+        const bool rows = t->gather_kernel == PIMDL_GATHER_ROWS ||
+                          (t->gather_kernel == PIMDL_GATHER_AUTO && !t->token_item && !t->cb_per_slice && !t->xcd_col_split &&
+                           (!t->col_block || (g.gather_kind == 0 && t->col_block == g.col_block)));
+        if (int rc = geometry_as(a, rows ? 0 : 2, &g)) return rc;
+    }
+    if ((t->col_block && t->col_block != g.col_block) || (t->gather_kernel && t->gather_kernel != kernel_of(g)))
         return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_set_tuning: col_block and gather_kernel fix the resident table; "
                                                  "create the operator with them (pimdl_amm_create_with)");
     std::string why;
-    AmmGeom g = a->g;
     if (!apply_runtime_tuning(&g, *t, &why)) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_set_tuning: %s", why.c_str());
+    void* table;
+    if (int rc = table_as(a, g, &table)) return rc;
+    if (table != a->d_lut) std::swap(a->d_lut, a->d_lut_other);
     a->g = g;
+    a->lut_bytes = table_bytes(*a, g);
     return PIMDL_OK;
 }
 
@@ -656,7 +740,7 @@ int pimdl_amm_get_tuning(const pimdl_amm* a, pimdl_amm_tuning* t)
 {
     if (!a || !t) return PIMDL_ERR_INVALID;
     t->col_block = a->g.col_block;
-    t->gather_kernel = a->g.gather_kind == 0 ? PIMDL_GATHER_ROWS : a->g.gather_kind == 1 ? PIMDL_GATHER_ONEHOT : PIMDL_GATHER_SPARSE;
+    t->gather_kernel = kernel_of(a->g);
     t->token_item = a->g.tune_token_item;
     t->cb_per_slice = a->g.tune_cb_per_slice;
     t->xcd_col_split = a->g.tune_xcd_col_split;
@@ -696,6 +780,7 @@ int pimdl_amm_create_with(pimdl_ctx* ctx, const pimdl_amm_desc* desc, const floa
     a->g = g;
     a->d_centroids = nullptr;
     a->d_lut = nullptr;
+    a->d_lut_other = nullptr;
     a->d_scales = nullptr;
     a->d_bias = nullptr;
     a->grouped = grouped;
@@ -707,9 +792,8 @@ int pimdl_amm_create_with(pimdl_ctx* ctx, const pimdl_amm_desc* desc, const floa
     a->h_scale0 = i8 ? scales[0] : 1.0f;
 
     const size_t cent_bytes = (size_t)g.CB * g.C * g.v * sizeof(float);
-    const size_t elem = i8 ? 1 : 4;
     const uint32_t row_elems = g.col_block;
-    a->lut_bytes = (size_t)g.M_pad * g.CB_pad * g.C_tile * elem;
+    a->lut_bytes = table_bytes(*a, g);
     std::vector<unsigned char> tiled;
     try {
         tiled.assign(a->lut_bytes, 0);
@@ -808,6 +892,7 @@ int pimdl_amm_destroy(pimdl_amm* a)
     (void)hipStreamSynchronize(a->ctx->stream);
     (void)hipFree(a->d_centroids);
     (void)hipFree(a->d_lut);
+    (void)hipFree(a->d_lut_other);
     (void)hipFree(a->d_scales);
     (void)hipFree(a->d_bias);
     delete a;
@@ -877,6 +962,7 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
         m.d_centroids = nullptr;
         m.d_scales = nullptr;
         m.d_lut = nullptr;
+        m.d_lut_other = nullptr;
         m.d_bias = nullptr;
         m.d_op_scales = nullptr;
         m.g.M = m.g.M_pad = first->g.M * count;

@@ -37,7 +37,8 @@ struct AmmGeom {
                             // 2: one-hot on the sparse matrix instruction (int8, C <= 32: a codebook of 17..32
                             //    centroids is two of 16 side by side; table laid out as for 1, with the columns
                             //    of a tile permuted by sparse_tile_column)
-    uint32_t auto_rows;     // 17..32 centroids, kind 0 by the library's own choice (the caller named no gather setting)
+    uint32_t auto_rows;     // 17..32 centroids, created with no gather setting: kind 0 by the library's choice, until a tuning names
+                            // a setting of the sparse kernel
     uint32_t q;             // 16-byte chunks per LUT row in LDS
     uint32_t col_block;     // columns per workgroup (int8: 16*q -- the byte adder picks its own at launch --, fp32: 4*q)
     uint32_t row_pitch;     // bytes between LUT rows in LDS
@@ -77,6 +78,7 @@ struct Amm {
     float* d_centroids;  // [CB][C][v], then the derived search data (ccs_centroid_bytes)
     void* d_lut;         // tiled
     size_t lut_bytes;
+    void* d_lut_other;   // auto_rows: the table as the kernel that is not in use reads it, once it has been needed (else null)
     float* d_scales;     // int8: scales
     uint32_t nscales;
     float* d_bias;       // [M]

@@ -786,3 +786,86 @@ def test_search_of_one_codebook_takes_no_longer_than_that_of_eight(ctx, v, C):
             us.append(min(amm.profile(x.data_ptr(), N, y.data_ptr(), warmup=5, iters=20)["ccs_ms"] for _ in range(5)) * 1e3)
             amm.close()
         assert us[0] < 1.2 * us[1] + 1, (N, us)
+
+
+def test_tuning_of_an_operator_the_library_gave_to_the_byte_adder(ctx):
+    """17..32 centroids, created without settings: a setting of the sparse kernel takes effect (as it does at creation), what
+    get_tuning reports is accepted by set_tuning and by the creation of another operator, no settings lead back to the byte adder."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    N, CB, v, C, M = 700, 41, 4, 27, 200
+    x, cent, lut, bias = make_case(61, N, CB * v, v, C, M)
+    amm = ctx.amm(cent, lut, np.float32(0.01), bias, max_n=N)
+    want = oracle.amm_cpu(x, cent, lut, bias, v, 0.01, 0.0, threads=THREADS)[0]
+
+    def run(op):
+        assert np.array_equal(op.run(x).view(np.uint32), want.view(np.uint32))
+        return op.last_gather_kernel()
+
+    assert run(amm).startswith("gather_i8_kernel") and amm.tuning()["gather_kernel"] == pimdl.GATHER_ROWS
+    untuned = amm.tuning()
+    for setting in ({"token_item": 128}, {"token_item": 256}, {"cb_per_slice": 16}, {"gather_kernel": pimdl.GATHER_SPARSE},
+                    {"token_item": 128, "xcd_col_split": 2, "search_kernel": 1}, {}, {"xcd_col_split": pimdl.XCD_PLAIN}, {"search_kernel": 3}):
+        amm.set_tuning(**setting)
+        sparse = any(k != "search_kernel" for k in setting)
+        kernel, tuned = run(amm), amm.tuning()
+        assert kernel.startswith("gather_sparse_kernel" if sparse else "gather_i8_kernel"), (setting, kernel)
+        assert tuned["gather_kernel"] == (pimdl.GATHER_SPARSE if sparse else pimdl.GATHER_ROWS)
+        assert all(tuned[k] == val for k, val in setting.items())
+        if "token_item" in setting:
+            assert amm.geometry()["tokens_per_wg"] == setting["token_item"]
+        same = ctx.amm(cent, lut, np.float32(0.01), bias, max_n=N, tuning=tuned)
+        assert same.tuning() == tuned and run(same) == kernel
+        same.close()
+        amm.set_tuning(**tuned)
+        assert amm.tuning() == tuned and run(amm) == kernel
+    for bad in ({"token_item": 100}, {"token_item": 512}, {"cb_per_slice": 64}, {"gather_kernel": pimdl.GATHER_ONEHOT},
+                {"gather_kernel": pimdl.GATHER_ROWS, "token_item": 128}, {"gather_kernel": pimdl.GATHER_SPARSE, "col_block": 80}):
+        before = amm.tuning()
+        with pytest.raises(pimdl.PimdlError) as e:
+            amm.set_tuning(**bad)
+        assert e.value.code == pimdl.ERR_INVALID and amm.tuning() == before, bad
+    amm.set_tuning()
+    assert amm.tuning() == untuned
+    amm.set_tuning(token_item=128)
+    amm.run(x[:1])   # one token: the setting is the sparse kernel's
+    assert amm.last_gather_kernel().startswith("gather_sparse_kernel")
+    amm.set_tuning()
+    amm.run(x[:1])
+    assert "_few_" in amm.last_gather_kernel()
+    amm.close()
+
+
+def test_a_graph_captured_before_a_change_of_tables_replays(ctx):
+    """A captured run holds the address of the table it was captured with."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    import torch
+    N, CB, v, C, M = 600, 32, 4, 32, 192
+    x, cent, lut, bias = make_case(62, N, CB * v, v, C, M)
+    local = pimdl.Context(0)
+    amm = local.amm(cent, lut, np.float32(0.01), bias, max_n=N)
+    stream = torch.cuda.Stream()
+    xd, out, eager = torch.from_numpy(x).cuda(), torch.empty(N, M, device="cuda"), torch.empty(N, M, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        local.set_stream(stream.cuda_stream)
+        amm.run_ptr(xd.data_ptr(), N, out.data_ptr())
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+            amm.run_ptr(xd.data_ptr(), N, out.data_ptr())
+            with pytest.raises(pimdl.PimdlError):   # the other table cannot be laid out here
+                amm.set_tuning(token_item=128)
+        want = oracle.amm_cpu(x, cent, lut, bias, v, 0.01, 0.0, threads=THREADS)[0]
+        for setting in ({"token_item": 128}, {}, {"token_item": 256}, {}):
+            amm.set_tuning(**setting)
+            eager.zero_()
+            out.zero_()
+            amm.run_ptr(xd.data_ptr(), N, eager.data_ptr())
+            graph.replay()
+            stream.synchronize()
+            assert np.array_equal(eager.cpu().numpy(), want) and np.array_equal(out.cpu().numpy(), want), setting
+    local.set_stream(None)
+    amm.close()
+    local.close()
