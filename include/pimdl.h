@@ -236,8 +236,8 @@ PIMDL_API int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uin
                                      pimdl_amm_group** out);
 PIMDL_API int pimdl_amm_group_run(pimdl_amm_group* group, const float* in, uint32_t n, float* const* outs);
 PIMDL_API int pimdl_amm_group_destroy(pimdl_amm_group* group);
-/* When the members are int8 operators of one shape served by the matrix-core gather (up to 16
- * centroids, output_feature_len a multiple of the column tile, same LUT bias and activation), the
+/* When the members are int8 operators of one shape with up to 32 centroids on one gather kernel (not a byte
+ * adder the caller asked for; output_feature_len a multiple of the column tile, same LUT bias and activation), the
  * group can also run ONE gather launch over all of them and write one buffer
  *   out fp32 [n][count * M], operator i in columns i*M .. (i+1)*M - 1
  * (the layout of the reference's fused qkv output, src/host/transformer_layer.cpp:301), each column

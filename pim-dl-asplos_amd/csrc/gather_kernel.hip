@@ -935,7 +935,9 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
         if (ct < 16) ct = 16;
         g->C_tile = ct;
         g->idx_tiled = 1;
-        g->q = hinted ? col_block_hint / 16 : ct <= 64 ? 4 : ct == 128 ? 2 : 1;
+        // (auto_rows: the width that divides M if one does, which is what operators side by side in one launch need)
+        g->q = hinted ? col_block_hint / 16 : g->auto_rows && M % 64 != 0 && M % 48 == 0 ? 3 : ct <= 64 ? 4 : ct == 128 ? 2 : 1;
+        g->cols = hinted ? col_block_hint : 0;
         g->gq = 4;
         g->cb_per_slice = 16;
         g->col_block = 16 * g->q;

@@ -339,7 +339,8 @@ int launch_gather_rows(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_ou
     ep.op_col_tiles = a.op_col_tiles;
     ep.op_idx_stride = a.op_idx_stride;
     const RowsLaunch l{ctx, a, d_idx, d_out, d_acc, n, ep};
-    if (a.g.q == 3) {  // 48-column tiles, on request
+    // 48-column tiles: on request, and for operators side by side that tiles of two and four chunks do not divide
+    if (a.g.cols == 48 || (ep.op_col_tiles * a.g.q) % 2 != 0) {
         switch (a.g.C_tile) {
             case 16: return launch_rows<16, 4, RowsShape<3, 8, 4>, RowsShape<3, 8, 2>, RowsShape<3, 8, 1>>(l);
             case 32: return launch_rows<32, 8, RowsShape<3, 8, 4>, RowsShape<3, 8, 2>, RowsShape<3, 8, 1>>(l);

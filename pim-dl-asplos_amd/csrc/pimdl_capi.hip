@@ -945,20 +945,34 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
                                            hipMemcpyDeviceToDevice, ctx->stream), "D2D centroids");
     if (!rc) rc = launch_ccs_prep(ctx, g, grp->d_centroids);
     if (!rc) rc = ensure(ctx, &ctx->d_idx, &ctx->idx_bytes, idx_buffer_bytes(g, max_n), "hipMalloc(index scratch)");
-    // one gather launch for all members?
-    bool same = first->desc.lut_dtype == PIMDL_LUT_I8 && !first->grouped && (first->g.gather_kind != 0 || first->g.auto_rows) &&
-                first->g.M % first->g.col_block == 0;
+    // One gather launch for all members?  The kernel is the one that every member has a table for: that of the members with a single
+    // one, the byte adder for auto_rows members of which one runs on it.
+    uint32_t kind = first->g.gather_kind;
+    bool every_auto = true;
+    for (uint32_t i = 0; i < count; ++i) {
+        if (every_auto) kind = amms[i]->g.gather_kind && kind ? kind : 0;
+        if (!amms[i]->g.auto_rows) {
+            every_auto = false;
+            kind = amms[i]->g.gather_kind;
+        }
+    }
+    AmmGeom mg[16];  // the members' geometries with that kernel
+    void* mtab[16];  // ... and tables
+    bool same = first->desc.lut_dtype == PIMDL_LUT_I8 && !first->grouped && (kind != 0 || every_auto) &&
+                geometry_as(first, kind, &mg[0]) == PIMDL_OK && mg[0].M % mg[0].col_block == 0;
     const float lbt0 = first->desc.bias_mode == PIMDL_BIAS_TIMES_CB ? first->desc.lut_bias * (float)first->g.CB : first->desc.lut_bias;
     for (uint32_t i = 1; i < count && same; ++i) {
         const Amm* a = amms[i];
         const float lbt = a->desc.bias_mode == PIMDL_BIAS_TIMES_CB ? a->desc.lut_bias * (float)a->g.CB : a->desc.lut_bias;
-        same = a->desc.lut_dtype == PIMDL_LUT_I8 && !a->grouped && a->g.gather_kind == first->g.gather_kind && a->g.auto_rows == first->g.auto_rows && a->g.M == first->g.M &&
-               a->g.q == first->g.q && a->g.C_tile == first->g.C_tile && a->g.CB_pad == first->g.CB_pad &&
-               a->lut_bytes == first->lut_bytes && a->desc.activation == first->desc.activation && lbt == lbt0;
+        same = a->desc.lut_dtype == PIMDL_LUT_I8 && !a->grouped && geometry_as(a, kind, &mg[i]) == PIMDL_OK && mg[i].M == mg[0].M &&
+               mg[i].q == mg[0].q && mg[i].C_tile == mg[0].C_tile && mg[i].CB_pad == mg[0].CB_pad &&
+               a->desc.activation == first->desc.activation && lbt == lbt0;
     }
+    for (uint32_t i = 0; i < count && same && !rc; ++i) rc = table_as(amms[i], mg[i], &mtab[i]);
     if (!rc && same) {
         Amm& m = grp->merged;
-        m = *first;  // geometry, epilogue constants; the pointers below are the group's own
+        m = *first;  // epilogue constants; geometry and pointers below are the group's own
+        m.g = mg[0];
         m.d_centroids = nullptr;
         m.d_scales = nullptr;
         m.d_lut = nullptr;
@@ -969,17 +983,18 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
         m.desc.output_feature_len = m.g.M;
         m.desc.max_n = max_n;
         m.g.idx_row_bytes = g.idx_row_bytes;
-        m.op_col_tiles = first->g.M / first->g.col_block;
+        m.op_col_tiles = mg[0].M / mg[0].col_block;
         m.op_idx_stride = first->g.idx_row_bytes * 64;  // tiled index rows: a byte range is a range of 256-byte blocks
-        m.lut_bytes = first->lut_bytes * count;
+        const size_t one_table = table_bytes(*first, mg[0]);
+        m.lut_bytes = one_table * count;
         std::vector<float> sc(count);
         for (uint32_t i = 0; i < count; ++i) sc[i] = amms[i]->h_scale0;
         rc = hip_check(ctx, hipMalloc(&m.d_lut, m.lut_bytes), "hipMalloc(group lut)");
         if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&m.d_bias), (size_t)m.g.M * sizeof(float)), "hipMalloc(group bias)");
         if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&m.d_op_scales), count * sizeof(float)), "hipMalloc(group scales)");
         for (uint32_t i = 0; i < count && !rc; ++i) {
-            rc = hip_check(ctx, hipMemcpyAsync(static_cast<char*>(m.d_lut) + (size_t)i * first->lut_bytes, amms[i]->d_lut,
-                                               first->lut_bytes, hipMemcpyDeviceToDevice, ctx->stream), "D2D lut");
+            rc = hip_check(ctx, hipMemcpyAsync(static_cast<char*>(m.d_lut) + (size_t)i * one_table, mtab[i],
+                                               one_table, hipMemcpyDeviceToDevice, ctx->stream), "D2D lut");
             if (!rc) rc = hip_check(ctx, hipMemcpyAsync(m.d_bias + (size_t)i * first->g.M, amms[i]->d_bias,
                                                         (size_t)first->g.M * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream), "D2D bias");
         }

@@ -869,3 +869,38 @@ def test_a_graph_captured_before_a_change_of_tables_replays(ctx):
     local.set_stream(None)
     amm.close()
     local.close()
+
+
+@pytest.mark.parametrize("M", [48, 96, 720, 1056, 64, 320])
+@pytest.mark.parametrize("settings", [({}, {}, {}), ({}, {"token_item": 128}, {}), ({"token_item": 128}, {"token_item": 128}, {}),
+                                      ({"gather_kernel": pimdl.GATHER_SPARSE}, {}, {"token_item": 256}), ({"token_item": 256},) * 3])
+def test_operators_side_by_side_of_17_to_32_centroids(ctx, M, settings):
+    """One gather launch over operators whose widths are multiples of 48 or 64, whichever kernel each of them runs on: a few
+    tokens and many, every column bit for bit that of the operator alone."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    N, CB, v, C = 2100, 32, 4, 20
+    x = make_case(70, N, CB * v, v, C, M)[0]
+    amms = []
+    for i, setting in enumerate(settings):
+        _, cent, lut, bias = make_case(71 + i, 1, CB * v, v, C, M)
+        created = {k: val for k, val in setting.items() if k == "gather_kernel"}
+        if created:
+            created["col_block"] = 48 if M % 64 else 64
+        amms.append(ctx.amm(cent, lut, np.float32(0.01 * (i + 1)), bias, max_n=N, tuning=created))
+        if not created:
+            amms[i].set_tuning(**setting)
+    group = ctx.amm_group(amms)
+    one_table = not any("gather_kernel" in s for s in settings) and not all(settings)
+    if one_table:   # the byte adder's, whose columns are dealt out sixteen at a time
+        assert group.fused_cols == 3 * M
+    elif all(s == settings[0] for s in settings):
+        assert (group.fused_cols > 0) == (M % amms[0].geometry()["col_block"] == 0)
+    for n in (N, 40):
+        want = np.concatenate([a.run(x[:n]) for a in amms], axis=1)
+        assert np.array_equal(np.concatenate(group.run(x[:n]), axis=1).view(np.uint32), want.view(np.uint32))
+        if group.fused_cols:
+            assert np.array_equal(group.run_fused(x[:n]).view(np.uint32), want.view(np.uint32))
+    group.close()
+    for a in amms:
+        a.close()
