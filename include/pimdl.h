@@ -229,7 +229,7 @@ PIMDL_API int pimdl_amm_run_debug(pimdl_amm* amm, const float* in, uint32_t n, f
  * in ONE launch (the input is read once and the launch's fixed cost is paid once), then runs each
  * operator's gather; results are bit for bit those of pimdl_amm_run on each operator.
  *   Conditions: same context, input_feature_len, sub_vec_len (2, 4 or 8) and num_centroid (<= 32), the same
- *   LUT type, num_codebook a multiple of 32; otherwise PIMDL_ERR_UNSUPPORTED / PIMDL_ERR_INVALID and the
+ *   LUT type (int8 operators created with PIMDL_GATHER_ROWS also go with fp32 ones), num_codebook a multiple of 32; otherwise PIMDL_ERR_UNSUPPORTED / PIMDL_ERR_INVALID and the
  *   caller runs the operators one by one.  The group borrows its operators: destroy it before them.
  *   outs[i]: fp32 [n][M_i] of operator i, host or device; n <= the smallest max_n. */
 PIMDL_API int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t count,

@@ -2135,6 +2135,25 @@ int launch_pack_idx(Ctx* ctx, const AmmGeom& g, const uint16_t* d_idx16, uint8_t
 }
 
 namespace {
+// index rows [N][row_words] -> [N/64][row_words][64 tokens] (idx_offset); words of tokens past N stay as they are
+__global__ void tile_idx_kernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, uint32_t N, uint32_t row_words)
+{
+    const uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (gid >= (uint64_t)N * row_words) return;
+    const uint32_t n = gid / row_words, w = gid % row_words;
+    out[((size_t)(n >> 6) * row_words + w) * 64 + (n & 63)] = in[gid];
+}
+}  // namespace
+
+int launch_tile_idx(Ctx* ctx, const uint8_t* d_rows, uint8_t* d_tiled, uint32_t n, uint32_t row_bytes)
+{
+    const uint64_t total = (uint64_t)n * (row_bytes / 4);
+    hipLaunchKernelGGL(tile_idx_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, ctx->stream,
+                       reinterpret_cast<const uint32_t*>(d_rows), reinterpret_cast<uint32_t*>(d_tiled), n, row_bytes / 4);
+    return hip_check(ctx, hipGetLastError(), "tile_idx_kernel launch");
+}
+
+namespace {
 // row-major [N][M] -> the order the reference's DPUs hand the output back in (test_amm.cpp:193-202)
 __global__ void retile_output_kernel(const float* __restrict__ in, float* __restrict__ out, uint32_t N, uint32_t M,
                                      uint32_t n_stile, uint32_t f_stile, uint32_t f_mtile)

@@ -531,6 +531,9 @@ struct pimdl_amm_group {
     float* d_centroids;   // the members' centroids, concatenated, + derived search data
     uint32_t x_cols;      // floats per input row (one member's K)
     uint32_t max_n;
+    // Byte-adder members (as the caller asked for) beside tables resident as floats: the search writes index rows, which the
+    // floats' gathers read, and a copy in the tiled layout is made for the byte adder.
+    bool both_layouts;
     // Members that are matrix-core gathers of one shape also run as ONE gather launch over their column
     // tiles side by side, into one [n][members * M] output (pimdl_amm_group_run_fused): `merged` borrows the
     // members' geometry and owns concatenated copies of their tables, biases and scales.
@@ -600,6 +603,14 @@ static int table_as(Amm* a, const AmmGeom& g, void** table)
     }
     *table = a->d_lut_other = fresh;
     return PIMDL_OK;
+}
+
+// index scratch of a group's call: one layout, or both one behind the other
+static size_t group_idx_bytes(const pimdl_amm_group& grp, uint32_t n)
+{
+    AmmGeom tiled = grp.g;
+    tiled.idx_tiled = 1;
+    return idx_buffer_bytes(grp.g, n) + (grp.both_layouts ? idx_buffer_bytes(tiled, n) : 0);
 }
 
 extern "C" {
@@ -910,14 +921,17 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
     const Amm* first = amms[0];
     if (!first) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_group_create: null operator");
     uint32_t max_n = first->desc.max_n;
+    bool both_layouts = false;
+    auto by_rows = [](const Amm* a) { return !a->g.idx_tiled || (a->g.gather_kind == 0 && !a->g.auto_rows); };
     for (uint32_t i = 0; i < count; ++i) {
         const Amm* a = amms[i];
         if (!a) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_group_create: null operator");
         if (a->ctx != ctx) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_group_create: operator %u belongs to another context", i);
         if (a->g.K != first->g.K || a->g.v != first->g.v || a->g.C != first->g.C)
             return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_group_create: operator %u differs in input_feature_len, sub_vec_len or num_centroid", i);
-        if (a->g.idx_tiled != first->g.idx_tiled || a->g.idx_bits != first->g.idx_bits)
+        if (by_rows(a) != by_rows(first) || a->g.idx_bits != first->g.idx_bits)
             return set_error(ctx, PIMDL_ERR_UNSUPPORTED, "pimdl_amm_group_create: operator %u uses another index layout (LUT type differs)", i);
+        both_layouts |= a->g.idx_tiled != first->g.idx_tiled;
         max_n = a->desc.max_n < max_n ? a->desc.max_n : max_n;
     }
     if (first->g.CB != first->g.CB_pad)
@@ -927,6 +941,7 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
     g.CB *= count;
     g.CB_pad *= count;
     g.idx_row_bytes *= count;
+    if (both_layouts) g.idx_tiled = 0;
     if (!ccs_supports_shared_input(g, first->g.K))
         return set_error(ctx, PIMDL_ERR_UNSUPPORTED, "pimdl_amm_group_create: no shared-input search for sub_vec_len=%u, num_centroid=%u, input_feature_len=%u",
                          g.v, g.C, first->g.K);
@@ -937,6 +952,7 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
     grp->d_centroids = nullptr;
     grp->x_cols = first->g.K;
     grp->max_n = max_n;
+    grp->both_layouts = both_layouts;
     grp->has_merged = false;
     rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&grp->d_centroids), ccs_centroid_bytes(g)), "hipMalloc(group centroids)");
     const size_t one = (size_t)first->g.CB * g.C * g.v;  // raw centroid floats of one member
@@ -944,7 +960,7 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
         rc = hip_check(ctx, hipMemcpyAsync(grp->d_centroids + i * one, amms[i]->d_centroids, one * sizeof(float),
                                            hipMemcpyDeviceToDevice, ctx->stream), "D2D centroids");
     if (!rc) rc = launch_ccs_prep(ctx, g, grp->d_centroids);
-    if (!rc) rc = ensure(ctx, &ctx->d_idx, &ctx->idx_bytes, idx_buffer_bytes(g, max_n), "hipMalloc(index scratch)");
+    if (!rc) rc = ensure(ctx, &ctx->d_idx, &ctx->idx_bytes, group_idx_bytes(*grp, max_n), "hipMalloc(index scratch)");
     // One gather launch for all members?  The kernel is the one that every member has a table for: that of the members with a single
     // one, the byte adder for auto_rows members of which one runs on it.
     uint32_t kind = first->g.gather_kind;
@@ -1063,14 +1079,16 @@ int pimdl_amm_group_run(pimdl_amm_group* grp, const float* in, uint32_t n, float
     if (rc || n == 0) return rc;
     const float* d_in;
     if ((rc = stage_input(ctx, grp->members[0]->g, in, n, &d_in))) return rc;
-    if ((rc = ensure(ctx, &ctx->d_idx, &ctx->idx_bytes, idx_buffer_bytes(grp->g, n), "hipMalloc(index scratch)"))) return rc;
+    if ((rc = ensure(ctx, &ctx->d_idx, &ctx->idx_bytes, group_idx_bytes(*grp, n), "hipMalloc(index scratch)"))) return rc;
     if ((rc = launch_ccs(ctx, grp->g, d_in, grp->d_centroids, ctx->d_idx, n, grp->x_cols))) return rc;
+    uint8_t* d_tiled = ctx->d_idx + (grp->both_layouts ? idx_buffer_bytes(grp->g, n) : 0);  // (index rows are whole 16-byte pieces)
+    if (grp->both_layouts && (rc = launch_tile_idx(ctx, ctx->d_idx, d_tiled, n, grp->g.idx_row_bytes))) return rc;
     for (size_t i = 0; i < grp->members.size(); ++i) {
         // member i's index bytes are bytes i*rb .. (i+1)*rb-1 of every row of the common buffer
         Amm view = *grp->members[i];
         const size_t rb = view.g.idx_row_bytes;
         view.g.idx_row_bytes = grp->g.idx_row_bytes;
-        const uint8_t* idx_i = ctx->d_idx + (grp->g.idx_tiled ? i * rb * 64 : i * rb);
+        const uint8_t* idx_i = view.g.idx_tiled ? d_tiled + i * rb * 64 : ctx->d_idx + i * rb;
         float* d_out;
         bool out_host;
         if ((rc = stage_output(ctx, view.g, outs[i], n, &d_out, &out_host))) return rc;

@@ -172,6 +172,8 @@ int launch_unpack_idx(Ctx* ctx, const AmmGeom& g, const uint8_t* d_idx, uint16_t
                       uint32_t n_stile, uint32_t cb_mtile);
 int launch_pack_idx(Ctx* ctx, const AmmGeom& g, const uint16_t* d_idx16, uint8_t* d_idx, uint32_t n,
                     uint32_t n_stile, uint32_t cb_mtile);
+// the same index rows in the tiled layout (idx_offset)
+int launch_tile_idx(Ctx* ctx, const uint8_t* d_rows, uint8_t* d_tiled, uint32_t n, uint32_t row_bytes);
 int launch_retile_output(Ctx* ctx, const float* d_rowmajor, float* d_tiled, uint32_t n, uint32_t M,
                          uint32_t n_stile, uint32_t f_stile, uint32_t f_mtile);
 // part: [CB][lutgen_parts()] floats, the largest magnitude that each workgroup wrote

@@ -904,3 +904,36 @@ def test_operators_side_by_side_of_17_to_32_centroids(ctx, M, settings):
     group.close()
     for a in amms:
         a.close()
+
+
+@pytest.mark.parametrize("C,v", [(16, 4), (7, 2), (32, 4)])
+@pytest.mark.parametrize("order", [("rows", "f32", "scales"), ("f32", "rows"), ("scales", "rows", "rows")])
+def test_byte_adder_and_float_tables_in_one_group(ctx, C, v, order):
+    """Operators created for the byte adder share a search with tables resident as floats, whose index rows lie differently;
+    those on the matrix-core gathers do not."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about what the caller names")
+    N, CB = 333, 64
+    x = make_case(80, N, CB * v, v, C, 1)[0]
+
+    def make(kind, i):
+        M = (96, 50, 130)[i]
+        _, cent, table, bias = make_case(81 + i, 1, CB * v, v, C, M, "f32" if kind == "f32" else "i8")
+        if kind == "scales":
+            return ctx.amm(cent, table, np.linspace(0.001, 0.02, CB, dtype=np.float32), bias, max_n=N, scale_group=1)
+        return ctx.amm(cent, table, None if kind == "f32" else np.float32(0.01), bias, max_n=N,
+                       tuning={"gather_kernel": pimdl.GATHER_ROWS} if kind == "rows" else {})
+
+    amms = [make(kind, i) for i, kind in enumerate(order)]
+    group = ctx.amm_group(amms)
+    assert group.fused_cols == 0
+    for n in (N, 1, 64, 65):
+        for a, o in zip(amms, group.run(x[:n])):
+            assert np.array_equal(o.view(np.uint32), a.run(x[:n]).view(np.uint32)), (n, a.last_gather_kernel())
+    group.close()
+    default = make("i8", 0)   # the matrix-core gather, or the byte adder by the library's own choice
+    with pytest.raises(pimdl.PimdlError) as e:
+        ctx.amm_group([amms[0], default])
+    assert e.value.code == pimdl.ERR_UNSUPPORTED
+    for a in amms + [default]:
+        a.close()
