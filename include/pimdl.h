@@ -171,7 +171,8 @@ PIMDL_API int pimdl_amm_create_with(pimdl_ctx* ctx, const pimdl_amm_desc* desc, 
                                     const pimdl_amm_tuning* tuning, pimdl_amm** out);
 /* Changes the choices that do not touch resident data (token_item, cb_per_slice, xcd_col_split,
  * search_kernel, search_token_tile) on an existing operator, so that a search need not upload the table once per candidate;
- * col_block and gather_kernel must be 0 or what the operator was created with.  An int8 operator of 17..32 centroids
+ * col_block and gather_kernel must be 0 or what the operator was created with (col_block of a byte adder of up to 64
+ * centroids that was created without one: also 48 or 64, 0 = the launch picks).  An int8 operator of 17..32 centroids
  * created without any of the gather's settings runs on the byte adder until settings of the sparse kernel are named here
  * (gather_kernel, its token_item, cb_per_slice, xcd_col_split or col_block), and again when none is: the choice
  * pimdl_amm_create_with makes.  The first such change lays out a second table, which cannot happen while the context's

@@ -937,11 +937,12 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
         g->idx_tiled = 1;
         // (auto_rows: the width that divides M if one does, which is what operators side by side in one launch need)
         g->q = hinted ? col_block_hint / 16 : g->auto_rows && M % 64 != 0 && M % 48 == 0 ? 3 : ct <= 64 ? 4 : ct == 128 ? 2 : 1;
-        g->cols = hinted ? col_block_hint : 0;
+        g->cols = hinted || (ct == 16 && (col_block_hint == 48 || col_block_hint == 64)) ? col_block_hint : 0;  // (C <= 8: not fixed by it)
+        g->cols_named = hinted;
         g->gq = 4;
         g->cb_per_slice = 16;
         g->col_block = 16 * g->q;
-        g->gather_threads = ct <= 32 ? 512 : 1024;
+        g->gather_threads = ct <= 128 ? 512 : 1024;
         g->tokens_per_wg = g->gather_threads;
     } else {
         g->gq = 0;

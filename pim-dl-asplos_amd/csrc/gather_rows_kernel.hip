@@ -339,12 +339,18 @@ int launch_gather_rows(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_ou
     ep.op_col_tiles = a.op_col_tiles;
     ep.op_idx_stride = a.op_idx_stride;
     const RowsLaunch l{ctx, a, d_idx, d_out, d_acc, n, ep};
-    // 48-column tiles: on request, and for operators side by side that tiles of two and four chunks do not divide
+    // A width that the caller has named, and 48 columns for operators side by side that tiles of two and four chunks do not
+    // divide; the launch's own choice below.
     if (a.g.cols == 48 || (ep.op_col_tiles * a.g.q) % 2 != 0) {
         switch (a.g.C_tile) {
             case 16: return launch_rows<16, 4, RowsShape<3, 8, 4>, RowsShape<3, 8, 2>, RowsShape<3, 8, 1>>(l);
             case 32: return launch_rows<32, 8, RowsShape<3, 8, 4>, RowsShape<3, 8, 2>, RowsShape<3, 8, 1>>(l);
             case 64: return launch_rows<64, 8, RowsShape<3, 16, 4>, RowsShape<3, 16, 2>, RowsShape<3, 16, 1>>(l);
+        }
+    } else if (a.g.cols == 64 && a.g.C_tile >= 32) {
+        switch (a.g.C_tile) {
+            case 32: return launch_rows<32, 8, RowsShape<4, 8, 4>, RowsShape<4, 8, 2>, RowsShape<4, 8, 1>>(l);
+            case 64: return launch_rows<64, 8, RowsShape<4, 16, 4>, RowsShape<4, 16, 2>, RowsShape<4, 16, 1>>(l);
         }
     } else {
         switch (a.g.C_tile) {

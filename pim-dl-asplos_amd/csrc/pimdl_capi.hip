@@ -734,7 +734,13 @@ int pimdl_amm_set_tuning(pimdl_amm* a, const pimdl_amm_tuning* t)
                            (!t->col_block || (g.gather_kind == 0 && t->col_block == g.col_block)));
         if (int rc = geometry_as(a, rows ? 0 : 2, &g)) return rc;
     }
-    if ((t->col_block && t->col_block != g.col_block) || (t->gather_kernel && t->gather_kernel != kernel_of(g)))
+    bool width_ok = !t->col_block || t->col_block == g.col_block;
+    if (g.gather_kind == 0 && g.idx_tiled && !g.cols_named) {
+        // byte adder: the table does not depend on the width of an item (128 centroids and more: one width was offered, 32)
+        width_ok |= g.C_tile <= 64 ? t->col_block == 48 || t->col_block == 64 : t->col_block == 32;
+        if (width_ok && g.C_tile <= 64) g.cols = t->col_block;
+    }
+    if (!width_ok || (t->gather_kernel && t->gather_kernel != kernel_of(g)))
         return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_set_tuning: col_block and gather_kernel fix the resident table; "
                                                  "create the operator with them (pimdl_amm_create_with)");
     std::string why;
@@ -750,7 +756,7 @@ int pimdl_amm_set_tuning(pimdl_amm* a, const pimdl_amm_tuning* t)
 int pimdl_amm_get_tuning(const pimdl_amm* a, pimdl_amm_tuning* t)
 {
     if (!a || !t) return PIMDL_ERR_INVALID;
-    t->col_block = a->g.col_block;
+    t->col_block = a->g.gather_kind == 0 ? a->g.cols : a->g.col_block;
     t->gather_kernel = kernel_of(a->g);
     t->token_item = a->g.tune_token_item;
     t->cb_per_slice = a->g.tune_cb_per_slice;
@@ -1468,7 +1474,7 @@ int pimdl_amm_get_geometry(const pimdl_amm* a, pimdl_amm_geometry* out)
     out->num_codebook_padded = g.CB_pad;
     out->idx_bits = g.idx_bits;
     out->idx_row_bytes = g.idx_row_bytes;
-    out->col_block = g.col_block;
+    out->col_block = g.cols ? g.cols : g.col_block;
     out->row_pitch = g.row_pitch;
     // the gather launcher picks among instances of its kernel by the batch it is given: report the last launch's
     // shape once there has been one, the plan's defaults before

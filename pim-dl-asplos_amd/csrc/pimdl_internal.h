@@ -40,8 +40,9 @@ struct AmmGeom {
     uint32_t auto_rows;     // 17..32 centroids, created with no gather setting: kind 0 by the library's choice, until a tuning names
                             // a setting of the sparse kernel
     uint32_t q;             // 16-byte chunks per LUT row in LDS
-    uint32_t col_block;     // columns per workgroup (int8: 16*q -- the byte adder picks its own at launch --, fp32: 4*q)
-    uint32_t cols;          // byte adder: columns per item that the caller has named (0: the launch picks)
+    uint32_t col_block;     // columns per workgroup (int8: 16*q -- the byte adder picks its own at launch, see cols --, fp32: 4*q)
+    uint32_t cols;          // byte adder of up to 64 centroids: columns per item that the caller has named (0: the launch picks)
+    uint32_t cols_named;    // ... at creation
     uint32_t row_pitch;     // bytes between LUT rows in LDS
     uint32_t gq;            // int8: codebooks per lane group per slice
     uint32_t cb_per_slice;

@@ -937,3 +937,63 @@ def test_byte_adder_and_float_tables_in_one_group(ctx, C, v, order):
     assert e.value.code == pimdl.ERR_UNSUPPORTED
     for a in amms + [default]:
         a.close()
+
+
+@pytest.mark.parametrize("C", [8, 16, 20, 64])
+@pytest.mark.parametrize("N,CB,M", [(1500, 33, 200), (200, 40, 1030), (9000, 16, 130)])
+def test_column_width_of_the_byte_adder(ctx, C, N, CB, M):
+    """A width that the caller names is the width of the launch's items, at creation and on the operator; without one the launch
+    picks, get_tuning says so, and an operator created with what it says launches the same."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about what the caller names")
+    v = 2
+    x, cent, lut, bias = make_case(90 + C, N, CB * v, v, C, M)
+    want = oracle.amm_cpu(x, cent, lut, bias, v, 0.01, 0.0, threads=THREADS)[0]
+    make = lambda **t: ctx.amm(cent, lut, np.float32(0.01), bias, max_n=N, tuning=t)
+
+    def kernel(op):
+        assert np.array_equal(op.run_debug(x)[0].view(np.uint32), want.view(np.uint32))
+        name = op.last_gather_kernel()
+        assert name.startswith("gather_i8_kernel<"), name
+        return name
+
+    rows = {"gather_kernel": pimdl.GATHER_ROWS}
+    free = make(**rows)
+    picked = kernel(free)
+    assert free.tuning()["col_block"] == 0
+    again = make(**free.tuning())
+    assert kernel(again) == picked and again.tuning() == free.tuning()
+    for width in (48, 64):
+        hinted = make(**rows, col_block=width)
+        assert kernel(hinted).split(", ")[1] == str(width // 16)
+        assert hinted.tuning()["col_block"] == hinted.geometry()["col_block"] == width
+        if C > 8:   # (up to 8 centroids the width given at creation is not binding)
+            with pytest.raises(pimdl.PimdlError):
+                hinted.set_tuning(col_block=112 - width)
+            hinted.set_tuning()
+            assert kernel(hinted).split(", ")[1] == str(width // 16)
+        free.set_tuning(col_block=width)
+        assert kernel(free) == kernel(hinted) and free.tuning() == hinted.tuning()
+        hinted.close()
+    free.set_tuning()
+    assert kernel(free) == picked
+    with pytest.raises(pimdl.PimdlError):
+        free.set_tuning(col_block=96)
+    free.close()
+    again.close()
+
+
+@pytest.mark.parametrize("C", [100, 200])
+def test_wide_tables_have_one_column_width(ctx, C):
+    x, cent, lut, bias = make_case(95, 300, 64, 4, C, 50)
+    amm = ctx.amm(cent, lut, np.float32(0.01), bias, max_n=300)
+    want = amm.run(x)
+    for t in ({"col_block": 32}, amm.tuning(), {}):
+        amm.set_tuning(**t)
+        assert np.array_equal(amm.run(x), want)
+    again = ctx.amm(cent, lut, np.float32(0.01), bias, max_n=300, tuning=amm.tuning())
+    assert np.array_equal(again.run(x), want) and again.tuning() == amm.tuning()
+    with pytest.raises(pimdl.PimdlError):
+        amm.set_tuning(col_block=64)
+    amm.close()
+    again.close()
