@@ -208,8 +208,8 @@ PIMDL_API int pimdl_amm_run(pimdl_amm* amm, const float* in, uint32_t n, float* 
  * the library runs on holds its copy until the process ends) instead of the context's grow-only scratch.
  *   in_dev, out_dev  DEVICE pointers, fp32 [n][K] and [n][M]; queued on the context's stream, returns at once.
  *   PIMDL_ERR_INVALID when a pointer is a host pointer, or when n tokens need more index bytes than the array
- *   holds: n rounded up to 64, times num_codebook rounded up to 32, times 1/2 byte (up to 16 centroids) or
- *   1 byte (more).  BERT-base's 3072 -> 768 matrix at n = 8192 needs 3 MiB.
+ *   holds: n rounded up to 64 (int8 tables of up to 32 centroids; else n), times num_codebook rounded up to 32,
+ *   times 1/2 byte (up to 16 centroids) or 1 byte (more).  BERT-base's 3072 -> 768 matrix at n = 8192 needs 3 MiB.
  * Output bits are those of pimdl_amm_run.  Every call on one GPU, from any context or thread, shares that
  * GPU's array: calls that overlap in time on one GPU race (calls queued on one stream do not overlap). */
 #define PIMDL_NOALLOC_SCRATCH_BYTES (8u << 20)

@@ -546,6 +546,10 @@ static uint32_t kernel_of(const AmmGeom& g)
     return g.gather_kind == 0 ? PIMDL_GATHER_ROWS : g.gather_kind == 1 ? PIMDL_GATHER_ONEHOT : PIMDL_GATHER_SPARSE;
 }
 
+// Index rows, or the byte adder's tiled words where no other kernel could have been the library's choice: such operators share
+// searches with each other, and a token counts for its own index bytes only.
+static bool by_rows(const Amm* a) { return !a->g.idx_tiled || (a->g.gather_kind == 0 && !a->g.auto_rows); }
+
 static size_t table_bytes(const Amm& a, const AmmGeom& g)
 {
     return (size_t)g.M_pad * g.CB_pad * g.C_tile * (a.desc.lut_dtype == PIMDL_LUT_I8 && !a.grouped ? 1 : 4);
@@ -928,7 +932,6 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
     if (!first) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_group_create: null operator");
     uint32_t max_n = first->desc.max_n;
     bool both_layouts = false;
-    auto by_rows = [](const Amm* a) { return !a->g.idx_tiled || (a->g.gather_kind == 0 && !a->g.auto_rows); };
     for (uint32_t i = 0; i < count; ++i) {
         const Amm* a = amms[i];
         if (!a) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_group_create: null operator");
@@ -1126,7 +1129,14 @@ int pimdl_amm_run_noalloc(pimdl_amm* a, const float* in_dev, uint32_t n, float* 
     Ctx* ctx = a->ctx;
     if (!is_device_ptr(in_dev) || !is_device_ptr(out_dev))
         return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_run_noalloc: in and out must be device pointers (staging host buffers would allocate)");
-    const size_t need = idx_buffer_bytes(a->g, n);
+    // Tiled index words take whole blocks of 64 tokens.  Where the index layout is a matter of the byte adder alone (what the tokens
+    // need is what counts), the tokens of a last block that does not fit go through the scratch on their own.
+    uint32_t head = n;
+    size_t need = idx_buffer_bytes(a->g, n);
+    if (need > (size_t)PIMDL_NOALLOC_SCRATCH_BYTES && by_rows(a) && n > 64 && (size_t)n * a->g.idx_row_bytes <= (size_t)PIMDL_NOALLOC_SCRATCH_BYTES) {
+        head = n / 64 * 64;
+        need = idx_buffer_bytes(a->g, head);
+    }
     if (need > (size_t)PIMDL_NOALLOC_SCRATCH_BYTES)
         return set_error(ctx, PIMDL_ERR_INVALID,
                          "pimdl_amm_run_noalloc: n=%u tokens x %u index bytes per token = %zu bytes of packed indices exceed the "
@@ -1136,8 +1146,11 @@ int pimdl_amm_run_noalloc(pimdl_amm* a, const float* in_dev, uint32_t n, float* 
     // Nothing in the scratch has to start at zero: the search kernel writes every index byte the gather reads,
     // padded codebooks included, and index bytes of tokens past n only reach accumulators that are never stored.
     uint8_t* d_idx = ctx->d_static_scratch;  // the device address from hipGetSymbolAddress, never the array's name
-    if ((rc = launch_ccs(ctx, a->g, in_dev, a->d_centroids, d_idx, n))) return rc;
-    return launch_gather(ctx, *a, d_idx, out_dev, nullptr, n);
+    for (uint32_t at = 0, count = head; at < n && !rc; at += count, count = n - at) {
+        rc = launch_ccs(ctx, a->g, in_dev + (size_t)at * a->g.K, a->d_centroids, d_idx, count);
+        if (!rc) rc = launch_gather(ctx, *a, d_idx, out_dev + (size_t)at * a->g.M, nullptr, count);
+    }
+    return rc;
 }
 
 int pimdl_amm_run_debug(pimdl_amm* a, const float* in, uint32_t n, float* out, uint16_t* idx_out, int32_t* acc_out)

@@ -172,3 +172,25 @@ def test_noalloc_refuses_what_it_cannot_hold(ctx):
         amm.run_noalloc_ptr(xh.ctypes.data, 4, od.data_ptr())
     assert e.value.code == pimdl.ERR_INVALID and "device pointers" in str(e.value)
     amm.close()
+
+
+@pytest.mark.parametrize("K,v,C,tuning", [(384, 2, 64, {}), (3072, 2, 16, {"gather_kernel": pimdl.GATHER_ROWS})])
+def test_noalloc_up_to_the_last_token_that_fits(ctx, K, v, C, tuning):
+    """Byte adder: the scratch is counted by what the tokens need, though their index words lie in blocks of 64 tokens; one more is refused."""
+    import torch
+
+    M, row = 16, K // v // (2 if C <= 16 else 1)
+    N = pimdl.NOALLOC_SCRATCH_BYTES // row
+    assert N % 64 != 0
+    rng = np.random.default_rng(K + C)
+    cent = rng.standard_normal((K // v, C, v)).astype(np.float32)
+    lut = rng.integers(-128, 128, (K // v, C, M)).astype(np.int8)
+    amm = ctx.amm(cent, lut, np.float32(0.01), rng.standard_normal(M).astype(np.float32), max_n=N + 1, tuning=tuning)
+    assert amm.geometry()["idx_row_bytes"] == row
+    xd = torch.randn(N + 1, K, device="cuda")
+    ref, got = _both(amm, xd, N, M)
+    assert np.array_equal(ref.view(np.uint32), got.view(np.uint32))
+    with pytest.raises(pimdl.PimdlError) as e:
+        amm.run_noalloc_ptr(xd.data_ptr(), N + 1, torch.empty(N + 1, M, device="cuda").data_ptr())
+    assert e.value.code == pimdl.ERR_INVALID
+    amm.close()
