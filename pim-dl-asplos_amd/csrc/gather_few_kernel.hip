@@ -58,7 +58,7 @@ __device__ __forceinline__ uint32_t few_column(uint32_t tn, uint32_t c, uint32_t
 //   FEW_ROWS    the byte adder: lane (g, token j) reads its 16 columns of codebook 4 s + g, the constant operand
 //               A[i][16 g + b] = (b == i) adds them
 template <FewTable T, int TM, int NW>
-__global__ __launch_bounds__(NW * 64) void gather_few_kernel(FewArgs a, Epilogue ep)
+__device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep)
 {
     constexpr int PITCH = T == FEW_ROWS ? FEW_PITCH_ROWS : FEW_PITCH_ONEHOT;
     extern __shared__ __attribute__((aligned(16))) int part[];  // [wave][4 TM registers][PITCH]
@@ -180,18 +180,34 @@ __global__ __launch_bounds__(NW * 64) void gather_few_kernel(FewArgs a, Epilogue
     }
 }
 
+// (a name for each, which says in a profile which of the large kernels it stands in for)
+template <int TM, int NW>
+__global__ __launch_bounds__(NW * 64) void gather_sparse_few_kernel(FewArgs a, Epilogue ep)
+{
+    gather_few<FEW_SPARSE, TM, NW>(a, ep);
+}
+template <int TM, int NW>
+__global__ __launch_bounds__(NW * 64) void gather_onehot_few_kernel(FewArgs a, Epilogue ep)
+{
+    gather_few<FEW_PAIRED, TM, NW>(a, ep);
+}
+template <int TM, int NW>
+__global__ __launch_bounds__(NW * 64) void gather_i8_few_kernel(FewArgs a, Epilogue ep)
+{
+    gather_few<FEW_ROWS, TM, NW>(a, ep);
+}
+
 template <FewTable T, int TM, int NW>
 int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
 {
     constexpr int LDS = few_lds_bytes(NW, TM, T == FEW_ROWS ? FEW_PITCH_ROWS : FEW_PITCH_ONEHOT);
-    auto kern = gather_few_kernel<T, TM, NW>;
+    auto kern = T == FEW_SPARSE ? gather_sparse_few_kernel<TM, NW> : T == FEW_PAIRED ? gather_onehot_few_kernel<TM, NW> : gather_i8_few_kernel<TM, NW>;
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_few)")) return rc;
-    // (the name says which of the large kernels it stands in for)
     static const char* const names[] = {"gather_sparse_few_kernel", "gather_onehot_few_kernel", "gather_i8_few_kernel"};
     snprintf(a.last_gather, sizeof(a.last_gather), "%s<%d, %d>", names[T], TM, NW);
     a.note_launch(0, LDS, 16 * TM, NW * 64);
     hipLaunchKernelGGL(kern, dim3(f.groups * ((f.N + 16 * TM - 1) / (16 * TM))), dim3(NW * 64), LDS, ctx->stream, f, ep);
-    return hip_check(ctx, hipGetLastError(), "gather_few_kernel launch");
+    return hip_check(ctx, hipGetLastError(), "gather_few launch");
 }
 
 // tokens of an item, by what the launch has: 16, 32 or 64

@@ -997,3 +997,25 @@ def test_wide_tables_have_one_column_width(ctx, C):
         amm.set_tuning(col_block=64)
     amm.close()
     again.close()
+
+
+def test_the_reported_gather_kernel_is_a_kernel_of_the_library(ctx):
+    """What last_gather_kernel names is what a profile of the launch lists: a kernel of the library, template arguments included
+    (the sparse gather's last one is left out where it is 1)."""
+    import subprocess
+    listed = subprocess.run(["nm", "-C", pimdl.LIB_PATH], check=True, capture_output=True, text=True).stdout
+    kernels = {line.split("(anonymous namespace)::", 1)[1].split(">(")[0] + ">" for line in listed.splitlines() if "::gather_" in line and ">(" in line}
+    seen = set()
+    for N, CB, v, C, M, lut, group in FEW_SHAPES + [(3000, 64, 4, C, 768, lut, g) for C in (8, 16, 32, 64, 200)
+                                                    for lut, g in (("i8", 0), ("f32", 0), ("i8", 4))]:
+        x, cent, table, _ = make_case(N + C, N, CB * v, v, C, M, lut)
+        scales = None if lut == "f32" else np.full((CB + group - 1) // group, 0.01, np.float32) if group else np.float32(0.01)
+        amm = ctx.amm(cent, table, scales, None, max_n=N, scale_group=group)
+        amm.run(x)
+        name = amm.last_gather_kernel()
+        assert name in kernels or name[:-1] + ", 1>" in kernels, name
+        seen.add(name.split("<")[0])
+        amm.close()
+    if not kernel_switches():
+        assert {"gather_sparse_few_kernel", "gather_onehot_few_kernel", "gather_i8_few_kernel", "gather_f32_few_kernel", "gather_sparse_kernel",
+                "gather_i8_kernel", "gather_f32_rows_kernel", "gather_f32_kernel"} <= seen, seen
