@@ -126,8 +126,9 @@ def test_fp32_lut_export(ctx):
 
 
 def test_lutgen_beside_other_threads_of_one_context(ctx):
-    """Table construction in two threads while a third runs an operator on host buffers: each result is that of a lone call."""
-    import threading
+    """Table construction in two threads while a third runs an operator on host buffers: each result is that of a lone call,
+    and every call succeeds."""
+    import concurrent.futures
     rng = np.random.default_rng(77)
     jobs = []
     for CB, C, v, M in [(96, 16, 4, 2048), (64, 16, 8, 1537)]:
@@ -138,23 +139,19 @@ def test_lutgen_beside_other_threads_of_one_context(ctx):
     amm = ctx.amm(cent, table, scales[0], np.zeros(2048, np.float32), max_n=1500)
     x = rng.standard_normal((1500, 384)).astype(np.float32)
     out = amm.run(x).copy()
-    wrong = []
 
     def construct(cent, weight, table, scales):
         for _ in range(6):
             got, s = ctx.lutgen(cent, weight)
-            if not (np.array_equal(got, table) and np.array_equal(s, scales)):
-                wrong.append("table")
+            assert np.array_equal(got, table) and np.array_equal(s, scales), "table"
+        return True
 
     def gather():
         for _ in range(6):
-            if not np.array_equal(amm.run(x), out):
-                wrong.append("output")
+            assert np.array_equal(amm.run(x), out), "output"
+        return True
 
-    threads = [threading.Thread(target=construct, args=j) for j in jobs] + [threading.Thread(target=gather)]
-    for t in threads:
-        t.start()
-    for t in threads:
-        t.join(60)
-    assert not wrong and not any(t.is_alive() for t in threads)
+    with concurrent.futures.ThreadPoolExecutor(3) as pool:   # result() raises what a call in the thread raised
+        running = [pool.submit(construct, *j) for j in jobs] + [pool.submit(gather)]
+        assert all(r.result(timeout=60) for r in running)
     amm.close()
