@@ -117,8 +117,11 @@ def test_every_item_is_computed_once_however_items_are_dealt_to_the_xcds(ctx, N,
     if os.environ.get("PIMDL_GATHER_ROWS") == "1":
         pytest.skip("the matrix-core gather is switched off")
     x, cent, lut, bias = make_case(N + M, N, 128, 4, 16, M)
-    amm = ctx.amm(cent, lut, np.float32(0.01), bias, max_n=N, col_block=96)
+    # (naming the items also keeps the kernel for few tokens away, which deals nothing to the XCDs)
+    amm = ctx.amm(cent, lut, np.float32(0.01), bias, max_n=N, tuning={"col_block": 96, "token_item": 128})
     out, idx, acc = amm.run_debug(x)
+    assert amm.last_gather_kernel().startswith(("gather_sparse_kernel<", "gather_onehot_kernel<")), amm.last_gather_kernel()
+    assert amm.geometry()["tokens_per_wg"] == 128
     want_idx = oracle.index_calculation(x, cent, 4, threads=THREADS)
     want_acc = oracle.gather_i8(want_idx, lut, threads=THREADS)
     assert np.array_equal(idx, want_idx)
@@ -258,21 +261,26 @@ def test_scale_per_codebook_group(ctx, group, C, v, CB, M):
     amm.close()
 
 
-@pytest.mark.parametrize("kind", ["f32", "grouped"])
-def test_two_tokens_per_lane_in_the_fp32_table_gather(ctx, kind):
-    """Wide outputs make the fp32-table gather give each lane two tokens (rows t and t + 256 of a 512-token
-    block); the last block is ragged in both halves' sense: 1100 = 2 * 512 + 76."""
-    N, v, CB, C, M = 1100, 4, 8, 16, 2752
+@pytest.mark.parametrize("C,M", [(64, 2752), (16, 2752), (130, 1376), (100, 1376), (40, 2750)])
+@pytest.mark.parametrize("kind", ["f32", "grouped", "prescaled"])
+def test_two_tokens_per_lane_in_the_fp32_table_gather(ctx, kind, C, M):
+    """Wide outputs make the fp32-table gather of more than 32 centroids give each lane two tokens (rows t and t + 256 of a
+    512-token block); the last block is ragged in both halves' sense: 1100 = 2 * 512 + 76.  (Up to 32 centroids the same sizes run on
+    the kernel that reads its rows in pieces.)"""
+    N, v, CB = 1100, 4, 8
     x, cent, lut, bias = make_case(77, N, CB * v, v, C, M, "f32" if kind == "f32" else "i8")
     want_idx = oracle.index_calculation(x, cent, v, threads=THREADS)
     if kind == "f32":
         amm = ctx.amm(cent, lut, None, bias, max_n=N)
-        np.testing.assert_allclose(amm.run(x), oracle.gather_f32(want_idx, lut, bias, threads=THREADS), rtol=1e-5, atol=1e-6)
+        want = oracle.gather_f32(want_idx, lut, bias, threads=THREADS)
     else:
-        scales = np.random.default_rng(3).uniform(1e-3, 0.1, 3).astype(np.float32)
-        amm = ctx.amm(cent, lut, scales, bias, max_n=N, scale_group=3)
-        want = oracle.gather_i8_grouped(want_idx, lut, scales, bias, 3, threads=THREADS)
-        assert np.array_equal(amm.run(x).view(np.uint32), want.view(np.uint32))
+        group = 3 if kind == "grouped" else 1
+        scales = np.random.default_rng(3).uniform(1e-3, 0.1, (CB + group - 1) // group).astype(np.float32)
+        amm = ctx.amm(cent, lut, scales, bias, max_n=N, scale_group=group)
+        want = oracle.gather_i8_grouped(want_idx, lut, scales, bias, group, threads=THREADS)
+    assert np.array_equal(amm.run_debug(x, want_acc=False)[0].view(np.uint32), want.view(np.uint32))
+    name = amm.last_gather_kernel()
+    assert name.startswith("gather_f32_kernel<") and name.endswith(", 2>") if C > 32 else name.startswith("gather_f32_rows_kernel<"), name
     amm.close()
 
 
@@ -1019,3 +1027,41 @@ def test_the_reported_gather_kernel_is_a_kernel_of_the_library(ctx):
     if not kernel_switches():
         assert {"gather_sparse_few_kernel", "gather_onehot_few_kernel", "gather_i8_few_kernel", "gather_f32_few_kernel", "gather_sparse_kernel",
                 "gather_i8_kernel", "gather_f32_rows_kernel", "gather_f32_kernel"} <= seen, seen
+
+
+@pytest.mark.parametrize("kernel,C,widths", [("ONEHOT", 16, (48, 64, 96)), ("ONEHOT", 5, (48, 64)), ("SPARSE", 16, (48, 64, 96)),
+                                             ("SPARSE", 7, (64,)), ("SPARSE", 20, (48, 64, 96))])
+@pytest.mark.parametrize("N,CB,M", [(255, 6, 63), (1000, 64, 130), (700, 33, 1001), (513, 32, 52), (257, 96, 1)])
+def test_matrix_core_gathers_at_ragged_sizes(ctx, kernel, C, widths, N, CB, M):
+    """The gathers of large launches, kept on small ones by naming their items: ragged token tiles, ragged and odd widths (scalar
+    stores), padded codebooks, every item size and slice depth; indices, accumulators, output bits and the rows behind the output."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about what the caller names")
+    import torch
+    v = 4
+    x, cent, lut, bias = make_case(9900 + N + C, N, CB * v, v, C, M)
+    want, want_idx, want_acc = oracle.amm_cpu(x, cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)
+    xd = torch.from_numpy(x).cuda()
+    entries = (CB + 31) // 32 * 32 * (2 if C > 16 else 1)   # table entries of 16 slots
+    for width in widths:
+        amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=N, tuning={"gather_kernel": getattr(pimdl, "GATHER_" + kernel), "col_block": width})
+        items = [{"token_item": 128}, {"token_item": 256}, {"token_item": 256, "cb_per_slice": 16}]
+        if kernel == "SPARSE" and C <= 16:
+            items += [{"token_item": 512}]
+            if width == 48 and entries % 64 == 0:
+                items += [{"token_item": t, "cb_per_slice": 64} for t in (256, 512)]   # (256: the split between the waves of a SIMD)
+        for item in items:
+            amm.set_tuning(**item)
+            out, idx, acc = amm.run_debug(x)
+            name = amm.last_gather_kernel()
+            assert name.startswith(f"gather_{kernel.lower()}_kernel<{width // 16}, "), (name, item)
+            assert amm.geometry()["tokens_per_wg"] == item["token_item"], (name, item)
+            assert np.array_equal(idx, want_idx) and np.array_equal(acc, want_acc), (name, item)
+            assert np.array_equal(out.view(np.uint32), want.view(np.uint32)), (name, item)
+            guarded = torch.full((N + 3, M), -5.0, device="cuda")
+            torch.cuda.synchronize()
+            amm.run_ptr(xd.data_ptr(), N, guarded.data_ptr())
+            ctx.synchronize()
+            got = guarded.cpu().numpy()
+            assert np.array_equal(got[:N].view(np.uint32), want.view(np.uint32)) and (got[N:] == -5.0).all(), (name, item)
+        amm.close()
