@@ -1460,6 +1460,9 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
             found |= ((__float_as_uint(best) & 15u) + (up ? 16u : 0u) + 32u * (up ? sg[1] : sg[0])) << (8 * tg);
             // 2 * [ (v+1)u (|c|^2) + 16u (omitted products) + 2.02 (6v + NM + 1) u (that many additions, each within u of a
             //       partial sum below 2.02 mag) + 2(v+2)u (the reference's own chain) ], and the tags
+            // (What this takes for granted of the matrix core, launch_diag_mfma_error measures on chains of three instructions that
+            // start from any accumulator: v = 16 and 32 are two and four of them one after the other, whose errors add up.  The
+            // device stays below 25.5 u per chain, which makes 51 and 102 of the 208 and 414 u allowed here.)
             constexpr float A2 = 2.0f * ((V + 1) + 16.0f + 2.02f * (6 * V + NM + 1) + 2 * (V + 2)) * 5.9604645e-8f;
             constexpr float B2 = 2.0f * 16.0f * 2.3841858e-7f;  // 2 * 2^(4-22)
             const float thr = fmaf(A2, mag[tg], fmaf(B2, fabsf(second), 1.001e-6f));

@@ -512,7 +512,7 @@ int launch_onehot(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, in
 // ---------------------------------------------------------------------------------------------
 constexpr int GF_THREADS = 256;
 
-template <int C_T, int Q, int GS, int IDX_BITS, bool GROUPED, int TPL>
+template <int C_T, int Q, int GS, bool GROUPED, int TPL>
 __global__ __launch_bounds__(GF_THREADS) void gather_f32_kernel(const uint8_t* __restrict__ idx,
                                                                const float* __restrict__ lut,
                                                                float* __restrict__ out, uint32_t N,
@@ -529,9 +529,8 @@ __global__ __launch_bounds__(GF_THREADS) void gather_f32_kernel(const uint8_t* _
     constexpr int SLICE_LDS = GS * CB_BYTES;
     constexpr int SLICE_UNITS = GS * C_T * Q;
     constexpr int UPT = (SLICE_UNITS + GF_THREADS - 1) / GF_THREADS;
-    constexpr int IDX_BYTES = GS * IDX_BITS / 8;
-    constexpr int IDX_WORDS = (IDX_BYTES + 3) / 4;
-    static_assert(IDX_BYTES % 4 == 0, "index fetch is in dwords");
+    constexpr int IDX_WORDS = GS / 4;  // a byte per codebook
+    static_assert(GS % 4 == 0, "index fetch is in dwords");
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     // TPL tokens per lane: the staged slice serves TPL * 256 tokens, so the table is streamed from L2
@@ -594,7 +593,6 @@ __global__ __launch_bounds__(GF_THREADS) void gather_f32_kernel(const uint8_t* _
     PIMDL_COMMIT_SLICE(0)
     __syncthreads();
 
-    constexpr int per_word = 32 / IDX_BITS;
     for (uint32_t s = 0; s < nslices; ++s) {
         const uint32_t sn = s + 1 < nslices ? s + 1 : s;
         PIMDL_FETCH_SLICE(sn)
@@ -610,11 +608,11 @@ __global__ __launch_bounds__(GF_THREADS) void gather_f32_kernel(const uint8_t* _
             for (int t = 0; t < TPL; ++t) word[t] = idx_cur[t][w];
             // ascending codebook order; partial unroll keeps the loads in flight within the VGPR budget
 #pragma unroll 2
-            for (int h = 0; h < per_word; ++h) {
+            for (int h = 0; h < 4; ++h) {
 #pragma unroll
                 for (int t = 0; t < TPL; ++t) {
-                    const uint32_t r = word[t] & ((1u << IDX_BITS) - 1);
-                    word[t] >>= IDX_BITS;
+                    const uint32_t r = word[t] & 255u;
+                    word[t] >>= 8;
                     const unsigned char* row = cbbase + r * PITCH;
 #pragma unroll
                     for (int c = 0; c < Q; ++c) {
@@ -676,17 +674,17 @@ __global__ __launch_bounds__(GF_THREADS) void gather_f32_kernel(const uint8_t* _
     }
 }
 
-template <int C_T, int Q, int GS, int IDX_BITS, bool GROUPED, int TPL>
+template <int C_T, int Q, int GS, bool GROUPED, int TPL>
 int launch_f32_impl(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, uint32_t n)
 {
     constexpr int LDS = 2 * GS * C_T * (16 * Q + 16);
-    auto kern = gather_f32_kernel<C_T, Q, GS, IDX_BITS, GROUPED, TPL>;
+    auto kern = gather_f32_kernel<C_T, Q, GS, GROUPED, TPL>;
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_f32)")) return rc;
     const uint32_t n_token_tiles = (n + GF_THREADS * TPL - 1) / (GF_THREADS * TPL), colblocks = a.g.M_pad / (4 * Q);
     const uint64_t wgs = (uint64_t)n_token_tiles * colblocks;
     if (wgs > 0x7FFFFFFFull) return set_error(ctx, PIMDL_ERR_UNSUPPORTED, "gather: %llu workgroups", (unsigned long long)wgs);
     const uint32_t by_xcd = colblocks % 8 == 0 ? 1u : 0u;
-    snprintf(a.last_gather, sizeof(a.last_gather), "gather_f32_kernel<%d, %d, %d, %d, %s, %d>", C_T, Q, GS, IDX_BITS, GROUPED ? "true" : "false", TPL);
+    snprintf(a.last_gather, sizeof(a.last_gather), "gather_f32_kernel<%d, %d, %d, %s, %d>", C_T, Q, GS, GROUPED ? "true" : "false", TPL);
     a.note_launch(GS, LDS, GF_THREADS * TPL, GF_THREADS);
     hipLaunchKernelGGL(kern, dim3((uint32_t)wgs), dim3(GF_THREADS), LDS, ctx->stream, d_idx,
                        reinterpret_cast<const float*>(a.d_lut), d_out, n, a.g.M, a.g.CB_pad, a.g.idx_row_bytes,
@@ -695,14 +693,14 @@ int launch_f32_impl(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, 
 }
 
 // workgroups of gather_f32_kernel that one CU holds at a time (asked once per variant)
-template <int C_T, int Q, int GS, int IDX_BITS, bool GROUPED, int TPL>
+template <int C_T, int Q, int GS, bool GROUPED, int TPL>
 int f32_wgs_per_cu()
 {
     static int cached = 0;
     if (cached == 0) {
         constexpr int LDS = 2 * GS * C_T * (16 * Q + 16);
         int q = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, gather_f32_kernel<C_T, Q, GS, IDX_BITS, GROUPED, TPL>, GF_THREADS,
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, gather_f32_kernel<C_T, Q, GS, GROUPED, TPL>, GF_THREADS,
                                                          LDS) != hipSuccess || q < 1) {
             (void)hipGetLastError();
             q = 1;
@@ -712,7 +710,7 @@ int f32_wgs_per_cu()
     return cached;
 }
 
-template <int C_T, int Q, int GS, int IDX_BITS, bool GROUPED>
+template <int C_T, int Q, int GS, bool GROUPED>
 int launch_f32_tpl(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, uint32_t n)
 {
     // Two tokens per lane halve the table traffic from L2 for batches that still give every CU two workgroups.
@@ -725,19 +723,19 @@ int launch_f32_tpl(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, u
     bool two = wgs2 >= 2 * cus;
     if (two && a.lut_bytes > (64ull << 20)) {
         const uint64_t wgs1 = (uint64_t)((n + GF_THREADS - 1) / GF_THREADS) * colblocks;
-        const uint64_t slots1 = cus * (uint64_t)f32_wgs_per_cu<C_T, Q, GS, IDX_BITS, GROUPED, 1>();
-        const uint64_t slots2 = cus * (uint64_t)f32_wgs_per_cu<C_T, Q, GS, IDX_BITS, GROUPED, 2>();
+        const uint64_t slots1 = cus * (uint64_t)f32_wgs_per_cu<C_T, Q, GS, GROUPED, 1>();
+        const uint64_t slots2 = cus * (uint64_t)f32_wgs_per_cu<C_T, Q, GS, GROUPED, 2>();
         two = 200 * ((wgs2 + slots2 - 1) / slots2) <= 106 * ((wgs1 + slots1 - 1) / slots1);
     }
-    if (two) return launch_f32_impl<C_T, Q, GS, IDX_BITS, GROUPED, 2>(ctx, a, d_idx, d_out, n);
-    return launch_f32_impl<C_T, Q, GS, IDX_BITS, GROUPED, 1>(ctx, a, d_idx, d_out, n);
+    if (two) return launch_f32_impl<C_T, Q, GS, GROUPED, 2>(ctx, a, d_idx, d_out, n);
+    return launch_f32_impl<C_T, Q, GS, GROUPED, 1>(ctx, a, d_idx, d_out, n);
 }
 
-template <int C_T, int Q, int GS, int IDX_BITS>
+template <int C_T, int Q, int GS>
 int launch_f32(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, uint32_t n)
 {
-    return a.grouped && !a.prescaled ? launch_f32_tpl<C_T, Q, GS, IDX_BITS, true>(ctx, a, d_idx, d_out, n)
-                     : launch_f32_tpl<C_T, Q, GS, IDX_BITS, false>(ctx, a, d_idx, d_out, n);
+    return a.grouped && !a.prescaled ? launch_f32_tpl<C_T, Q, GS, true>(ctx, a, d_idx, d_out, n)
+                     : launch_f32_tpl<C_T, Q, GS, false>(ctx, a, d_idx, d_out, n);
 }
 
 }  // namespace
@@ -1002,9 +1000,9 @@ int launch_gather(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, in
         if (gather_few_wanted(ctx, a, n)) return launch_gather_few(ctx, a, d_idx, d_out, nullptr, n, 0.0f, 0.0f);
         if (g.C_tile <= 32) return launch_gather_f32_rows(ctx, a, d_idx, d_out, n);
         switch (g.C_tile) {
-            case 64: return launch_f32<64, 4, 8, 8>(ctx, a, d_idx, d_out, n);
-            case 128: return launch_f32<128, 2, 8, 8>(ctx, a, d_idx, d_out, n);
-            case 256: return launch_f32<256, 2, 4, 8>(ctx, a, d_idx, d_out, n);
+            case 64: return launch_f32<64, 4, 8>(ctx, a, d_idx, d_out, n);
+            case 128: return launch_f32<128, 2, 8>(ctx, a, d_idx, d_out, n);
+            case 256: return launch_f32<256, 2, 4>(ctx, a, d_idx, d_out, n);
         }
     }
     return set_error(ctx, PIMDL_ERR_UNSUPPORTED, "no gather kernel for C_tile=%u", g.C_tile);
