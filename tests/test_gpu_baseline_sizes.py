@@ -141,10 +141,11 @@ def test_codebook_split_between_the_waves_of_a_simd(env, N):
     assert np.array_equal(acc[rows], w_acc)
     assert np.array_equal(out[rows].view(np.uint32), w_out.view(np.uint32))
     assert np.array_equal(amm.run(x).view(np.uint32), out.view(np.uint32))  # the launch without the accumulator copy
-    # the same operator told to take 128-token items gives the same bits
-    other = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=N, tuning={"token_item": 128})
-    assert np.array_equal(other.run(x).view(np.uint32), out.view(np.uint32))
-    other.close()
+    # the same operator told to take 128-token items gives the same bits (the byte adder has no such setting)
+    if "PIMDL_GATHER_ROWS" not in kernel_switches():
+        other = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=N, tuning={"token_item": 128})
+        assert np.array_equal(other.run(x).view(np.uint32), out.view(np.uint32))
+        other.close()
     amm.close()
 
 
