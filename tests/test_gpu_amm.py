@@ -1065,3 +1065,25 @@ def test_matrix_core_gathers_at_ragged_sizes(ctx, kernel, C, widths, N, CB, M):
             got = guarded.cpu().numpy()
             assert np.array_equal(got[:N].view(np.uint32), want.view(np.uint32)) and (got[N:] == -5.0).all(), (name, item)
         amm.close()
+
+
+def gather_us(ctx, N, CB, C, M, lut="i8", tuning=None, v=4):
+    """Shortest of a few timings of an operator's gather, us."""
+    import torch
+    _, cent, table, bias = make_case(1, 1, CB * v, v, C, M, lut)
+    amm = ctx.amm(cent, table, None if lut == "f32" else np.float32(0.01), bias, max_n=N, tuning=tuning or {})
+    x, y = torch.randn(N, CB * v, device="cuda"), torch.empty(N, M, device="cuda")
+    torch.cuda.synchronize()
+    us = min(amm.profile(x.data_ptr(), N, y.data_ptr(), warmup=8, iters=10)["gather_ms"] for _ in range(5)) * 1e3
+    amm.close()
+    return us
+
+
+def test_byte_adder_writes_large_outputs_like_the_sparse_gather(ctx):
+    """One codebook: the launch is its stores.  No wait of the epilogue stands between them: 1.02 of the sparse kernel's time, 1.45 with
+    the bias of a column chunk loaded behind the stores of the chunk before it.  (Not at every width: rows of 4096 floats, a power of
+    two apart, take 1.33, and took 1.58.)"""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about what the caller names")
+    rows, sparse = (gather_us(ctx, 38004, 1, 16, 3131, tuning={"gather_kernel": k}) for k in (pimdl.GATHER_ROWS, pimdl.GATHER_SPARSE))
+    assert rows < 1.25 * sparse, (rows, sparse)
