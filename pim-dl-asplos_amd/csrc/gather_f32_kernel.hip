@@ -63,13 +63,13 @@ __global__ __launch_bounds__(F32_THREADS, 4) void gather_f32_rows_kernel(
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // Workgroup p of the 1-D grid: column block p / n_token_tiles, token tile p % n_token_tiles -- or, by_xcd
-    // (column blocks a multiple of 8): workgroups go to the 8 XCDs round-robin, and XCD p % 8 takes every token
-    // tile of the column blocks congruent to it, so that a column block's part of the table is streamed
-    // through one L2 instead of all eight.
+    // Workgroup p of the 1-D grid: column block p / n_token_tiles, token tile p % n_token_tiles -- or, by_xcd: workgroups go to the 8
+    // XCDs round-robin, and XCD p % 8 takes every token tile of the column blocks congruent to it, so that a column block's part of
+    // the table is streamed through one L2 instead of all eight (column blocks past the last: nothing to do).
     const uint32_t pq = by_xcd ? blockIdx.x / 8 : blockIdx.x;
     const uint32_t tile = pq % n_token_tiles;
     const uint32_t colblk = by_xcd ? blockIdx.x % 8 + 8 * (pq / n_token_tiles) : pq / n_token_tiles;
+    if (colblk * 16 >= M) return;  // whole workgroup
     const uint32_t tok = SPLIT ? tile * 64 + lane : tile * F32_THREADS + threadIdx.x;
     const uint32_t nslices = CB_pad / GS;  // even
     // 16 bytes of an index row are the codebooks of two slices
@@ -210,9 +210,18 @@ int launch_f32_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, ui
     auto kern = gather_f32_rows_kernel<C_T, IDX_BITS, GROUPED, SPLIT>;
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_f32)")) return rc;
     const uint32_t n_token_tiles = (n + TOKENS - 1) / TOKENS, colblocks = a.g.M_pad / 16;
-    const uint64_t wgs = (uint64_t)n_token_tiles * colblocks;
+    // By XCD where the table's traffic counts and the column blocks divide evenly enough (an eighth more at most).  Not for outputs
+    // beyond the caches, and larger than the table, in whole float4s: eight column blocks side by side then write pieces of the same
+    // rows at the same time (us, by XCD / in order: 16 centroids, 1 codebook, N = 27003, M = 3072 358 / 252; 64 codebooks, N = 6664,
+    // M = 4096 127 / 102; 192 codebooks, N = 12608, M = 3072 291 / 292, N = 2048 61 / 64; 32 centroids, 256 codebooks, N = 2048,
+    // M = 3072 86 / 116, N = 6664, M = 4096 347 / 375; 768 codebooks, N = 12608, M = 768 368 / 488; odd widths, 128 codebooks, N = 9919,
+    // M = 4095 317 / 344; few tokens, 192 codebooks, N = 328, M = 2157 26 / 53).
+    const uint64_t out_bytes = (uint64_t)n * a.g.M * 4;
+    const uint32_t padded = (colblocks + 7) / 8 * 8;
+    const bool wide_output = a.g.M % 4 == 0 && out_bytes >= (40ull << 20) && a.lut_bytes < out_bytes;
+    const uint32_t by_xcd = 8 * (padded - colblocks) <= colblocks && !wide_output ? 1u : 0u;
+    const uint64_t wgs = (uint64_t)n_token_tiles * (by_xcd ? padded : colblocks);
     if (wgs > 0x7FFFFFFFull) return set_error(ctx, PIMDL_ERR_UNSUPPORTED, "gather: %llu workgroups", (unsigned long long)wgs);
-    const uint32_t by_xcd = colblocks % 8 == 0 ? 1u : 0u;
     snprintf(a.last_gather, sizeof(a.last_gather), "gather_f32_rows_kernel<%d, %d, %s, %s>", C_T, IDX_BITS, GROUPED ? "true" : "false",
              SPLIT ? "true" : "false");
     a.note_launch(f32_slice_cbs(C_T), LDS, TOKENS, F32_THREADS);

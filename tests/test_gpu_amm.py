@@ -1087,3 +1087,32 @@ def test_byte_adder_writes_large_outputs_like_the_sparse_gather(ctx):
         pytest.skip("the environment keeps one kernel for every shape; this test is about what the caller names")
     rows, sparse = (gather_us(ctx, 38004, 1, 16, 3131, tuning={"gather_kernel": k}) for k in (pimdl.GATHER_ROWS, pimdl.GATHER_SPARSE))
     assert rows < 1.25 * sparse, (rows, sparse)
+
+
+@pytest.mark.parametrize("N,CB,C,M", [(328, 40, 32, 2157), (1500, 33, 16, 905), (1500, 40, 8, 898), (3000, 33, 16, 140),   # column blocks: 135, 57, 57, 9
+                                      (2600, 33, 16, 4096), (2600, 3, 32, 4096), (2600, 40, 7, 4095)])                 # outputs of 40 MB
+def test_float_tables_whose_column_blocks_do_not_divide_among_the_xcds(ctx, N, CB, C, M):
+    """Column blocks dealt out by XCD with some past the last, and in order: every output bit, and the guard rows."""
+    import torch
+    x, cent, table, bias = make_case(9700 + N + M, N, CB * 4, 4, C, M, "f32")
+    amm = ctx.amm(cent, table, None, bias, max_n=N)
+    guarded = torch.full((N + 3, M), -1e30, device="cuda")  # no sum of the case comes near it
+    xd = torch.from_numpy(x).cuda()
+    torch.cuda.synchronize()
+    amm.run_ptr(xd.data_ptr(), N, guarded.data_ptr())
+    ctx.synchronize()
+    assert "_f32_rows_" in amm.last_gather_kernel(), amm.last_gather_kernel()
+    got = guarded.cpu().numpy()
+    rows = np.unique(np.concatenate([np.arange(min(N, 70)), np.arange(max(0, N - 70), N), np.arange(250, min(N, 260))]))
+    want = oracle.gather_f32(oracle.index_calculation(x[rows], cent, 4, threads=THREADS), table, bias, threads=THREADS)
+    assert np.array_equal(got[rows].view(np.uint32), want.view(np.uint32)) and (got[N:] < -9e29).all() and (got[:N] > -9e29).all()
+    amm.close()
+
+
+def test_float_gathers_do_not_depend_on_a_multiple_of_eight_column_blocks(ctx):
+    """135 and 136 column blocks of a table beyond the caches, few tokens (2.1 times as long when the 135 were not dealt out by XCD);
+    256 and 254 of one codebook, an output beyond the caches (1.5 times when the 256 were)."""
+    few = [gather_us(ctx, 328, 192, 32, M, "f32") for M in (2157, 2173)]
+    wide = [gather_us(ctx, 6664, 1, 16, M, "f32") for M in (4096, 4064)]   # not 4080: rows just short of 16 KiB take 1.5 times as long in either order
+    assert few[0] < 1.4 * few[1], few
+    assert wide[0] < 1.3 * wide[1], wide
