@@ -40,6 +40,9 @@ namespace pimdl {
 namespace {
 
 typedef int v8i __attribute__((ext_vector_type(8)));
+// four columns of a row of any width: 16-byte stores need dword alignment only
+typedef float v4f_dw __attribute__((ext_vector_type(4), aligned(4)));
+typedef int v4i_dw __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int N>
 __device__ __forceinline__ void lgkm_wait()
@@ -150,7 +153,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void gather_i8_kernel(
     // ---- epilogue: lane (j, g) holds columns 4 g .. 4 g + 3 of every chunk for token j of every group --------
     // All bias values first, then the stores row by row: with a chunk's bias loaded behind the chunk before it, every chunk waited for
     // the stores so far, and the rows were written in Q passes (us, before / now: one codebook, N = 38004, M = 3131, 16 centroids
-    // 354 / 249, 64 centroids 338 / 275; N = 25265, M = 3072, 96 codebooks, 64 centroids 160 / 139).
+    // 354 / 249, 64 centroids 338 / 275; N = 25265, M = 3072, 96 codebooks, 64 centroids 160 / 139).  Four columns in one store at any
+    // width (us, float by float where M % 4 != 0 / now: 32 centroids, N = 20000, M = 1001, 1 codebook 49 / 27, 192 codebooks 76 / 56;
+    // 64 centroids, N = 38004, M = 3131, 33 codebooks 349 / 281).
     auto epilogue_as = [&](uint32_t item, auto actc) __attribute__((always_inline)) {
         constexpr bool ACT = decltype(actc)::value;
         const uint32_t col = col_of(item);
@@ -160,7 +165,6 @@ __global__ __launch_bounds__(NW * 64, WPS) void gather_i8_kernel(
         uint32_t je = j, ge = g;
         asm volatile("" : "+v"(je), "+v"(ge));
         const uint32_t tok0 = tok_tile_of(item) * TOK_ITEM + wave * (TG * 16) + je;
-        const bool vec_store = (M % 4 == 0);
         float bv[Q][4];
 #pragma unroll
         for (int c = 0; c < Q; ++c)
@@ -182,9 +186,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void gather_i8_kernel(
 #pragma unroll
                 for (int e = 0; e < 4; ++e) o[e] = dequant<ACT>(a[e], epl, bv[c][e]);
                 const size_t at = (size_t)tok * M + f;
-                if (vec_store) {  // M % 4 == 0 and f % 4 == 0: the whole float4 is in range and aligned
-                    *reinterpret_cast<float4*>(out + at) = make_float4(o[0], o[1], o[2], o[3]);
-                    if (acc_out) *reinterpret_cast<v4i*>(acc_out + at) = a;
+                if (f + 4 <= M) {
+                    *reinterpret_cast<v4f_dw*>(out + at) = (v4f_dw){o[0], o[1], o[2], o[3]};
+                    if (acc_out) *reinterpret_cast<v4i_dw*>(acc_out + at) = (v4i_dw){a[0], a[1], a[2], a[3]};
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e)

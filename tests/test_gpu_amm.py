@@ -1080,13 +1080,44 @@ def gather_us(ctx, N, CB, C, M, lut="i8", tuning=None, v=4):
 
 
 def test_byte_adder_writes_large_outputs_like_the_sparse_gather(ctx):
-    """One codebook: the launch is its stores.  No wait of the epilogue stands between them: 1.02 of the sparse kernel's time, 1.45 with
+    """One codebook: the launch is its stores.  No wait of the epilogue stands between them: 0.94 of the sparse kernel's time, 1.45 with
     the bias of a column chunk loaded behind the stores of the chunk before it.  (Not at every width: rows of 4096 floats, a power of
     two apart, take 1.33, and took 1.58.)"""
     if kernel_switches():
         pytest.skip("the environment keeps one kernel for every shape; this test is about what the caller names")
     rows, sparse = (gather_us(ctx, 38004, 1, 16, 3131, tuning={"gather_kernel": k}) for k in (pimdl.GATHER_ROWS, pimdl.GATHER_SPARSE))
     assert rows < 1.25 * sparse, (rows, sparse)
+
+
+@pytest.mark.parametrize("M", [99, 258, 1001, 5])
+@pytest.mark.parametrize("C", [20, 64, 130])
+def test_byte_adder_stores_rows_of_any_width(ctx, C, M):
+    """Rows that are no whole float4s, behind an address that is a multiple of 4 bytes only: every bit, and what lies around them."""
+    import torch
+    N, CB = 700, 40
+    x, cent, lut, bias = make_case(9800 + C + M, N, CB * 4, 4, C, M)
+    amm = ctx.amm(cent, lut, np.float32(0.02), bias, max_n=N)
+    guarded = torch.full((1 + N * M + 64,), -1e30, device="cuda")
+    xd = torch.from_numpy(x).cuda()
+    torch.cuda.synchronize()
+    amm.run_ptr(xd.data_ptr(), N, guarded.data_ptr() + 4)
+    ctx.synchronize()
+    assert "gather_i8_" in amm.last_gather_kernel() or kernel_switches(), amm.last_gather_kernel()
+    got = guarded.cpu().numpy()
+    acc = oracle.gather_i8(oracle.index_calculation(x, cent, 4, threads=THREADS), lut, threads=THREADS)
+    want = oracle.dequant(acc, bias, CB, 0.02, 0.0, 0, threads=THREADS)
+    assert np.array_equal(got[1:1 + N * M].reshape(N, M).view(np.uint32), want.view(np.uint32))
+    assert got[0] == np.float32(-1e30) and (got[1 + N * M:] == np.float32(-1e30)).all()
+    amm.close()
+
+
+def test_odd_widths_of_17_to_32_centroids_are_not_slower_than_the_sparse_gather(ctx):
+    """The library gives them to the byte adder: 0.7 of the sparse kernel's time, 1.25 and 1.4 when it stored float by float."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    for N, CB, M in ((20000, 1, 1001), (20000, 33, 258)):
+        auto, sparse = (gather_us(ctx, N, CB, 32, M, tuning=t) for t in (None, {"gather_kernel": pimdl.GATHER_SPARSE}))
+        assert auto < 1.1 * sparse, (N, CB, M, auto, sparse)
 
 
 @pytest.mark.parametrize("N,CB,C,M", [(328, 40, 32, 2157), (1500, 33, 16, 905), (1500, 40, 8, 898), (3000, 33, 16, 140),   # column blocks: 135, 57, 57, 9
