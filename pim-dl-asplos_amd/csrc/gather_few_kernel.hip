@@ -317,7 +317,9 @@ int launch_f32_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, u
 // 24.1 / 40.8 at 300.  Floats, 16 centroids (the large kernel with 64-token workgroups): 3072 -> 768 23.7 / 14.4 at 1,
 // 24.0 / 19.6 at 13, 25.5 / 28.7 at 64; 768 -> 3072 8.6 / 5.2 at 1, 8.4 / 9.3 at 13; 32 centroids 3072 -> 768 44 / 33 at 1,
 // 47 / 71 at 64; 200 centroids (whole rows) 1000 -> 1001 49 / 5.3 at 1, 51 / 32 at 64, 56 / 73 at 150; a scale per 5
-// codebooks 19.8 / 18.7 at 1, 19.7 / 22.6 at 13.  The estimates are fits to these.
+// codebooks 19.8 / 18.7 at 1, 19.7 / 22.6 at 13; 64 centroids (large / few; a piece costs more where the caches do not hold the
+// table), 96 codebooks, M = 2441 16.2 / 10.2 at 32, 16.5 / 24.3 at 93; M = 554 15.7 / 9.1 at 150, 17.5 / 17.2 at 400; 768 codebooks,
+// M = 2441 122 / 63 at 32, 123 / 183 at 93; a scale per 8 codebooks, M = 1001 25 / 31 at 283.  The estimates are fits to these.
 bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
 {
     const AmmGeom& g = a.g;
@@ -327,7 +329,7 @@ bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
     if (a.desc.lut_dtype == PIMDL_LUT_F32 || a.grouped) {
         const bool bounds = a.grouped && !a.prescaled;  // a scale to apply at the end of every group
         if (g.lut_chunk) return pieces * (g.lut_chunk == 2 ? 18e-6 : 7.5e-6) < (bounds ? 1.0 : 1.4 + 0.0103 * g.CB_pad);
-        const double piece = g.q != 4 ? 32e-6 : 4e-6;
+        const double piece = g.q != 4 ? 32e-6 : bounds || a.lut_bytes > (48u << 20) ? 6.5e-6 : 5e-6;
         return 2.7 + g.CB_pad * (bounds ? 0.062 : 0.0137) + pieces * piece < 4.0 + g.CB_pad * (bounds ? 0.14 : 0.07);
     }
     if (g.gather_kind == 0)

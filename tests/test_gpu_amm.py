@@ -1067,11 +1067,12 @@ def test_matrix_core_gathers_at_ragged_sizes(ctx, kernel, C, widths, N, CB, M):
         amm.close()
 
 
-def gather_us(ctx, N, CB, C, M, lut="i8", tuning=None, v=4):
+def gather_us(ctx, N, CB, C, M, lut="i8", tuning=None, v=4, group=0):
     """Shortest of a few timings of an operator's gather, us."""
     import torch
     _, cent, table, bias = make_case(1, 1, CB * v, v, C, M, lut)
-    amm = ctx.amm(cent, table, None if lut == "f32" else np.float32(0.01), bias, max_n=N, tuning=tuning or {})
+    scales = None if lut == "f32" else np.full((CB + group - 1) // group, 0.01, np.float32) if group else np.float32(0.01)
+    amm = ctx.amm(cent, table, scales, bias, max_n=N, tuning=tuning or {}, scale_group=group)
     x, y = torch.randn(N, CB * v, device="cuda"), torch.empty(N, M, device="cuda")
     torch.cuda.synchronize()
     us = min(amm.profile(x.data_ptr(), N, y.data_ptr(), warmup=8, iters=10)["gather_ms"] for _ in range(5)) * 1e3
@@ -1147,3 +1148,10 @@ def test_float_gathers_do_not_depend_on_a_multiple_of_eight_column_blocks(ctx):
     wide = [gather_us(ctx, 6664, 1, 16, M, "f32") for M in (4096, 4064)]   # not 4080: rows just short of 16 KiB take 1.5 times as long in either order
     assert few[0] < 1.4 * few[1], few
     assert wide[0] < 1.3 * wide[1], wide
+
+
+@pytest.mark.parametrize("CB,lut,group,M", [(96, "f32", 0, 2441), (768, "f32", 0, 2441), (96, "i8", 8, 3692)])
+def test_few_tokens_of_64_centroids_take_the_large_gather_where_it_is_shorter(ctx, CB, lut, group, M):
+    """93 tokens, gathered piece by piece, took 1.4 to 1.7 times as long as 150 on the large kernel."""
+    a, b = (gather_us(ctx, n, CB, 64, M, lut, v=1, group=group) for n in (93, 150))
+    assert a < 1.2 * b, (a, b)
