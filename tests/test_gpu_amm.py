@@ -1150,6 +1150,12 @@ def test_float_gathers_do_not_depend_on_a_multiple_of_eight_column_blocks(ctx):
     assert wide[0] < 1.3 * wide[1], wide
 
 
+def test_float_gathers_take_whole_workgroups_where_the_copies_are_the_chain(ctx):
+    """32 centroids: 283 tokens in two workgroups per column block, as 400 are (1.5 times their time in five of 64 tokens)."""
+    a, b = (gather_us(ctx, n, 768, 32, 3370, "f32", v=1) for n in (283, 400))
+    assert a < 1.2 * b, (a, b)
+
+
 @pytest.mark.parametrize("CB,lut,group,M", [(96, "f32", 0, 2441), (768, "f32", 0, 2441), (96, "i8", 8, 3692)])
 def test_few_tokens_of_64_centroids_take_the_large_gather_where_it_is_shorter(ctx, CB, lut, group, M):
     """93 tokens, gathered piece by piece, took 1.4 to 1.7 times as long as 150 on the large kernel."""
