@@ -211,14 +211,15 @@ int launch_f32_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, ui
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_f32)")) return rc;
     const uint32_t n_token_tiles = (n + TOKENS - 1) / TOKENS, colblocks = a.g.M_pad / 16;
     // By XCD where the table's traffic counts and the column blocks divide evenly enough (an eighth more at most).  Not for outputs
-    // beyond the caches, and larger than the table, in whole float4s: eight column blocks side by side then write pieces of the same
-    // rows at the same time (us, by XCD / in order: 16 centroids, 1 codebook, N = 27003, M = 3072 358 / 252; 64 codebooks, N = 6664,
-    // M = 4096 127 / 102; 192 codebooks, N = 12608, M = 3072 291 / 292, N = 2048 61 / 64; 32 centroids, 256 codebooks, N = 2048,
-    // M = 3072 86 / 116, N = 6664, M = 4096 347 / 375; 768 codebooks, N = 12608, M = 768 368 / 488; odd widths, 128 codebooks, N = 9919,
-    // M = 4095 317 / 344; few tokens, 192 codebooks, N = 328, M = 2157 26 / 53).
+    // beyond the caches, and larger than the table, in rows of more than 4 KiB of whole float4s: eight column blocks side by side then
+    // write pieces of the same rows at the same time (us, by XCD / in order: 16 centroids, 1 codebook, N = 27003, M = 3072 358 / 252;
+    // 64 codebooks, N = 6664, M = 4096 127 / 102; 192 codebooks, N = 12608, M = 3072 291 / 292, N = 2048 61 / 64; 32 centroids, 256
+    // codebooks, N = 2048, M = 3072 86 / 116, N = 6664, M = 4096 347 / 375; 768 codebooks, N = 12608, M = 768 368 / 488; odd widths,
+    // 128 codebooks, N = 9919, M = 4095 317 / 344; rows of up to 4 KiB, 1 codebook, 180 MB, M = 512 130 / 177, M = 1024 147 / 196,
+    // M = 768 135 / 134; few tokens, 192 codebooks, N = 328, M = 2157 26 / 53).
     const uint64_t out_bytes = (uint64_t)n * a.g.M * 4;
     const uint32_t padded = (colblocks + 7) / 8 * 8;
-    const bool wide_output = a.g.M % 4 == 0 && out_bytes >= (40ull << 20) && a.lut_bytes < out_bytes;
+    const bool wide_output = a.g.M % 4 == 0 && a.g.M > 1024 && out_bytes >= (40ull << 20) && a.lut_bytes < out_bytes;
     const uint32_t by_xcd = 8 * (padded - colblocks) <= colblocks && !wide_output ? 1u : 0u;
     const uint64_t wgs = (uint64_t)n_token_tiles * (by_xcd ? padded : colblocks);
     if (wgs > 0x7FFFFFFFull) return set_error(ctx, PIMDL_ERR_UNSUPPORTED, "gather: %llu workgroups", (unsigned long long)wgs);

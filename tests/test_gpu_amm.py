@@ -1150,6 +1150,12 @@ def test_float_gathers_do_not_depend_on_a_multiple_of_eight_column_blocks(ctx):
     assert wide[0] < 1.3 * wide[1], wide
 
 
+def test_float_gathers_of_rows_of_up_to_4_kib_are_dealt_out_by_xcd(ctx):
+    """32 and 33 column blocks of one codebook, outputs of 180 MB (1.36 times as long when the 32 were taken in order)."""
+    a, b = gather_us(ctx, 92160, 1, 16, 512, "f32"), gather_us(ctx, 89367, 1, 16, 528, "f32")
+    assert a < 1.2 * b, (a, b)
+
+
 def test_float_gathers_take_whole_workgroups_where_the_copies_are_the_chain(ctx):
     """32 centroids: 283 tokens in two workgroups per column block, as 400 are (1.5 times their time in five of 64 tokens)."""
     a, b = (gather_us(ctx, n, 768, 32, 3370, "f32", v=1) for n in (283, 400))
