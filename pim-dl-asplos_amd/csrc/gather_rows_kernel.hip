@@ -300,8 +300,15 @@ int launch_rows_as(const RowsLaunch& l)
     const uint32_t n_items = n_token_tiles * col_tiles;
     uint32_t grid = l.ctx->prop.multiProcessorCount * rw_wgs_per_cu(S::NW);
     if (grid > n_items) grid = n_items;
-    const XcdMap xmap = choose_xcd_map(col_tiles, n_token_tiles, grid, (uint64_t)g.CB_pad * C_T * g.M_pad,
-                                       (uint64_t)l.n * g.idx_row_bytes, g.tune_xcd_col_split);
+    // Outputs well beyond the last cache, of tables that are small beside them: an XCD writes whole rows (its own token tiles) instead of
+    // its own columns of all rows, which would have several XCDs write pieces of the same rows at the same time (us, by the table's
+    // traffic / by rows: 24 centroids, N = 36621, M = 3072, 1 codebook 154 / 134, 32 160 / 139, 96 208 / 200; N = 27465, M = 4096, 1
+    // codebook 161 / 148; 64 centroids 156 / 135, 157 / 146, 96 codebooks 270 / 261.  Not: 64 centroids, 192 codebooks, N = 36621, M = 2048
+    // 281 / 293; tiles of one chunk, 128 centroids, 32 codebooks 240 / 253; outputs of 300 MB, N = 24414, M = 3072 78 / 78).
+    const uint64_t table = (uint64_t)g.CB_pad * C_T * g.M_pad, out_bytes = (uint64_t)l.n * g.M * 4;
+    const bool by_tokens = S::Q > 1 && out_bytes > (320ull << 20) && table * 16 < out_bytes;
+    const uint32_t split = g.tune_xcd_col_split || !by_tokens ? g.tune_xcd_col_split : n_token_tiles % 8 == 0 ? 1u : PIMDL_XCD_PLAIN;
+    const XcdMap xmap = choose_xcd_map(col_tiles, n_token_tiles, grid, table, (uint64_t)l.n * g.idx_row_bytes, split);
     Epilogue ep = l.ep;
     ep.op_col_tiles = ep.op_col_tiles * g.q / S::Q;
     snprintf(l.a.last_gather, sizeof(l.a.last_gather), "gather_i8_kernel<%d, %d, %d, %d, %d, %d>", C_T, S::Q, S::NW, S::TG, WPS, IDX_BITS);

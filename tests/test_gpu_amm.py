@@ -1167,3 +1167,28 @@ def test_few_tokens_of_64_centroids_take_the_large_gather_where_it_is_shorter(ct
     """93 tokens, gathered piece by piece, took 1.4 to 1.7 times as long as 150 on the large kernel."""
     a, b = (gather_us(ctx, n, CB, 64, M, lut, v=1, group=group) for n in (93, 150))
     assert a < 1.2 * b, (a, b)
+
+
+def test_byte_adder_writes_whole_rows_of_outputs_beyond_the_caches(ctx):
+    """24 centroids, one codebook, 450 MB: 1.2 times the sparse kernel's time when an XCD wrote its own columns of all rows."""
+    rows, sparse = (gather_us(ctx, 36621, 1, 24, 3072, tuning={"gather_kernel": k}) for k in (pimdl.GATHER_ROWS, pimdl.GATHER_SPARSE))
+    assert rows < 1.12 * sparse, (rows, sparse)
+
+
+@pytest.mark.parametrize("N,C,M", [(20490, 24, 4096), (24570, 64, 3500)])  # 21 token tiles of 1024, and 24, which eight XCDs share
+def test_byte_adder_deals_outputs_beyond_the_caches_out_by_tokens(ctx, N, C, M):
+    import torch
+    x, cent, lut, bias = make_case(9900 + C, N, 12, 4, C, M)
+    amm = ctx.amm(cent, lut, np.float32(0.02), bias, max_n=N, tuning={"gather_kernel": pimdl.GATHER_ROWS})
+    guarded = torch.full((N + 3, M), -1e30, device="cuda")
+    xd = torch.from_numpy(x).cuda()
+    torch.cuda.synchronize()
+    amm.run_ptr(xd.data_ptr(), N, guarded.data_ptr())
+    ctx.synchronize()
+    assert "gather_i8_kernel" in amm.last_gather_kernel(), amm.last_gather_kernel()
+    got = guarded.cpu().numpy()
+    pick = np.unique(np.concatenate([np.arange(0, N, 97), np.arange(1000, 1050), np.arange(N - 70, N)]))
+    acc = oracle.gather_i8(oracle.index_calculation(x[pick], cent, 4, threads=THREADS), lut, threads=THREADS)
+    want = oracle.dequant(acc, bias, 3, 0.02, 0.0, 0, threads=THREADS)
+    assert np.array_equal(got[pick].view(np.uint32), want.view(np.uint32)) and (got[N:] < -9e29).all() and (got[:N] > -9e29).all()
+    amm.close()
