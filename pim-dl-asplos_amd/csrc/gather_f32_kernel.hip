@@ -238,13 +238,15 @@ int launch_f32_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, ui
 // 768 N = 64 25 / 42, 600 27 / 44, 1200 52 / 46, 8192 273 / 190; 8 centroids, 1024 -> 1024 N = 600 12 / 18, 1200 20 / 23,
 // 2500 38 / 37; 32 centroids (whose slices take longer to copy than to add, which two workgroups of the whole form share),
 // 768 -> 768 N = 600 12 / 19, 1200 23 / 21; 192 codebooks, M = 2048 N = 283 18.5 / 18.4, M = 4096 N = 130 19.5 / 19.8, 283 33 / 23;
-// 768 codebooks, M = 3370 N = 283 158 / 87.
+// 768 codebooks, M = 3370 N = 283 158 / 87.  A scale per group is work per codebook whatever the columns: 8 centroids, a
+// scale per 8, 192 codebooks, M = 3072 N = 300 31 / 34, 600 46 / 38, 1200 71 / 49, 768 codebooks, M = 768 N = 1200 94 / 102, 2500 152 / 104, 3080
+// 180 / 119.
 template <int C_T, int IDX_BITS, bool GROUPED>
 int launch_f32(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, uint32_t n)
 {
     const double per_cu = (double)(a.g.M_pad / 16) / ctx->prop.multiProcessorCount;
     const double w = (n + 63) / 64 * per_cu, w1 = (n + F32_THREADS - 1) / F32_THREADS * per_cu;
-    const double grow = (C_T == 8 ? 0.42 : 0.58) * w, grow1 = C_T == 32 ? 0.5 * w1 + 0.4 : 0.85 * w1 + 0.15;
+    const double grow = (C_T == 8 ? (GROUPED ? 0.49 : 0.42) : 0.58) * w, grow1 = C_T == 32 ? 0.5 * w1 + 0.4 : 0.85 * w1 + 0.15;
     if (0.57 * (grow > 1 ? grow : 1) < (grow1 > 1 ? grow1 : 1)) return launch_f32_as<C_T, IDX_BITS, GROUPED, true>(ctx, a, d_idx, d_out, n);
     return launch_f32_as<C_T, IDX_BITS, GROUPED, false>(ctx, a, d_idx, d_out, n);
 }

@@ -1192,3 +1192,9 @@ def test_byte_adder_deals_outputs_beyond_the_caches_out_by_tokens(ctx, N, C, M):
     want = oracle.dequant(acc, bias, 3, 0.02, 0.0, 0, threads=THREADS)
     assert np.array_equal(got[pick].view(np.uint32), want.view(np.uint32)) and (got[N:] < -9e29).all() and (got[:N] > -9e29).all()
     amm.close()
+
+
+def test_grouped_float_gathers_take_whole_workgroups_from_two_per_cu_on(ctx):
+    """8 centroids, a scale per 8 codebooks: 3080 tokens in workgroups of 64 took 1.5 times as long as 3400 in workgroups of 256."""
+    a, b = (gather_us(ctx, n, 768, 8, 768, group=8) for n in (3080, 3400))
+    assert a < 1.2 * b, (a, b)
