@@ -217,10 +217,14 @@ int launch_f32_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, ui
     // codebooks, N = 2048, M = 3072 86 / 116, N = 6664, M = 4096 347 / 375; 768 codebooks, N = 12608, M = 768 368 / 488; odd widths,
     // 128 codebooks, N = 9919, M = 4095 317 / 344; rows of up to 4 KiB, 1 codebook, 180 MB, M = 512 130 / 177, M = 1024 147 / 196,
     // M = 768 135 / 134; few tokens, 192 codebooks, N = 328, M = 2157 26 / 53).
+    // Uneven column blocks of the whole form only where the CUs of an XCD take at most an eighth more rounds (8 centroids, a scale per 8
+    // of 96 codebooks, N = 6444, M = 608, 38 column blocks 41.5 / 34.4).
     const uint64_t out_bytes = (uint64_t)n * a.g.M * 4;
-    const uint32_t padded = (colblocks + 7) / 8 * 8;
+    const uint64_t padded = (colblocks + 7) / 8 * 8, cus = ctx->prop.multiProcessorCount;
     const bool wide_output = a.g.M % 4 == 0 && a.g.M > 1024 && out_bytes >= (40ull << 20) && a.lut_bytes < out_bytes;
-    const uint32_t by_xcd = 8 * (padded - colblocks) <= colblocks && !wide_output ? 1u : 0u;
+    const bool even = 8 * (padded - colblocks) <= colblocks &&
+                      (SPLIT || 8 * ((n_token_tiles * padded + cus - 1) / cus) <= 9 * (((uint64_t)n_token_tiles * colblocks + cus - 1) / cus));
+    const uint32_t by_xcd = even && !wide_output ? 1u : 0u;
     const uint64_t wgs = (uint64_t)n_token_tiles * (by_xcd ? padded : colblocks);
     if (wgs > 0x7FFFFFFFull) return set_error(ctx, PIMDL_ERR_UNSUPPORTED, "gather: %llu workgroups", (unsigned long long)wgs);
     snprintf(a.last_gather, sizeof(a.last_gather), "gather_f32_rows_kernel<%d, %d, %s, %s>", C_T, IDX_BITS, GROUPED ? "true" : "false",

@@ -1198,3 +1198,9 @@ def test_grouped_float_gathers_take_whole_workgroups_from_two_per_cu_on(ctx):
     """8 centroids, a scale per 8 codebooks: 3080 tokens in workgroups of 64 took 1.5 times as long as 3400 in workgroups of 256."""
     a, b = (gather_us(ctx, n, 768, 8, 768, group=8) for n in (3080, 3400))
     assert a < 1.2 * b, (a, b)
+
+
+def test_float_gathers_of_uneven_column_blocks_do_not_wait_for_one_xcd(ctx):
+    """38 column blocks on 8 XCDs: 26 token tiles of them took a fifth round of the CUs (1.24 times as long as 24 tiles)."""
+    a, b = (gather_us(ctx, n, 96, 8, 608, group=8) for n in (6444, 6144))
+    assert a < 1.15 * b, (a, b)
