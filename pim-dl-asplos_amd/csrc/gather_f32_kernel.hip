@@ -202,6 +202,20 @@ __global__ __launch_bounds__(F32_THREADS, 4) void gather_f32_rows_kernel(
     }
 }
 
+// Outputs beyond the last cache in rows of whole 8 KiB: their columns fall on few memory channels, and 256 rows at a time
+// (a wave's stores of the whole form, times the column blocks under way) thrash what holds them.  Workgroups of 64 rows, an XCD its own columns,
+// write 590 MB in 0.54 ms instead of 1.5 (us, whole in order / whole by XCD / split by XCD: 1 codebook of 16 centroids, M = 4096 N = 36000
+// 1502 / 1234 / 541, N = 20000 496 / 597 / 315, M = 2048 N = 36000 320 / 400 / 267; 96 codebooks 8 centroids 1222 / 1338 / 754, 443 /
+// 615 / 412, 382 / 393 / 374, 16 centroids 1258 / 1316 / 932, 518 / 627 / 531, 454 / 400 / 490, 32 centroids 1684 / 1332 / 1432, 759 / 699 /
+// 868, 672 / 543 / 780; 32 codebooks 32 centroids 1302 / 1321 / 694, 441 / 617 / 394, 356 / 391 / 346; a scale per 8, M = 2048 N = 36000,
+// 96 codebooks of 8 centroids 424 / 394 / 583, 64 of 16 379 / 401 / 529).  Below: 12608 x 4096 172 / 266 /
+// 182; other widths: 36000 x 3072 364 / 464 / 423, x 4095 680 / 680 / 799.
+bool rows_of_8k(const Amm& a, uint32_t n)
+{
+    const uint64_t out_bytes = (uint64_t)n * a.g.M * 4;
+    return a.g.M % 2048 == 0 && out_bytes > (256ull << 20) && a.lut_bytes < out_bytes;
+}
+
 template <int C_T, int IDX_BITS, bool GROUPED, bool SPLIT>
 int launch_f32_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, uint32_t n)
 {
@@ -217,11 +231,13 @@ int launch_f32_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, ui
     // codebooks, N = 2048, M = 3072 86 / 116, N = 6664, M = 4096 347 / 375; 768 codebooks, N = 12608, M = 768 368 / 488; odd widths,
     // 128 codebooks, N = 9919, M = 4095 317 / 344; rows of up to 4 KiB, 1 codebook, 180 MB, M = 512 130 / 177, M = 1024 147 / 196,
     // M = 768 135 / 134; few tokens, 192 codebooks, N = 328, M = 2157 26 / 53).
-    // Uneven column blocks of the whole form only where the CUs of an XCD take at most an eighth more rounds (8 centroids, a scale per 8
-    // of 96 codebooks, N = 6444, M = 608, 38 column blocks 41.5 / 34.4).
+    // Rows of whole 8 KiB that together exceed the last cache are the exception: by XCD, in the split form where its chain is short and
+    // with 32 centroids (rows_of_8k).  Uneven column blocks of the whole form only where the CUs of an XCD take at most an eighth more
+    // rounds (8 centroids, a scale per 8 of 96 codebooks, N = 6444, M = 608, 38 column blocks 41.5 / 34.4).
     const uint64_t out_bytes = (uint64_t)n * a.g.M * 4;
     const uint64_t padded = (colblocks + 7) / 8 * 8, cus = ctx->prop.multiProcessorCount;
-    const bool wide_output = a.g.M % 4 == 0 && a.g.M > 1024 && out_bytes >= (40ull << 20) && a.lut_bytes < out_bytes;
+    const bool wide_output = a.g.M % 4 == 0 && a.g.M > 1024 && out_bytes >= (40ull << 20) && a.lut_bytes < out_bytes &&
+                             !((SPLIT || C_T == 32) && rows_of_8k(a, n));
     const bool even = 8 * (padded - colblocks) <= colblocks &&
                       (SPLIT || 8 * ((n_token_tiles * padded + cus - 1) / cus) <= 9 * (((uint64_t)n_token_tiles * colblocks + cus - 1) / cus));
     const uint32_t by_xcd = even && !wide_output ? 1u : 0u;
@@ -251,7 +267,9 @@ int launch_f32(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, uint3
     const double per_cu = (double)(a.g.M_pad / 16) / ctx->prop.multiProcessorCount;
     const double w = (n + 63) / 64 * per_cu, w1 = (n + F32_THREADS - 1) / F32_THREADS * per_cu;
     const double grow = (C_T == 8 ? (GROUPED ? 0.49 : 0.42) : 0.58) * w, grow1 = C_T == 32 ? 0.5 * w1 + 0.4 : 0.85 * w1 + 0.15;
-    if (0.57 * (grow > 1 ? grow : 1) < (grow1 > 1 ? grow1 : 1)) return launch_f32_as<C_T, IDX_BITS, GROUPED, true>(ctx, a, d_idx, d_out, n);
+    const bool short_chain = a.g.CB_pad <= (C_T == 32 ? 32u : C_T == 8 ? (GROUPED ? 64u : 96u) : (GROUPED ? 32u : 64u));
+    if ((short_chain && rows_of_8k(a, n)) || 0.57 * (grow > 1 ? grow : 1) < (grow1 > 1 ? grow1 : 1))
+        return launch_f32_as<C_T, IDX_BITS, GROUPED, true>(ctx, a, d_idx, d_out, n);
     return launch_f32_as<C_T, IDX_BITS, GROUPED, false>(ctx, a, d_idx, d_out, n);
 }
 

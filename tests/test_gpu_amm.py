@@ -1122,7 +1122,8 @@ def test_odd_widths_of_17_to_32_centroids_are_not_slower_than_the_sparse_gather(
 
 
 @pytest.mark.parametrize("N,CB,C,M", [(328, 40, 32, 2157), (1500, 33, 16, 905), (1500, 40, 8, 898), (3000, 33, 16, 140),   # column blocks: 135, 57, 57, 9
-                                      (2600, 33, 16, 4096), (2600, 3, 32, 4096), (2600, 40, 7, 4095)])                 # outputs of 40 MB
+                                      (2600, 33, 16, 4096), (2600, 3, 32, 4096), (2600, 40, 7, 4095),                  # outputs of 40 MB
+                                      (16400, 3, 16, 4096), (32801, 33, 32, 2048)])                                    # of 256 MB, rows of whole 8 KiB
 def test_float_tables_whose_column_blocks_do_not_divide_among_the_xcds(ctx, N, CB, C, M):
     """Column blocks dealt out by XCD with some past the last, and in order: every output bit, and the guard rows."""
     import torch
@@ -1169,6 +1170,24 @@ def test_few_tokens_of_64_centroids_take_the_large_gather_where_it_is_shorter(ct
     assert a < 1.2 * b, (a, b)
 
 
+def test_float_gathers_write_rows_of_whole_8_kib_as_fast_as_others(ctx):
+    """Outputs of 590 and 440 MB, one codebook (2.9 times as long per byte in workgroups of 256 tokens, column blocks in order)."""
+    a, b = (gather_us(ctx, 36000, 1, 16, M, "f32") / M for M in (4096, 3072))
+    assert a < 1.5 * b, (a, b)
+
+
+def test_float_gathers_of_uneven_column_blocks_do_not_wait_for_one_xcd(ctx):
+    """38 column blocks on 8 XCDs: 26 token tiles of them took a fifth round of the CUs (1.24 times as long as 24 tiles)."""
+    a, b = (gather_us(ctx, n, 96, 8, 608, group=8) for n in (6444, 6144))
+    assert a < 1.15 * b, (a, b)
+
+
+def test_grouped_float_gathers_take_whole_workgroups_from_two_per_cu_on(ctx):
+    """8 centroids, a scale per 8 codebooks: 3080 tokens in workgroups of 64 took 1.5 times as long as 3400 in workgroups of 256."""
+    a, b = (gather_us(ctx, n, 768, 8, 768, group=8) for n in (3080, 3400))
+    assert a < 1.2 * b, (a, b)
+
+
 def test_byte_adder_writes_whole_rows_of_outputs_beyond_the_caches(ctx):
     """24 centroids, one codebook, 450 MB: 1.2 times the sparse kernel's time when an XCD wrote its own columns of all rows."""
     rows, sparse = (gather_us(ctx, 36621, 1, 24, 3072, tuning={"gather_kernel": k}) for k in (pimdl.GATHER_ROWS, pimdl.GATHER_SPARSE))
@@ -1192,15 +1211,3 @@ def test_byte_adder_deals_outputs_beyond_the_caches_out_by_tokens(ctx, N, C, M):
     want = oracle.dequant(acc, bias, 3, 0.02, 0.0, 0, threads=THREADS)
     assert np.array_equal(got[pick].view(np.uint32), want.view(np.uint32)) and (got[N:] < -9e29).all() and (got[:N] > -9e29).all()
     amm.close()
-
-
-def test_grouped_float_gathers_take_whole_workgroups_from_two_per_cu_on(ctx):
-    """8 centroids, a scale per 8 codebooks: 3080 tokens in workgroups of 64 took 1.5 times as long as 3400 in workgroups of 256."""
-    a, b = (gather_us(ctx, n, 768, 8, 768, group=8) for n in (3080, 3400))
-    assert a < 1.2 * b, (a, b)
-
-
-def test_float_gathers_of_uneven_column_blocks_do_not_wait_for_one_xcd(ctx):
-    """38 column blocks on 8 XCDs: 26 token tiles of them took a fifth round of the CUs (1.24 times as long as 24 tiles)."""
-    a, b = (gather_us(ctx, n, 96, 8, 608, group=8) for n in (6444, 6144))
-    assert a < 1.15 * b, (a, b)
