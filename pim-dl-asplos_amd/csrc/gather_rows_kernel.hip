@@ -28,7 +28,7 @@
 // Measured (us; before: rows of one codebook side by side, dense matrix instruction; the floor is N * CB * M bytes at
 // 256 bytes per clock, CU and 2.4 GHz): N = 8192, 768 -> 3072, v = 4: 64 centroids 140 -> 61, 128 186 -> 74, 256
 // 338 -> 83 (floor 31); N = 12608, 32 centroids (before: the sparse one-hot kernel) 768 -> 3072 119 -> 94, 3072 -> 768
-// 122 -> 93 (floor 47).  Counters: no bank conflicts, LDS busy 61 % of the CUs' cycles at 64
+// 122 -> 93 (floor 47).  Counters: no bank conflicts, LDS busy 63 % of the CUs' cycles at 64
 // centroids and 73 % at 32; the rest is the copies of the slices (43 bytes per clock and CU), the barriers and the last items of
 // the grid.
 //
