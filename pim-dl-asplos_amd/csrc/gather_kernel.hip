@@ -882,8 +882,12 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
                 const uint32_t blocks = (M + 16 * tn - 1) / (16 * tn);
                 const uint64_t items = (uint64_t)tiles * blocks;
                 const uint64_t items_small = (uint64_t)((d.max_n + 127) / 128) * blocks;
-                const double t256 = grid_rounds(items, slots) * item_cost(tn, false);
-                const double t128 = grid_rounds(items_small, slots) * item_cost(tn, true);
+                // Outputs beyond the caches in rows of whole 16 KiB: 64 columns of a row are 256-byte pieces on their
+                // own memory channels, 96 are not (1024 -> 4096, N = 32768, us, 96 / 64 columns: v = 4 311 / 267, v = 8
+                // 218 / 161, v = 16 166 / 106; M = 3072, where no tile width meets the channels again: 163 / 174 at v = 4).
+                const double width = tn == 4 && M % 4096 == 0 && (uint64_t)d.max_n * M * 4 >= SP_LARGE_OUTPUT ? 0.9 : 1.0;
+                const double t256 = grid_rounds(items, slots) * item_cost(tn, false) * width;
+                const double t128 = grid_rounds(items_small, slots) * item_cost(tn, true) * width;
                 const double t = t128 < t256 ? t128 : t256;  // the launcher takes the better item size
                 if (t < best - 1e-9) {
                     best = t;

@@ -551,8 +551,18 @@ int launch_sparse_tm(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out,
     const uint32_t n_items = n_token_tiles * (a.g.M_pad / (16 * TN));
     uint32_t grid = ctx->prop.multiProcessorCount * sp_wgs_per_cu(TM, NW);
     if (grid > n_items) grid = n_items;
+    // Outputs that do not fit the last cache: an XCD takes its token tiles in blocks of about 1024 tokens (2048 with
+    // 64-column tiles) through all of its columns, so that the rows it is writing are written whole within a short time,
+    // instead of a few columns of all of its rows.  With more tokens to a block fewer workgroups share the rows, with fewer
+    // every column's table is fetched again for each of them.  Tiles of 64 / 96 columns, N = 32768, us without blocks and with
+    // blocks of 512, 1024, 2048, 4096 tokens: 24 codebooks, M = 3072 91 80 79 79 85 / 78 67 68 68 68; M = 4096 117 105 106 107 106 /
+    // 140 113 120 128 140; 192 codebooks, M = 3072 185 174 176 174 172 / 177 165 163 164 164; M = 4096 236 230 236 231 233 /
+    // 271 232 236 233 265; N = 16384, 48 codebooks, M = 4096 76 64 62 58 57 / 58 67 58 58 57.  Not below: N = 16384, M = 3072 (201 MB),
+    // 192 codebooks 83 84 84 84 85 / 80 83 84 81 84, 24 codebooks 35 36 36 36 36 / 37 37 37 37 38.
+    const bool blocks = (uint64_t)n * a.g.M * 4 >= SP_LARGE_OUTPUT;
+    const uint32_t tok_block = !blocks ? 0 : (TN == 4 ? 2048 : 1024) / TOK_ITEM;
     const XcdMap xmap = choose_xcd_map(a.g.M_pad / (16 * TN), n_token_tiles, grid, (uint64_t)cb16 * 16 * a.g.M_pad,
-                                       (uint64_t)n * a.g.idx_row_bytes, a.g.tune_xcd_col_split);
+                                       (uint64_t)n * a.g.idx_row_bytes, a.g.tune_xcd_col_split, tok_block);
     if (KS == 1) snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_kernel<%d, %d, %d, %d, %s>", TN, TM, GS, NW, WIDE ? "true" : "false");
     else snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_kernel<%d, %d, %d, %d, %s, %d>", TN, TM, GS, NW, WIDE ? "true" : "false", KS);
     a.note_launch(GS, LDS, TOK_ITEM, NW * 64);

@@ -1067,6 +1067,39 @@ def test_matrix_core_gathers_at_ragged_sizes(ctx, kernel, C, widths, N, CB, M):
         amm.close()
 
 
+@pytest.mark.parametrize("N,M,tuning", [(16384, 4096, {}), (16640, 4160, {}), (17000, 4001, {}), (34000, 2112, {"col_block": 48}),
+                                        (33792, 2048, {"col_block": 64, "xcd_col_split": 2}), (65600, 1030, {"token_item": 128}),
+                                        (17408, 4096, {"col_block": 96, "xcd_col_split": pimdl.XCD_PLAIN})])
+def test_sparse_gather_of_large_outputs(ctx, N, M, tuning):
+    """Outputs from 256 MiB on go through the launch in blocks of token tiles, dealt by XCD or in plain order, the last block smaller:
+    every row as in launches of a few thousand tokens, which have no blocks, and nothing behind the output."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the sparse gather")
+    import torch
+    assert N * M * 4 >= 256 << 20
+    v, CB, C = 4, 8, 16
+    _, cent, lut, bias = make_case(515 + M, 1, CB * v, v, C, M)
+    x = torch.randn((N, CB * v), device="cuda", generator=torch.Generator(device="cuda").manual_seed(N))
+    amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=N, tuning=tuning)
+    out = torch.full((N + 2, M), -5.0, device="cuda")
+    part = torch.empty((4096, M), device="cuda")
+    torch.cuda.synchronize()
+    amm.run_ptr(x.data_ptr(), N, out.data_ptr())
+    ctx.synchronize()
+    assert amm.last_gather_kernel().startswith("gather_sparse_kernel<"), amm.last_gather_kernel()
+    assert bool((out[N:] == -5.0).all())
+    for i in range(0, N, 4096):
+        n = min(4096, N - i)
+        torch.cuda.synchronize()
+        amm.run_ptr(x[i:].data_ptr(), n, part.data_ptr())
+        ctx.synchronize()
+        assert torch.equal(out[i:i + n], part[:n]), i
+    n = 300
+    want = oracle.amm_cpu(x[:n].cpu().numpy(), cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)[0]
+    assert np.array_equal(out[:n].cpu().numpy().view(np.uint32), want.view(np.uint32))
+    amm.close()
+
+
 def gather_us(ctx, N, CB, C, M, lut="i8", tuning=None, v=4, group=0):
     """Shortest of a few timings of an operator's gather, us."""
     import torch
