@@ -9,6 +9,8 @@
 // instead of sequentially, which can move the float mean or variance by one ulp in rare rows.
 // The centred value x - mean is computed once and reused (the reference computes the identical
 // expression twice).
+#include <type_traits>
+
 #include "pimdl_internal.h"
 
 namespace pimdl {
@@ -172,11 +174,12 @@ __global__ __launch_bounds__(256) void layer_norm_vec_kernel(const float* __rest
 // KQ = K Q, scale by 1/sqrt(head_dim), soft_max, V KQ, permute back to [n][token_dim]); inputs and
 // output stay in the layer's [token][head * 64 + d] order, so no head transposes are needed.
 //
-// A workgroup = 64 queries of one (batch, head), a wave = 16 of them.  Keys come in chunks of 128
-// through LDS (K, then V in the same buffer; V is fetched into registers while the scores are computed from
-// K), with the running maximum / sum of a streaming softmax between chunks; 16-key tiles past the end of
-// the sequence are skipped.  Both products run on v_mfma_f32_16x16x4_f32, transposed so that nothing has to
-// change lanes in between:
+// A workgroup = 64 queries of one (batch, head), a wave = 16 of them.  Keys are taken in chunks of 128, with the running
+// maximum / sum of a streaming softmax between chunks.  A chunk's K and then its V go through LDS in pieces of 32 keys, copied without
+// registers (global_load_lds) into a ring of four: when a piece is worked on, the next two have been requested and the
+// third goes into the place of the piece before, so there is one barrier per piece and the first products wait for 32 keys, not
+// for 128.  Key tiles of 16 past the end of the sequence are skipped.  Both products run on v_mfma_f32_16x16x4_f32,
+// transposed so that nothing has to change lanes in between:
 //   S^T[key][query]  = K Q^T:  A = K rows (keys), B = this lane's query, 16 steps of 4 dims.  The K
 //                      index of lane group g in step s is dim 16 g + s (a sum does not care in which
 //                      order its terms are paired), so a lane's operands are 16 consecutive floats.
@@ -184,99 +187,181 @@ __global__ __launch_bounds__(256) void layer_norm_vec_kernel(const float* __rest
 //   out^T[d][query] += V^T P^T: the B operand of step (kt, i) is that very register (key 16 kt + 4 g + i
 //                      from group g), A = V[that key][16 dt + j].  Result: lane (j, g) holds dims
 //                      16 dt + 4 g + i of its query: one float4 store per 16-dim tile.
-// LDS rows are 68 floats apart: 16 keys x 4 groups (first product) and 16 dims x 4 keys (second) then
-// fall into 64 different banks.
+// A row of a piece is 64 floats, all LDS banks once.  Rows lie in fours, 64 bytes between one four and the next, and the 16-byte
+// parts of a row in the order part ^ (row % 4): so the 16 keys x 4 groups of the first product's reads and the 16 dims x 4 keys
+// of the second's fall into different banks, and everything but the lane's own place is an immediate offset of the read.
+// What bounds it: the fp32 matrix instructions and the vector ones share a unit, so the kernel takes the sum of their
+// times; everything that a whole chunk does not need (masks, clamped rows, zeroed rows) is compiled for the last chunk alone.
+// us, before (whole chunks through registers, four barriers each, masks in every chunk, three workgroups per CU) / now, same bits:
+// 32 x 128 tokens, 12 heads 24.6 / 21.4; 64 x 128, 16 heads 51.9 / 46; 64 x 197, 12 heads 112 / 102; 16 x 512, 12 heads 131 / 115 (82 of
+// them matrix instructions at 2.4 GHz); 300 x 17, 12 heads 33 / 27; 1 x 128, 12 heads 9.9 / 8.2.  (The ring alone, with the masks and
+// clamped addresses left in every chunk: 24.5, 51.3, 112.8, 129, 41, 10.2 -- it is the vector instructions that count.)
 // ---------------------------------------------------------------------------------------------
-constexpr int AT_KC = 128, AT_PITCH = 68, AT_THREADS = 256;
+constexpr int AT_KC = 128, AT_PK = 32, AT_PIECES = AT_KC / AT_PK, AT_THREADS = 256;
+constexpr int AT_FOUR = 4 * 256 + 64, AT_TILE = 4 * AT_FOUR, AT_PIECE_BYTES = 2 * AT_TILE;  // bytes of 4, 16 and 32 rows
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(AT_THREADS, 3) void attention_hd64_kernel(const float* __restrict__ q,
+template <int OFF>
+__device__ __forceinline__ void at_read(v4f& dst, uint32_t addr)
+{
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
+}
+template <int OFF>
+__device__ __forceinline__ void at_read(float& dst, uint32_t addr)
+{
+    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
+}
+template <int N>
+__device__ __forceinline__ void at_lgkm_wait()
+{
+    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+__global__ __launch_bounds__(AT_THREADS, 4) void attention_hd64_kernel(const float* __restrict__ q,
                                                                    const float* __restrict__ k,
                                                                    const float* __restrict__ v,
                                                                    float* __restrict__ out, uint32_t S,
                                                                    uint32_t in_stride, uint32_t out_stride,
                                                                    float scale)
 {
-    __shared__ __attribute__((aligned(16))) float kv[AT_KC * AT_PITCH];
+    __shared__ __attribute__((aligned(1024))) unsigned char kv[AT_PIECES * AT_PIECE_BYTES];
     const uint32_t h = blockIdx.y, b = blockIdx.z;
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t j = lane & 15, g = lane >> 4;
     const size_t in_base = (size_t)b * S * in_stride + (size_t)h * 64;
     const uint32_t q_tok = blockIdx.x * 64 + wave * 16 + j;
     const uint32_t q_tok_c = q_tok < S ? q_tok : S - 1;  // rows past S repeat the last query; never stored
 
-    float qreg[16];
+    v4f qraw[4];
     {
         const float* qp = q + in_base + (size_t)q_tok_c * in_stride + 16 * g;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4 t = *reinterpret_cast<const float4*>(qp + 4 * i);
-            qreg[4 * i + 0] = t.x * scale;
-            qreg[4 * i + 1] = t.y * scale;
-            qreg[4 * i + 2] = t.z * scale;
-            qreg[4 * i + 3] = t.w * scale;
-        }
+        for (int i = 0; i < 4; ++i) qraw[i] = *reinterpret_cast<const v4f*>(qp + 4 * i);
     }
-    // 128 keys x 64 floats, zero past S: into registers (eight 16-byte pieces per thread), then into LDS.  The two
-    // halves are separate so that V is already on its way while the scores are computed from K.
-    constexpr int AT_PIECES = AT_KC * 16 / AT_THREADS;
-    auto fetch_chunk = [&](float4 (&r)[AT_PIECES], const float* src, uint32_t kc) {
+    // Copies this wave's 8 rows of a piece (two operations of 4 rows).  CLAMP: rows past the sequence repeat its last one.
+    const uint32_t part = (j & 12) | ((j & 3) ^ g);  // that this lane copies of its row
+    const size_t copy_off[2] = {((size_t)(wave * 8 + g) * in_stride + 4 * part) * 4, ((size_t)(wave * 8 + 4 + g) * in_stride + 4 * part) * 4};
+    auto copy_piece = [&](const float* src, uint32_t key0, auto slotc, auto clampc) __attribute__((always_inline)) {
+        constexpr int slot = decltype(slotc)::value;
 #pragma unroll
-        for (int p = 0; p < AT_PIECES; ++p) {
-            const uint32_t i = threadIdx.x + p * AT_THREADS, key = i / 16, c4 = i % 16, tok = kc + key;
-            r[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (tok < S) r[p] = *reinterpret_cast<const float4*>(src + in_base + (size_t)tok * in_stride + 4 * c4);
+        for (int u = 0; u < 2; ++u) {
+            const char* p;
+            if constexpr (decltype(clampc)::value) {
+                const uint32_t key = key0 + wave * 8 + 4 * u + g, tok = key < S ? key : S - 1;
+                p = reinterpret_cast<const char*>(src + in_base + (size_t)tok * in_stride + 4 * part);
+            } else {
+                p = reinterpret_cast<const char*>(src + in_base + (size_t)key0 * in_stride) + copy_off[u];
+            }
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)p,
+                                             (__attribute__((address_space(3))) void*)(kv + slot * AT_PIECE_BYTES + (2 * wave + u) * AT_FOUR), 16, 0, 0);
         }
     };
-    auto store_chunk = [&](const float4 (&r)[AT_PIECES]) {
-#pragma unroll
-        for (int p = 0; p < AT_PIECES; ++p) {
-            const uint32_t i = threadIdx.x + p * AT_THREADS, key = i / 16, c4 = i % 16;
-            *reinterpret_cast<float4*>(&kv[key * AT_PITCH + 4 * c4]) = r[p];
-        }
+    // The piece about to be used has landed (`behind` operations have been issued since), then everybody's part of it; after
+    // that everybody is done with the piece before.
+    auto arrive = [&](auto behindc) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(behindc)::value) : "memory");
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
     };
-    float4 stage[AT_PIECES];
+    const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)kv);
+    // K rows: part 4 g + i of row j; V: float j % 4 of part 4 dt + j / 4 of row 4 g + i
+    uint32_t k_addr[4], v_addr[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        k_addr[i] = lds0 + j / 4 * AT_FOUR + j % 4 * 256 + (4 * g + (i ^ (j & 3))) * 16;
+        v_addr[i] = lds0 + g * AT_FOUR + i * 256 + ((j / 4) ^ i) * 16 + (j % 4) * 4;
+    }
+
+    constexpr std::integral_constant<int, 0> c0;
+    constexpr std::integral_constant<int, 1> c1;
+    constexpr std::integral_constant<int, 2> c2;
+    constexpr std::integral_constant<int, 3> c3;
+    // The three pieces that the chunk at kc begins with: of K -- or, where at most 64 keys are left (short chunk), K, K and V,
+    // whose places are 2 and 3 then.
+    auto begin_piece = [&](uint32_t kc, auto pc) __attribute__((always_inline)) {
+        constexpr int p = decltype(pc)::value;
+        if (kc + AT_KC <= S) copy_piece(k, kc + p * AT_PK, pc, std::false_type{});
+        else if (p < 2 || kc + 2 * AT_PK < S) copy_piece(k, kc + p * AT_PK, pc, std::true_type{});
+        else copy_piece(v, kc, pc, std::true_type{});
+    };
+    begin_piece(0, c0);
+    begin_piece(0, c1);
+    begin_piece(0, c2);
+    float qreg[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) qreg[i] = qraw[i / 4][i % 4] * scale;
 
     float m_run = -__builtin_inff(), l_run = 0.0f;
     v4f o[4];
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt) o[dt] = (v4f){0.f, 0.f, 0.f, 0.f};
 
-    for (uint32_t kc = 0; kc < S; kc += AT_KC) {
-        fetch_chunk(stage, k, kc);
-        __syncthreads();  // the previous chunk's V has been consumed
-        store_chunk(stage);
-        __syncthreads();
-        fetch_chunk(stage, v, kc);  // lands while the scores are computed
-        v4f s[AT_KC / 16];
+    // WHOLE: 128 keys, SHORT: at most 64; LAST: no chunk follows
+    auto chunk = [&](uint32_t kc, auto wholec, auto shortc, auto lastc) __attribute__((always_inline)) {
+        constexpr bool WHOLE = decltype(wholec)::value, SHORT = decltype(shortc)::value, LAST = decltype(lastc)::value;
+        constexpr std::bool_constant<!WHOLE> tail;
+        constexpr int TILES = SHORT ? 4 : AT_KC / 16, V0 = SHORT ? 2 : 0;  // key tiles; place of the first piece of V
+        const bool two = kc + AT_PK < S;  // (SHORT) pieces
+        v4f s[TILES];
+        auto scores = [&](auto pc) __attribute__((always_inline)) {
+            constexpr int p = decltype(pc)::value;
+            v4f a[2][4];
+            auto request = [&](auto tc) {
+                constexpr int t = decltype(tc)::value, off = p * AT_PIECE_BYTES + t * AT_TILE;
+                at_read<off>(a[t][0], k_addr[0]);
+                at_read<off>(a[t][1], k_addr[1]);
+                at_read<off>(a[t][2], k_addr[2]);
+                at_read<off>(a[t][3], k_addr[3]);
+            };
+            auto product = [&](auto tc) {
+                constexpr int t = decltype(tc)::value, kt = 2 * p + t;
 #pragma unroll
-        for (int kt = 0; kt < AT_KC / 16; ++kt) {
-            if (kc + 16 * kt >= S) {  // (uniform) a key tile past the sequence: nothing to compute
+                for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(a[t][i]));
                 s[kt] = (v4f){0.f, 0.f, 0.f, 0.f};
-                continue;
-            }
-            const float* kp = kv + (16 * kt + j) * AT_PITCH + 16 * g;
-            float areg[16];
+                if (WHOLE || kc + 16 * kt < S) {  // (uniform) else a key tile past the sequence: nothing to compute
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float4 t = *reinterpret_cast<const float4*>(kp + 4 * i);
-                areg[4 * i + 0] = t.x;
-                areg[4 * i + 1] = t.y;
-                areg[4 * i + 2] = t.z;
-                areg[4 * i + 3] = t.w;
+                    for (int st = 0; st < 16; ++st) s[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t][st / 4][st % 4], qreg[st], s[kt], 0, 0, 0);
+                }
+            };
+            request(c0);
+            request(c1);
+            at_lgkm_wait<4>();
+            product(c0);
+            at_lgkm_wait<0>();
+            product(c1);
+        };
+        arrive(std::integral_constant<int, 4>{});
+        if constexpr (SHORT) {
+            if (two) copy_piece(v, kc + AT_PK, c3, tail);
+            scores(c0);
+            if (two) {
+                arrive(std::integral_constant<int, 4>{});
+                scores(c1);
+            } else {
+                s[2] = s[3] = (v4f){0.f, 0.f, 0.f, 0.f};
             }
-            v4f acc = (v4f){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int st = 0; st < 16; ++st) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(areg[st], qreg[st], acc, 0, 0, 0);
-            s[kt] = acc;
+        } else {
+            copy_piece(k, kc + 3 * AT_PK, c3, tail);
+            scores(c0);
+            arrive(std::integral_constant<int, 4>{});
+            copy_piece(v, kc, c0, tail);
+            scores(c1);
+            arrive(std::integral_constant<int, 4>{});
+            copy_piece(v, kc + AT_PK, c1, tail);
+            scores(c2);
+            arrive(std::integral_constant<int, 4>{});
+            copy_piece(v, kc + 2 * AT_PK, c2, tail);
+            scores(c3);
         }
+
         // keys past S do not take part
         float mx = -__builtin_inff();
 #pragma unroll
-        for (int kt = 0; kt < AT_KC / 16; ++kt)
+        for (int kt = 0; kt < TILES; ++kt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                if (kc + 16 * kt + 4 * g + i >= S) s[kt][i] = -__builtin_inff();
+                if (!WHOLE && kc + 16 * kt + 4 * g + i >= S) s[kt][i] = -__builtin_inff();
                 mx = fmaxf(mx, s[kt][i]);
             }
         mx = fmaxf(mx, __shfl_xor(mx, 16));
@@ -285,7 +370,7 @@ __global__ __launch_bounds__(AT_THREADS, 3) void attention_hd64_kernel(const flo
         const float alpha = __expf(m_run - m_new);  // 0 for the first chunk
         float psum = 0.0f;
 #pragma unroll
-        for (int kt = 0; kt < AT_KC / 16; ++kt)
+        for (int kt = 0; kt < TILES; ++kt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float p = __expf(s[kt][i] - m_new);
@@ -299,21 +384,102 @@ __global__ __launch_bounds__(AT_THREADS, 3) void attention_hd64_kernel(const flo
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) o[dt] *= alpha;
 
-        __syncthreads();  // every wave is done with K
-        store_chunk(stage);
-        __syncthreads();
+        // rows of V past the sequence must be zeros (their probabilities are, but zero times infinity is not)
+        auto zero_rows = [&](auto pc) {
+            constexpr int p = decltype(pc)::value;
+            const uint32_t key0 = kc + p * AT_PK;
+            if (WHOLE || key0 + AT_PK <= S || key0 >= S) return;  // (uniform)
 #pragma unroll
-        for (int kt = 0; kt < AT_KC / 16; ++kt) {
-            if (kc + 16 * kt >= S) continue;  // (uniform) its probabilities are all zero
+            for (int u = 0; u < 2; ++u)
+                if (key0 + wave * 8 + 4 * u + g >= S)
+                    *reinterpret_cast<v4f*>(kv + (V0 + p) * AT_PIECE_BYTES + (2 * wave + u) * AT_FOUR + lane * 16) = (v4f){0.f, 0.f, 0.f, 0.f};
+        };
+        auto values = [&](auto pc) __attribute__((always_inline)) {
+            constexpr int p = decltype(pc)::value;
+            float a[4][4];
+            auto request = [&](auto tc, auto ic) {
+                constexpr int off = (V0 + p) * AT_PIECE_BYTES + decltype(tc)::value * AT_TILE, i = decltype(ic)::value;
+                at_read<off>(a[i][0], v_addr[i]);
+                at_read<off + 64>(a[i][1], v_addr[i]);
+                at_read<off + 128>(a[i][2], v_addr[i]);
+                at_read<off + 192>(a[i][3], v_addr[i]);
+            };
+            auto product = [&](auto tc, auto ic) {
+                constexpr int kt = 2 * p + decltype(tc)::value, i = decltype(ic)::value;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float* vp = kv + (16 * kt + 4 * g + i) * AT_PITCH + j;
+                for (int dt = 0; dt < 4; ++dt) asm volatile("" : "+v"(a[i][dt]));
+                if (WHOLE || kc + 16 * kt < S) {  // (uniform) else its probabilities are all zero
 #pragma unroll
-                for (int dt = 0; dt < 4; ++dt)
-                    o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vp[16 * dt], s[kt][i], o[dt], 0, 0, 0);
+                    for (int dt = 0; dt < 4; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][dt], s[kt][i], o[dt], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            request(c0, c0);
+            request(c0, c1);
+            request(c0, c2);
+            request(c0, c3);
+            at_lgkm_wait<12>();
+            product(c0, c0);
+            request(c1, c0);
+            at_lgkm_wait<12>();
+            product(c0, c1);
+            request(c1, c1);
+            at_lgkm_wait<12>();
+            product(c0, c2);
+            request(c1, c2);
+            at_lgkm_wait<12>();
+            product(c0, c3);
+            request(c1, c3);
+            at_lgkm_wait<12>();
+            product(c1, c0);
+            at_lgkm_wait<8>();
+            product(c1, c1);
+            at_lgkm_wait<4>();
+            product(c1, c2);
+            at_lgkm_wait<0>();
+            product(c1, c3);
+        };
+        auto arrive_v = [&](auto pc, auto behindc) {  // (behindc: where no chunk follows)
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LAST ? decltype(behindc)::value : 4) : "memory");
+            zero_rows(pc);
+            __syncthreads();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto next_piece = [&](auto pc) {
+            if constexpr (!LAST) begin_piece(kc + AT_KC, pc);
+        };
+        if constexpr (SHORT) {
+            if (two) {
+                arrive_v(c0, std::integral_constant<int, 2>{});
+                values(c0);
+                arrive_v(c1, std::integral_constant<int, 0>{});
+                values(c1);
+            } else {
+                arrive_v(c0, std::integral_constant<int, 0>{});
+                values(c0);
             }
+        } else {
+            arrive_v(c0, std::integral_constant<int, 4>{});
+            copy_piece(v, kc + 3 * AT_PK, c3, tail);
+            values(c0);
+            arrive_v(c1, std::integral_constant<int, 4>{});
+            next_piece(c0);
+            values(c1);
+            arrive_v(c2, std::integral_constant<int, 2>{});
+            next_piece(c1);
+            values(c2);
+            arrive_v(c3, std::integral_constant<int, 0>{});
+            next_piece(c2);
+            values(c3);
         }
-    }
+    };
+    constexpr std::true_type yes;
+    constexpr std::false_type no;
+    uint32_t kc = 0;
+    for (; kc + AT_KC < S; kc += AT_KC) chunk(kc, yes, no, no);
+    if (kc + AT_KC == S) chunk(kc, yes, no, yes);
+    else if (kc + 2 * AT_PK < S) chunk(kc, no, no, yes);
+    else chunk(kc, no, yes, yes);
     if (q_tok < S) {
         const float inv = 1.0f / l_run;
         float* op = out + ((size_t)b * S + q_tok) * out_stride + (size_t)h * 64 + 4 * g;

@@ -124,6 +124,31 @@ def test_attention_kernel_against_float64(ctx, B, S, H, fused):
         ctx.attention_ptr(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), B, S, H, 32, in_stride, D, 0.125)
 
 
+@pytest.mark.parametrize("S", [1, 31, 32, 33, 63, 64, 65, 96, 97, 127, 128, 129, 160, 191, 192, 193, 256, 257])
+def test_attention_at_the_edges_of_its_pieces(ctx, S):
+    """Keys go through LDS 32 at a time, 128 to a chunk, the last chunk in a form of its own up to 64 and beyond: every length at an
+    edge against float64, with infinities and NaN in the rows behind each sequence (the next head batch's), which must not leak in,
+    and nothing written behind the output."""
+    import torch
+    B, H = 2, 2
+    D, n = H * 64, B * S
+    gen = torch.Generator(device="cuda").manual_seed(S)
+    buf = torch.randn((n + 128, 3 * D), device="cuda", generator=gen) * 2.0
+    buf[n:] = float("nan")
+    buf[n:, ::2] = float("inf")
+    out = torch.full((n + 2, D), -5.0, device="cuda")
+    at = buf.data_ptr()
+    torch.cuda.synchronize()
+    ctx.attention_ptr(at, at + 4 * D, at + 8 * D, out.data_ptr(), B, S, H, 64, 3 * D, D, 0.125)
+    ctx.synchronize()
+    q64, k64, v64 = (buf[:n, i * D:(i + 1) * D].double().cpu().reshape(B, S, H, 64).permute(0, 2, 1, 3).contiguous() for i in range(3))
+    p = torch.softmax(q64 @ k64.transpose(-1, -2).contiguous() * 0.125, dim=-1)
+    want = (p @ v64).permute(0, 2, 1, 3).reshape(n, D)
+    assert bool((out[n:] == -5.0).all())
+    # as test_attention_kernel_against_float64
+    torch.testing.assert_close(out[:n].double().cpu(), want, rtol=1e-5, atol=1e-5)
+
+
 def test_qkv_modes_give_the_same_bits(ctx):
     """Q/K/V as a group (one search launch), on three streams, and one by one."""
     import torch
