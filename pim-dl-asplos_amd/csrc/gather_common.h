@@ -62,22 +62,27 @@ inline bool prefer_small_items(uint64_t items256, uint64_t items128, uint64_t sl
 struct XcdMap {
     uint32_t col_split, tok_split, tok_per_xcd;  // tok_per_xcd = n_token_tiles / tok_split
     uint32_t tok_block, block_items;             // block_items = tok_block x the column tiles that a block goes through
+    // BLOCKS: a kernel for launches with tok_block (the divisions more are latency that a launch of few slices would feel)
+    template <bool BLOCKS = false>
     __device__ __forceinline__ void decode(uint32_t p, uint32_t n_token_tiles, uint32_t& col, uint32_t& tok) const
     {
-        const uint32_t x = col_split ? p % 8 : 0, q = col_split ? p / 8 : p;
-        const uint32_t tiles = col_split ? tok_per_xcd : n_token_tiles;
-        uint32_t c = q / tiles, t = q % tiles;
-        if (tok_block) {
+        if constexpr (BLOCKS) {
+            const uint32_t x = col_split ? p % 8 : 0, q = col_split ? p / 8 : p;
+            const uint32_t tiles = col_split ? tok_per_xcd : n_token_tiles;
             const uint32_t block = q / block_items, r = q % block_items, first = block * tok_block;
             const uint32_t width = tiles - first < tok_block ? tiles - first : tok_block;  // the last one may be smaller
-            c = r / width;
-            t = first + r % width;
+            // (the same in every lane: the positions are)
+            const uint32_t c = __builtin_amdgcn_readfirstlane(r / width), t = __builtin_amdgcn_readfirstlane(first + r % width);
+            col = col_split ? x % col_split + col_split * c : c;
+            tok = col_split ? x / col_split + tok_split * t : t;
+        } else if (col_split == 0) {
+            col = p / n_token_tiles;
+            tok = p % n_token_tiles;
+        } else {
+            const uint32_t x = p % 8, q = p / 8;
+            col = x % col_split + col_split * (q / tok_per_xcd);
+            tok = x / col_split + tok_split * (q % tok_per_xcd);
         }
-        // (the same in every lane: the positions are)
-        c = __builtin_amdgcn_readfirstlane(c);
-        t = __builtin_amdgcn_readfirstlane(t);
-        col = col_split ? x % col_split + col_split * c : c;
-        tok = col_split ? x / col_split + tok_split * t : t;
     }
 };
 
@@ -88,10 +93,10 @@ inline XcdMap choose_xcd_map(uint32_t n_col_tiles, uint32_t n_token_tiles, uint3
                              uint64_t idx_bytes, uint32_t forced = 0, uint32_t tok_block = 0)
 {
     auto dealt = [&](uint32_t cs) {
-        const uint32_t per_xcd = n_token_tiles / (8 / cs), block = tok_block < per_xcd ? tok_block : 0;
+        const uint32_t per_xcd = n_token_tiles / (8 / cs), block = tok_block < per_xcd ? tok_block : tok_block ? per_xcd : 0;
         return XcdMap{cs, 8 / cs, per_xcd, block, block * (n_col_tiles / cs)};
     };
-    const uint32_t plain_block = 8 * tok_block < n_token_tiles ? 8 * tok_block : 0;
+    const uint32_t plain_block = 8 * tok_block < n_token_tiles ? 8 * tok_block : tok_block ? n_token_tiles : 0;
     XcdMap best{0, 0, 0, plain_block, plain_block * n_col_tiles};
     if (grid % 8 != 0 || forced == PIMDL_XCD_PLAIN) return best;
     if (forced && n_col_tiles % forced == 0 && n_token_tiles % (8 / forced) == 0) return dealt(forced);

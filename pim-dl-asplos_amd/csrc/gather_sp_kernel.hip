@@ -117,8 +117,9 @@ __device__ __forceinline__ T* uniform_ptr(T* p)
 // KS = 2 (eight waves): waves w and w + 4 hold the same 64 tokens and take one half of every slice's codebooks each;
 // the halves are added through LDS before the epilogue.  An item is then 256 tokens: a launch too small to give
 // every CU a 512-token item still fills the chip with TM = 4 tiles and copies a slice once per 256 tokens.
-template <int TN, int TM, int GS, int NW, bool WIDE, int KS = 1>
-__global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TM, NW) * NW / 4 /* waves per SIMD */) void gather_sparse_kernel(
+// BLOCKS: the launch deals its items in blocks of token tiles (XcdMap).
+template <int TN, int TM, int GS, int NW, bool WIDE, int KS, bool BLOCKS>
+__device__ __forceinline__ void gather_sparse(
     const uint8_t* __restrict__ idx, const int8_t* __restrict__ lut, float* __restrict__ out,
     int32_t* __restrict__ acc_out, uint32_t N, uint32_t M, uint32_t CB_pad, uint32_t idx_row_bytes,
     uint32_t n_token_tiles, uint32_t n_items, Epilogue ep, XcdMap xmap)
@@ -192,8 +193,8 @@ __global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TM, NW) * NW / 4 /* waves pe
         reinterpret_cast<uint32_t*>(smem + POS0)[b] = word;
     }
 
-    auto col_of = [&](uint32_t p) { uint32_t c, t; xmap.decode(p, n_token_tiles, c, t); return c; };
-    auto tok_tile_of = [&](uint32_t p) { uint32_t c, t; xmap.decode(p, n_token_tiles, c, t); return t; };
+    auto col_of = [&](uint32_t p) { uint32_t c, t; xmap.decode<BLOCKS>(p, n_token_tiles, c, t); return c; };
+    auto tok_tile_of = [&](uint32_t p) { uint32_t c, t; xmap.decode<BLOCKS>(p, n_token_tiles, c, t); return t; };
     uint32_t lut_item = blockIdx.x, lut_s = 0, ix_item = blockIdx.x, ix_s = 0;
     const int8_t* dma_base;   // uniform: start of the slice at the LUT stream position
     const uint8_t* ix_base;   // uniform: the 256-byte block of index words at the index stream position
@@ -312,7 +313,7 @@ __global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TM, NW) * NW / 4 /* waves pe
         asm volatile("" : "+v"(je), "+v"(ge));  // keeps the address arithmetic below out of the slice loop
         const uint32_t colblk = col_of(item);
         Epilogue epl = ep;
-        if (ep.op_col_tiles) epl.scale = scalar_load1(ep.op_scales + colblk / ep.op_col_tiles);
+        if (ep.op_col_tiles) epl.scale = scalar_load1(ep.op_scales + __builtin_amdgcn_readfirstlane(colblk / ep.op_col_tiles));
         const uint32_t tile_tok0 = tok_tile_of(item) * TOK_ITEM;
         const uint32_t tok0 = tile_tok0 + tw * (TM * 16) + 4 * ge;
         const bool vec_ok = (M % 4 == 0);
@@ -537,14 +538,32 @@ __global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TM, NW) * NW / 4 /* waves pe
     }
 }
 
-template <int TN, int TM, int GS, int NW = 4, bool WIDE = false, int KS = 1>
-int launch_sparse_tm(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc, uint32_t n,
+template <int TN, int TM, int GS, int NW, bool WIDE, int KS = 1>
+__global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TM, NW) * NW / 4 /* waves per SIMD */) void gather_sparse_kernel(
+    const uint8_t* __restrict__ idx, const int8_t* __restrict__ lut, float* __restrict__ out, int32_t* __restrict__ acc_out, uint32_t N,
+    uint32_t M, uint32_t CB_pad, uint32_t idx_row_bytes, uint32_t n_token_tiles, uint32_t n_items, Epilogue ep, XcdMap xmap)
+{
+    gather_sparse<TN, TM, GS, NW, WIDE, KS, false>(idx, lut, out, acc_out, N, M, CB_pad, idx_row_bytes, n_token_tiles, n_items, ep, xmap);
+}
+template <int TN, int TM, int GS, int NW>
+__global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TM, NW) * NW / 4) void gather_sparse_blocks_kernel(
+    const uint8_t* __restrict__ idx, const int8_t* __restrict__ lut, float* __restrict__ out, int32_t* __restrict__ acc_out, uint32_t N,
+    uint32_t M, uint32_t CB_pad, uint32_t idx_row_bytes, uint32_t n_token_tiles, uint32_t n_items, Epilogue ep, XcdMap xmap)
+{
+    gather_sparse<TN, TM, GS, NW, false, 1, true>(idx, lut, out, acc_out, N, M, CB_pad, idx_row_bytes, n_token_tiles, n_items, ep, xmap);
+}
+
+template <int TN, int TM, int GS, int NW, bool WIDE, int KS, bool BLOCKS>
+int launch_sparse_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc, uint32_t n,
                      const Epilogue& ep)
 {
     constexpr int LDS = sp_lds_bytes_tm(TN, TM, GS, NW, WIDE, KS);
     static_assert(sp_wgs_per_cu(TM, NW) * LDS <= 160 * 1024, "the CU's LDS holds the workgroups that its registers hold");
     constexpr int TOK_ITEM = sp_tok_item(TM, NW / KS);
-    auto kern = gather_sparse_kernel<TN, TM, GS, NW, WIDE, KS>;
+    auto kern = [] {
+        if constexpr (BLOCKS) return gather_sparse_blocks_kernel<TN, TM, GS, NW>;
+        else return gather_sparse_kernel<TN, TM, GS, NW, WIDE, KS>;
+    }();
     const uint32_t cb16 = sparse_codebooks(a.g);  // codebooks of 16 centroids in the tiled table
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_sparse)")) return rc;
     const uint32_t n_token_tiles = (n + TOK_ITEM - 1) / TOK_ITEM;
@@ -559,16 +578,25 @@ int launch_sparse_tm(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out,
     // 140 113 120 128 140; 192 codebooks, M = 3072 185 174 176 174 172 / 177 165 163 164 164; M = 4096 236 230 236 231 233 /
     // 271 232 236 233 265; N = 16384, 48 codebooks, M = 4096 76 64 62 58 57 / 58 67 58 58 57.  Not below: N = 16384, M = 3072 (201 MB),
     // 192 codebooks 83 84 84 84 85 / 80 83 84 81 84, 24 codebooks 35 36 36 36 36 / 37 37 37 37 38.
-    const bool blocks = (uint64_t)n * a.g.M * 4 >= SP_LARGE_OUTPUT;
-    const uint32_t tok_block = !blocks ? 0 : (TN == 4 ? 2048 : 1024) / TOK_ITEM;
+    const uint32_t tok_block = BLOCKS ? (TN == 4 ? 2048 : 1024) / TOK_ITEM : 0;
     const XcdMap xmap = choose_xcd_map(a.g.M_pad / (16 * TN), n_token_tiles, grid, (uint64_t)cb16 * 16 * a.g.M_pad,
                                        (uint64_t)n * a.g.idx_row_bytes, a.g.tune_xcd_col_split, tok_block);
-    if (KS == 1) snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_kernel<%d, %d, %d, %d, %s>", TN, TM, GS, NW, WIDE ? "true" : "false");
+    if (BLOCKS) snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_blocks_kernel<%d, %d, %d, %d>", TN, TM, GS, NW);
+    else if (KS == 1) snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_kernel<%d, %d, %d, %d, %s>", TN, TM, GS, NW, WIDE ? "true" : "false");
     else snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_kernel<%d, %d, %d, %d, %s, %d>", TN, TM, GS, NW, WIDE ? "true" : "false", KS);
     a.note_launch(GS, LDS, TOK_ITEM, NW * 64);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), LDS, ctx->stream, d_idx, reinterpret_cast<const int8_t*>(a.d_lut),
                        d_out, d_acc, n, a.g.M, cb16, a.g.idx_row_bytes, n_token_tiles, n_items, ep, xmap);
     return hip_check(ctx, hipGetLastError(), "gather_sparse_kernel launch");
+}
+
+template <int TN, int TM, int GS, int NW = 4, bool WIDE = false, int KS = 1>
+int launch_sparse_tm(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc, uint32_t n, const Epilogue& ep)
+{
+    // (17..32 centroids are here on request only, and a split of the codebooks is for launches of one round)
+    if constexpr (!WIDE && KS == 1)
+        if ((uint64_t)n * a.g.M * 4 >= SP_LARGE_OUTPUT) return launch_sparse_as<TN, TM, GS, NW, WIDE, KS, true>(ctx, a, d_idx, d_out, d_acc, n, ep);
+    return launch_sparse_as<TN, TM, GS, NW, WIDE, KS, false>(ctx, a, d_idx, d_out, d_acc, n, ep);
 }
 
 // 256- or 128-token items, whichever gives the shorter launch (the rule of the dense kernel)

@@ -1086,7 +1086,7 @@ def test_sparse_gather_of_large_outputs(ctx, N, M, tuning):
     torch.cuda.synchronize()
     amm.run_ptr(x.data_ptr(), N, out.data_ptr())
     ctx.synchronize()
-    assert amm.last_gather_kernel().startswith("gather_sparse_kernel<"), amm.last_gather_kernel()
+    assert amm.last_gather_kernel().startswith("gather_sparse_blocks_kernel<"), amm.last_gather_kernel()
     assert bool((out[N:] == -5.0).all())
     for i in range(0, N, 4096):
         n = min(4096, N - i)
