@@ -39,6 +39,7 @@ struct FewArgs {
     uint32_t c_tile;        // rows: rows per codebook in the table
     uint32_t idx_row_bytes;
     uint32_t op_groups;     // operators side by side: 16-column groups of each (0: one operator)
+    uint32_t token_tiles, by_xcd;
 };
 
 // Column of position s of a tile of one-hot tables (sparse_tile_column on the device)
@@ -50,45 +51,65 @@ __device__ __forceinline__ uint32_t few_column(uint32_t tn, uint32_t c, uint32_t
     return 16 * c + j;
 }
 
-// One workgroup per (16 columns, 16 * TM tokens).  Operands of a K-step, lane l = 16 g + j:
+// One workgroup per (16 * TC columns, 16 * TM tokens).  Operands of a K-step, lane l = 16 g + j:
 //   FEW_SPARSE  the sparse one-hot product (8 codebooks of 16): lane (g, token j) turns byte g of index word s into value
 //               bytes and positions, lane (g, column j) reads the table entries of codebooks g and g + 4
 //   FEW_PAIRED  the same instruction on the paired table (up to 8 centroids): an entry's 16 slots are two codebooks of
 //               8, whose one-hots fall into different groups of four, so a K-step covers 16 codebooks
 //   FEW_ROWS    the byte adder: lane (g, token j) reads its 16 columns of codebook 4 s + g, the constant operand
 //               A[i][16 g + b] = (b == i) adds them
-template <FewTable T, int TM, int NW>
+template <FewTable T, int TM, int NW, int TC = 1>
 __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep)
 {
+    static_assert(TC == 1 || T == FEW_SPARSE, "several column groups: sparse table only");
+    constexpr int UNROLL = TC == 1 ? FEW_UNROLL : 2;  // (registers)
     constexpr int PITCH = T == FEW_ROWS ? FEW_PITCH_ROWS : FEW_PITCH_ONEHOT;
     extern __shared__ __attribute__((aligned(16))) int part[];  // [wave][4 TM registers][PITCH]
     const uint32_t lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t col_group = blockIdx.x % a.groups, tok0 = blockIdx.x / a.groups * (16 * TM);
+    const uint32_t col_blocks = a.groups / TC;
+    // First of the TC column groups (of one tile) and first token.  by_xcd: XCD p % 8 takes every token tile of the column blocks congruent
+    // to it, so that one L2 streams a block's part of the table (blocks past the last: nothing to do).
+    uint32_t col_group = blockIdx.x, tok0 = 0;  // (items of 16 and 32 tokens: the launch has no more)
+    if constexpr (TM == 4) {
+        if (a.by_xcd) {
+            const uint32_t q = blockIdx.x / 8;
+            col_group = blockIdx.x % 8 + 8 * (q / a.token_tiles);
+            if (col_group >= col_blocks) return;  // whole workgroup
+            tok0 = q % a.token_tiles * (16 * TM);
+        } else {
+            tok0 = blockIdx.x / col_blocks * (16 * TM);
+            col_group = blockIdx.x % col_blocks;
+        }
+        col_group *= TC;
+    }
     const uint32_t tile = col_group / a.tile_groups, c = col_group % a.tile_groups;
     const uint32_t op = a.op_groups ? col_group / a.op_groups : 0u;
     const uint32_t wn = 16 * a.tile_groups;
     // 64-token block of the tiled index buffer (16 TM tokens lie in one block), this operator's words
     const uint8_t* ix = a.idx + (size_t)op * ep.op_idx_stride + (size_t)(tok0 / 64) * a.idx_row_bytes * 64 + ((tok0 & 63) + j) * 4;
 
-    v4i acc[TM];
+    v4i acc[TC][TM];
 #pragma unroll
-    for (int t = 0; t < TM; ++t) acc[t] = (v4i){0, 0, 0, 0};
+    for (int t = 0; t < TC * TM; ++t) acc[t / TM][t % TM] = (v4i){0, 0, 0, 0};
 
     if constexpr (T != FEW_ROWS) {
         // entry e of column j: ((tile * entries + e) * wn + 16 c + j) * 16 bytes; a K-step is 8 entries
         const int8_t* tab = a.lut + (((size_t)tile * a.steps * 8 + g) * wn + 16 * c + j) * 16;
         ix += T == FEW_SPARSE ? g : (g >> 1) * 256 + (g & 1) * 2;
-        for (uint32_t s0 = wave; s0 < a.steps; s0 += NW * FEW_UNROLL) {
-            v4i lo[FEW_UNROLL], hi[FEW_UNROLL];
-            uint32_t raw[FEW_UNROLL][TM];
+        for (uint32_t s0 = wave; s0 < a.steps; s0 += NW * UNROLL) {
+            v4i lo[UNROLL][TC], hi[UNROLL][TC];
+            uint32_t raw[UNROLL][TM];
 #pragma unroll
-            for (int u = 0; u < FEW_UNROLL; ++u) {
+            for (int u = 0; u < UNROLL; ++u) {
                 const uint32_t s = s0 + u * NW;
                 if (s < a.steps) {  // uniform
                     const int8_t* p = tab + (size_t)s * 8 * wn * 16;
-                    lo[u] = *reinterpret_cast<const v4i*>(p);
-                    hi[u] = *reinterpret_cast<const v4i*>(p + (size_t)4 * wn * 16);
+#pragma unroll
+                    for (int e = 0; e < TC; ++e) {
+                        lo[u][e] = *reinterpret_cast<const v4i*>(p + e * 256);
+                        hi[u][e] = *reinterpret_cast<const v4i*>(p + (size_t)4 * wn * 16 + e * 256);
+                    }
 #pragma unroll
                     for (int t = 0; t < TM; ++t) {
                         if constexpr (T == FEW_SPARSE) raw[u][t] = ix[(size_t)s * 256 + t * 64];
@@ -97,9 +118,8 @@ __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep)
                 }
             }
 #pragma unroll
-            for (int u = 0; u < FEW_UNROLL; ++u) {
+            for (int u = 0; u < UNROLL; ++u) {
                 if (s0 + u * NW >= a.steps) break;  // uniform
-                const v8i bb = {lo[u][0], lo[u][1], lo[u][2], lo[u][3], hi[u][0], hi[u][1], hi[u][2], hi[u][3]};
 #pragma unroll
                 for (int t = 0; t < TM; ++t) {
                     const uint32_t r = raw[u][t];
@@ -117,7 +137,12 @@ __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep)
                         aa = (v4i){val(0), val(1), val(2), val(3)};
                         pw = pos(r & 7) | pos(r >> 4 & 7) << 8 | pos(r >> 8 & 7) << 16 | pos(r >> 12 & 7) << 24;
                     }
-                    acc[t] = __builtin_amdgcn_smfmac_i32_16x16x128_i8(aa, bb, acc[t], (int)pw, 0, 0);
+#pragma unroll
+                    for (int e = 0; e < TC; ++e) {
+                        const v4i l = lo[u][e], h = hi[u][e];
+                        const v8i bb = {l[0], l[1], l[2], l[3], h[0], h[1], h[2], h[3]};
+                        acc[e][t] = __builtin_amdgcn_smfmac_i32_16x16x128_i8(aa, bb, acc[e][t], (int)pw, 0, 0);
+                    }
                 }
             }
         }
@@ -151,32 +176,36 @@ __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep)
             for (int u = 0; u < FEW_UNROLL; ++u) {
                 if (s0 + u * NW >= a.steps) break;
 #pragma unroll
-                for (int t = 0; t < TM; ++t) acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(one, row[u][t], acc[t], 0, 0, 0);
+                for (int t = 0; t < TM; ++t) acc[0][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(one, row[u][t], acc[0][t], 0, 0, 0);
             }
         }
     }
 
     // lane (g, j) holds: one-hot forms tokens 4 g + r of column position j, byte adder columns 4 g + r of token j
 #pragma unroll
-    for (int t = 0; t < TM; ++t)
+    for (int e = 0; e < TC; ++e) {
+        if (e) __syncthreads();  // the exchange of the group before has been read
 #pragma unroll
-        for (int r = 0; r < 4; ++r) part[((size_t)wave * TM * 4 + t * 4 + r) * PITCH + lane] = acc[t][r];
-    __syncthreads();
-    for (uint32_t o = threadIdx.x; o < TM * 256; o += NW * 64) {
-        const uint32_t x = o % 16, tok = o / 16;  // column position, token of the item
-        const uint32_t reg = tok / 16 * 4 + (T == FEW_ROWS ? x % 4 : tok % 4);
-        const uint32_t src = T == FEW_ROWS ? x / 4 * 16 + tok % 16 : (tok % 16) / 4 * 16 + x;
-        int32_t sum = 0;
+        for (int t = 0; t < TM; ++t)
 #pragma unroll
-        for (int w = 0; w < NW; ++w) sum += part[((size_t)w * TM * 4 + reg) * PITCH + src];
-        const uint32_t n = tok0 + tok;
-        const uint32_t f = T == FEW_SPARSE ? tile * wn + few_column(a.tile_groups, c, x) : 16 * col_group + x;
-        if (n >= a.N || f >= a.M) continue;
-        Epilogue epl = ep;
-        if (a.op_groups) epl.scale = ep.op_scales[op];
-        const float b = ep.bias ? ep.bias[f] : 0.0f;
-        a.out[(size_t)n * a.M + f] = ep.act == PIMDL_ACT_GELU_TANH ? dequant<true>(sum, epl, b) : dequant<false>(sum, epl, b);
-        if (a.acc_out) a.acc_out[(size_t)n * a.M + f] = sum;
+            for (int r = 0; r < 4; ++r) part[((size_t)wave * TM * 4 + t * 4 + r) * PITCH + lane] = acc[e][t][r];
+        __syncthreads();
+        for (uint32_t o = threadIdx.x; o < TM * 256; o += NW * 64) {
+            const uint32_t x = o % 16, tok = o / 16;  // column position, token of the item
+            const uint32_t reg = tok / 16 * 4 + (T == FEW_ROWS ? x % 4 : tok % 4);
+            const uint32_t src = T == FEW_ROWS ? x / 4 * 16 + tok % 16 : (tok % 16) / 4 * 16 + x;
+            int32_t sum = 0;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) sum += part[((size_t)w * TM * 4 + reg) * PITCH + src];
+            const uint32_t n = tok0 + tok;
+            const uint32_t f = T == FEW_SPARSE ? tile * wn + few_column(a.tile_groups, c + e, x) : 16 * col_group + x;
+            if (n >= a.N || f >= a.M) continue;
+            Epilogue epl = ep;
+            if (a.op_groups) epl.scale = ep.op_scales[op];
+            const float b = ep.bias ? ep.bias[f] : 0.0f;
+            a.out[(size_t)n * a.M + f] = ep.act == PIMDL_ACT_GELU_TANH ? dequant<true>(sum, epl, b) : dequant<false>(sum, epl, b);
+            if (a.acc_out) a.acc_out[(size_t)n * a.M + f] = sum;
+        }
     }
 }
 
@@ -185,6 +214,14 @@ template <int TM, int NW>
 __global__ __launch_bounds__(NW * 64) void gather_sparse_few_kernel(FewArgs a, Epilogue ep)
 {
     gather_few<FEW_SPARSE, TM, NW>(a, ep);
+}
+// Sparse table, TC column groups of a tile per workgroup: the operands made from index bytes serve all of them, and a launch has
+// fewer workgroups, each with as many loads in flight.  (16 waves, one or two token groups, and all four groups of a
+// 64-column tile were slower or spill: N = 1024, 768 codebooks, M = 768 us 8 waves 12.5, 16 12.6, 4 14.8.)
+template <int TM, int NW, int TC>
+__global__ __launch_bounds__(NW * 64, 4) void gather_sparse_few_wide_kernel(FewArgs a, Epilogue ep)
+{
+    gather_few<FEW_SPARSE, TM, NW, TC>(a, ep);
 }
 template <int TM, int NW>
 __global__ __launch_bounds__(NW * 64) void gather_onehot_few_kernel(FewArgs a, Epilogue ep)
@@ -197,8 +234,20 @@ __global__ __launch_bounds__(NW * 64) void gather_i8_few_kernel(FewArgs a, Epilo
     gather_few<FEW_ROWS, TM, NW>(a, ep);
 }
 
+// Workgroups of a launch.  By XCD where the column blocks do not divide by eight by themselves and several token tiles read the same table:
+// us, in order / by XCD, three column groups: 2048 codebooks, M = 2048 N = 256 41.1 / 24.8, 1280 x 1280 N = 512 33.2 / 17.6, 256, M =
+// 5120 N = 128 10.6 / 7.7; one column group: 2048 N = 128 32.8 / 26.4, 1280 N = 256 22.9 / 18.8; with a CU for every workgroup
+// of one column group 1024 N = 100 9.2 / 9.5, 1280 N = 128 11.6 / 11.1.
+uint32_t few_grid(FewArgs& f, uint32_t tm, uint32_t tc, uint32_t cus)
+{
+    const uint32_t blocks = f.groups / tc;
+    f.token_tiles = (f.N + 16 * tm - 1) / (16 * tm);
+    f.by_xcd = f.token_tiles > 1 && blocks % 8 != 0 && (tc > 1 || f.token_tiles * blocks > cus);
+    return f.token_tiles * (f.by_xcd ? (blocks + 7) / 8 * 8 : blocks);
+}
+
 template <FewTable T, int TM, int NW>
-int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
+int launch_few_as(Ctx* ctx, const Amm& a, FewArgs f, const Epilogue& ep)
 {
     constexpr int LDS = few_lds_bytes(NW, TM, T == FEW_ROWS ? FEW_PITCH_ROWS : FEW_PITCH_ONEHOT);
     auto kern = T == FEW_SPARSE ? gather_sparse_few_kernel<TM, NW> : T == FEW_PAIRED ? gather_onehot_few_kernel<TM, NW> : gather_i8_few_kernel<TM, NW>;
@@ -206,8 +255,20 @@ int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
     static const char* const names[] = {"gather_sparse_few_kernel", "gather_onehot_few_kernel", "gather_i8_few_kernel"};
     snprintf(a.last_gather, sizeof(a.last_gather), "%s<%d, %d>", names[T], TM, NW);
     a.note_launch(0, LDS, 16 * TM, NW * 64);
-    hipLaunchKernelGGL(kern, dim3(f.groups * ((f.N + 16 * TM - 1) / (16 * TM))), dim3(NW * 64), LDS, ctx->stream, f, ep);
+    hipLaunchKernelGGL(kern, dim3(few_grid(f, TM, 1, ctx->prop.multiProcessorCount)), dim3(NW * 64), LDS, ctx->stream, f, ep);
     return hip_check(ctx, hipGetLastError(), "gather_few launch");
+}
+
+template <int TC>
+int launch_few_wide(Ctx* ctx, const Amm& a, FewArgs f, const Epilogue& ep)
+{
+    constexpr int TM = 4, NW = 8, LDS = few_lds_bytes(NW, TM, FEW_PITCH_ONEHOT);
+    auto kern = gather_sparse_few_wide_kernel<TM, NW, TC>;
+    if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_few_wide)")) return rc;
+    snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_few_wide_kernel<%d, %d, %d>", TM, NW, TC);
+    a.note_launch(0, LDS, 16 * TM, NW * 64);
+    hipLaunchKernelGGL(kern, dim3(few_grid(f, TM, TC, ctx->prop.multiProcessorCount)), dim3(NW * 64), LDS, ctx->stream, f, ep);
+    return hip_check(ctx, hipGetLastError(), "gather_few_wide launch");
 }
 
 // tokens of an item, by what the launch has: 16, 32 or 64
@@ -307,6 +368,25 @@ int launch_f32_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, u
 
 }  // namespace
 
+// Column groups that a workgroup of a launch on the sparse kernel's table takes (0: the large kernel is the shorter launch): as few as leave
+// every workgroup a CU of its own.  us, large / one group / several, N tokens: 768 codebooks, M = 768 N = 512 19.1 / 12.6 / 12.1 (three), 1024 19.3 /
+// 17.7 / 12.6, 2048 19.7 / 30.9 / 20.0; 1024, M = 1024 N = 512 26.0 / 16.8 / 12.0 (two), 700 27 / 24 / 20; 2048, M = 2048 N = 400 53 / 51 / 35 (two);
+// 192, M = 3072 N = 256 8.1 / 8.1 / 6.7 (three), 512 8.6 / 13.5 / 9.3; 384, M = 1280 N = 256 11.9 / 8.0 / 8.3 (three), 400 12.8 / 11.2 / 8.6; 256, M =
+// 4096 N = 128 9.5 / 7.8 / 6.5 (two), 200 10.8 / 11.7 / 9.2; 96-column tiles 192, M = 2304 N = 256 11.7 / 9.1 / 7.3 (three), 400 12.5 / 11.2 / 8.3 (two).
+// One token tile (the large kernel's chain is the same for one token): 512, M = 8192 N = 1 17.6 / 12.6, 32 18.2 / 12.7, 64 18.3 /
+// 14.4 / 14.2 (three); 192, M = 8192 N = 1 8.2 / 3.8, M = 12000 9.8 / 6.2, N = 64 10.7 / 9.3 / 8.8 (three).
+uint32_t few_column_groups(const Ctx* ctx, const AmmGeom& g, uint32_t n)
+{
+    const uint64_t cus = ctx->prop.multiProcessorCount, item = few_item(n), groups = g.M_pad / 16, tiles = (n + item - 1) / item;
+    const uint64_t wgs = tiles * groups;
+    if (wgs <= cus) return 1;
+    if (n <= 32) return wgs <= 4 * cus ? 1 : 0;
+    const uint32_t tc = g.q % 2 == 0 && (wgs / 2 <= cus || g.q % 3 != 0) ? 2 : 3;
+    const uint64_t wide = wgs / tc;
+    if (g.q == 3) return wgs <= 2 * cus ? (g.CB_pad >= 640 ? 3 : 1) : wide <= cus ? 3 : 0;
+    return wide <= cus || (wide <= 2 * cus && g.CB_pad >= 128) ? tc : wgs <= 2 * cus ? 1 : 0;
+}
+
 // Whether these kernels are the shorter launch.  The large kernels' time is flat while their items do not fill the chip
 // (us, large / few): one-hot tables 768 -> 3072 8.1 / 3.0 at N = 1, 8.7 / 4.1 at 64, 9.1 / 9.7 at 300; 3072 -> 768
 // 19.8 / 4.5 at 1, 20.2 / 7.7 at 150, 19.8 / 13.1 at 512, 20.3 / 18.2 at 1024; 8 centroids 3072 -> 768 15.4 / 5.9 at 64,
@@ -336,7 +416,7 @@ bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
         return g.idx_bits == 8 && 2.6 + pieces * (g.C_tile <= 32 ? 0.5e-3 : 1e-3) / (double)(wgs < cus ? wgs : cus) <
                                       3.3 + (g.CB + 15) / 16 * (0.2 + 0.003 * g.C_tile);
     if (g.gather_kind == 2 ? g.C_tile == 32 : g.C_tile != 8) return false;  // tables only a tuning asks for
-    return wgs <= 2 * cus;
+    return g.gather_kind == 2 ? few_column_groups(ctx, g, n) != 0 : wgs <= 2 * cus;
 }
 
 int launch_gather_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc, uint32_t n, float scale,
@@ -365,6 +445,10 @@ int launch_gather_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out
                  g.idx_row_bytes, a.op_col_tiles * g.q};
     if (g.gather_kind == 2) {
         f.steps = g.CB_pad / 8;
+        switch (few_column_groups(ctx, g, n)) {
+            case 2: return launch_few_wide<2>(ctx, a, f, ep);
+            case 3: return launch_few_wide<3>(ctx, a, f, ep);
+        }
         return launch_few<FEW_SPARSE>(ctx, a, f, ep);
     }
     if (g.gather_kind == 1) {

@@ -1067,6 +1067,37 @@ def test_matrix_core_gathers_at_ragged_sizes(ctx, kernel, C, widths, N, CB, M):
         amm.close()
 
 
+@pytest.mark.parametrize("N,CB,M,C,width,groups", [(1000, 8, 768, 16, 48, 3), (513, 640, 760, 16, 48, 3), (300, 33, 1000, 16, 64, 2), (200, 70, 1500, 9, 96, 2),
+                                                   (449, 12, 1500, 16, 96, 3), (400, 130, 2049, 16, 64, 2), (65, 96, 9001, 16, 48, 0), (64, 40, 9001, 16, 48, 3),
+                                                   (20, 40, 9001, 16, 48, 1), (1, 5, 16001, 16, 48, 1), (700, 129, 1100, 13, 96, 3)])
+def test_launches_of_few_tokens_with_several_column_groups(ctx, N, CB, M, C, width, groups):
+    """Between the launches of few tokens and the large ones: workgroups of two and three column groups, their column blocks dealt to the
+    XCDs (those past the last do nothing), waves with and without K-steps, ragged tokens and columns: accumulators and output bits of the oracle,
+    nothing behind the output.  `groups`: column groups of a workgroup on 256 CUs (0: the large kernel)."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    import torch
+    v = 2
+    x, cent, lut, bias = make_case(3100 + N + M, N, CB * v, v, C, M)
+    want, want_idx, want_acc = oracle.amm_cpu(x, cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)
+    amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=N, tuning={"gather_kernel": pimdl.GATHER_SPARSE, "col_block": width})
+    out, idx, acc = amm.run_debug(x)
+    name = amm.last_gather_kernel()
+    if ctx.device_info()["compute_units"] == 256:
+        assert name.startswith("gather_sparse_kernel<" if groups == 0 else "gather_sparse_few_kernel<" if groups == 1 else "gather_sparse_few_wide_kernel<"), name
+        assert groups < 2 or name.endswith(f", {groups}>"), name
+    assert np.array_equal(idx, want_idx) and np.array_equal(acc, want_acc), name
+    assert np.array_equal(out.view(np.uint32), want.view(np.uint32)), name
+    guarded = torch.full((N + 3, M), -5.0, device="cuda")
+    xd = torch.from_numpy(x).cuda()
+    torch.cuda.synchronize()
+    amm.run_ptr(xd.data_ptr(), N, guarded.data_ptr())
+    ctx.synchronize()
+    got = guarded.cpu().numpy()
+    assert np.array_equal(got[:N].view(np.uint32), want.view(np.uint32)) and (got[N:] == -5.0).all(), name
+    amm.close()
+
+
 @pytest.mark.parametrize("N,M,tuning", [(16384, 4096, {}), (16640, 4160, {}), (17000, 4001, {}), (34000, 2112, {"col_block": 48}),
                                         (33792, 2048, {"col_block": 64, "xcd_col_split": 2}), (65600, 1030, {"token_item": 128}),
                                         (17408, 4096, {"col_block": 96, "xcd_col_split": pimdl.XCD_PLAIN})])
