@@ -39,7 +39,9 @@ struct FewArgs {
     uint32_t c_tile;        // rows: rows per codebook in the table
     uint32_t idx_row_bytes;
     uint32_t op_groups;     // operators side by side: 16-column groups of each (0: one operator)
-    uint32_t token_tiles, by_xcd;
+};
+struct FewGrid {
+    uint32_t token_tiles, by_xcd;  // see gather_few
 };
 
 // Column of position s of a tile of one-hot tables (sparse_tile_column on the device)
@@ -59,7 +61,7 @@ __device__ __forceinline__ uint32_t few_column(uint32_t tn, uint32_t c, uint32_t
 //   FEW_ROWS    the byte adder: lane (g, token j) reads its 16 columns of codebook 4 s + g, the constant operand
 //               A[i][16 g + b] = (b == i) adds them
 template <FewTable T, int TM, int NW, int TC = 1>
-__device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep)
+__device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep, const FewGrid& grid)
 {
     static_assert(TC == 1 || T == FEW_SPARSE, "several column groups: sparse table only");
     constexpr int UNROLL = TC == 1 ? FEW_UNROLL : 2;  // (registers)
@@ -72,11 +74,11 @@ __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep)
     // to it, so that one L2 streams a block's part of the table (blocks past the last: nothing to do).
     uint32_t col_group = blockIdx.x, tok0 = 0;  // (items of 16 and 32 tokens: the launch has no more)
     if constexpr (TM == 4) {
-        if (a.by_xcd) {
+        if (grid.by_xcd) {
             const uint32_t q = blockIdx.x / 8;
-            col_group = blockIdx.x % 8 + 8 * (q / a.token_tiles);
+            col_group = blockIdx.x % 8 + 8 * (q / grid.token_tiles);
             if (col_group >= col_blocks) return;  // whole workgroup
-            tok0 = q % a.token_tiles * (16 * TM);
+            tok0 = q % grid.token_tiles * (16 * TM);
         } else {
             tok0 = blockIdx.x / col_blocks * (16 * TM);
             col_group = blockIdx.x % col_blocks;
@@ -211,43 +213,43 @@ __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep)
 
 // (a name for each, which says in a profile which of the large kernels it stands in for)
 template <int TM, int NW>
-__global__ __launch_bounds__(NW * 64) void gather_sparse_few_kernel(FewArgs a, Epilogue ep)
+__global__ __launch_bounds__(NW * 64) void gather_sparse_few_kernel(FewArgs a, Epilogue ep, FewGrid grid)
 {
-    gather_few<FEW_SPARSE, TM, NW>(a, ep);
+    gather_few<FEW_SPARSE, TM, NW>(a, ep, grid);
 }
 // Sparse table, TC column groups of a tile per workgroup: the operands made from index bytes serve all of them, and a launch has
 // fewer workgroups, each with as many loads in flight.  (16 waves, one or two token groups, and all four groups of a
 // 64-column tile were slower or spill: N = 1024, 768 codebooks, M = 768 us 8 waves 12.5, 16 12.6, 4 14.8.)
 template <int TM, int NW, int TC>
-__global__ __launch_bounds__(NW * 64, 4) void gather_sparse_few_wide_kernel(FewArgs a, Epilogue ep)
+__global__ __launch_bounds__(NW * 64, 4) void gather_sparse_few_wide_kernel(FewArgs a, Epilogue ep, FewGrid grid)
 {
-    gather_few<FEW_SPARSE, TM, NW, TC>(a, ep);
+    gather_few<FEW_SPARSE, TM, NW, TC>(a, ep, grid);
 }
 template <int TM, int NW>
-__global__ __launch_bounds__(NW * 64) void gather_onehot_few_kernel(FewArgs a, Epilogue ep)
+__global__ __launch_bounds__(NW * 64) void gather_onehot_few_kernel(FewArgs a, Epilogue ep, FewGrid grid)
 {
-    gather_few<FEW_PAIRED, TM, NW>(a, ep);
+    gather_few<FEW_PAIRED, TM, NW>(a, ep, grid);
 }
 template <int TM, int NW>
-__global__ __launch_bounds__(NW * 64) void gather_i8_few_kernel(FewArgs a, Epilogue ep)
+__global__ __launch_bounds__(NW * 64) void gather_i8_few_kernel(FewArgs a, Epilogue ep, FewGrid grid)
 {
-    gather_few<FEW_ROWS, TM, NW>(a, ep);
+    gather_few<FEW_ROWS, TM, NW>(a, ep, grid);
 }
 
 // Workgroups of a launch.  By XCD where the column blocks do not divide by eight by themselves and several token tiles read the same table:
 // us, in order / by XCD, three column groups: 2048 codebooks, M = 2048 N = 256 41.1 / 24.8, 1280 x 1280 N = 512 33.2 / 17.6, 256, M =
 // 5120 N = 128 10.6 / 7.7; one column group: 2048 N = 128 32.8 / 26.4, 1280 N = 256 22.9 / 18.8; with a CU for every workgroup
 // of one column group 1024 N = 100 9.2 / 9.5, 1280 N = 128 11.6 / 11.1.
-uint32_t few_grid(FewArgs& f, uint32_t tm, uint32_t tc, uint32_t cus)
+uint32_t few_grid(const FewArgs& f, uint32_t tm, uint32_t tc, uint32_t cus, FewGrid* grid)
 {
-    const uint32_t blocks = f.groups / tc;
-    f.token_tiles = (f.N + 16 * tm - 1) / (16 * tm);
-    f.by_xcd = f.token_tiles > 1 && blocks % 8 != 0 && (tc > 1 || f.token_tiles * blocks > cus);
-    return f.token_tiles * (f.by_xcd ? (blocks + 7) / 8 * 8 : blocks);
+    const uint32_t blocks = f.groups / tc, tiles = (f.N + 16 * tm - 1) / (16 * tm);
+    grid->token_tiles = tiles;
+    grid->by_xcd = tiles > 1 && blocks % 8 != 0 && (tc > 1 || tiles * blocks > cus);
+    return tiles * (grid->by_xcd ? (blocks + 7) / 8 * 8 : blocks);
 }
 
 template <FewTable T, int TM, int NW>
-int launch_few_as(Ctx* ctx, const Amm& a, FewArgs f, const Epilogue& ep)
+int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
 {
     constexpr int LDS = few_lds_bytes(NW, TM, T == FEW_ROWS ? FEW_PITCH_ROWS : FEW_PITCH_ONEHOT);
     auto kern = T == FEW_SPARSE ? gather_sparse_few_kernel<TM, NW> : T == FEW_PAIRED ? gather_onehot_few_kernel<TM, NW> : gather_i8_few_kernel<TM, NW>;
@@ -255,19 +257,23 @@ int launch_few_as(Ctx* ctx, const Amm& a, FewArgs f, const Epilogue& ep)
     static const char* const names[] = {"gather_sparse_few_kernel", "gather_onehot_few_kernel", "gather_i8_few_kernel"};
     snprintf(a.last_gather, sizeof(a.last_gather), "%s<%d, %d>", names[T], TM, NW);
     a.note_launch(0, LDS, 16 * TM, NW * 64);
-    hipLaunchKernelGGL(kern, dim3(few_grid(f, TM, 1, ctx->prop.multiProcessorCount)), dim3(NW * 64), LDS, ctx->stream, f, ep);
+    FewGrid grid;
+    const uint32_t wgs = few_grid(f, TM, 1, ctx->prop.multiProcessorCount, &grid);
+    hipLaunchKernelGGL(kern, dim3(wgs), dim3(NW * 64), LDS, ctx->stream, f, ep, grid);
     return hip_check(ctx, hipGetLastError(), "gather_few launch");
 }
 
 template <int TC>
-int launch_few_wide(Ctx* ctx, const Amm& a, FewArgs f, const Epilogue& ep)
+int launch_few_wide(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
 {
     constexpr int TM = 4, NW = 8, LDS = few_lds_bytes(NW, TM, FEW_PITCH_ONEHOT);
     auto kern = gather_sparse_few_wide_kernel<TM, NW, TC>;
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_few_wide)")) return rc;
     snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_few_wide_kernel<%d, %d, %d>", TM, NW, TC);
     a.note_launch(0, LDS, 16 * TM, NW * 64);
-    hipLaunchKernelGGL(kern, dim3(few_grid(f, TM, TC, ctx->prop.multiProcessorCount)), dim3(NW * 64), LDS, ctx->stream, f, ep);
+    FewGrid grid;
+    const uint32_t wgs = few_grid(f, TM, TC, ctx->prop.multiProcessorCount, &grid);
+    hipLaunchKernelGGL(kern, dim3(wgs), dim3(NW * 64), LDS, ctx->stream, f, ep, grid);
     return hip_check(ctx, hipGetLastError(), "gather_few_wide launch");
 }
 
