@@ -1580,6 +1580,102 @@ __global__ __launch_bounds__(CCS_THREADS) void ccs_few_kernel(const float* __res
     }
 }
 
+// Few tokens, up to 32 centroids: a wave takes 4 codebooks (2 from 17 centroids on) of one token after the other, a lane one centroid.
+// The distances are the reference's own (every operation rounded on its own, dimensions ascending), so nothing is replayed: where only one
+// centroid is within the hysteresis of the smallest distance the scan returns it whatever the order -- the subtraction that decides is
+// the scan's --, else every group goes through its distances in the scan's order.
+// Bound by the launch and one round trip to memory (the matrix search makes operands for 64 tokens and 16 codebooks first);
+// beyond some thousand (token, 4 codebooks) by the vector ALU.  Search of 64 tokens, 192 codebooks of 16, v = 4: 4.1 -> 2.8 us; 1 token 3.6 -> 2.5.
+template <int V, bool WIDE>
+__global__ __launch_bounds__(CCS_THREADS) void ccs_small_kernel(const float* __restrict__ x, const float* __restrict__ cent,
+                                                                uint8_t* __restrict__ idx, uint32_t N, uint32_t x_row, uint32_t CB,
+                                                                uint32_t CB_pad, uint32_t C, uint32_t idx_row_bytes, int idx_tiled,
+                                                                uint32_t tokens_per_wave, int x_aligned)
+{
+    constexpr uint32_t GROUP = WIDE ? 32 : 16, PER = 64 / GROUP;
+    const uint32_t lane = threadIdx.x & 63, c = lane % GROUP, quads = CB_pad / PER;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(blockIdx.x * (CCS_THREADS / 64) + (threadIdx.x >> 6));
+    const uint32_t q = w % quads, tok0 = w / quads * tokens_per_wave;
+    if (tok0 >= N) return;  // whole wave, past the last chunk of tokens
+    const uint32_t tok1 = tok0 + tokens_per_wave < N ? tok0 + tokens_per_wave : N;
+    const uint32_t cb = q * PER + lane / GROUP, cb_r = cb < CB ? cb : 0;  // (padding codebooks: index 0)
+    float cr[V];
+    {
+        const float* cp = cent + ((size_t)cb_r * C + (c < C ? c : 0)) * V;
+#pragma unroll
+        for (int t = 0; t < V; ++t) cr[t] = cp[t];
+    }
+    const float* xp = x + cb_r * V % x_row;  // (several operators' codebooks read the same columns)
+    auto fetch = [&](float (&xr)[V], uint32_t tok) {
+        const float* p = xp + (size_t)tok * x_row;
+        if (V % 4 == 0 && x_aligned) {  // uniform
+#pragma unroll
+            for (int t = 0; t < V; t += 4) {
+                const float4 f = *reinterpret_cast<const float4*>(p + t);
+                xr[t] = f.x;
+                xr[t + 1] = f.y;
+                xr[t + 2] = f.z;
+                xr[t + 3] = f.w;
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < V; ++t) xr[t] = p[t];
+        }
+    };
+    float xr[V], xn[V];
+    fetch(xr, tok0);
+    for (uint32_t tok = tok0; tok < tok1; ++tok) {
+        fetch(xn, tok + 1 < tok1 ? tok + 1 : tok);
+        float d = 0.0f;
+#pragma unroll
+        for (int t = 0; t < V; ++t) {
+            const float diff = __fsub_rn(xr[t], cr[t]);
+            d = __fadd_rn(d, __fmul_rn(diff, diff));
+        }
+        float best = c < C ? d : __builtin_inff();
+        auto rotate = [](float f, auto nc) {
+            return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), 0x120 + decltype(nc)::value, 0xf, 0xf, true));
+        };
+        best = vmin(best, rotate(best, std::integral_constant<int, 8>{}));
+        best = vmin(best, rotate(best, std::integral_constant<int, 4>{}));
+        best = vmin(best, rotate(best, std::integral_constant<int, 2>{}));
+        best = vmin(best, rotate(best, std::integral_constant<int, 1>{}));
+        if constexpr (WIDE) {
+            const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(best), __float_as_uint(best), false, false);
+            best = vmin(__uint_as_float(s[0]), __uint_as_float(s[1]));
+        }
+        // (NaN: a distance that is one counts as near, and alone the group is gone through)
+        const uint64_t near = __builtin_amdgcn_ballot_w64(c < C && !(__fsub_rn(d, best) > 1e-6f));
+        uint32_t found[PER];
+        bool several = false;
+#pragma unroll
+        for (uint32_t g = 0; g < PER; ++g) {
+            const uint32_t m = (uint32_t)(near >> (GROUP * g)) & (WIDE ? ~0u : 0xFFFFu);
+            several |= (m & (m - 1)) != 0;
+            found[g] = m ? (uint32_t)__builtin_ctz(m) : 0u;
+        }
+        if (several) {
+            float b = __shfl(d, lane & ~(GROUP - 1));
+            uint32_t k = 0;
+            for (uint32_t i = 1; i < C; ++i) {
+                const float di = __shfl(d, (lane & ~(GROUP - 1)) + i);
+                const bool take = __fsub_rn(b, di) > 1e-6f;
+                b = take ? di : b;
+                k = take ? i : k;
+            }
+#pragma unroll
+            for (uint32_t g = 0; g < PER; ++g) found[g] = __builtin_amdgcn_readlane(k, GROUP * g);
+        }
+        uint32_t word = 0;
+#pragma unroll
+        for (uint32_t g = 0; g < PER; ++g)
+            if (q * PER + g < CB) word |= found[g] << (16 / PER * g);
+        if (lane == 0) *reinterpret_cast<uint16_t*>(idx + idx_offset(tok, 2 * q, idx_row_bytes, idx_tiled)) = (uint16_t)word;
+#pragma unroll
+        for (int t = 0; t < V; ++t) xr[t] = xn[t];
+    }
+}
+
 // Generic sub-vector length (any v): one lane per (token, codebook), operands straight from
 // global memory.  Correct for every shape; only used where no specialisation exists.
 template <int IDX_BITS>
@@ -1815,6 +1911,19 @@ int launch_ccs_few(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_
     return hip_check(ctx, hipGetLastError(), "ccs_few_kernel launch");
 }
 
+template <int V>
+int launch_ccs_small(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent, uint8_t* d_idx, uint32_t n, uint32_t x_cols)
+{
+    constexpr uint32_t WAVES = CCS_THREADS / 64;
+    const uint64_t waves = 32ull * ctx->prop.multiProcessorCount, quads = g.CB_pad / (g.C > 16 ? 2 : 4);
+    const uint32_t per = (uint32_t)((n * quads + waves - 1) / waves), chunks = (n + per - 1) / per;
+    auto kern = g.C > 16 ? ccs_small_kernel<V, true> : ccs_small_kernel<V, false>;
+    hipLaunchKernelGGL(kern, dim3((uint32_t)((chunks * quads + WAVES - 1) / WAVES)), dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent, d_idx, n,
+                       x_cols ? x_cols : g.K, g.CB, g.CB_pad, g.C, g.idx_row_bytes, (int)g.idx_tiled, per,
+                       (int)((reinterpret_cast<uintptr_t>(d_x) & 15) == 0));
+    return hip_check(ctx, hipGetLastError(), "ccs_small_kernel launch");
+}
+
 template <int IDX_BITS>
 int launch_ccs_bits(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent, uint8_t* d_idx, uint32_t n,
                     uint32_t x_cols)
@@ -1822,6 +1931,23 @@ int launch_ccs_bits(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     // the operator's own choice (pimdl_amm_tuning.search_kernel) comes before the environment's
     const bool exact = g.tune_search ? g.tune_search == PIMDL_SEARCH_SCAN : ccs_exact_only();
     const bool f32 = g.tune_search ? g.tune_search == PIMDL_SEARCH_MFMA_F32 : ccs_f32_only();
+    // Few pairs: a wave per token and 4 (2 from 17 centroids on) codebooks takes 2.6 us + 0.13 ns each (v = 16 0.3, v = 32 1.1 ns, whose
+    // rows a lane fetches for itself), the matrix searches 3.5 to 5.5 us until they fill the chip.  us, matrix / this: 16
+    // centroids, v = 4 192 codebooks N = 1 3.6 / 2.5, N = 64 4.1 / 2.8, N = 256 4.7 / 3.9, N = 512 4.3 / 5.7, 2048 codebooks N = 8 4.2 / 2.7,
+    // N = 32 4.3 / 4.6; v = 2 384 codebooks N = 64 4.1 / 2.9, N = 128 4.1 / 3.7, N = 256 4.1 / 5.4; v = 8 96 codebooks N = 512 6.1 / 4.3, 1024 6.2 / 6.2,
+    // 1024 codebooks N = 64 6.1 / 4.9, 128 6.4 / 7.3; v = 16 64 codebooks N = 128 4.0 / 2.9, 256 4.0 / 3.8; v = 32 160 codebooks N = 8 3.9 /
+    // 3.2, 32 4.7 / 4.6; 32 centroids, v = 4 192 codebooks N = 64 4.8 / 2.8, 256 5.9 / 4.8, 512 5.9 / 7.1; v = 2 1536 codebooks N = 32 5.6 / 4.6.
+    const uint64_t waves = (uint64_t)n * (g.CB_pad / (g.C > 16 ? 2 : 4));
+    const uint32_t most = g.v == 32 ? 1200 : g.v == 16 ? 3500 : g.v == 8 || g.C > 16 ? 20000 : 13500;
+    if (g.C <= 32 && waves <= most && !g.tune_search && !g.tune_search_tile && !exact && !f32) {
+        switch (g.v) {
+            case 2: return launch_ccs_small<2>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+            case 4: return launch_ccs_small<4>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+            case 8: return launch_ccs_small<8>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+            case 16: return launch_ccs_small<16>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+            case 32: return launch_ccs_small<32>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+        }
+    }
     if (IDX_BITS == 8 && g.C <= 32 && !exact && !f32) {
         switch (g.v) {
             case 2: return launch_ccs_bf16<2, true>(ctx, g, d_x, d_cent, d_idx, n, x_cols);

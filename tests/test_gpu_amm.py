@@ -1067,6 +1067,47 @@ def test_matrix_core_gathers_at_ragged_sizes(ctx, kernel, C, widths, N, CB, M):
         amm.close()
 
 
+@pytest.mark.parametrize("N,CB,v,C", [(1, 1, 4, 16), (3, 33, 4, 9), (64, 70, 2, 16), (230, 192, 4, 16), (5, 35, 8, 1), (600, 97, 8, 16), (70, 30, 16, 13),
+                                      (9, 24, 32, 16), (1, 3, 2, 17), (40, 100, 4, 32), (333, 34, 8, 24), (50, 33, 16, 32), (17, 9, 32, 20)])
+@pytest.mark.parametrize("lut", ["i8", "f32"])
+def test_search_of_few_pairs_up_to_32_centroids(ctx, N, CB, v, C, lut):
+    """A wave per token and a few codebooks: indices of the oracle for random rows, near ties on either side of the hysteresis, repeated and
+    equal-to-a-centroid rows, NaN and infinities in rows and centroids, padded codebooks, several tokens per wave, both index
+    layouts, and rows that are only 4-byte aligned."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one search for every shape")
+    import torch
+    M = 20
+    x, cent, table, bias = make_case(700 + N + CB, N, CB * v, v, C, M, lut)
+    rng = np.random.default_rng(N + C)
+    if C > 2:
+        cent[::3, C // 2] = cent[::3, 0]                                   # repeated centroids
+        cent[1::3, C - 1] = cent[1::3, 1] + np.float32(3e-7)               # ... nearly so: the hysteresis decides
+    xv = x.reshape(N, CB, v)
+    rows = rng.integers(0, C, (N, CB))
+    near = cent[np.arange(CB), rows]                                       # [N][CB][v]
+    pick = rng.random((N, CB)) < 0.4
+    xv[pick] = near[pick] + rng.choice([0.0, 1e-4, 5e-4], (int(pick.sum()), 1)).astype(np.float32)
+    xv[rng.random((N, CB)) < 0.02] = np.nan
+    xv[rng.random((N, CB)) < 0.02] = np.inf
+    if CB > 4 and C > 1:
+        cent[3, rng.integers(0, C)] = np.nan
+        cent[4, rng.integers(0, C), 0] = -np.inf
+    scales = np.float32(0.0123) if lut == "i8" else None
+    want = oracle.index_calculation(x, cent, v, threads=THREADS)
+    amm = ctx.amm(cent, table, scales, bias, max_n=N)
+    out, idx, _ = amm.run_debug(x, want_acc=False)
+    assert np.array_equal(idx, want.reshape(N, CB))
+    shifted = torch.empty(N * CB * v + 1, device="cuda")[1:]
+    shifted.copy_(torch.from_numpy(x.reshape(-1)).cuda())
+    od = torch.empty((N, M), device="cuda")
+    torch.cuda.synchronize()
+    amm.run_ptr(shifted.data_ptr(), N, od.data_ptr())
+    ctx.synchronize()
+    assert np.array_equal(od.cpu().numpy().view(np.uint32), out.view(np.uint32))
+    amm.close()
+
+
 @pytest.mark.parametrize("N,CB,M,C,width,groups", [(1000, 8, 768, 16, 48, 3), (513, 640, 760, 16, 48, 3), (300, 33, 1000, 16, 64, 2), (200, 70, 1500, 9, 96, 2),
                                                    (449, 12, 1500, 16, 96, 3), (400, 130, 2049, 16, 64, 2), (65, 96, 9001, 16, 48, 0), (64, 40, 9001, 16, 48, 3),
                                                    (20, 40, 9001, 16, 48, 1), (1, 5, 16001, 16, 48, 1), (700, 129, 1100, 13, 96, 3)])
