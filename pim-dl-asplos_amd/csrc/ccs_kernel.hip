@@ -43,6 +43,7 @@
 #include <vector>
 
 #include "pimdl_internal.h"
+#include "search_quad.h"
 
 #include <stdlib.h>
 
@@ -1580,10 +1581,8 @@ __global__ __launch_bounds__(CCS_THREADS) void ccs_few_kernel(const float* __res
     }
 }
 
-// Few tokens, up to 32 centroids: a wave takes 4 codebooks (2 from 17 centroids on) of one token after the other, a lane one centroid.
-// The distances are the reference's own (every operation rounded on its own, dimensions ascending), so nothing is replayed: where only one
-// centroid is within the hysteresis of the smallest distance the scan returns it whatever the order -- the subtraction that decides is
-// the scan's --, else every group goes through its distances in the scan's order.
+// Few tokens, up to 32 centroids: a wave takes 4 codebooks (2 from 17 centroids on) of one token after the other, a lane one centroid
+// (quad_scan): the reference's own distances, so nothing is replayed.
 // Bound by the launch and one round trip to memory (the matrix search makes operands for 64 tokens and 16 codebooks first);
 // beyond some thousand (token, 4 codebooks) by the vector ALU.  Search of 64 tokens, 192 codebooks of 16, v = 4: 4.1 -> 2.8 us; 1 token 3.6 -> 2.5.
 template <int V, bool WIDE>
@@ -1606,70 +1605,11 @@ __global__ __launch_bounds__(CCS_THREADS) void ccs_small_kernel(const float* __r
         for (int t = 0; t < V; ++t) cr[t] = cp[t];
     }
     const float* xp = x + cb_r * V % x_row;  // (several operators' codebooks read the same columns)
-    auto fetch = [&](float (&xr)[V], uint32_t tok) {
-        const float* p = xp + (size_t)tok * x_row;
-        if (V % 4 == 0 && x_aligned) {  // uniform
-#pragma unroll
-            for (int t = 0; t < V; t += 4) {
-                const float4 f = *reinterpret_cast<const float4*>(p + t);
-                xr[t] = f.x;
-                xr[t + 1] = f.y;
-                xr[t + 2] = f.z;
-                xr[t + 3] = f.w;
-            }
-        } else {
-#pragma unroll
-            for (int t = 0; t < V; ++t) xr[t] = p[t];
-        }
-    };
     float xr[V], xn[V];
-    fetch(xr, tok0);
+    quad_row<V>(xr, xp + (size_t)tok0 * x_row, x_aligned);
     for (uint32_t tok = tok0; tok < tok1; ++tok) {
-        fetch(xn, tok + 1 < tok1 ? tok + 1 : tok);
-        float d = 0.0f;
-#pragma unroll
-        for (int t = 0; t < V; ++t) {
-            const float diff = __fsub_rn(xr[t], cr[t]);
-            d = __fadd_rn(d, __fmul_rn(diff, diff));
-        }
-        float best = c < C ? d : __builtin_inff();
-        auto rotate = [](float f, auto nc) {
-            return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(f), 0x120 + decltype(nc)::value, 0xf, 0xf, true));
-        };
-        best = vmin(best, rotate(best, std::integral_constant<int, 8>{}));
-        best = vmin(best, rotate(best, std::integral_constant<int, 4>{}));
-        best = vmin(best, rotate(best, std::integral_constant<int, 2>{}));
-        best = vmin(best, rotate(best, std::integral_constant<int, 1>{}));
-        if constexpr (WIDE) {
-            const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(best), __float_as_uint(best), false, false);
-            best = vmin(__uint_as_float(s[0]), __uint_as_float(s[1]));
-        }
-        // (NaN: a distance that is one counts as near, and alone the group is gone through)
-        const uint64_t near = __builtin_amdgcn_ballot_w64(c < C && !(__fsub_rn(d, best) > 1e-6f));
-        uint32_t found[PER];
-        bool several = false;
-#pragma unroll
-        for (uint32_t g = 0; g < PER; ++g) {
-            const uint32_t m = (uint32_t)(near >> (GROUP * g)) & (WIDE ? ~0u : 0xFFFFu);
-            several |= (m & (m - 1)) != 0;
-            found[g] = m ? (uint32_t)__builtin_ctz(m) : 0u;
-        }
-        if (several) {
-            float b = __shfl(d, lane & ~(GROUP - 1));
-            uint32_t k = 0;
-            for (uint32_t i = 1; i < C; ++i) {
-                const float di = __shfl(d, (lane & ~(GROUP - 1)) + i);
-                const bool take = __fsub_rn(b, di) > 1e-6f;
-                b = take ? di : b;
-                k = take ? i : k;
-            }
-#pragma unroll
-            for (uint32_t g = 0; g < PER; ++g) found[g] = __builtin_amdgcn_readlane(k, GROUP * g);
-        }
-        uint32_t word = 0;
-#pragma unroll
-        for (uint32_t g = 0; g < PER; ++g)
-            if (q * PER + g < CB) word |= found[g] << (16 / PER * g);
+        quad_row<V>(xn, xp + (size_t)(tok + 1 < tok1 ? tok + 1 : tok) * x_row, x_aligned);
+        const uint32_t word = quad_scan<V, WIDE>(xr, cr, C, lane, CB > q * PER ? CB - q * PER : 0);
         if (lane == 0) *reinterpret_cast<uint16_t*>(idx + idx_offset(tok, 2 * q, idx_row_bytes, idx_tiled)) = (uint16_t)word;
 #pragma unroll
         for (int t = 0; t < V; ++t) xr[t] = xn[t];
@@ -1808,16 +1748,6 @@ int launch_ccs_mfma(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     hipLaunchKernelGGL((ccs_mfma_kernel<V>), grid, dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent, aux_a, cnmax_pad,
                        d_idx, n, g.K, g.CB, g.C, g.idx_row_bytes, (int)g.idx_tiled, vec_ok, tiles_cb, total);
     return hip_check(ctx, hipGetLastError(), "ccs_mfma_kernel launch");
-}
-
-// PIMDL_CCS_F32=1 keeps the fp32 matrix-core search (same results; for comparison)
-static bool ccs_f32_only()
-{
-    static const bool v = [] {
-        const char* e = getenv("PIMDL_CCS_F32");
-        return e && e[0] == '1';
-    }();
-    return v;
 }
 
 template <int V, bool WIDE, int TTOK>
@@ -2153,6 +2083,16 @@ bool ccs_exact_only()
 {
     static const bool v = [] {
         const char* e = getenv("PIMDL_CCS_EXACT");
+        return e && e[0] == '1';
+    }();
+    return v;
+}
+
+// PIMDL_CCS_F32=1 keeps the fp32 matrix-core search (same results; for comparison)
+bool ccs_f32_only()
+{
+    static const bool v = [] {
+        const char* e = getenv("PIMDL_CCS_F32");
         return e && e[0] == '1';
     }();
     return v;

@@ -7,6 +7,7 @@
 // 96 columns to a workgroup, which goes through all codebooks slice by slice; a launch with fewer items than CUs
 // then takes the time of that chain -- copy, barrier, operands, 32 codebooks further -- however few its tokens are.
 #include "gather_common.h"
+#include "search_quad.h"
 
 namespace pimdl {
 namespace {
@@ -40,6 +41,13 @@ struct FewArgs {
     uint32_t idx_row_bytes;
     uint32_t op_groups;     // operators side by side: 16-column groups of each (0: one operator)
 };
+// the search of a launch that has no index buffer
+struct FewSearch {
+    const float* x;
+    const float* cent;
+    uint32_t K, CB, C, aligned;
+};
+constexpr int FEW_FUSED_TOKENS = 2;
 struct FewGrid {
     uint32_t token_tiles, by_xcd;  // see gather_few
 };
@@ -60,11 +68,13 @@ __device__ __forceinline__ uint32_t few_column(uint32_t tn, uint32_t c, uint32_t
 //               8, whose one-hots fall into different groups of four, so a K-step covers 16 codebooks
 //   FEW_ROWS    the byte adder: lane (g, token j) reads its 16 columns of codebook 4 s + g, the constant operand
 //               A[i][16 g + b] = (b == i) adds them
-template <FewTable T, int TM, int NW, int TC = 1>
-__device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep, const FewGrid& grid)
+// V > 0: up to FEW_FUSED_TOKENS tokens whose index bytes are searched here, by the wave that needs them (sub-vectors of V floats).
+template <FewTable T, int TM, int NW, int TC = 1, int V = 0>
+__device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep, const FewGrid& grid, const FewSearch& fs = {})
 {
     static_assert(TC == 1 || T == FEW_SPARSE, "several column groups: sparse table only");
-    constexpr int UNROLL = TC == 1 ? FEW_UNROLL : 2;  // (registers)
+    static_assert(V == 0 || (T == FEW_SPARSE && TM == 1 && TC == 1), "searched where it is gathered: 16-token items of the sparse table");
+    constexpr int UNROLL = V == 8 ? 1 : TC > 1 || V > 0 ? 2 : FEW_UNROLL;  // (registers)
     constexpr int PITCH = T == FEW_ROWS ? FEW_PITCH_ROWS : FEW_PITCH_ONEHOT;
     extern __shared__ __attribute__((aligned(16))) int part[];  // [wave][4 TM registers][PITCH]
     const uint32_t lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
@@ -102,10 +112,22 @@ __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep,
         for (uint32_t s0 = wave; s0 < a.steps; s0 += NW * UNROLL) {
             v4i lo[UNROLL][TC], hi[UNROLL][TC];
             uint32_t raw[UNROLL][TM];
+            constexpr int W = V > 0 ? V : 1;
+            float cr[UNROLL][2][W], xr[UNROLL][2][FEW_FUSED_TOKENS][W];  // codebooks 8 s + 4 h + g
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u) {
                 const uint32_t s = s0 + u * NW;
                 if (s < a.steps) {  // uniform
+                    if constexpr (V > 0) {
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const uint32_t cb = 8 * s + 4 * h + g, cbr = cb < fs.CB ? cb : 0;  // (padding: index 0)
+                            quad_row<V>(cr[u][h], fs.cent + ((size_t)cbr * fs.C + (j < fs.C ? j : 0)) * V, true);
+#pragma unroll
+                            for (int t = 0; t < FEW_FUSED_TOKENS; ++t)
+                                quad_row<V>(xr[u][h][t], fs.x + (size_t)((uint32_t)t < a.N ? t : 0) * fs.K + cbr * V, fs.aligned);
+                        }
+                    }
                     const int8_t* p = tab + (size_t)s * 8 * wn * 16;
 #pragma unroll
                     for (int e = 0; e < TC; ++e) {
@@ -114,7 +136,8 @@ __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep,
                     }
 #pragma unroll
                     for (int t = 0; t < TM; ++t) {
-                        if constexpr (T == FEW_SPARSE) raw[u][t] = ix[(size_t)s * 256 + t * 64];
+                        if constexpr (V > 0) continue;
+                        else if constexpr (T == FEW_SPARSE) raw[u][t] = ix[(size_t)s * 256 + t * 64];
                         else raw[u][t] = *reinterpret_cast<const uint16_t*>(ix + (size_t)s * 512 + t * 64);
                     }
                 }
@@ -122,6 +145,17 @@ __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep,
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u) {
                 if (s0 + u * NW >= a.steps) break;  // uniform
+                if constexpr (V > 0) {
+                    const uint32_t cb = 8 * (s0 + u * NW), real = fs.CB > cb ? fs.CB - cb : 0;
+                    uint32_t word[FEW_FUSED_TOKENS];
+#pragma unroll
+                    for (int t = 0; t < FEW_FUSED_TOKENS; ++t)
+                        if (t == 0 || (uint32_t)t < a.N)  // uniform
+                            word[t] = quad_scan<V, false>(xr[u][0][t], cr[u][0], fs.C, lane, real) |
+                                      quad_scan<V, false>(xr[u][1][t], cr[u][1], fs.C, lane, real > 4 ? real - 4 : 0) << 16;
+                        else word[t] = 0;
+                    raw[u][0] = ((j == 1 ? word[1] : word[0]) >> (8 * g)) & 255u;  // (lanes past the tokens: any)
+                }
 #pragma unroll
                 for (int t = 0; t < TM; ++t) {
                     const uint32_t r = raw[u][t];
@@ -216,6 +250,14 @@ template <int TM, int NW>
 __global__ __launch_bounds__(NW * 64) void gather_sparse_few_kernel(FewArgs a, Epilogue ep, FewGrid grid)
 {
     gather_few<FEW_SPARSE, TM, NW>(a, ep, grid);
+}
+// One or two tokens: search and gather in one launch.  Every workgroup searches all codebooks for its 16 columns, which is less
+// than a second launch: the centroids and the rows are requested with the table, so there is one round trip, and a wave turns the
+// winners of its own codebooks into its operands without LDS or a barrier.
+template <int V, int NW>
+__global__ __launch_bounds__(NW * 64) void gather_sparse_few_fused_kernel(FewArgs a, Epilogue ep, FewGrid grid, FewSearch fs)
+{
+    gather_few<FEW_SPARSE, 1, NW, 1, V>(a, ep, grid, fs);
 }
 // Sparse table, TC column groups of a tile per workgroup: the operands made from index bytes serve all of them, and a launch has
 // fewer workgroups, each with as many loads in flight.  (16 waves, one or two token groups, and all four groups of a
@@ -423,6 +465,39 @@ bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
                                       3.3 + (g.CB + 15) / 16 * (0.2 + 0.003 * g.C_tile);
     if (g.gather_kind == 2 ? g.C_tile == 32 : g.C_tile != 8) return false;  // tables only a tuning asks for
     return g.gather_kind == 2 ? few_column_groups(ctx, g, n) != 0 : wgs <= 2 * cus;
+}
+
+// Whether one launch searches and gathers: up to 256 (token, codebook) pairs, which the 16 waves of every workgroup search side by side while
+// the table is on its way.  us a pass, two launches / one, launched one by one (replayed from a graph): 192 codebooks, v = 4, M = 3072 N = 1
+// 6.8 / 4.5 (4.9 / 4.2), N = 2 6.9 / 5.4 (4.8 / 5.1); 96 codebooks, v = 8, M = 2304 N = 1 7.1 / 3.9 (4.4 / 3.7), N = 2 7.1 / 4.6 (4.6 / 4.2); 25
+// codebooks 6.9 / 4.0 (4.1 / 2.6); 384 codebooks, v = 2, M = 768 N = 1 7.0 / 6.2 (5.4 / 5.8); 512, v = 4 6.8 / 7.7 (6.0 / 7.5).  Nor with more
+// workgroups than CUs, each of which would search again: 256, v = 4, M = 4096 6.2 / 8.3 (5.6 / 8.2), 128, v = 8 6.3 / 6.3 (4.8 / 6.1).
+bool amm_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
+{
+    const AmmGeom& g = a.g;
+    return n <= FEW_FUSED_TOKENS && n * g.CB_pad <= 256 && a.desc.lut_dtype == PIMDL_LUT_I8 && !a.grouped && g.gather_kind == 2 && g.C <= 16 &&
+           (g.v == 2 || g.v == 4 || g.v == 8) && !g.tune_search && !g.tune_search_tile && !ccs_exact_only() && !ccs_f32_only() &&
+           g.M_pad / 16 <= (uint32_t)ctx->prop.multiProcessorCount && gather_few_wanted(ctx, a, n);
+}
+
+int launch_amm_few(Ctx* ctx, const Amm& a, const float* d_x, float* d_out, uint32_t n, float scale, float lut_bias_term)
+{
+    const AmmGeom& g = a.g;
+    constexpr int NW = 16, LDS = few_lds_bytes(NW, 1, FEW_PITCH_ONEHOT);
+    Epilogue ep = {};
+    ep.scale = scale;
+    ep.lut_bias_term = lut_bias_term;
+    ep.bias = a.d_bias;
+    ep.act = a.desc.activation;
+    const FewArgs f = {nullptr, reinterpret_cast<const int8_t*>(a.d_lut), d_out, nullptr, n, g.M, g.M_pad / 16, g.CB_pad / 8, g.q, g.C_tile,
+                       g.idx_row_bytes, 0};
+    const FewSearch fs = {d_x, a.d_centroids, g.K, g.CB, g.C, (reinterpret_cast<uintptr_t>(d_x) & 15) == 0};
+    auto kern = g.v == 2 ? gather_sparse_few_fused_kernel<2, NW> : g.v == 4 ? gather_sparse_few_fused_kernel<4, NW> : gather_sparse_few_fused_kernel<8, NW>;
+    if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_few_fused)")) return rc;
+    snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_few_fused_kernel<%u, %d>", g.v, NW);
+    a.note_launch(0, LDS, 16, NW * 64);
+    hipLaunchKernelGGL(kern, dim3(f.groups), dim3(NW * 64), LDS, ctx->stream, f, ep, FewGrid{1, 0}, fs);
+    return hip_check(ctx, hipGetLastError(), "gather_few_fused launch");
 }
 
 int launch_gather_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc, uint32_t n, float scale,

@@ -969,6 +969,15 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
     return apply_runtime_tuning(g, tune, why);
 }
 
+int launch_amm(Ctx* ctx, const Amm& a, const float* d_x, uint8_t* d_idx, float* d_out, uint32_t n)
+{
+    if (n == 0) return PIMDL_OK;
+    if (amm_few_wanted(ctx, a, n))
+        return launch_amm_few(ctx, a, d_x, d_out, n, a.h_scale0, a.desc.bias_mode == PIMDL_BIAS_TIMES_CB ? a.desc.lut_bias * (float)a.g.CB : a.desc.lut_bias);
+    if (int rc = launch_ccs(ctx, a.g, d_x, a.d_centroids, d_idx, n)) return rc;
+    return launch_gather(ctx, a, d_idx, d_out, nullptr, n);
+}
+
 int launch_gather(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc, uint32_t n)
 {
     if (n == 0) return PIMDL_OK;

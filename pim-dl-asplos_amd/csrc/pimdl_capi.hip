@@ -1114,8 +1114,7 @@ int pimdl_amm_run(pimdl_amm* a, const float* in, uint32_t n, float* out)
     Ctx* ctx = a->ctx;
     if ((rc = ensure(ctx, &ctx->d_idx, &ctx->idx_bytes, idx_buffer_bytes(a->g, n), "hipMalloc(index scratch)"))) return rc;
     auto run_rows = [&](const float* d_in, float* d_out, uint32_t tokens) -> int {
-        int r = launch_ccs(ctx, a->g, d_in, a->d_centroids, ctx->d_idx, tokens);
-        return r ? r : launch_gather(ctx, *a, ctx->d_idx, d_out, nullptr, tokens);
+        return launch_amm(ctx, *a, d_in, ctx->d_idx, d_out, tokens);
     };
     const bool in_host = !is_device_ptr(in), out_host = !is_device_ptr(out);
     if (in_host || out_host) return run_piped(ctx, a->g.K, a->g.M, in, in_host, out, out_host, n, run_rows);
@@ -1147,8 +1146,7 @@ int pimdl_amm_run_noalloc(pimdl_amm* a, const float* in_dev, uint32_t n, float* 
     // padded codebooks included, and index bytes of tokens past n only reach accumulators that are never stored.
     uint8_t* d_idx = ctx->d_static_scratch;  // the device address from hipGetSymbolAddress, never the array's name
     for (uint32_t at = 0, count = head; at < n && !rc; at += count, count = n - at) {
-        rc = launch_ccs(ctx, a->g, in_dev + (size_t)at * a->g.K, a->d_centroids, d_idx, count);
-        if (!rc) rc = launch_gather(ctx, *a, d_idx, out_dev + (size_t)at * a->g.M, nullptr, count);
+        rc = launch_amm(ctx, *a, in_dev + (size_t)at * a->g.K, d_idx, out_dev + (size_t)at * a->g.M, count);
     }
     return rc;
 }

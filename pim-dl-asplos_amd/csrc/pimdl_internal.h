@@ -206,6 +206,12 @@ int launch_gather_rows(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_ou
 bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n);
 int launch_gather_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc_or_null, uint32_t n,
                       float scale, float lut_bias_term);
+// one or two tokens: search and gather in one launch (gather_few_kernel.hip); the same bits as the two launches
+bool amm_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n);
+int launch_amm_few(Ctx* ctx, const Amm& a, const float* d_x, float* d_out, uint32_t n, float scale, float lut_bias_term);
+// search and gather of n tokens on device buffers
+int launch_amm(Ctx* ctx, const Amm& a, const float* d_x, uint8_t* d_idx, float* d_out, uint32_t n);
+bool ccs_f32_only();
 uint32_t rows_lds_bytes(uint32_t c_tile, uint32_t q);
 uint32_t sparse_tile_column(uint32_t tn, uint32_t s);  // column of a tile stored at position s of the tile
 uint32_t sparse_lds_bytes(uint32_t tn, bool wide);

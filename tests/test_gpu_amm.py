@@ -1067,6 +1067,45 @@ def test_matrix_core_gathers_at_ragged_sizes(ctx, kernel, C, widths, N, CB, M):
         amm.close()
 
 
+@pytest.mark.parametrize("N,CB,v,C,M", [(1, 192, 4, 16, 3072), (2, 96, 8, 16, 2300), (1, 256, 2, 16, 768), (2, 128, 4, 9, 100), (1, 1, 4, 16, 1),
+                                        (2, 3, 2, 1, 17), (1, 97, 8, 16, 4000), (2, 33, 4, 13, 63), (1, 200, 4, 10, 1000)])
+def test_one_launch_for_one_or_two_tokens(ctx, N, CB, v, C, M):
+    """Search and gather in one launch: the output bits of the oracle and of the two launches, with near ties, repeated centroids, NaN and
+    infinities in the row, rows that are only 4-byte aligned, and through the allocation-free entry; nothing behind the output."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape")
+    import torch
+    x, cent, lut, bias = make_case(8100 + N + CB, N, CB * v, v, C, M)
+    rng = np.random.default_rng(CB + C)
+    if C > 2:
+        cent[::3, C // 2] = cent[::3, 0]
+        cent[1::3, C - 1] = cent[1::3, 1] + np.float32(3e-7)
+    xv = x.reshape(N, CB, v)
+    near = cent[np.arange(CB), rng.integers(0, C, (N, CB))]
+    pick = rng.random((N, CB)) < 0.4
+    xv[pick] = near[pick] + rng.choice([0.0, 1e-4, 5e-4], (int(pick.sum()), 1)).astype(np.float32)
+    xv[rng.random((N, CB)) < 0.02] = np.nan
+    xv[rng.random((N, CB)) < 0.02] = np.inf
+    want = oracle.amm_cpu(x, cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)[0]
+    amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=8, tuning={"gather_kernel": pimdl.GATHER_SPARSE})
+    two = amm.run_debug(x)[0]
+    assert "_fused_" not in amm.last_gather_kernel()
+    assert np.array_equal(two.view(np.uint32), want.view(np.uint32))
+    for shift in (0, 1):
+        xd = torch.empty(N * CB * v + shift, device="cuda")[shift:]
+        xd.copy_(torch.from_numpy(x.reshape(-1)).cuda())
+        for run in (amm.run_ptr, amm.run_noalloc_ptr):
+            out = torch.full((N + 1, M), -5.0, device="cuda")
+            torch.cuda.synchronize()
+            run(xd.data_ptr(), N, out.data_ptr())
+            ctx.synchronize()
+            got = out.cpu().numpy()
+            if ctx.device_info()["compute_units"] == 256:
+                assert amm.last_gather_kernel().startswith(f"gather_sparse_few_fused_kernel<{v}, "), amm.last_gather_kernel()
+            assert np.array_equal(got[:N].view(np.uint32), want.view(np.uint32)) and (got[N:] == -5.0).all(), (shift, run.__name__)
+    amm.close()
+
+
 @pytest.mark.parametrize("N,CB,v,C", [(1, 1, 4, 16), (3, 33, 4, 9), (64, 70, 2, 16), (230, 192, 4, 16), (5, 35, 8, 1), (600, 97, 8, 16), (70, 30, 16, 13),
                                       (9, 24, 32, 16), (1, 3, 2, 17), (40, 100, 4, 32), (333, 34, 8, 24), (50, 33, 16, 32), (17, 9, 32, 20)])
 @pytest.mark.parametrize("lut", ["i8", "f32"])
