@@ -56,26 +56,11 @@ inline bool prefer_small_items(uint64_t items256, uint64_t items128, uint64_t sl
 // col_split and the token tiles congruent to tx mod tok_split (col_split * tok_split = 8), and its L2
 // fetches only that share of the LUT and of the index buffer instead of all of both.
 // col_split = 0: plain order, position p = column tile p / n_token_tiles, token tile p % n_token_tiles.
-// tok_block = 0: an XCD takes one column tile after the other through all its token tiles.  tok_block > 0: its token
-// tiles are taken in blocks of so many, a block through all of the XCD's column tiles before the next (in plain order
-// the blocks are those of the launch, and a multiple of 8 tiles keeps a token tile on one XCD).
 struct XcdMap {
     uint32_t col_split, tok_split, tok_per_xcd;  // tok_per_xcd = n_token_tiles / tok_split
-    uint32_t tok_block, block_items;             // block_items = tok_block x the column tiles that a block goes through
-    // BLOCKS: a kernel for launches with tok_block (the divisions more are latency that a launch of few slices would feel)
-    template <bool BLOCKS = false>
     __device__ __forceinline__ void decode(uint32_t p, uint32_t n_token_tiles, uint32_t& col, uint32_t& tok) const
     {
-        if constexpr (BLOCKS) {
-            const uint32_t x = col_split ? p % 8 : 0, q = col_split ? p / 8 : p;
-            const uint32_t tiles = col_split ? tok_per_xcd : n_token_tiles;
-            const uint32_t block = q / block_items, r = q % block_items, first = block * tok_block;
-            const uint32_t width = tiles - first < tok_block ? tiles - first : tok_block;  // the last one may be smaller
-            // (the same in every lane: the positions are)
-            const uint32_t c = __builtin_amdgcn_readfirstlane(r / width), t = __builtin_amdgcn_readfirstlane(first + r % width);
-            col = col_split ? x % col_split + col_split * c : c;
-            tok = col_split ? x / col_split + tok_split * t : t;
-        } else if (col_split == 0) {
+        if (col_split == 0) {
             col = p / n_token_tiles;
             tok = p % n_token_tiles;
         } else {
@@ -86,20 +71,41 @@ struct XcdMap {
     }
 };
 
+// The same dealing with an XCD's token tiles taken in blocks of tok_block, a block through all of the XCD's column tiles before the next
+// (in plain order the blocks are those of the launch, and a multiple of 8 tiles keeps a token tile on one XCD).  A map of its
+// own: the divisions more are latency that a launch of few slices would feel.
+struct XcdBlocks {
+    XcdMap map;
+    uint32_t tok_block, block_items;  // block_items = tok_block x the column tiles that a block goes through
+    __device__ __forceinline__ void decode(uint32_t p, uint32_t n_token_tiles, uint32_t& col, uint32_t& tok) const
+    {
+        const uint32_t split = map.col_split, x = split ? p % 8 : 0, q = split ? p / 8 : p;
+        const uint32_t tiles = split ? map.tok_per_xcd : n_token_tiles;
+        const uint32_t block = q / block_items, r = q % block_items, first = block * tok_block;
+        const uint32_t width = tiles - first < tok_block ? tiles - first : tok_block;  // the last one may be smaller
+        // (the same in every lane: the positions are)
+        const uint32_t c = __builtin_amdgcn_readfirstlane(r / width), t = __builtin_amdgcn_readfirstlane(first + r % width);
+        col = split ? x % split + split * c : c;
+        tok = split ? x / split + map.tok_split * t : t;
+    }
+};
+// tok_block: token tiles of an XCD per block
+inline XcdBlocks xcd_blocks(const XcdMap& map, uint32_t n_col_tiles, uint32_t n_token_tiles, uint32_t tok_block)
+{
+    const uint32_t split = map.col_split, tiles = split ? map.tok_per_xcd : n_token_tiles, want = split ? tok_block : 8 * tok_block;
+    const uint32_t block = want < tiles ? want : tiles;
+    return XcdBlocks{map, block, block * (split ? n_col_tiles / split : n_col_tiles)};
+}
+
 // Picks the split with the least L2 fill traffic: 8 * (lut_bytes / col_split + idx_bytes / tok_split).
 // forced: the caller's column split (pimdl_amm_tuning.xcd_col_split), used when it divides the tile counts
-// tok_block: token tiles per block of an XCD (0: none)
 inline XcdMap choose_xcd_map(uint32_t n_col_tiles, uint32_t n_token_tiles, uint32_t grid, uint64_t lut_bytes,
-                             uint64_t idx_bytes, uint32_t forced = 0, uint32_t tok_block = 0)
+                             uint64_t idx_bytes, uint32_t forced = 0)
 {
-    auto dealt = [&](uint32_t cs) {
-        const uint32_t per_xcd = n_token_tiles / (8 / cs), block = tok_block < per_xcd ? tok_block : tok_block ? per_xcd : 0;
-        return XcdMap{cs, 8 / cs, per_xcd, block, block * (n_col_tiles / cs)};
-    };
-    const uint32_t plain_block = 8 * tok_block < n_token_tiles ? 8 * tok_block : tok_block ? n_token_tiles : 0;
-    XcdMap best{0, 0, 0, plain_block, plain_block * n_col_tiles};
+    XcdMap best{0, 0, 0};
     if (grid % 8 != 0 || forced == PIMDL_XCD_PLAIN) return best;
-    if (forced && n_col_tiles % forced == 0 && n_token_tiles % (8 / forced) == 0) return dealt(forced);
+    if (forced && n_col_tiles % forced == 0 && n_token_tiles % (8 / forced) == 0)
+        return XcdMap{forced, 8 / forced, n_token_tiles / (8 / forced)};
     uint64_t best_cost = lut_bytes + idx_bytes / 8 + 1;  // plain order: every XCD reads the whole LUT
     best_cost *= 8;
     for (uint32_t cs = 8; cs >= 1; cs /= 2) {
@@ -108,7 +114,7 @@ inline XcdMap choose_xcd_map(uint32_t n_col_tiles, uint32_t n_token_tiles, uint3
         const uint64_t cost = 8 * (lut_bytes / cs + idx_bytes / ts);
         if (cost < best_cost) {
             best_cost = cost;
-            best = dealt(cs);
+            best = XcdMap{cs, ts, n_token_tiles / ts};
         }
     }
     return best;

@@ -282,7 +282,7 @@ __global__ __launch_bounds__(OH_THREADS, 2) void gather_onehot_kernel(
         asm volatile("" : "+v"(je), "+v"(ge));
         const uint32_t colblk = col_of(item);
         Epilogue epl = ep;
-        if (ep.op_col_tiles) epl.scale = scalar_load1(ep.op_scales + __builtin_amdgcn_readfirstlane(colblk / ep.op_col_tiles));
+        if (ep.op_col_tiles) epl.scale = scalar_load1(ep.op_scales + colblk / ep.op_col_tiles);
         const uint32_t tile_tok0 = tok_tile_of(item) * OH_TOK_ITEM;
         const uint32_t tok0 = tile_tok0 + wave * (TM * 16);
         const bool vec_store = (M % 4 == 0);

@@ -160,7 +160,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void gather_i8_kernel(
         constexpr bool ACT = decltype(actc)::value;
         const uint32_t col = col_of(item);
         Epilogue epl = ep;
-        if (ep.op_col_tiles) epl.scale = scalar_load1(ep.op_scales + __builtin_amdgcn_readfirstlane(col / ep.op_col_tiles));
+        if (ep.op_col_tiles) epl.scale = scalar_load1(ep.op_scales + col / ep.op_col_tiles);
         // (opaque, so that none of the address arithmetic is kept in registers through the slices)
         uint32_t je = j, ge = g;
         asm volatile("" : "+v"(je), "+v"(ge));
