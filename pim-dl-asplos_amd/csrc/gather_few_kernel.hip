@@ -442,7 +442,7 @@ uint32_t few_column_groups(const Ctx* ctx, const AmmGeom& g, uint32_t n)
 // Whether these kernels are the shorter launch.  The large kernels' time is flat while their items do not fill the chip
 // (us, large / few): one-hot tables 768 -> 3072 8.1 / 3.0 at N = 1, 8.7 / 4.1 at 64, 9.1 / 9.7 at 300; 3072 -> 768
 // 19.8 / 4.5 at 1, 20.2 / 7.7 at 150, 19.8 / 13.1 at 512, 20.3 / 18.2 at 1024; 8 centroids 3072 -> 768 15.4 / 5.9 at 64,
-// 15.6 / 10.0 at 512: up to two workgroups of this launch per CU.
+// 15.6 / 10.0 at 512: up to two workgroups of this launch per CU (the paired table; for the sparse one few_column_groups decides).
 // The byte adder and the floats read every gathered piece from the caches on its own, which costs in proportion to
 // tokens x codebooks x columns; against that stands the large kernels' chain of slices.  Byte adder, 3072 -> 768,
 // 32 centroids: 17.6 / 4.4 at N = 1, 17.7 / 7.9 at 13, 17.8 / 27.4 at 64; 1000 -> 1001, 200 centroids: 18.9 / 5.8 at 13,
