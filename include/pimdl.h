@@ -191,7 +191,7 @@ PIMDL_API int pimdl_amm_destroy(pimdl_amm* amm);
 /* The AMM itself.  Replaces amm_host (src/host/amm_host.h:8-10, amm_host.cpp:10-30) =
  * index_calculation + pim_lut, with row-major input and output.
  *   in   fp32 [n][K], host or device
- *   out  fp32 [n][M], host or device
+ *   out  fp32 [n][M], host or device; on the device it may overlap an `in` there
  * Synchronous for host pointers.  For device pointers the kernels are queued on the context's
  * stream and the call returns at once; use pimdl_synchronize() or stream ordering.
  * Host buffers may be ordinary pageable memory: the batch is cut into chunks of tokens that are copied into
@@ -207,6 +207,7 @@ PIMDL_API int pimdl_amm_run(pimdl_amm* amm, const float* in, uint32_t n, float* 
  * kernel live in a fixed array of PIMDL_NOALLOC_SCRATCH_BYTES inside the library's device image (each GPU
  * the library runs on holds its copy until the process ends) instead of the context's grow-only scratch.
  *   in_dev, out_dev  DEVICE pointers, fp32 [n][K] and [n][M]; queued on the context's stream, returns at once.
+ *   With K == M they may be the same.
  *   PIMDL_ERR_INVALID when a pointer is a host pointer, or when n tokens need more index bytes than the array
  *   holds: n rounded up to 64 (int8 tables of up to 32 centroids; else n), times num_codebook rounded up to 32,
  *   times 1/2 byte (up to 16 centroids) or 1 byte (more).  BERT-base's 3072 -> 768 matrix at n = 8192 needs 3 MiB.

@@ -972,7 +972,11 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
 int launch_amm(Ctx* ctx, const Amm& a, const float* d_x, uint8_t* d_idx, float* d_out, uint32_t n)
 {
     if (n == 0) return PIMDL_OK;
-    if (amm_few_wanted(ctx, a, n))
+    // Of two launches the first has read every row before the second writes, so the output may lie on the input, in whole or in part; the
+    // workgroups of one launch read all rows while others write, which only buffers apart from each other bear.
+    const uintptr_t x = reinterpret_cast<uintptr_t>(d_x), out = reinterpret_cast<uintptr_t>(d_out);
+    const bool apart = x + (size_t)n * a.g.K * 4 <= out || out + (size_t)n * a.g.M * 4 <= x;
+    if (apart && amm_few_wanted(ctx, a, n))
         return launch_amm_few(ctx, a, d_x, d_out, n, a.h_scale0, a.desc.bias_mode == PIMDL_BIAS_TIMES_CB ? a.desc.lut_bias * (float)a.g.CB : a.desc.lut_bias);
     if (int rc = launch_ccs(ctx, a.g, d_x, a.d_centroids, d_idx, n)) return rc;
     return launch_gather(ctx, a, d_idx, d_out, nullptr, n);

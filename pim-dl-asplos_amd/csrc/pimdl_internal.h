@@ -206,7 +206,7 @@ int launch_gather_rows(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_ou
 bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n);
 int launch_gather_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc_or_null, uint32_t n,
                       float scale, float lut_bias_term);
-// one or two tokens: search and gather in one launch (gather_few_kernel.hip); the same bits as the two launches
+// one or two tokens: search and gather in one launch (gather_few_kernel.hip); the same bits as the two launches.  d_out must not overlap d_x.
 bool amm_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n);
 int launch_amm_few(Ctx* ctx, const Amm& a, const float* d_x, float* d_out, uint32_t n, float scale, float lut_bias_term);
 // search and gather of n tokens on device buffers

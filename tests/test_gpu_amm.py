@@ -1106,6 +1106,31 @@ def test_one_launch_for_one_or_two_tokens(ctx, N, CB, v, C, M):
     amm.close()
 
 
+@pytest.mark.parametrize("N", [1, 2, 3])
+@pytest.mark.parametrize("K,M,v,shift", [(512, 512, 4, 0), (256, 256, 2, 0), (256, 256, 2, 100), (512, 512, 8, -300), (256, 700, 4, 255), (512, 100, 4, 30),
+                                         (256, 256, 4, -1), (256, 700, 4, None), (512, 100, 4, None)])
+def test_output_that_lies_on_the_input(ctx, N, K, M, v, shift):
+    """The output's first float `shift` floats behind the input's: every row is searched as it was before the call, for one and two tokens too.
+    (None: right behind the input's last float, which one launch bears.)"""
+    import torch
+    x, cent, lut, bias = make_case(910 + N + K, N, K, v, 16, M)
+    want = oracle.amm_cpu(x, cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)[0]
+    amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=4)
+    at = N * K if shift is None else shift
+    start = 1000  # of the input in the buffer
+    for run in (amm.run_ptr, amm.run_noalloc_ptr):
+        buf = torch.full((start + N * (K + M) + 1000,), -5.0, device="cuda")
+        buf[start:start + N * K] = torch.from_numpy(x.reshape(-1)).cuda()
+        torch.cuda.synchronize()
+        run(buf.data_ptr() + 4 * start, N, buf.data_ptr() + 4 * (start + at))
+        ctx.synchronize()
+        got = buf[start + at:start + at + N * M].cpu().numpy().reshape(N, M)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), run.__name__
+        if ctx.device_info()["compute_units"] == 256 and not kernel_switches():
+            assert ("_fused_" in amm.last_gather_kernel()) == (shift is None and N <= 2), amm.last_gather_kernel()
+    amm.close()
+
+
 @pytest.mark.parametrize("N,CB,v,C", [(1, 1, 4, 16), (3, 33, 4, 9), (64, 70, 2, 16), (230, 192, 4, 16), (5, 35, 8, 1), (600, 97, 8, 16), (70, 30, 16, 13),
                                       (9, 24, 32, 16), (1, 3, 2, 17), (40, 100, 4, 32), (333, 34, 8, 24), (50, 33, 16, 32), (17, 9, 32, 20)])
 @pytest.mark.parametrize("lut", ["i8", "f32"])
