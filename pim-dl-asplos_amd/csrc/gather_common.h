@@ -76,15 +76,23 @@ struct XcdMap {
 // own: the divisions more are latency that a launch of few slices would feel.
 struct XcdBlocks {
     XcdMap map;
+    static __host__ __device__ __forceinline__ uint32_t uniform(uint32_t i)  // the same in every lane: the positions are
+    {
+#ifdef __HIP_DEVICE_COMPILE__
+        return __builtin_amdgcn_readfirstlane(i);
+#else
+        return i;
+#endif
+    }
     uint32_t tok_block, block_items;  // block_items = tok_block x the column tiles that a block goes through
-    __device__ __forceinline__ void decode(uint32_t p, uint32_t n_token_tiles, uint32_t& col, uint32_t& tok) const
+    __host__ __device__ __forceinline__ void decode(uint32_t p, uint32_t n_token_tiles, uint32_t& col, uint32_t& tok) const
     {
         const uint32_t split = map.col_split, x = split ? p % 8 : 0, q = split ? p / 8 : p;
         const uint32_t tiles = split ? map.tok_per_xcd : n_token_tiles;
         const uint32_t block = q / block_items, r = q % block_items, first = block * tok_block;
-        const uint32_t width = tiles - first < tok_block ? tiles - first : tok_block;  // the last one may be smaller
-        // (the same in every lane: the positions are)
-        const uint32_t c = __builtin_amdgcn_readfirstlane(r / width), t = __builtin_amdgcn_readfirstlane(first + r % width);
+        // The last block may be smaller.  (Behind the last item a workgroup decodes one position that it never uses: no tiles are left there.)
+        const uint32_t left = first < tiles ? tiles - first : 1, width = left < tok_block ? left : tok_block;
+        const uint32_t c = uniform(r / width), t = uniform(first + r % width);
         col = split ? x % split + split * c : c;
         tok = split ? x / split + map.tok_split * t : t;
     }
