@@ -71,38 +71,52 @@ struct XcdMap {
     }
 };
 
+// Quotient and remainder by a number that the launch knows, on the scalar unit: the estimate is the quotient or one less
+// (m > 2^32 / d - 1, so i m / 2^32 > i / d - 1).
+struct DivideBy {
+    uint32_t d, m;  // m = 2^32 / d rounded down, all ones for d = 1
+    __host__ __device__ __forceinline__ uint32_t quotient(uint32_t i, uint32_t& rest) const
+    {
+        uint32_t q = (uint32_t)((uint64_t)i * m >> 32);
+        rest = i - q * d;
+        if (rest >= d) {
+            rest -= d;
+            ++q;
+        }
+        return q;
+    }
+};
+inline DivideBy divide_by(uint32_t d) { return DivideBy{d, d > 1 ? (uint32_t)((1ull << 32) / d) : 0xFFFFFFFFu}; }
+
 // The same dealing with an XCD's token tiles taken in blocks of tok_block, a block through all of the XCD's column tiles before the next
 // (in plain order the blocks are those of the launch, and a multiple of 8 tiles keeps a token tile on one XCD).  A map of its
-// own: the divisions more are latency that a launch of few slices would feel.
+// own, and without a division: a workgroup decodes a position several times per item, which a launch of few slices feels.
+// Gather, us, with divisions / as it is: 64 codebooks of 8 floats, N = 24000, M = 3000 77 / 72, 100 codebooks 106 / 98; 32 codebooks, N = 22000,
+// M = 3500 75.8 / 72.8; 24 codebooks, N = 31894, M = 2304 54.7 / 53.9.
 struct XcdBlocks {
-    XcdMap map;
-    static __host__ __device__ __forceinline__ uint32_t uniform(uint32_t i)  // the same in every lane: the positions are
+    uint32_t xcd_bits, col_bits, tok_bits;  // 3 = col_bits + tok_bits of a position choose the XCD; all 0 in plain order
+    uint32_t last;                          // block, which may be smaller
+    uint32_t tok_block;
+    DivideBy items, width, last_width;      // items of a block, its token tiles
+    __host__ __device__ __forceinline__ void decode(uint32_t p, uint32_t /* n_token_tiles */, uint32_t& col, uint32_t& tok) const
     {
-#ifdef __HIP_DEVICE_COMPILE__
-        return __builtin_amdgcn_readfirstlane(i);
-#else
-        return i;
-#endif
-    }
-    uint32_t tok_block, block_items;  // block_items = tok_block x the column tiles that a block goes through
-    __host__ __device__ __forceinline__ void decode(uint32_t p, uint32_t n_token_tiles, uint32_t& col, uint32_t& tok) const
-    {
-        const uint32_t split = map.col_split, x = split ? p % 8 : 0, q = split ? p / 8 : p;
-        const uint32_t tiles = split ? map.tok_per_xcd : n_token_tiles;
-        const uint32_t block = q / block_items, r = q % block_items, first = block * tok_block;
-        // The last block may be smaller.  (Behind the last item a workgroup decodes one position that it never uses: no tiles are left there.)
-        const uint32_t left = first < tiles ? tiles - first : 1, width = left < tok_block ? left : tok_block;
-        const uint32_t c = uniform(r / width), t = uniform(first + r % width);
-        col = split ? x % split + split * c : c;
-        tok = split ? x / split + map.tok_split * t : t;
+        const uint32_t x = p & ((1u << xcd_bits) - 1);
+        uint32_t r, t;
+        const uint32_t block = items.quotient(p >> xcd_bits, r);
+        // (behind the last item a workgroup decodes one position that it never uses)
+        const uint32_t c = (block < last ? width : last_width).quotient(r, t);
+        col = (x & ((1u << col_bits) - 1)) + (c << col_bits);
+        tok = (x >> col_bits) + (block * tok_block + t << tok_bits);
     }
 };
 // tok_block: token tiles of an XCD per block
 inline XcdBlocks xcd_blocks(const XcdMap& map, uint32_t n_col_tiles, uint32_t n_token_tiles, uint32_t tok_block)
 {
     const uint32_t split = map.col_split, tiles = split ? map.tok_per_xcd : n_token_tiles, want = split ? tok_block : 8 * tok_block;
-    const uint32_t block = want < tiles ? want : tiles;
-    return XcdBlocks{map, block, block * (split ? n_col_tiles / split : n_col_tiles)};
+    const uint32_t block = want < tiles ? want : tiles, last = (tiles - 1) / block;
+    const uint32_t col_bits = split == 8 ? 3 : split == 4 ? 2 : split == 2 ? 1 : 0;
+    return XcdBlocks{split ? 3u : 0u, col_bits, split ? 3 - col_bits : 0, last, block,
+                     divide_by(block * (split ? n_col_tiles / split : n_col_tiles)), divide_by(block), divide_by(tiles - last * block)};
 }
 
 // Picks the split with the least L2 fill traffic: 8 * (lut_bytes / col_split + idx_bytes / tok_split).
