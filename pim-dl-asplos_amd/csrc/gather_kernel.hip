@@ -873,7 +873,7 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
         // leave room for two workgroups per CU
         const uint32_t slots = 2 * (num_cus ? num_cus : 256);
         const uint32_t tiles = (d.max_n + 255) / 256;
-        auto pick_tn = [&](bool paired_layout) {
+        auto pick_tn = [&](bool paired_layout, bool by_rows = true) {  // by_rows: with what whole 16 KiB rows are worth
             double best = 1e300;
             uint32_t pick = 0;
             for (uint32_t tn : {6u, 4u, 3u}) {
@@ -885,7 +885,7 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
                 // Outputs beyond the caches in rows of whole 16 KiB: 64 columns of a row are 256-byte pieces on their
                 // own memory channels, 96 are not (1024 -> 4096, N = 32768, us, 96 / 64 columns: v = 4 311 / 267, v = 8
                 // 218 / 161, v = 16 166 / 106; M = 3072, where no tile width meets the channels again: 163 / 174 at v = 4).
-                const double width = tn == 4 && M % 4096 == 0 && (uint64_t)d.max_n * M * 4 >= SP_LARGE_OUTPUT ? 0.9 : 1.0;
+                const double width = by_rows && tn == 4 && M % 4096 == 0 && (uint64_t)d.max_n * M * 4 >= SP_LARGE_OUTPUT ? 0.9 : 1.0;
                 const double t256 = grid_rounds(items, slots) * item_cost(tn, false) * width;
                 const double t128 = grid_rounds(items_small, slots) * item_cost(tn, true) * width;
                 const double t = t128 < t256 ? t128 : t256;  // the launcher takes the better item size
@@ -901,9 +901,11 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
         // Measured over N 2048..12608, K and M 768..4096, vec_len 2..8: the sparse kernel is 3 to 38 % faster where
         // the launch is large against its codebook count (tokens x columns >= 65536 x codebooks) and either
         // 96-column tiles are its best launch or there are at most 128 codebooks; elsewhere 0 to 20 % slower.
+        // (Rows of whole 16 KiB, where it takes 64-column tiles instead, are no exception: passes, us, paired / sparse, M = 4096: 256 codebooks
+        // N = 32768 350 / 270, N = 16384 163 / 138; 160 codebooks N = 16384 124 / 97; M = 8192, 256 codebooks N = 8192 160 / 141.)
         if (C <= 8 && g->gather_kind == 1 && tune.gather_kernel == PIMDL_GATHER_AUTO && !gather_dense_only() &&
             (col_block_hint == 96 ||  // (only the sparse kernel has that tile)
-             ((uint64_t)d.max_n * M >= 65536ull * g->CB && (pick_tn(false) == 6 || g->CB <= 128))))
+             ((uint64_t)d.max_n * M >= 65536ull * g->CB && (pick_tn(false, false) == 6 || g->CB <= 128))))
             g->gather_kind = 2;
         const bool paired = C <= 8 && g->gather_kind == 1;
         g->C_tile = paired ? 8 : C > 16 ? 32 : 16;

@@ -1236,6 +1236,32 @@ def test_sparse_gather_of_large_outputs(ctx, N, M, tuning):
     amm.close()
 
 
+@pytest.mark.parametrize("N,CB,C,M", [(16384, 130, 8, 4096), (16384, 160, 3, 4096), (16640, 130, 8, 4160)])
+def test_large_outputs_of_up_to_8_centroids(ctx, N, CB, C, M):
+    """More than 128 codebooks and 96-column tiles by themselves the best launch: the sparse kernel, also where rows of whole 16 KiB make it
+    64-column tiles; the bits of the paired kernel's operator, and of the oracle."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    import torch
+    v = 2
+    _, cent, lut, bias = make_case(615 + M + C, 1, CB * v, v, C, M)
+    x = torch.randn((N, CB * v), device="cuda", generator=torch.Generator(device="cuda").manual_seed(N + C))
+    outs = [torch.full((N + 2, M), -5.0, device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    for tuning, out in zip(({}, {"gather_kernel": pimdl.GATHER_ONEHOT}), outs):
+        amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=N, tuning=tuning)
+        amm.run_ptr(x.data_ptr(), N, out.data_ptr())
+        ctx.synchronize()
+        name = amm.last_gather_kernel()
+        if ctx.device_info()["compute_units"] == 256:
+            assert name.startswith("gather_onehot_kernel<" if tuning else "gather_sparse_blocks_kernel<"), name
+        amm.close()
+    assert torch.equal(outs[0][:N], outs[1][:N]) and bool((outs[0][N:] == -5.0).all())
+    n = 200
+    want = oracle.amm_cpu(x[:n].cpu().numpy(), cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)[0]
+    assert np.array_equal(outs[0][:n].cpu().numpy().view(np.uint32), want.view(np.uint32))
+
+
 def gather_us(ctx, N, CB, C, M, lut="i8", tuning=None, v=4, group=0):
     """Shortest of a few timings of an operator's gather, us."""
     import torch
