@@ -93,7 +93,7 @@ typedef struct pimdl_amm_group pimdl_amm_group; /* operators that read the same 
 typedef struct pimdl_amm_timing {
     float ccs_ms;    /* closest-centroid search kernel */
     float gather_ms; /* LUT gather-accumulate (+ epilogue) kernel */
-    float total_ms;  /* both, back to back, as pimdl_amm_run issues them */
+    float total_ms;  /* what pimdl_amm_run issues: both, back to back, or the one launch it makes of one or two tokens */
 } pimdl_amm_timing;
 
 /* ---- context ---------------------------------------------------------------------------
@@ -248,7 +248,7 @@ PIMDL_API int pimdl_amm_group_destroy(pimdl_amm_group* group);
 PIMDL_API int pimdl_amm_group_fused_cols(const pimdl_amm_group* group, uint32_t* cols);
 PIMDL_API int pimdl_amm_group_run_fused(pimdl_amm_group* group, const float* in, uint32_t n, float* out);
 
-/* Runs the two kernels `iters` times each on device-resident buffers and reports the average
+/* Runs the two kernels and the whole pass `iters` times each on device-resident buffers and reports the average
  * device time of each.  in/out must be DEVICE pointers. */
 PIMDL_API int pimdl_amm_profile(pimdl_amm* amm, const float* in_dev, uint32_t n, float* out_dev,
                                 uint32_t warmup, uint32_t iters, pimdl_amm_timing* timing);

@@ -1194,12 +1194,15 @@ int pimdl_amm_profile(pimdl_amm* a, const float* in_dev, uint32_t n, float* out_
         if ((rc = launch_ccs(ctx, a->g, in_dev, a->d_centroids, ctx->d_idx, n))) return rc;
         if ((rc = launch_gather(ctx, *a, ctx->d_idx, out_dev, nullptr, n))) return rc;
     }
+    if (warmup && (rc = launch_amm(ctx, *a, in_dev, ctx->d_idx, out_dev, n))) return rc;  // (one or two tokens: another kernel)
     float ms[3] = {0, 0, 0};
     for (int phase = 0; phase < 3; ++phase) {
         if ((rc = hip_check(ctx, hipEventRecord(ctx->ev[0], ctx->stream), "hipEventRecord"))) return rc;
         for (uint32_t i = 0; i < iters; ++i) {
-            if (phase != 1 && (rc = launch_ccs(ctx, a->g, in_dev, a->d_centroids, ctx->d_idx, n))) return rc;
-            if (phase != 0 && (rc = launch_gather(ctx, *a, ctx->d_idx, out_dev, nullptr, n))) return rc;
+            if (phase == 0) rc = launch_ccs(ctx, a->g, in_dev, a->d_centroids, ctx->d_idx, n);
+            else if (phase == 1) rc = launch_gather(ctx, *a, ctx->d_idx, out_dev, nullptr, n);
+            else rc = launch_amm(ctx, *a, in_dev, ctx->d_idx, out_dev, n);
+            if (rc) return rc;
         }
         if ((rc = hip_check(ctx, hipEventRecord(ctx->ev[1], ctx->stream), "hipEventRecord"))) return rc;
         if ((rc = hip_check(ctx, hipEventSynchronize(ctx->ev[1]), "hipEventSynchronize"))) return rc;

@@ -1107,6 +1107,27 @@ def test_one_launch_for_one_or_two_tokens(ctx, N, CB, v, C, M):
 
 
 @pytest.mark.parametrize("N", [1, 2, 3])
+def test_profile_times_the_pass_that_a_run_makes(ctx, N):
+    """total_ms is of the launches of pimdl_amm_run, one or two; the last of them is what the operator names afterwards."""
+    import torch
+    x, cent, lut, bias = make_case(930 + N, N, 512, 4, 16, 300)
+    want = oracle.amm_cpu(x, cent, lut, bias, 4, 0.0123, 0.0, threads=THREADS)[0]
+    amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=4)
+    xd, out = torch.from_numpy(x).cuda(), torch.empty((N, 300), device="cuda")
+    torch.cuda.synchronize()
+    t = amm.profile(xd.data_ptr(), N, out.data_ptr(), warmup=2, iters=3)
+    profiled = amm.last_gather_kernel()
+    assert all(ms > 0 for ms in t.values())
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    amm.run_ptr(xd.data_ptr(), N, out.data_ptr())
+    ctx.synchronize()
+    assert profiled == amm.last_gather_kernel()
+    if ctx.device_info()["compute_units"] == 256 and not kernel_switches():
+        assert ("_fused_" in profiled) == (N <= 2), profiled
+    amm.close()
+
+
+@pytest.mark.parametrize("N", [1, 2, 3])
 @pytest.mark.parametrize("K,M,v,shift", [(512, 512, 4, 0), (256, 256, 2, 0), (256, 256, 2, 100), (512, 512, 8, -300), (256, 700, 4, 255), (512, 100, 4, 30),
                                          (256, 256, 4, -1), (256, 700, 4, None), (512, 100, 4, None)])
 def test_output_that_lies_on_the_input(ctx, N, K, M, v, shift):
