@@ -1106,6 +1106,33 @@ def test_one_launch_for_one_or_two_tokens(ctx, N, CB, v, C, M):
     amm.close()
 
 
+@pytest.mark.parametrize("N,v,lut_bias,mode,with_bias,act", [(1, 4, 0.25, 0, True, 0), (2, 8, 0.25, 1, True, 0), (1, 2, -0.125, 1, False, 0), (2, 4, 0.0, 0, False, 0),
+                                                             (1, 8, 0.25, 1, True, 1), (2, 2, 0.0, 0, False, 1)])
+def test_epilogue_of_one_launch(ctx, N, v, lut_bias, mode, with_bias, act):
+    """Bias or none, the table's own bias once or per codebook, GELU: the bits of the two launches, and without GELU the oracle's."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape")
+    import torch
+    CB, C, M = 75, 16, 500
+    x, cent, lut, bias = make_case(8300 + N + v, N, CB * v, v, C, M)
+    bias = bias if with_bias else None
+    amm = ctx.amm(cent, lut, np.float32(0.0371), bias, max_n=8, lut_bias=lut_bias, bias_mode=mode,
+                  activation=pimdl.ACT_GELU_TANH if act else pimdl.ACT_NONE)
+    two, idx, acc = amm.run_debug(x)
+    if not act:
+        want = oracle.dequant(acc, np.zeros(M, np.float32) if bias is None else bias, CB, 0.0371, lut_bias, mode, threads=THREADS)
+        assert np.array_equal(two.view(np.uint32), want.view(np.uint32))
+    xd, out = torch.from_numpy(x).cuda(), torch.full((N + 1, M), -5.0, device="cuda")
+    torch.cuda.synchronize()
+    amm.run_ptr(xd.data_ptr(), N, out.data_ptr())
+    ctx.synchronize()
+    if ctx.device_info()["compute_units"] == 256:
+        assert "_fused_" in amm.last_gather_kernel(), amm.last_gather_kernel()
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:N].view(np.uint32), two.view(np.uint32)) and (got[N:] == -5.0).all()
+    amm.close()
+
+
 @pytest.mark.parametrize("N", [1, 2, 3])
 def test_profile_times_the_pass_that_a_run_makes(ctx, N):
     """total_ms is of the launches of pimdl_amm_run, one or two; the last of them is what the operator names afterwards."""
@@ -1255,6 +1282,78 @@ def test_sparse_gather_of_large_outputs(ctx, N, M, tuning):
     want = oracle.amm_cpu(x[:n].cpu().numpy(), cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)[0]
     assert np.array_equal(out[:n].cpu().numpy().view(np.uint32), want.view(np.uint32))
     amm.close()
+
+
+@pytest.mark.parametrize("N,CB,M,act,tuning,form", [
+    (32700, 64, 2060, 0, {"col_block": 48}, "<3, 4, 64, 8>"),               # eight waves by the launch rule
+    (17000, 70, 4001, 0, {"col_block": 48, "token_item": 512, "cb_per_slice": 32}, "<3, 4, 32, 8>"),
+    (17000, 70, 4001, 0, {"col_block": 64, "token_item": 512}, "<4, 4, 32, 8>"),
+    (16500, 40, 4096, 0, {"col_block": 64, "token_item": 512, "cb_per_slice": 16}, "<4, 4, 16, 8>"),
+    (18000, 40, 3800, 0, {"col_block": 96, "token_item": 512, "cb_per_slice": 16}, "<6, 4, 16, 8>"),
+    (17000, 200, 4000, 1, {"col_block": 96}, "<6, 4, 16, 4>"),              # many slices, GELU
+    (16390, 96, 4096, 1, {"col_block": 64}, "<4, 4, 32, 4>"),
+    (33000, 33, 2100, 1, {"col_block": 48, "token_item": 128}, "<3, 2, 32, 4>"),
+])
+def test_forms_of_the_sparse_gather_of_large_outputs(ctx, N, CB, M, act, tuning, form):
+    """Four and eight waves, slices of 16, 32 and 64 codebooks, several to an item, with GELU too: every row as in launches without blocks."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the sparse gather")
+    import torch
+    assert N * M * 4 >= 256 << 20
+    v, C = 2, 16
+    _, cent, lut, bias = make_case(717 + M + CB, 1, CB * v, v, C, M)
+    x = torch.randn((N, CB * v), device="cuda", generator=torch.Generator(device="cuda").manual_seed(N))
+    amm = ctx.amm(cent, lut, np.float32(0.0023), bias, max_n=N, tuning=tuning, activation=pimdl.ACT_GELU_TANH if act else pimdl.ACT_NONE)
+    out = torch.full((N + 2, M), -5.0, device="cuda")
+    part = torch.empty((4096, M), device="cuda")
+    torch.cuda.synchronize()
+    amm.run_ptr(x.data_ptr(), N, out.data_ptr())
+    ctx.synchronize()
+    if ctx.device_info()["compute_units"] == 256:
+        assert amm.last_gather_kernel() == "gather_sparse_blocks_kernel" + form
+    assert bool((out[N:] == -5.0).all())
+    for i in range(0, N, 4096):
+        n = min(4096, N - i)
+        torch.cuda.synchronize()
+        amm.run_ptr(x[i:].data_ptr(), n, part.data_ptr())
+        ctx.synchronize()
+        assert torch.equal(out[i:i + n], part[:n]), i
+    if not act:
+        n = 200
+        want = oracle.amm_cpu(x[:n].cpu().numpy(), cent, lut, bias, v, 0.0023, 0.0, threads=THREADS)[0]
+        assert np.array_equal(out[:n].cpu().numpy().view(np.uint32), want.view(np.uint32))
+    amm.close()
+
+
+@pytest.mark.parametrize("N,M,count", [(29200, 768, 3), (22100, 1536, 2), (32768, 1024, 3)])
+def test_operators_side_by_side_with_a_large_output(ctx, N, M, count):
+    """One gather launch for several operators whose common output is dealt out in blocks: every column as of the operator alone, whose
+    output has no blocks."""
+    if kernel_switches():
+        pytest.skip("a kernel this test is about is switched off by the environment")
+    import torch
+    assert N * M * count * 4 >= 256 << 20 > N * M * 4
+    v, CB, C = 4, 32, 16
+    amms = []
+    for i in range(count):
+        _, cent, lut, bias = make_case(818 + i, 1, CB * v, v, C, M)
+        amms.append(ctx.amm(cent, lut, np.float32(0.01 * (i + 1)), bias, max_n=N))
+    group = ctx.amm_group(amms)
+    assert group.fused_cols == M * count
+    x = torch.randn((N, CB * v), device="cuda", generator=torch.Generator(device="cuda").manual_seed(N))
+    out = torch.full((N + 1, M * count), -5.0, device="cuda")
+    alone = torch.empty((N, M), device="cuda")
+    torch.cuda.synchronize()
+    group.run_fused_ptr(x.data_ptr(), N, out.data_ptr())
+    for i, amm in enumerate(amms):
+        amm.run_ptr(x.data_ptr(), N, alone.data_ptr())
+        ctx.synchronize()
+        assert torch.equal(out[:N, i * M:(i + 1) * M], alone), i
+        torch.cuda.synchronize()
+    assert bool((out[N:] == -5.0).all())
+    group.close()
+    for amm in amms:
+        amm.close()
 
 
 @pytest.mark.parametrize("N,CB,C,M", [(16384, 130, 8, 4096), (16384, 160, 3, 4096), (16640, 130, 8, 4160)])
