@@ -1867,6 +1867,7 @@ int launch_ccs_bits(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     // N = 32 4.3 / 4.6; v = 2 384 codebooks N = 64 4.1 / 2.9, N = 128 4.1 / 3.7, N = 256 4.1 / 5.4; v = 8 96 codebooks N = 512 6.1 / 4.3, 1024 6.2 / 6.2,
     // 1024 codebooks N = 64 6.1 / 4.9, 128 6.4 / 7.3; v = 16 64 codebooks N = 128 4.0 / 2.9, 256 4.0 / 3.8; v = 32 160 codebooks N = 8 3.9 /
     // 3.2, 32 4.7 / 4.6; 32 centroids, v = 4 192 codebooks N = 64 4.8 / 2.8, 256 5.9 / 4.8, 512 5.9 / 7.1; v = 2 1536 codebooks N = 32 5.6 / 4.6.
+    // (Beyond 16 centroids the line is v = 8's, 20000: two of these points, 24576 each, lie past it and would gain a microsecond; 49152 loses one.)
     const uint64_t waves = (uint64_t)n * (g.CB_pad / (g.C > 16 ? 2 : 4));
     const uint32_t most = g.v == 32 ? 1200 : g.v == 16 ? 3500 : g.v == 8 || g.C > 16 ? 20000 : 13500;
     if (g.C <= 32 && waves <= most && !g.tune_search && !g.tune_search_tile && !exact && !f32) {

@@ -15,7 +15,7 @@ namespace {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 
-// An int8 launch: a workgroup takes 16 columns of 16 * TM tokens, its NW waves deal out the K-steps of the matrix
+// An int8 launch: a workgroup takes 16 columns (32 or 48 of the sparse table between few and many tokens) of 16 * TM tokens, its NW waves deal out the K-steps of the matrix
 // instruction, every operand comes straight from memory (nothing is shared between waves, so nothing is staged), and the
 // waves' int32 sums meet in LDS once, at the end.  All loads of a wave are in flight together: a launch is one
 // round trip for the indices and the table, not one per slice.  What bounds it: up to 16 tokens the launch itself and
@@ -252,8 +252,9 @@ __global__ __launch_bounds__(NW * 64) void gather_sparse_few_kernel(FewArgs a, E
     gather_few<FEW_SPARSE, TM, NW>(a, ep, grid);
 }
 // One or two tokens: search and gather in one launch.  Every workgroup searches all codebooks for its 16 columns, which is less
-// than a second launch: the centroids and the rows are requested with the table, so there is one round trip, and a wave turns the
-// winners of its own codebooks into its operands without LDS or a barrier.
+// than a second launch: a wave requests the centroids, the rows and its part of the table together, 16 codebooks at a time (v = 8: 8, for
+// registers), and turns the winners of its own codebooks into its operands without LDS or a barrier.  So there is one round trip up to 256
+// codebooks, 128 at v = 8, two beyond.
 template <int V, int NW>
 __global__ __launch_bounds__(NW * 64) void gather_sparse_few_fused_kernel(FewArgs a, Epilogue ep, FewGrid grid, FewSearch fs)
 {
@@ -471,11 +472,14 @@ bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
     return g.gather_kind == 2 ? few_column_groups(ctx, g, n) != 0 : wgs <= 2 * cus;
 }
 
-// Whether one launch searches and gathers: up to 256 (token, codebook) pairs, which the 16 waves of every workgroup search side by side while
-// the table is on its way.  us a pass, two launches / one, launched one by one (replayed from a graph): 192 codebooks, v = 4, M = 3072 N = 1
+// Whether one launch searches and gathers: up to 256 (token, codebook) pairs, which the 16 waves of every workgroup search side by side.
+// us a pass, two launches / one, launched one by one (replayed from a graph): 192 codebooks, v = 4, M = 3072 N = 1
 // 6.8 / 4.5 (4.9 / 4.2), N = 2 6.9 / 5.4 (4.8 / 5.1); 96 codebooks, v = 8, M = 2304 N = 1 7.1 / 3.9 (4.4 / 3.7), N = 2 7.1 / 4.6 (4.6 / 4.2); 25
 // codebooks 6.9 / 4.0 (4.1 / 2.6); 384 codebooks, v = 2, M = 768 N = 1 7.0 / 6.2 (5.4 / 5.8); 512, v = 4 6.8 / 7.7 (6.0 / 7.5).  Nor with more
 // workgroups than CUs, each of which would search again: 256, v = 4, M = 4096 6.2 / 8.3 (5.6 / 8.2), 128, v = 8 6.3 / 6.3 (4.8 / 6.1).
+// At the line, 256 workgroups: 192 codebooks, v = 4 8.1 / 4.7 (5.1 / 4.5), 256 8.1 / 5.8 (5.3 / 5.3); 256, v = 2 8.2 / 5.8 (5.3 / 5.3).  v = 8,
+// whose second round trip begins beyond 128 codebooks, M = 2304: 128 6.8 / 4.7 (4.7 / 4.2), 160 7.0 / 5.0 (4.9 / 4.6), 192 7.0 / 5.6 (5.0 / 4.9), 224 6.7 /
+// 6.1 (5.2 / 5.5), 256 7.9 / 6.5 (5.3 / 5.9): what a program that launches one by one gains there outweighs what a graph loses.
 bool amm_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
 {
     const AmmGeom& g = a.g;

@@ -885,6 +885,10 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
                 // Outputs beyond the caches in rows of whole 16 KiB: 64 columns of a row are 256-byte pieces on their
                 // own memory channels, 96 are not (1024 -> 4096, N = 32768, us, 96 / 64 columns: v = 4 311 / 267, v = 8
                 // 218 / 161, v = 16 166 / 106; M = 3072, where no tile width meets the channels again: 163 / 174 at v = 4).
+                // Passes through buffers that take turns, 96 / 64 columns: M = 4096 64 codebooks N = 16384 84.9 / 70.5, N = 32768 153 / 131, 16 codebooks
+                // N = 16384 84 / 76; M = 8192 64 codebooks N = 8192 75.4 / 72.4, N = 12288 110 / 104, 16 codebooks N = 8192 71.7 / 70.0; M = 12288 64
+                // codebooks N = 8192 101.7 / 98.0.  (One buffer written over and over, which the last cache holds in part, at 256 MiB: up to 32
+                // codebooks 62 / 66 at M = 4096, 58 / 66 at 8192; 64 codebooks 71.1 / 68.9 and 65.0 / 67.7.  From 512 MiB on as above.)
                 const double width = by_rows && tn == 4 && M % 4096 == 0 && (uint64_t)d.max_n * M * 4 >= SP_LARGE_OUTPUT ? 0.9 : 1.0;
                 const double t256 = grid_rounds(items, slots) * item_cost(tn, false) * width;
                 const double t128 = grid_rounds(items_small, slots) * item_cost(tn, true) * width;

@@ -1,4 +1,7 @@
-// Body of gather_sparse_kernel and gather_sparse_blocks_kernel (gather_sp_kernel.hip), which differ in the type of xmap.
+// Body of gather_sparse_kernel and gather_sparse_blocks_kernel (gather_sp_kernel.hip), included inside each of them and nowhere else.  It
+// takes from the kernel: the template's TN, TM, GS, NW, WIDE and KS, the arguments idx, lut, out, acc_out, N, M, CB_pad, idx_row_bytes,
+// n_token_tiles, n_items and ep, and xmap, whose type is all that the two differ in: decode(position, n_token_tiles, column tile, token
+// tile), which is also called for the position behind a workgroup's last item and must return then, with any values.
     constexpr int SP_WAVES = NW;
     constexpr int NWT = NW / KS;                   // waves with tokens of their own
     static_assert(KS == 1 || (KS == 2 && NW == 8), "the codebook split is between the two waves of a SIMD");

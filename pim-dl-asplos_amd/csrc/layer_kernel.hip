@@ -188,8 +188,9 @@ __global__ __launch_bounds__(256) void layer_norm_vec_kernel(const float* __rest
 //                      from group g), A = V[that key][16 dt + j].  Result: lane (j, g) holds dims
 //                      16 dt + 4 g + i of its query: one float4 store per 16-dim tile.
 // A row of a piece is 64 floats, all LDS banks once.  Rows lie in fours, 64 bytes between one four and the next, and the 16-byte
-// parts of a row in the order part ^ (row % 4): so the 16 keys x 4 groups of the first product's reads and the 16 dims x 4 keys
-// of the second's fall into different banks, and everything but the lane's own place is an immediate offset of the read.
+// parts of a row in the order part ^ (row % 4): so the 16 dims x 4 keys of the second product's reads fall into different banks, and
+// everything but the lane's own place is an immediate offset of the read.  Of the first product's reads (16 keys x 4 groups, served 16
+// lanes at a time) two lanes meet in a bank, 4 cycles more for each: a quarter of the LDS's cycles, which are 15 to 17 % of the kernel's.
 // What bounds it: the fp32 matrix instructions and the vector ones share a unit, so the kernel takes the sum of their
 // times; everything that a whole chunk does not need (masks, clamped rows, zeroed rows) is compiled for the last chunk alone.
 // us, before (whole chunks through registers, four barriers each, masks in every chunk, three workgroups per CU) / now, same bits:
