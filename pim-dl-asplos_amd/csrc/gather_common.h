@@ -49,6 +49,39 @@ inline bool prefer_small_items(uint64_t items256, uint64_t items128, uint64_t sl
     return grid_rounds(items128, slots) * 0.62 < grid_rounds(items256, slots);
 }
 
+// The sparse gather with 48- or 64-column tiles and up to 16 centroids: a launch of more 256-token items than two workgroups per CU take at
+// once, and of enough codebooks for its K-loop to weigh, goes to three per CU.  One against the other, us a pass over three operators,
+// inputs and outputs in turn, two / three: 64 columns, 768 -> 3072 N = 3072 (576 items) 29.8 / 28.8, N = 4096 (768) 31.5 / 30.0, N = 6000 (1152)
+// 44.5 / 44.3, N = 12608 (2400) 82.8 / 75.0, 3072 -> 768 N = 11000 (516) 105 / 98; up to 512 items 1024 -> 4096 N = 2048 27.5 / 28.2, 4096 -> 1024
+// N = 8192 97.5 / 104.  Up to 96 codebooks stores and first loads are what a launch spends its time on, and 32-codebook slices have
+// fewer of them: 48 codebooks -> 3072 N = 8192 29.7 / 31.1, N = 16384 52.8 / 51.7; 64 -> 2048 N = 6000 22.6 / 24.0; 96 -> 1024 N = 12608 31.8 / 32.3.
+inline bool sparse_three_per_cu(uint64_t items256, uint32_t cb16, uint64_t cus) { return items256 > 2 * cus && cb16 >= 128; }
+
+// Time of that kernel's launch of n tokens x M columns, in rounds of 64-column 256-token items with two workgroups per CU, for the choice
+// of the column tile.  A round of three per CU takes 1.46 of one of two (which is half as many items again); of a partly filled one
+// the part counts 1.2-fold.  A 48-column item takes 0.85 of a 64-column one; eight waves and the split of the codebooks
+// between the waves of a SIMD as in launch_sparse_tn.  What the figures give against passes timed with either tile, 48 / 64
+// columns: 3072 -> 768 N = 4096 39.9 / 44.9, N = 5000 58.0 / 51.6, N = 6000 58.8 / 63.0, N = 8192 68.3 / 72.6, N = 12608 115 / 105; 768 -> 768 N = 4096 19.6 / 20.1,
+// N = 16384 40.9 / 38.3; 768 -> 3072 N = 3072 26.5 / 28.8, N = 8192 54.3 / 50.7; 1024 -> 4096 N = 8192 84.7 / 76.3; 1280 -> 1280 N = 8192 52.3 / 46.0.
+// (96-column tiles, whose rows are pieces of 256 and 128 bytes, used to be the choice of most wide outputs; they are 0.5 to 25 % slower than
+// 64-column ones once outputs take turns instead of staying in the last cache: 768 -> 3072 N = 8192 66.6 / 57.1, N = 16384 119 / 104, 2048 -> 2048
+// N = 4096 60.5 / 47.5, before either had three workgroups per CU.)
+inline double sparse_launch_cost(uint32_t tn, uint64_t n, uint64_t M, uint32_t cb16, uint64_t cus)
+{
+    const uint64_t cols = (M + 16 * tn - 1) / (16 * tn), items = (n + 255) / 256 * cols, items_small = (n + 127) / 128 * cols;
+    const double item = tn == 3 ? 0.85 : 1.0;
+    if (tn == 3 && cb16 % 64 == 0 && cb16 >= 384 && items <= cus && 10 * items >= 7 * cus) return 0.48;
+    double t = grid_rounds(items, 2 * cus);
+    if (grid_rounds(items_small, 2 * cus) * 0.62 < t) t = grid_rounds(items_small, 2 * cus) * 0.62;
+    if (sparse_three_per_cu(items, cb16, cus)) {
+        const uint64_t rest = items % (3 * cus);
+        const double part = 1.2 * (double)rest / (double)(3 * cus);
+        const double t3 = 1.46 * ((double)(items / (3 * cus)) + (part < 1.0 ? part : 1.0));
+        if (t3 < t) t = t3;
+    }
+    return t * item;
+}
+
 // How the items (column tile x token tile) of a gather are dealt to the 8 XCDs.  Workgroup b takes
 // positions b, b + grid, ... of the item sequence and the hardware places workgroups on the XCDs
 // round-robin, so (for a grid that is a multiple of 8) positions congruent mod 8 run on one XCD, each
@@ -106,7 +139,7 @@ struct XcdBlocks {
         // (behind the last item a workgroup decodes one position that it never uses)
         const uint32_t c = (block < last ? width : last_width).quotient(r, t);
         col = (x & ((1u << col_bits) - 1)) + (c << col_bits);
-        tok = (x >> col_bits) + (block * tok_block + t << tok_bits);
+        tok = (x >> col_bits) + ((block * tok_block + t) << tok_bits);
     }
 };
 // tok_block: token tiles of an XCD per block

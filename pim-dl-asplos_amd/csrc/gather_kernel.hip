@@ -866,14 +866,13 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
     }
     g->idx_tiled = g->gather_kind != 0;
     if (g->gather_kind != 0) {
-        // One-hot matrix-core kernel: an item is 256 tokens x 16*TN columns.  Take the TN with the shortest
-        // launch for the largest batch this operator will see: rounds of the persistent grid (two workgroups
-        // per CU; grid_rounds) x the cost of an item of that width; among equals the widest.
-        // up to 8 centroids: two codebooks share a lane's 16 K-slots (C_tile 8); 96-column tiles then do not
-        // leave room for two workgroups per CU
-        const uint32_t slots = 2 * (num_cus ? num_cus : 256);
+        // One-hot matrix-core kernels: an item is 256 tokens x 16*TN columns.  Take the TN with the shortest
+        // launch for the largest batch this operator will see.  Dense kernel (up to 8 centroids, where two codebooks share a lane's
+        // 16 K-slots, C_tile 8: no 96-column tiles, which would not leave room for two workgroups per CU), and 17..32 centroids:
+        // rounds of the persistent grid (two workgroups per CU; grid_rounds) x the cost of an item of that width; among equals the widest.
+        const uint32_t cus = num_cus ? num_cus : 256, slots = 2 * cus;
         const uint32_t tiles = (d.max_n + 255) / 256;
-        auto pick_tn = [&](bool paired_layout, bool by_rows = true) {  // by_rows: with what whole 16 KiB rows are worth
+        auto pick_dense = [&](bool paired_layout) {
             double best = 1e300;
             uint32_t pick = 0;
             for (uint32_t tn : {6u, 4u, 3u}) {
@@ -882,16 +881,8 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
                 const uint32_t blocks = (M + 16 * tn - 1) / (16 * tn);
                 const uint64_t items = (uint64_t)tiles * blocks;
                 const uint64_t items_small = (uint64_t)((d.max_n + 127) / 128) * blocks;
-                // Outputs beyond the caches in rows of whole 16 KiB: 64 columns of a row are 256-byte pieces on their
-                // own memory channels, 96 are not (1024 -> 4096, N = 32768, us, 96 / 64 columns: v = 4 311 / 267, v = 8
-                // 218 / 161, v = 16 166 / 106; M = 3072, where no tile width meets the channels again: 163 / 174 at v = 4).
-                // Passes through buffers that take turns, 96 / 64 columns: M = 4096 64 codebooks N = 16384 84.9 / 70.5, N = 32768 153 / 131, 16 codebooks
-                // N = 16384 84 / 76; M = 8192 64 codebooks N = 8192 75.4 / 72.4, N = 12288 110 / 104, 16 codebooks N = 8192 71.7 / 70.0; M = 12288 64
-                // codebooks N = 8192 101.7 / 98.0.  (One buffer written over and over, which the last cache holds in part, at 256 MiB: up to 32
-                // codebooks 62 / 66 at M = 4096, 58 / 66 at 8192; 64 codebooks 71.1 / 68.9 and 65.0 / 67.7.  From 512 MiB on as above.)
-                const double width = by_rows && tn == 4 && M % 4096 == 0 && (uint64_t)d.max_n * M * 4 >= SP_LARGE_OUTPUT ? 0.9 : 1.0;
-                const double t256 = grid_rounds(items, slots) * item_cost(tn, false) * width;
-                const double t128 = grid_rounds(items_small, slots) * item_cost(tn, true) * width;
+                const double t256 = grid_rounds(items, slots) * item_cost(tn, false);
+                const double t128 = grid_rounds(items_small, slots) * item_cost(tn, true);
                 const double t = t128 < t256 ? t128 : t256;  // the launcher takes the better item size
                 if (t < best - 1e-9) {
                     best = t;
@@ -899,6 +890,13 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
                 }
             }
             return pick;
+        };
+        // Sparse kernel, up to 16 centroids: 64 or 48 columns (96 on request).  An output of a multiple of 48 columns that 64 does not
+        // divide takes 48, which lets operators of such outputs share a gather launch.
+        auto pick_sparse = [&] {
+            if (col_block_hint) return col_block_hint / 16;
+            if (M % 48 == 0 && M % 64 != 0) return 3u;
+            return sparse_launch_cost(3, d.max_n, M, g->CB_pad, cus) < sparse_launch_cost(4, d.max_n, M, g->CB_pad, cus) - 1e-9 ? 3u : 4u;
         };
         // Up to 8 centroids, kernel not named by the caller: the paired dense kernel has the cheaper K-loop, the
         // sparse kernel (the table as 16 centroids with empty rows) the cheaper epilogue and the 96-column tile.
@@ -909,7 +907,7 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
         // N = 32768 350 / 270, N = 16384 163 / 138; 160 codebooks N = 16384 124 / 97; M = 8192, 256 codebooks N = 8192 160 / 141.)
         if (C <= 8 && g->gather_kind == 1 && tune.gather_kernel == PIMDL_GATHER_AUTO && !gather_dense_only() &&
             (col_block_hint == 96 ||  // (only the sparse kernel has that tile)
-             ((uint64_t)d.max_n * M >= 65536ull * g->CB && (pick_tn(false, false) == 6 || g->CB <= 128))))
+             ((uint64_t)d.max_n * M >= 65536ull * g->CB && (pick_dense(false) == 6 || g->CB <= 128))))
             g->gather_kind = 2;
         const bool paired = C <= 8 && g->gather_kind == 1;
         g->C_tile = paired ? 8 : C > 16 ? 32 : 16;
@@ -918,7 +916,7 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
                           : "column tile hint must be 48, 64 or 96 for this operator";
             return false;
         }
-        g->q = pick_tn(paired);
+        g->q = g->gather_kind == 2 && C <= 16 ? pick_sparse() : pick_dense(paired);
         g->gq = 4;
         g->cb_per_slice = 16;
         g->col_block = 16 * g->q;

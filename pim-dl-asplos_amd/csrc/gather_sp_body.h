@@ -19,7 +19,7 @@
 
     // LDS: value table(s) | position words (1 KB) | NBUF LUT slice buffers | NIBUF index buffers
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    constexpr int NBUF = sp_nbuf(GS), NIBUF = NBUF;
+    constexpr int NBUF = sp_nbuf(TN, TM, GS, NW, WIDE), NIBUF = NBUF;
     constexpr int PD = NBUF - 1;  // prefetch distance of the LUT stream, in slices
     constexpr uint32_t POS0 = sp_value_table_bytes(WIDE);  // position words
     constexpr uint32_t BUF0 = sp_table_bytes(WIDE);

@@ -63,29 +63,32 @@ namespace {
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 
-// Waves per workgroup (NW): 4, two workgroups per CU -- or 8, one workgroup per CU: the same two waves per
+// Waves per workgroup (NW): 4, two or three workgroups per CU -- or 8, one workgroup per CU: two waves per
 // SIMD, but a LUT slice is copied into LDS once for 512 tokens instead of 256 and the CU's whole LDS belongs
 // to one workgroup (slices twice as deep, half as many barriers).
 constexpr int sp_tok_item(int tm, int nw = 4) { return nw * tm * 16; }
-// workgroups per CU: two of four waves or one of eight, two waves per SIMD either way.  (Eight waves of 32 tokens
-// each, two such workgroups per CU -- four waves per SIMD on 128 registers -- were measured 17 % slower on 64-column
-// tiles: a wave then re-reads every table entry for two token groups instead of four, and 96-column tiles spill.)
-constexpr int sp_wgs_per_cu(int, int nw) { return nw == 4 ? 2 : 1; }
+// Workgroups per CU: 48- and 64-column tiles of 64 tokens per wave fit 168 registers, and with slices of 16 codebooks (64 columns: in two
+// buffers) three workgroups fit a CU.  The third wave of a SIMD runs where the other two wait for operands, slices or stores: three
+// operators, inputs and outputs taking turns, two against three, us a pass: 768 -> 3072 N = 8192 57.1 / 56.2, N = 12608 85.1 / 80.9; 1024 -> 4096 N = 32768
+// 319 / 308.  (Eight waves of 32 tokens each, two such workgroups per CU -- four waves per SIMD -- are slower: a wave then re-reads every
+// table entry for two token groups instead of four.  Four workgroups of 48 columns on 128 registers spill: 60 -> 77 us.  Position
+// words from vector operations instead of the table in LDS: 79 -> 88 us at 768 -> 3072, N = 12608.)
+constexpr bool sp_three_per_cu(int tn, int tm, int gs, int nw, bool wide) { return nw == 4 && tm == 4 && gs == 16 && tn <= 4 && !wide; }
+constexpr int sp_wgs_per_cu(int tn, int tm, int gs, int nw, bool wide)
+{
+    return nw != 4 ? 1 : sp_three_per_cu(tn, tm, gs, nw, wide) ? 3 : 2;
+}
 // 64-token index blocks a workgroup keeps per slice: a wave of 32 tokens shares its block with its neighbour (both
 // copy the same bytes to the same place)
 constexpr int sp_ix_blocks(int tm, int nw) { return nw * tm * 16 / 64; }
-constexpr int sp_nbuf(int gs) { return gs > 16 ? 2 : 3; }
+constexpr int sp_nbuf(int tn, int tm, int gs, int nw, bool wide) { return gs > 16 || (tn == 4 && sp_three_per_cu(tn, tm, gs, nw, wide)) ? 2 : 3; }
 // value tables (17..32 centroids only: two tables of 32 entries of 16 bytes); then the position words, one per index byte
 constexpr int sp_value_table_bytes(bool wide) { return wide ? 1024 : 0; }
 constexpr int sp_table_bytes(bool wide) { return sp_value_table_bytes(wide) + 1024; }
-constexpr int sp_lds_bytes(int tn, int gs, int nw = 4, bool wide = false)
-{
-    return sp_table_bytes(wide) + sp_nbuf(gs) * gs * 16 * tn * 16 + sp_nbuf(gs) * nw * 64 * 4 * (gs / 8);
-}
 // ks: waves that share a token block and split the codebooks of a slice between them (1 or 2)
-constexpr int sp_lds_bytes_tm(int tn, int tm, int gs, int nw, bool wide, int ks = 1)
+constexpr int sp_lds_bytes(int tn, int tm, int gs, int nw, bool wide, int ks = 1)
 {
-    return sp_table_bytes(wide) + sp_nbuf(gs) * gs * 16 * tn * 16 + sp_nbuf(gs) * sp_ix_blocks(tm, nw / ks) * 64 * 4 * (gs / 8);
+    return sp_table_bytes(wide) + sp_nbuf(tn, tm, gs, nw, wide) * (gs * 16 * tn * 16 + sp_ix_blocks(tm, nw / ks) * 64 * 4 * (gs / 8));
 }
 
 template <int OFF>
@@ -119,7 +122,7 @@ __device__ __forceinline__ T* uniform_ptr(T* p)
 // every CU a 512-token item still fills the chip with TM = 4 tiles and copies a slice once per 256 tokens.
 // The body of both kernels is gather_sp_body.h: a shared function compiles to other code than the kernel alone.
 template <int TN, int TM, int GS, int NW, bool WIDE, int KS = 1>
-__global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TM, NW) * NW / 4 /* waves per SIMD */) void gather_sparse_kernel(
+__global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TN, TM, GS, NW, WIDE) * NW / 4 /* waves per SIMD */) void gather_sparse_kernel(
     const uint8_t* __restrict__ idx, const int8_t* __restrict__ lut, float* __restrict__ out,
     int32_t* __restrict__ acc_out, uint32_t N, uint32_t M, uint32_t CB_pad, uint32_t idx_row_bytes,
     uint32_t n_token_tiles, uint32_t n_items, Epilogue ep, XcdMap xmap)
@@ -128,7 +131,7 @@ __global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TM, NW) * NW / 4 /* waves pe
 }
 // the launch deals its items in blocks of token tiles
 template <int TN, int TM, int GS, int NW>
-__global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TM, NW) * NW / 4) void gather_sparse_blocks_kernel(
+__global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TN, TM, GS, NW, false) * NW / 4) void gather_sparse_blocks_kernel(
     const uint8_t* __restrict__ idx, const int8_t* __restrict__ lut, float* __restrict__ out,
     int32_t* __restrict__ acc_out, uint32_t N, uint32_t M, uint32_t CB_pad, uint32_t idx_row_bytes,
     uint32_t n_token_tiles, uint32_t n_items, Epilogue ep, XcdBlocks xmap)
@@ -142,8 +145,9 @@ template <int TN, int TM, int GS, int NW, bool WIDE, int KS, bool BLOCKS>
 int launch_sparse_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc, uint32_t n,
                      const Epilogue& ep)
 {
-    constexpr int LDS = sp_lds_bytes_tm(TN, TM, GS, NW, WIDE, KS);
-    static_assert(sp_wgs_per_cu(TM, NW) * LDS <= 160 * 1024, "the CU's LDS holds the workgroups that its registers hold");
+    constexpr int LDS = sp_lds_bytes(TN, TM, GS, NW, WIDE, KS);
+    constexpr int PER_CU = sp_wgs_per_cu(TN, TM, GS, NW, WIDE);
+    static_assert(PER_CU * LDS <= 160 * 1024, "the CU's LDS holds the workgroups that its registers hold");
     constexpr int TOK_ITEM = sp_tok_item(TM, NW / KS);
     auto kern = [] {
         if constexpr (BLOCKS) return gather_sparse_blocks_kernel<TN, TM, GS, NW>;
@@ -153,16 +157,17 @@ int launch_sparse_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out,
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_sparse)")) return rc;
     const uint32_t n_token_tiles = (n + TOK_ITEM - 1) / TOK_ITEM;
     const uint32_t n_items = n_token_tiles * (a.g.M_pad / (16 * TN));
-    uint32_t grid = ctx->prop.multiProcessorCount * sp_wgs_per_cu(TM, NW);
+    uint32_t grid = ctx->prop.multiProcessorCount * PER_CU;
     if (grid > n_items) grid = n_items;
-    // Outputs that do not fit the last cache: an XCD takes its token tiles in blocks of about 1024 tokens (2048 with
+    // Outputs of 16 MiB and more: an XCD takes its token tiles in blocks of about 1024 tokens (2048 with
     // 64-column tiles) through all of its columns, so that the rows it is writing are written whole within a short time,
     // instead of a few columns of all of its rows.  With more tokens to a block fewer workgroups share the rows, with fewer
-    // every column's table is fetched again for each of them.  Tiles of 64 / 96 columns, N = 32768, us without blocks and with
-    // blocks of 512, 1024, 2048, 4096 tokens: 24 codebooks, M = 3072 91 80 79 79 85 / 78 67 68 68 68; M = 4096 117 105 106 107 106 /
-    // 140 113 120 128 140; 192 codebooks, M = 3072 185 174 176 174 172 / 177 165 163 164 164; M = 4096 236 230 236 231 233 /
-    // 271 232 236 233 265; N = 16384, 48 codebooks, M = 4096 76 64 62 58 57 / 58 67 58 58 57.  Not below: N = 16384, M = 3072 (201 MB),
-    // 192 codebooks 83 84 84 84 85 / 80 83 84 81 84, 24 codebooks 35 36 36 36 36 / 37 37 37 37 38.
+    // every column's table is fetched again for each of them.  us a pass over three operators, inputs and outputs in turn (one output written
+    // over and over stays in the last cache up to 256 MiB, and shows nothing of this), 64-column tiles, three workgroups per CU, without blocks
+    // and with blocks of 512, 1024, 2048, 4096 tokens: 768 -> 3072 N = 4096 33.8 / 29.9 30.0 30.2 30.6, N = 8192 54.8 / 50.2 50.1 50.0 49.9, N = 16384
+    // 99 / 95 95 95 95; 2048 -> 2048 N = 16384 167 / 153 154 156 159; 1024 -> 4096 N = 8192 80 / 76 77 78 76; 3072 -> 768 N = 16384 124 / 119 119 119 120.
+    // Without a column split by XCD smaller blocks cost more (1024 -> 4096 N = 32768, split over 1 / 8: 323 / 298 with 512 tokens, 323 / 301 with 2048).
+    // Below 16 MiB there is no difference (768 -> 768, N = 2048 .. 4096).
     const uint32_t col_tiles = a.g.M_pad / (16 * TN);
     const XcdMap dealt = choose_xcd_map(col_tiles, n_token_tiles, grid, (uint64_t)cb16 * 16 * a.g.M_pad,
                                         (uint64_t)n * a.g.idx_row_bytes, a.g.tune_xcd_col_split);
@@ -184,7 +189,7 @@ int launch_sparse_tm(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out,
 {
     // (17..32 centroids are here on request only, and a split of the codebooks is for launches of one round)
     if constexpr (!WIDE && KS == 1)
-        if ((uint64_t)n * a.g.M * 4 >= SP_LARGE_OUTPUT) return launch_sparse_as<TN, TM, GS, NW, WIDE, KS, true>(ctx, a, d_idx, d_out, d_acc, n, ep);
+        if ((uint64_t)n * a.g.M * 4 >= SP_BLOCK_OUTPUT) return launch_sparse_as<TN, TM, GS, NW, WIDE, KS, true>(ctx, a, d_idx, d_out, d_acc, n, ep);
     return launch_sparse_as<TN, TM, GS, NW, WIDE, KS, false>(ctx, a, d_idx, d_out, d_acc, n, ep);
 }
 
@@ -210,7 +215,10 @@ int launch_sparse_tn(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out,
     if constexpr (TN == 3 && !WIDE) {
         const uint64_t cus = ctx->prop.multiProcessorCount;
         const uint64_t items8 = (uint64_t)((n + sp_tok_item(4, 8) - 1) / sp_tok_item(4, 8)) * col_tiles;
+        // (sums of fewer than 384 codebooks that three workgroups per CU take: 768 -> 2304 N = 8192 49.7 us a pass with eight waves, 46.2 with
+        // them, 768 -> 3072 59.3 / 55.9; 3072 -> 768 N = 16384 124.2 / 127.2)
         if (!a.g.tune_token_item && !a.g.tune_cb_per_slice && cb16 % 64 == 0 && !small_items && items8 >= cus &&
+            !(cb16 < 384 && sparse_three_per_cu(items4, cb16, cus)) &&
             0.96 * (double)((items8 + cus - 1) / cus) < grid_rounds(items4, slots))
             return launch_sparse_tm<TN, 4, 64, 8>(ctx, a, d_idx, d_out, d_acc, n, ep);
         // A launch of long sums that offers about one 256-token item per CU: 128-token items would fill the chip's
@@ -231,6 +239,9 @@ int launch_sparse_tn(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out,
         if (TN == 3 || a.g.tune_cb_per_slice != 16) return launch_sparse_tm<TN, 4, 32, 8>(ctx, a, d_idx, d_out, d_acc, n, ep);
         if constexpr (TN != 3) return launch_sparse_tm<TN, 4, 16, 8>(ctx, a, d_idx, d_out, d_acc, n, ep);
     }
+    if constexpr (TN <= 4 && !WIDE)
+        if (!a.g.tune_token_item && !a.g.tune_cb_per_slice && sparse_three_per_cu(items4, cb16, ctx->prop.multiProcessorCount))
+            return launch_sparse_tm<TN, 4, 16>(ctx, a, d_idx, d_out, d_acc, n, ep);
     constexpr int GSB = TN <= 4 ? 32 : 16;  // 32-codebook slices in two buffers where two workgroups still fit a CU
     if constexpr (GSB != 16) {
         if (cb16 % GSB == 0 && a.g.tune_cb_per_slice != 16) {
@@ -244,7 +255,7 @@ int launch_sparse_tn(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out,
 
 }  // namespace
 
-uint32_t sparse_lds_bytes(uint32_t tn, bool wide) { return (uint32_t)sp_lds_bytes((int)tn, 16, 4, wide); }
+uint32_t sparse_lds_bytes(uint32_t tn, bool wide) { return (uint32_t)sp_lds_bytes((int)tn, 4, 16, 4, wide); }
 
 int launch_gather_sparse(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, int32_t* d_acc, uint32_t n,
                          float scale, float lut_bias_term)

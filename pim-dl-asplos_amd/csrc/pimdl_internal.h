@@ -56,8 +56,8 @@ struct AmmGeom {
 // floats of the pieces in which the rows of an fp32 table are kept (0: whole rows)
 constexpr uint32_t f32_lut_chunk(uint32_t c_tile) { return c_tile == 32 ? 2 : c_tile <= 16 ? 4 : 0; }
 
-// bytes of output from which the sparse gather's launches count as larger than the last cache (256 MiB)
-constexpr uint64_t SP_LARGE_OUTPUT = 256ull << 20;
+// bytes of output from which a launch of the sparse gather takes its token tiles in blocks
+constexpr uint64_t SP_BLOCK_OUTPUT = 16ull << 20;
 
 // bytes of a packed index buffer for n tokens
 inline size_t idx_buffer_bytes(const AmmGeom& g, uint32_t n)

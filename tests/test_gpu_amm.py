@@ -1325,6 +1325,47 @@ def test_forms_of_the_sparse_gather_of_large_outputs(ctx, N, CB, M, act, tuning,
     amm.close()
 
 
+@pytest.mark.parametrize("N,CB,M,form", [
+    (8300, 97, 1100, "blocks_kernel<4, 4, 16, 4>"),        # three workgroups per CU: just beyond two of them, ragged tokens and columns
+    (7700, 128, 1088, "blocks_kernel<4, 4, 16, 4>"),
+    (8300, 100, 816, "blocks_kernel<3, 4, 16, 4>"),
+    (8192, 128, 1024, "blocks_kernel<4, 4, 32, 4>"),       # exactly two workgroups per CU
+    (8300, 96, 1100, "blocks_kernel<4, 4, 32, 4>"),        # a sum of 96 codebooks
+    (40000, 130, 104, "kernel<4, 4, 32, 4, false>"),       # below 16 MiB: no blocks
+    (65000, 130, 104, "blocks_kernel<4, 4, 32, 4>"),
+    (17000, 130, 2001, "blocks_kernel<4, 4, 16, 4>"),      # several rounds, odd columns
+])
+def test_sparse_gather_with_three_workgroups_per_cu(ctx, N, CB, M, form):
+    """Either side of the lines between two and three workgroups per CU and of the blocks of token tiles: every row as in launches of 900
+    tokens, which have neither, the oracle's bits in the first and last rows, nothing behind the output."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    import torch
+    v, C = 2, 16
+    _, cent, lut, bias = make_case(2025 + M + CB, 1, CB * v, v, C, M)
+    x = torch.randn((N, CB * v), device="cuda", generator=torch.Generator(device="cuda").manual_seed(N))
+    width = 16 * int(form.split("<")[1][0])
+    amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=N, tuning={"col_block": width})
+    out = torch.full((N + 2, M), -5.0, device="cuda")
+    part = torch.empty((900, M), device="cuda")
+    torch.cuda.synchronize()
+    amm.run_ptr(x.data_ptr(), N, out.data_ptr())
+    ctx.synchronize()
+    if ctx.device_info()["compute_units"] == 256:
+        assert amm.last_gather_kernel() == "gather_sparse_" + form, amm.last_gather_kernel()
+    assert bool((out[N:] == -5.0).all())
+    for i in range(0, N, 900):
+        n = min(900, N - i)
+        torch.cuda.synchronize()
+        amm.run_ptr(x[i:].data_ptr(), n, part.data_ptr())
+        ctx.synchronize()
+        assert torch.equal(out[i:i + n], part[:n]), i
+    rows = list(range(70)) + list(range(N - 70, N))
+    want = oracle.amm_cpu(x[rows].cpu().numpy(), cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)[0]
+    assert np.array_equal(out[rows].cpu().numpy().view(np.uint32), want.view(np.uint32))
+    amm.close()
+
+
 @pytest.mark.parametrize("N,M,count", [(29200, 768, 3), (22100, 1536, 2), (32768, 1024, 3)])
 def test_operators_side_by_side_with_a_large_output(ctx, N, M, count):
     """One gather launch for several operators whose common output is dealt out in blocks: every column as of the operator alone, whose
