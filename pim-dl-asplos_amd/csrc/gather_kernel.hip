@@ -899,15 +899,13 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
             return sparse_launch_cost(3, d.max_n, M, g->CB_pad, cus) < sparse_launch_cost(4, d.max_n, M, g->CB_pad, cus) - 1e-9 ? 3u : 4u;
         };
         // Up to 8 centroids, kernel not named by the caller: the paired dense kernel has the cheaper K-loop, the
-        // sparse kernel (the table as 16 centroids with empty rows) the cheaper epilogue and the 96-column tile.
-        // Measured over N 2048..12608, K and M 768..4096, vec_len 2..8: the sparse kernel is 3 to 38 % faster where
-        // the launch is large against its codebook count (tokens x columns >= 65536 x codebooks) and either
-        // 96-column tiles are its best launch or there are at most 128 codebooks; elsewhere 0 to 20 % slower.
-        // (Rows of whole 16 KiB, where it takes 64-column tiles instead, are no exception: passes, us, paired / sparse, M = 4096: 256 codebooks
-        // N = 32768 350 / 270, N = 16384 163 / 138; 160 codebooks N = 16384 124 / 97; M = 8192, 256 codebooks N = 8192 160 / 141.)
+        // sparse kernel (the table as 16 centroids with empty rows) the cheaper epilogue, three workgroups per CU and rows written whole.
+        // The sparse kernel where the launch is large against its codebook count (tokens x columns >= 65536 x codebooks); passes over three
+        // operators, inputs and outputs in turn, sparse / paired: there 0.70 .. 0.98 over N 2048..24000, K and M 512..4096, sub-vectors of 2..16 (768 -> 3072
+        // N = 8192 0.92, of 8 floats 0.80; 768 -> 1001 N = 16384 0.85; 1024 -> 1024 N = 16384 0.96); below 0.91 .. 1.26 (768 -> 768 N = 4096 1.01,
+        // 3072 -> 768 N = 2048 1.16, 2048 -> 2048 N = 8192 0.99).
         if (C <= 8 && g->gather_kind == 1 && tune.gather_kernel == PIMDL_GATHER_AUTO && !gather_dense_only() &&
-            (col_block_hint == 96 ||  // (only the sparse kernel has that tile)
-             ((uint64_t)d.max_n * M >= 65536ull * g->CB && (pick_dense(false) == 6 || g->CB <= 128))))
+            (col_block_hint == 96 || (uint64_t)d.max_n * M >= 65536ull * g->CB))  // (only the sparse kernel has that tile)
             g->gather_kind = 2;
         const bool paired = C <= 8 && g->gather_kind == 1;
         g->C_tile = paired ? 8 : C > 16 ? 32 : 16;
