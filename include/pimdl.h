@@ -144,7 +144,7 @@ typedef enum pimdl_search_kernel {
     PIMDL_SEARCH_AUTO = 0,
     PIMDL_SEARCH_SCAN = 1,      /* one lane per token, the reference's scan for every pair */
     PIMDL_SEARCH_MFMA_F32 = 2,  /* scores on the fp32 matrix instruction, exact replay of near ties; C <= 16 */
-    PIMDL_SEARCH_MFMA_BF16 = 3  /* scores from three bf16 pieces per value; C <= 32, sub_vec_len 2, 4, 8 */
+    PIMDL_SEARCH_MFMA_BF16 = 3  /* scores from 16-bit pieces of every value; C <= 32, sub_vec_len 2, 4, 8 */
 } pimdl_search_kernel;
 typedef struct pimdl_amm_tuning {
     uint32_t col_block;      /* output columns per work item of the gather: 48, 64 or 96 (what the kernel offers) */
@@ -161,7 +161,7 @@ typedef struct pimdl_amm_tuning {
                                 tiles; PIMDL_XCD_PLAIN = no dealing.  A split that does not divide a launch's
                                 tile counts is replaced by the library's choice for that launch. */
     uint32_t search_kernel;  /* pimdl_search_kernel */
-    uint32_t search_token_tile; /* tokens per tile of the bf16 matrix-core search: 64 or 128 */
+    uint32_t search_token_tile; /* tokens per tile of that search: 64 or 128 */
 } pimdl_amm_tuning;
 #define PIMDL_XCD_PLAIN 0xFFFFFFFFu
 /* pimdl_amm_create with these choices made by the caller (tuning NULL or all zero: pimdl_amm_create).
@@ -387,17 +387,18 @@ PIMDL_API int pimdl_diag_bandwidth(pimdl_ctx* ctx, uint64_t bytes, float* copy_g
  * into pinned memory and back, and the transfers between pinned memory and the device.  A measuring aid. */
 PIMDL_API int pimdl_diag_host_copy(pimdl_ctx* ctx, uint64_t bytes, float* to_pinned_gbps, float* from_pinned_gbps,
                                    float* h2d_gbps, float* d2h_gbps);
-/* Checks on this device what the bf16-split closest-centroid search takes for granted about the
- * matrix core: runs `trials` (1..4096) chains of three v_mfma_f32_32x32x16_bf16 on random operands of
+/* Checks on this device what the closest-centroid search from 16-bit pieces takes for granted about the
+ * matrix core: runs `trials` (1..4096) chains of three v_mfma_f32_32x32x16_f16 on random operands of
  * mixed magnitude and reports the largest |result - exact sum| in units of 2^-24 * sum|terms|.  The
- * search kernel's margin allows 51 of these units (sub_vec_len 4); index_calculation itself
+ * search kernel's margin allows 51 of these units for such a chain; index_calculation itself
  * (src/host/index_calc_host.cpp:8-53) has no counterpart of this: it is a property of this port. */
 PIMDL_API int pimdl_diag_mfma_error(pimdl_ctx* ctx, uint32_t trials, float* max_err_u);
 /* The same measurement on operands built to make an accumulator lose as much as it can, instead of random
  * ones: an accumulator of 1.0 that receives 48 equal products just below or just above 1/2, 1 and 2 units in its
  * last place, of either sign (an adder that rounds to nearest after every product drops all of the first kind,
  * 24 units in all; one that truncates would drop up to 96), and products that fall by a factor of four from
- * slot to slot (bits shifted out when the terms of one instruction are aligned).  The margin allows 51. */
+ * slot to slot (bits shifted out when the terms of one instruction are aligned), and sums of products with a subnormal half, which
+ * a matrix core that took those for zero would lose whole.  The margin allows 51. */
 PIMDL_API int pimdl_diag_mfma_error_crafted(pimdl_ctx* ctx, float* max_err_u);
 
 #ifdef __cplusplus

@@ -228,7 +228,7 @@ class Context:
         return c.value, l.value
 
     def diag_mfma_error(self, trials=256):
-        """Largest error of a chain of three bf16 MFMAs against the exact sum, in units of 2^-24 * sum|terms|."""
+        """Largest error of a chain of three half-precision MFMAs against the exact sum, in units of 2^-24 * sum|terms|."""
         e = ctypes.c_float(0)
         self._check(lib().pimdl_diag_mfma_error(self._h, trials, ctypes.byref(e)))
         return e.value

@@ -11,8 +11,8 @@ would otherwise decide by rule (pimdl_amm_tuning):
     token_item      tokens per work item (128, 256; 512 = eight waves per workgroup, sparse kernel)
     cb_per_slice    codebooks staged in LDS at a time (16, 32, 64)
     xcd_col_split   how the 8 XCDs share column tiles and token tiles (1, 2, 4, 8, plain order)
-    search_kernel   closest-centroid search: lane-per-token scan / fp32 matrix core / bf16 matrix core
-    search_token_tile  tokens per tile of the bf16 search (64, 128)
+    search_kernel   closest-centroid search: lane-per-token scan / fp32 matrix core / matrix core on 16-bit pieces
+    search_token_tile  tokens per tile of the last of these (64, 128)
 
 times the two kernels with events on the device (pimdl_amm_profile) and keeps the fastest setting of each
 kernel.  Gather and search are independent (they only share the packed index layout, which depends on the

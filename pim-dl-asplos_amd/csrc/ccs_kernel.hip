@@ -40,6 +40,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <utility>
 #include <vector>
 
 #include "pimdl_internal.h"
@@ -77,23 +78,24 @@ inline size_t ccs_aux_a_floats(const AmmGeom& g)
     return (size_t)(g.CB_pad / 2) * (g.v + 1) * 64 + g.CB_pad;  // A-operand images, padded cnmax
 }
 
-// bf16-split search (v = 4, C <= 16): offset in floats of its operands behind everything else, and
+// Search by half-precision pieces (C <= 32): offset in floats of its operands behind everything else, and
 // their size.  The offset is rounded up to 16 bytes (uint4 operand images).
-inline bool ccs_has_bf16(const AmmGeom& g) { return (g.v == 2 || g.v == 4 || g.v == 8) && g.C <= 32; }
+inline bool ccs_has_f16(const AmmGeom& g) { return (g.v == 2 || g.v == 4 || g.v == 8) && g.C <= 32; }
 // 17..32 centroids: a codebook fills all 32 rows of the matrix instruction by itself ("wide"); the operand
 // images are then per codebook instead of per pair of codebooks
-inline bool ccs_bf16_wide(const AmmGeom& g) { return g.C > 16; }
-inline size_t ccs_bf16_units(const AmmGeom& g) { return ccs_bf16_wide(g) ? g.CB_pad : g.CB_pad / 2; }
-// MFMAs (16 K-slots each) per codebook pair: 2 codebooks x v dims x 6 cross products
-constexpr uint32_t ccs_bf16_nm(uint32_t v) { return (12 * v + 15) / 16; }
-inline size_t ccs_bf16_offset(const AmmGeom& g)
+inline bool ccs_f16_wide(const AmmGeom& g) { return g.C > 16; }
+inline size_t ccs_f16_units(const AmmGeom& g) { return ccs_f16_wide(g) ? g.CB_pad : g.CB_pad / 2; }
+// matrix instructions (16 K-slots each) per unit: v dims x 4 cross products, of 2 codebooks or (wide) of one
+constexpr uint32_t ccs_f16_nm(uint32_t v, bool wide) { return ((wide ? 4 : 8) * v + 15) / 16; }
+inline size_t ccs_f16_offset(const AmmGeom& g)
 {
     const size_t o = (size_t)g.CB * g.C * g.v + ccs_aux_floats(g) + g.CB + ccs_aux_a_floats(g);
     return (o + 3) / 4 * 4;
 }
-inline size_t ccs_bf16_floats(const AmmGeom& g)
+inline size_t ccs_f16_floats(const AmmGeom& g)
 {
-    return ccs_has_bf16(g) ? ccs_bf16_units(g) * ccs_bf16_nm(g.v) * 64 * 4 + ccs_bf16_units(g) * 2 * 16 : 0;
+    // (and a scale for every 8 units, CB_pad being a multiple of 32; see half_scale)
+    return ccs_has_f16(g) ? ccs_f16_units(g) * ccs_f16_nm(g.v, ccs_f16_wide(g)) * 64 * 4 + ccs_f16_units(g) * 2 * 16 + ccs_f16_units(g) / 8 : 0;
 }
 
 // more than 32 centroids, or sub-vectors of 16 or 32 dimensions: the matrix search over groups of 32 centroids
@@ -657,39 +659,75 @@ __global__ __launch_bounds__(CCS_THREADS, V == 8 ? 2 : 4) void ccs_mfma_kernel(c
 }
 
 // =============================================================================================
-// bf16-split variant of the MFMA search for v in {2, 4, 8} (C <= 16).  The fp32 MFMA above shares the fp32
+// The matrix search from half-precision pieces, v in {2, 4, 8}, up to 32 centroids.  The fp32 MFMA above shares the fp32
 // units with the VALU, so its five instructions per item (147 ns) add to the ~50 VALU operations of
-// the top-two search (100 ns).  v_mfma_f32_32x32x16_bf16 is twice as fast per K-slot and runs beside
-// VALU work.  bf16 has 8 significand bits, so each fp32 value is cut into three bf16 pieces and six
-// of the nine cross products are kept (see `scores` below); the score then carries a known error
-// bound like the fp32 form's, only larger (A2 below), and everything after the scores -- tagged
-// keys, tournament, margin test, exact replay -- is the same.  Operands:
-//   aux_b [CB_pad/2 pairs][NM][64 lanes] uint4 A-operand images (bf16 pieces of -2c, by K-slot)
-//   cn16  [CB_pad][16] float                   |c|^2 (r for padded codebooks, 3e38 for ids past C)
+// the top-two search (100 ns).  v_mfma_f32_32x32x16_f16 is twice as fast per K-slot and runs beside
+// VALU work.  A half has 11 significand bits, so two pieces (x = xh + xm) hold a float up to 2^-21 of it, or up to 2^-24 where
+// the second one is subnormal; all four cross products with the pieces of -2c are taken.  The score then carries a known error
+// bound like the fp32 form's, only larger (A2, E2 below), and everything after the scores -- tagged
+// keys, tournament, margin test, exact replay -- is the same.
+// Bound by the vector ALU, of which the pieces are what a form can choose: cut in one v_cvt_pkrtz_f16_f32 per two values and piece, the
+// remainder by one v_fma_mix_f32, they are 8 operations per 64 pairs at v = 4, and two matrix instructions.  (Three bf16 pieces by
+// masking, six cross products, were 22 and three, with 1.4 times the margin at v = 4 and so as many more replays: search and gather, us
+// a pass, inputs and outputs in turn, before / now: v = 4 N = 8192 K = 3072 66.1 / 62.6, N = 4096 38.4 / 37.6, K = 768 18.5 / 18.1; v = 8 N =
+// 8192 K = 3072 50.5 / 46.9, v = 2 105.7 / 101.1; beyond 16 centroids, where it also counts that a lane decides a codebook instead of both lanes of
+// a token the same one, N = 12608 K = 3072 160 / 140.7, N = 8192 v = 8 72.8 / 65.0, v = 2 188 / 178.)
+// Halves end at 65504: a tile with a centroid longer than 1024 is searched at a power-of-two scale, and
+// sub-vectors longer than 31623 of that scale are replayed exactly.
+// Operands:
+//   aux_b [units][NM][64 lanes] uint4 A-operand images (pieces of -2c, by K-slot); a unit is two codebooks, or one (wide)
+//   cn16  [CB_pad][16] float          |c|^2 (r for padded codebooks, 3e38 for ids past C)
+//   scale [units / 8] float           what a tile's activations and centroids are multiplied with
 // =============================================================================================
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
-typedef unsigned int v6u __attribute__((ext_vector_type(6)));
 
-// K-slot registers (two bf16 K-slots each, four registers per MFMA) of lane (row i, half kh).  The lane
-// covers dims DL*kh .. DL*kh + DL-1 (DL = v/2) of both codebooks of the pair.
-//   DL >= 2: three MFMAs per pair of dims (d, d+1); a register holds (piece of d | piece of d+1 << 16).  The
-//            search kernel keeps six registers  xm(cb0) xm(cb1) xh(cb0) xh(cb1) xl(cb0) xl(cb1)  in a row and
-//            hands the MFMAs windows of four of them, so that no piece is copied:
-//              registers 0..3 against {ch, ch, ch, ch}   (xm*ch, xh*ch)
-//              registers 0..3 against {cm, cm, cm, cm}   (xm*cm, xh*cm)
-//              registers 2..5 against {cl, cl, ch, ch}   (xh*cl, xl*ch)
-//            with the pieces of -2c of the row's own codebook in that codebook's registers;
-//   DL == 1: codebook q owns registers 3q .. 3q+2 of the first two MFMAs: (ch | cm), (ch | cm), (cl | ch)
-//            against (xh | xh), (xm | xm), (xh | xl).
-// Registers of the other codebook, and registers past the last one used, hold zeros.
-// WIDE (17..32 centroids): "pair" p is codebook p alone, its half h holds centroids 16h .. 16h+15, and both
-// halves meet the same sub-vector (the search kernel feeds the activations of codebook p to both).
-template <uint32_t V, bool WIDE>
-__global__ void ccs_prep_bf16_kernel(const float* __restrict__ cent, uint4* __restrict__ aux_b,
-                                     float* __restrict__ cn16, uint32_t CB, uint32_t C)
+// two floats cut to halves (towards zero): a in the low one
+__device__ __forceinline__ uint32_t half_pair(float a, float b) { return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b)); }
+// what the low (HI: high) half of p leaves of a, exactly
+template <bool HI>
+__device__ __forceinline__ float half_rest(uint32_t p, float a)
 {
-    constexpr uint32_t DL = V / 2, NM = ccs_bf16_nm(V);
+    float r;
+    if constexpr (HI) asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(p), "v"(a));
+    else asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(p), "v"(a));
+    return r;
+}
+// a piece of -2c: rounded to nearest, what is left
+__device__ __forceinline__ uint32_t half_piece(float& a)
+{
+    const _Float16 p = (_Float16)a;
+    a = __fsub_rn(a, (float)p);
+    return __builtin_bit_cast(uint16_t, p);
+}
+
+// The power of two that the activations and centroids of n codebooks are multiplied with: 1 unless one of their centroids is longer than
+// 1024, else what makes the longest one shorter than that.  (A codebook with a centroid that is not finite has no say: it is replayed.)
+__device__ __forceinline__ float half_scale(const float* cnmax, uint32_t n)
+{
+    float m = 0.0f;
+    for (uint32_t i = 0; i < n; ++i) m = fmaxf(m, cnmax[i]);  // (a NaN gives way)
+    if (!(m > 1048576.0f)) return 1.0f;
+    const int e = ilogbf(m) - 20;  // m < 2^(21 + e), e >= 0
+    return ldexpf(1.0f, -(e / 2 + 1));
+}
+
+// K-slot registers (two half K-slots each, four registers per MFMA) of lane (row i, half kh).  The lane
+// covers dims DL*kh .. DL*kh + DL-1 (DL = v/2).  A register holds (piece of dim d | piece of d+1 << 16) and, at DL == 1, the
+// activations' (piece | the same piece) against (ch | cm).  The activations' registers and the images that meet them:
+//   two codebooks a, b (the images hold zeros in the registers of the codebook that the row does not belong to)
+//     DL == 1     xh(a) xm(a) xh(b) xm(b)                  once     (ch | cm) throughout
+//     DL >= 2     xh(a) xh(b) xm(a) xm(b), per two dims    twice    ch throughout, cm throughout
+//   WIDE (17..32 centroids): unit p is codebook p alone, row half h holds centroids 16h .. 16h+15
+//     DL == 1     xh xm 0 0                                once     (ch | cm) (ch | cm) 0 0
+//     DL == 2     xh xm xh xm                              once     ch ch cm cm
+//     DL == 4     xh(0,1) xh(2,3) xm(0,1) xm(2,3)          twice    ch(0,1) ch(2,3) ch(0,1) ch(2,3), the same of cm
+template <uint32_t V, bool WIDE>
+__global__ void ccs_prep_f16_kernel(const float* __restrict__ cent, const float* __restrict__ cnmax, uint4* __restrict__ aux_b,
+                                    float* __restrict__ cn16, float* __restrict__ scale, uint32_t CB, uint32_t C)
+{
+    constexpr uint32_t DL = V / 2, NM = ccs_f16_nm(V, WIDE);
     const uint32_t pair = blockIdx.x, lane = threadIdx.x;
     const uint32_t i = lane & 31, kh = lane >> 5;
     const uint32_t h = (i >> 2) & 1, r = (i & 3) + 4 * (i >> 3);
@@ -697,29 +735,26 @@ __global__ void ccs_prep_bf16_kernel(const float* __restrict__ cent, uint4* __re
     const uint32_t cid = WIDE ? 16 * h + r : r;  // centroid of row i
     const bool real = (cb < CB) && (cid < C);
     const float* cp = cent + ((size_t)cb * C + cid) * V;
-    uint32_t pc[DL][3];  // bf16 pieces ch, cm, cl of -2c for the lane's dims
+    constexpr uint32_t PER_TILE = WIDE ? 8 : 16;
+    const uint32_t first = pair / 8 * PER_TILE;
+    const float sc = half_scale(cnmax + first, first >= CB ? 0u : CB - first < PER_TILE ? CB - first : PER_TILE);
+    if (pair % 8 == 0 && lane == 0) scale[pair / 8] = sc;
+    uint32_t pc[DL][2];  // pieces ch, cm of -2c for the lane's dims
     for (uint32_t d = 0; d < DL; ++d) {
-        const float a = real ? -2.0f * cp[DL * kh + d] : 0.0f;
-        const uint32_t au = __float_as_uint(a);
-        const float r1 = __fsub_rn(a, __uint_as_float(au & 0xffff0000u));
-        const uint32_t r1u = __float_as_uint(r1);
-        const float r2 = __fsub_rn(r1, __uint_as_float(r1u & 0xffff0000u));
-        pc[d][0] = au >> 16;
-        pc[d][1] = r1u >> 16;
-        pc[d][2] = __float_as_uint(r2) >> 16;
+        float a = real ? -2.0f * (cp[DL * kh + d] * sc) : 0.0f;
+        pc[d][0] = half_piece(a);
+        pc[d][1] = half_piece(a);
     }
     for (uint32_t m = 0; m < NM; ++m) {
         uint32_t w[4];
         for (uint32_t q = 0; q < 4; ++q) {
-            const uint32_t rho = 4 * m + q;
             uint32_t val = 0;
             if (DL == 1) {
-                if (real && rho < 6 && rho / 3 == h)
-                    val = rho % 3 == 2 ? (pc[0][2] | (pc[0][0] << 16)) : (pc[0][0] | (pc[0][1] << 16));
-            } else if (real && (q & 1) == h) {
-                const uint32_t dp = m / 3, kind = m % 3;
-                const uint32_t t = kind == 2 ? (q < 2 ? 2u : 0u) : kind;  // ch, cm, or cl | ch
-                val = pc[2 * dp][t] | (pc[2 * dp + 1][t] << 16);
+                if (real && (WIDE ? q < 2 : q / 2 == h)) val = pc[0][0] | pc[0][1] << 16;
+            } else if (real && (WIDE || (q & 1) == h)) {
+                const uint32_t d = WIDE ? (DL == 2 ? 0 : 2 * (q & 1)) : 2 * (m / 2);
+                const uint32_t t = WIDE ? (DL == 2 ? q / 2 : m) : m % 2;
+                val = pc[d][t] | pc[d + 1][t] << 16;
             }
             w[q] = val;
         }
@@ -729,7 +764,10 @@ __global__ void ccs_prep_bf16_kernel(const float* __restrict__ cent, uint4* __re
         float cn = (float)cid;  // a padded codebook scores r against centroid r: index 0 with a margin of 1
         if (real) {
             cn = 0.0f;
-            for (uint32_t t = 0; t < V; ++t) cn = fmaf(cp[t], cp[t], cn);
+            for (uint32_t t = 0; t < V; ++t) {
+                const float c = cp[t] * sc;
+                cn = fmaf(c, c, cn);
+            }
         } else if (cb < CB) {
             cn = 3e38f;  // centroid ids past C never win
         }
@@ -741,10 +779,11 @@ __global__ void ccs_prep_bf16_kernel(const float* __restrict__ cent, uint4* __re
 // whose 64 prefetch registers do not fit: asked for three the compiler gives up and takes 288 (one workgroup per
 // CU); asked for two it takes 237 without spills, and the 76 KB of LDS allow no more than two anyway.
 template <int V, bool WIDE, int TTOK>
-__global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 : 3) void ccs_bf16_kernel(const float* __restrict__ x,
+__global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 : 3) void ccs_f16_kernel(const float* __restrict__ x,
                                                                  const float* __restrict__ cent,
                                                                  const uint4* __restrict__ aux_b,
                                                                  const float* __restrict__ cn16,
+                                                                 const float* __restrict__ scale,
                                                                  const float* __restrict__ cnmax_pad,
                                                                  uint8_t* __restrict__ idx, uint32_t N,
                                                                  uint32_t K, uint32_t CB, uint32_t C,
@@ -755,10 +794,13 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
     // that read the same row (tiles_x codebook tiles each), so the activation columns wrap around.
     using S = CcsMfmaShape<V, WIDE, TTOK>;
     constexpr int TF = S::TF, PITCH = S::PITCH, TT = S::TILE_TOKENS, CBW = S::CBW, TG = S::TG, RCB = S::RCB;
-    constexpr int XSTEP = WIDE ? V : 2 * V;  // activation floats per pair
-    constexpr int NM = (int)ccs_bf16_nm(V);  // MFMAs per item: 2 codebooks x v dims x 6 cross products, 16 K-slots each
+    constexpr int XSTEP = WIDE ? V : 2 * V;  // activation floats per unit
+    constexpr int NM = (int)ccs_f16_nm(V, WIDE);  // MFMAs per item
     constexpr int DL = V / 2;                // dims of each codebook this lane supplies
     constexpr int ITEMS = S::ITEMS;
+    constexpr int NCB = WIDE ? 1 : 2;        // codebooks of a unit
+    // items a lane decides: a codebook each, for TG (WIDE: both of the wave's units together) or 2 TG token groups
+    constexpr int OWN = WIDE ? TG : ITEMS;
     __shared__ __attribute__((aligned(16))) float tile[S::X_FLOATS];
     __shared__ __attribute__((aligned(16))) float cst[S::CENT_FLOATS];
     __shared__ __attribute__((aligned(16))) uint8_t ist[TT * (CBW / 2)];
@@ -812,7 +854,9 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
     uint32_t tiles_done = 0;
     uint32_t tcb_loaded = 0xFFFFFFFFu;  // codebook tile whose operands are resident (registers and LDS)
     uint4 aq[2][NM];
-    float cmax[2];
+    float cmax[NCB];
+    float sc = 1.0f;                        // the tile's scale (uniform)
+    bool plain = true;
     for (uint32_t tile_id = blockIdx.x; tile_id < total_tiles; tile_id += gridDim.x) {
         switch (4 * tiles_done / my_tiles) {
             case 0: __builtin_amdgcn_s_setprio(3); break;
@@ -830,6 +874,8 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
         const bool new_cb = tcb != tcb_loaded;  // workgroup-uniform
         tcb_loaded = tcb;
         if (new_cb) {
+            sc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(scale[tcb])));
+            plain = sc == 1.0f;
 #pragma unroll
             for (int pl = 0; pl < 2; ++pl)
 #pragma unroll
@@ -837,7 +883,16 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
             // every global load the search needs is issued here, ahead of the next tile's prefetch:
             // loads complete in order, so a later load would have to wait for the prefetch from HBM
 #pragma unroll
-            for (int pl = 0; pl < 2; ++pl) cmax[pl] = cnmax_pad[WIDE ? pair0 + pl : 2 * (pair0 + pl) + h];
+            for (int o = 0; o < NCB; ++o) cmax[o] = cnmax_pad[WIDE ? pair0 + h : 2 * (pair0 + o) + h] * sc * sc;
+        }
+        if (!plain) {
+#pragma unroll
+            for (int i = 0; i < PASSES; ++i) {
+                pf[i].x *= sc;
+                pf[i].y *= sc;
+                pf[i].z *= sc;
+                pf[i].w *= sc;
+            }
         }
 #pragma unroll
         for (int i = 0; i < PASSES; ++i)
@@ -856,19 +911,22 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
         __syncthreads();
         if (tile_id + gridDim.x < total_tiles) fetch(pf, tile_id + gridDim.x);
 
-        // Scores of item `it` (pair pl, token group tg) for this lane's token: this lane (half h) holds
-        // dims DL*h .. DL*h + DL-1 of both codebooks of the pair.  Each value is cut into three bf16 pieces
-        // by masking (x = xh + xm + xl exactly: 8 + 8 + 8 significand bits); the A operand holds the same
-        // pieces of -2c, and the K-slots pair them as  xh*ch, xh*cm, xm*ch, xm*cm, xh*cl, xl*ch  (the three
-        // omitted products are below 2^-20 |x||c|).  Products of bf16 values are exact in fp32; the
-        // accumulators start from |c|^2.  xx_out: |x|^2 over the lane's own codebook (for the bound).
+        // what the hysteresis is at this scale, and 2 * 1.25 v u for pieces below the smallest half
+        const float c0 = fmaf(1.001e-6f * sc, sc, 2.5f * V * 5.9604645e-8f);
+
+        // Scores of item `it` (unit pl, token group tg) for this lane's token: this lane (half h) holds
+        // dims DL*h .. DL*h + DL-1 of the unit's codebooks, cut into two halves each; the accumulators start from |c|^2.
+        // Products of halves are exact in fp32.  part: |x|^2 over the lane's dims, for the bound.
+        // WIDE: the two units take turns, so that the two halves of a wave, which hold the two halves of both codebooks' centroids, can
+        // decide one of them each.
+        auto unit_of = [](int it) { return WIDE ? it % 2 : it / TG; };
+        auto group_of = [](int it) { return WIDE ? it / 2 : it % TG; };
         // activations of item `it` for this lane; read two items ahead of their use (see the loop below)
-        auto load_x = [&](float (&xs)[2][DL], int it) {
-            const int pl = it / TG, tg = it % TG;
-            const float* brow = brow0 + tg * 32 * PITCH + pl * XSTEP;
+        auto load_x = [&](float (&xs)[NCB][DL], int it) {
+            const float* brow = brow0 + group_of(it) * 32 * PITCH + unit_of(it) * XSTEP;
 #pragma unroll
-            for (int cbh = 0; cbh < 2; ++cbh) {
-                const float* src = brow + (WIDE ? 0 : cbh * V) + DL * h;
+            for (int cbh = 0; cbh < NCB; ++cbh) {
+                const float* src = brow + cbh * V + DL * h;
                 if constexpr (DL == 1) {
                     xs[cbh][0] = src[0];
                 } else if constexpr (DL == 2) {
@@ -885,100 +943,83 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
                 }
             }
         };
-        floatx16 cn_pl;  // |c|^2 of the lane's 16 centroids of the current pair: what every accumulator starts from
-        auto scores = [&](floatx16& acc, float& xx_out, int it, const float (&xs)[2][DL]) {
-            const int pl = it / TG;
-            if (it % TG == 0) {  // (a constant once the item loop is unrolled) first token group of a pair
-                const float4* cnp = reinterpret_cast<const float4*>(cnl + (2 * (2 * wave + pl) + h) * 16);
+        floatx16 cn_pl[WIDE ? 2 : 1];  // |c|^2 of the lane's 16 centroids of a unit: what every accumulator starts from
+        auto load_cn = [&](floatx16& cn, int pl) {
+            const float4* cnp = reinterpret_cast<const float4*>(cnl + (2 * (2 * wave + pl) + h) * 16);
 #pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) {
-                    const float4 c4 = cnp[q4];
-                    cn_pl[4 * q4 + 0] = c4.x;
-                    cn_pl[4 * q4 + 1] = c4.y;
-                    cn_pl[4 * q4 + 2] = c4.z;
-                    cn_pl[4 * q4 + 3] = c4.w;
-                }
+            for (int q4 = 0; q4 < 4; ++q4) {
+                const float4 c4 = cnp[q4];
+                cn[4 * q4 + 0] = c4.x;
+                cn[4 * q4 + 1] = c4.y;
+                cn[4 * q4 + 2] = c4.z;
+                cn[4 * q4 + 3] = c4.w;
             }
-            // bf16 pieces of the lane's activations: x = xh + xm + xl exactly
-            uint32_t xu[2][DL], r1u[2][DL], r2u[2][DL];
-            float part[2];
+        };
+        auto scores = [&](floatx16& acc, float (&part)[NCB], int it, const float (&xs)[NCB][DL]) {
+            const int pl = unit_of(it);
+            floatx16& cn = cn_pl[WIDE ? pl : 0];
+            if (group_of(it) == 0) load_cn(cn, pl);  // (a constant once the item loop is unrolled)
+            constexpr int R = DL == 1 ? 1 : DL / 2;
+            uint32_t xh[NCB][R], xm[NCB][R];
 #pragma unroll
-            for (int cbh = 0; cbh < 2; ++cbh) {
+            for (int cbh = 0; cbh < NCB; ++cbh) {
                 float sq = 0.0f;
 #pragma unroll
-                for (int d = 0; d < DL; ++d) {
-                    const float a = xs[cbh][d];
-                    xu[cbh][d] = __float_as_uint(a);
-                    const float r1 = a - __uint_as_float(xu[cbh][d] & 0xffff0000u);
-                    r1u[cbh][d] = __float_as_uint(r1);
-                    r2u[cbh][d] = __float_as_uint(r1 - __uint_as_float(r1u[cbh][d] & 0xffff0000u));
-                    sq = d == 0 ? a * a : fmaf(a, a, sq);
-                }
+                for (int d = 0; d < DL; ++d) sq = d == 0 ? xs[cbh][0] * xs[cbh][0] : fmaf(xs[cbh][d], xs[cbh][d], sq);
                 part[cbh] = sq;
-            }
-            // |x|^2 of codebook h: lanes l and l+32 each hold half of it for both codebooks
-            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(part[0]), __float_as_uint(part[1]), false, false);
-            xx_out = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-            auto mfma = [&](int m, const v4u& b, bool first) {
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, aq[pl][m]), __builtin_bit_cast(bf16x8, b),
-                                                              first ? cn_pl : acc, 0, 0, 0);
-            };
-            // __builtin_amdgcn_perm(p, q, 0x07060302) = (bf16 of q | bf16 of p << 16)
-            if constexpr (DL == 1) {
-                uint32_t breg[8];
 #pragma unroll
-                for (int cbh = 0; cbh < 2; ++cbh) {
-                    breg[3 * cbh + 0] = __builtin_amdgcn_perm(xu[cbh][0], xu[cbh][0], 0x07060302u);    // (xh | xh)
-                    breg[3 * cbh + 1] = __builtin_amdgcn_perm(r1u[cbh][0], r1u[cbh][0], 0x07060302u);  // (xm | xm)
-                    breg[3 * cbh + 2] = __builtin_amdgcn_perm(r2u[cbh][0], xu[cbh][0], 0x07060302u);   // (xh | xl)
+                for (int q = 0; q < R; ++q) {
+                    const float a = xs[cbh][2 * q], b = xs[cbh][DL == 1 ? 0 : 2 * q + 1];
+                    xh[cbh][q] = half_pair(a, b);
+                    const float ra = half_rest<false>(xh[cbh][q], a), rb = DL == 1 ? ra : half_rest<true>(xh[cbh][q], b);
+                    xm[cbh][q] = half_pair(ra, rb);
                 }
-                breg[6] = breg[7] = 0;
-                mfma(0, v4u{breg[0], breg[1], breg[2], breg[3]}, true);
-                mfma(1, v4u{breg[4], breg[5], breg[6], breg[7]}, false);
+            }
+            auto mfma = [&](int m, const v4u& b) {
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, aq[pl][m]), __builtin_bit_cast(f16x8, b),
+                                                             m == 0 ? cn : acc, 0, 0, 0);
+            };
+            if constexpr (WIDE) {
+                const v4u b = DL == 1 ? v4u{xh[0][0], xm[0][0], 0, 0} : DL == 2 ? v4u{xh[0][0], xm[0][0], xh[0][0], xm[0][0]}
+                                                                               : v4u{xh[0][0], xh[0][R - 1], xm[0][0], xm[0][R - 1]};
+#pragma unroll
+                for (int m = 0; m < NM; ++m) mfma(m, b);
+            } else if constexpr (DL == 1) {
+                mfma(0, v4u{xh[0][0], xm[0][0], xh[1][0], xm[1][0]});
             } else {
 #pragma unroll
-                for (int dp = 0; dp < DL / 2; ++dp) {
-                    // six registers in a row, the MFMAs read windows of four of them (see ccs_prep_bf16_kernel)
-                    v6u s6;
-#pragma unroll
-                    for (int cbh = 0; cbh < 2; ++cbh) {
-                        s6[0 + cbh] = __builtin_amdgcn_perm(r1u[cbh][2 * dp + 1], r1u[cbh][2 * dp], 0x07060302u);  // xm
-                        s6[2 + cbh] = __builtin_amdgcn_perm(xu[cbh][2 * dp + 1], xu[cbh][2 * dp], 0x07060302u);    // xh
-                        s6[4 + cbh] = __builtin_amdgcn_perm(r2u[cbh][2 * dp + 1], r2u[cbh][2 * dp], 0x07060302u);  // xl
-                    }
-                    const v4u lo = __builtin_shufflevector(s6, s6, 0, 1, 2, 3), hi = __builtin_shufflevector(s6, s6, 2, 3, 4, 5);
-                    mfma(3 * dp + 0, lo, dp == 0);
-                    mfma(3 * dp + 1, lo, false);
-                    mfma(3 * dp + 2, hi, false);
+                for (int q = 0; q < R; ++q) {
+                    const v4u b = {xh[0][q], xh[1][q], xm[0][q], xm[1][q]};
+                    mfma(2 * q, b);
+                    mfma(2 * q + 1, b);
                 }
             }
         };
 
-        // words[tg / 2], 16 bits per token group: nibble of (pair pl, half h) at bit 8 pl + 4 h
+        // words[tg / 2], 16 bits per token group: nibble of (pair pl, half h) at bit 8 pl + 4 h, or (WIDE) the byte of unit h at bit 0
         uint32_t words[TG / 2];
 #pragma unroll
         for (int i = 0; i < TG / 2; ++i) words[i] = 0;
-        uint32_t need = 0;  // bit it: item it must be replayed exactly by this lane
+        uint32_t need = 0;  // bit o: the lane's item o must be replayed exactly
 
         floatx16 acc_cur, acc_nxt;
-        float xx_cur, xx_nxt;
+        float part_cur[NCB], part_nxt[NCB];
+        float m1_a = 0.0f, m2_a = 0.0f, part_a = 0.0f;  // WIDE: of the first unit
         // The activations of item it + 2 are read from LDS before item it + 1 is scored and item it searched, and
         // the read is kept there: left to itself the compiler sinks it to a few instructions before its use and
         // the wave waits out the LDS latency once per item.
-        float xs_ring[3][2][DL];
+        float xs_ring[3][NCB][DL];
         load_x(xs_ring[0], 0);
         if constexpr (ITEMS > 1) load_x(xs_ring[1], 1);
-        scores(acc_cur, xx_cur, 0, xs_ring[0]);
+        scores(acc_cur, part_cur, 0, xs_ring[0]);
         static_for<ITEMS>([&](auto itc) {
             constexpr int it = decltype(itc)::value;
-            constexpr int pl = it / TG, tg = it % TG;
-            (void)tg;
+            constexpr int pl = WIDE ? it % 2 : it / TG, tg = WIDE ? it / 2 : it % TG;
             if constexpr (it + 2 < ITEMS) {
                 load_x(xs_ring[(it + 2) % 3], it + 2);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if constexpr (it + 1 < ITEMS) scores(acc_nxt, xx_nxt, it + 1, xs_ring[(it + 1) % 3]);
-            const float xx = xx_cur;
+            if constexpr (it + 1 < ITEMS) scores(acc_nxt, part_nxt, it + 1, xs_ring[(it + 1) % 3]);
             // smallest (m1) and second smallest (m2) of the 16 id-tagged scores, 36 VALU operations:
             // five triples give (min3, med3) each; the overall second smallest is the smaller of
             // the second smallest of the six group minima and the smallest of the group medians.
@@ -996,36 +1037,43 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
             const float b1 = vmin3(lo[3], lo[4], key[15]), b2 = __builtin_amdgcn_fmed3f(lo[3], lo[4], key[15]);
             float m1 = vmin(a1, b1);
             float m2 = vmin3(vmin3(md[0], md[1], md[2]), vmin3(md[3], md[4], vmax(a1, b1)), vmin(a2, b2));
-            uint32_t bi = __float_as_uint(m1) & 15u;
-            if constexpr (WIDE) {
-                // the other 16 centroids of the codebook were searched by lane l ^ 32: both lanes merge the
-                // two (smallest, second smallest) pairs and reach the same outcome.  Equal tagged minima
-                // give m2 == m1, which fails the margin test.
-                const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m1), __float_as_uint(m1), false, false);
-                const auto s2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m2), __float_as_uint(m2), false, false);
-                const float m1lo = __uint_as_float(s1[0]), m1hi = __uint_as_float(s1[1]);
-                const float m2lo = __uint_as_float(s2[0]), m2hi = __uint_as_float(s2[1]);
-                m1 = vmin(m1lo, m1hi);
-                m2 = vmin3(vmax(m1lo, m1hi), m2lo, m2hi);
-                bi = (__float_as_uint(m1) & 15u) | (m1hi < m1lo ? 16u : 0u);
+            if constexpr (WIDE && pl == 0) {
+                m1_a = m1;
+                m2_a = m2;
+                part_a = part_cur[0];
+            } else {
+                // |x|^2 of codebook h (of unit h): lanes l and l+32 each hold half of it for both
+                const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(WIDE ? part_a : part_cur[0]), __float_as_uint(part_cur[NCB - 1]), false, false);
+                const float xx = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+                uint32_t bi;
+                if constexpr (WIDE) {
+                    // Lane l holds the first 16 centroids of both units, l ^ 32 the other 16: after the exchange lane half h has both
+                    // (smallest, second smallest) pairs of unit h.  Equal tagged minima give m2 == m1, which fails the margin test.
+                    const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m1_a), __float_as_uint(m1), false, false);
+                    const auto s2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m2_a), __float_as_uint(m2), false, false);
+                    const float m1lo = __uint_as_float(s1[0]), m1hi = __uint_as_float(s1[1]);
+                    m1 = vmin(m1lo, m1hi);
+                    m2 = vmin3(vmax(m1lo, m1hi), __uint_as_float(s2[0]), __uint_as_float(s2[1]));
+                    bi = (__float_as_uint(m1) & 15u) | (m1hi < m1lo ? 16u : 0u);
+                } else {
+                    bi = __float_as_uint(m1) & 15u;
+                }
+                const float mag = xx + cmax[WIDE ? 0 : pl];
+                // 2 * [ (v+1)u (|c|^2) + 12u (what the pieces leave: 8u of x, 2u of c, where subnormal u) + 2.02 * 17 NM u (16 NM products
+                //       and NM accumulators, each within u of a partial sum below 2.02 mag) + 2(v+2)u (the reference's own chain) ]
+                //       = 2 * {57, 98, 178} u  for v = {2, 4, 8}; WIDE {57, 63, 109}
+                constexpr float A2 = 2.0f * ((V + 1) + 12.0f + 2.02f * (17 * NM) + 2 * (V + 2)) * 5.9604645e-8f;
+                constexpr float B2 = 2.0f * 16.0f * 2.3841858e-7f;               // 2 * 2^(4-22)
+                const float thr = fmaf(A2, mag, fmaf(B2, fabsf(m2), c0));
+                // NaN anywhere makes a compare false, which counts as "not safe"; beyond 1e9 a half may have run out
+                const bool safe = ((m2 - m1) > thr) && (mag < 1e9f);
+                need |= (safe ? 0u : 1u) << (WIDE ? tg : it);
+                words[tg / 2] |= bi << (16 * (tg % 2) + (WIDE ? 0 : 8 * pl + 4 * h));
             }
-            const float mag = xx + cmax[pl];
-            // 2 * [ (v+1)u (|c|^2) + 16u (omitted products) + 2.02 (12v + NM) u (that many additions, each
-            //       within u of a partial sum below 2.02 mag) + 2(v+2)u (the reference's own chain) ]
-            //       = 2 * {80, 136, 251} u  for v = {2, 4, 8}
-            constexpr float A2 = 2.0f * ((V + 1) + 16.0f + 2.02f * (12 * V + NM) + 2 * (V + 2)) * 5.9604645e-8f;
-            constexpr float B2 = 2.0f * 16.0f * 2.3841858e-7f;               // 2 * 2^(4-22)
-            const float thr = fmaf(A2, mag, fmaf(B2, fabsf(m2), 1.001e-6f));
-            // NaN anywhere makes a compare false, which counts as "not safe"
-            const bool safe = ((m2 - m1) > thr) && (mag < 1e36f);
-            need |= (safe ? 0u : 1u) << it;
-            if constexpr (WIDE)
-                words[tg / 2] |= (h == 0 ? bi : 0u) << (16 * (tg % 2) + 8 * pl);  // one byte per codebook
-            else
-                words[tg / 2] |= bi << (16 * (tg % 2) + 8 * pl + 4 * h);
             if constexpr (it + 1 < ITEMS) {
                 acc_cur = acc_nxt;
-                xx_cur = xx_nxt;
+#pragma unroll
+                for (int o = 0; o < NCB; ++o) part_cur[o] = part_nxt[o];
             }
         });
 
@@ -1034,12 +1082,24 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
         // pass over the centroids in order that moves to a centroid closer by more than 1e-6.
         const uint64_t replay_mask = __builtin_amdgcn_ballot_w64(need != 0);
         constexpr int COOP_MAX = V / 2;  // up to that many lanes: one at a time, by the whole wave (8 measured the same)
-        if (replay_mask != 0 && __builtin_popcountll(WIDE ? (replay_mask & 0xFFFFFFFFull) : replay_mask) <= COOP_MAX) {
+        // a token's sub-vector of codebook cbl of the tile as it came (the tile holds it scaled)
+        auto raw_x = [&](float (&xr)[V], uint32_t row, uint32_t cbl) __attribute__((always_inline)) {
+            const uint32_t tok = tok0 + row < N ? tok0 + row : N - 1;
+            if (plain) {
+#pragma unroll
+                for (int t = 0; t < V; ++t) xr[t] = tile[row * PITCH + cbl * V + t];
+            } else {
+                const float* xo = x + (size_t)tok * K + (tcb % tiles_x) * TF + cbl * V;
+#pragma unroll
+                for (int t = 0; t < V; ++t) xr[t] = xo[t];
+            }
+        };
+        constexpr uint32_t keep_mask = WIDE ? 255u : 15u;
+        if (replay_mask != 0 && __builtin_popcountll(replay_mask) <= COOP_MAX) {
             // A lane's replay done by the wave: lane c computes the distance to centroid c, the pass over the
             // centroids reads them lane by lane.  A single lane doing all of it (below) keeps the other 63 waiting
             // for C x (3v + 4) operations; this is 3v + 5C.
-            // wide: lanes l and l + 32 hold the same outcome, and lane l (h = 0) keeps the byte
-            uint64_t mask = WIDE ? (replay_mask & 0xFFFFFFFFull) : replay_mask;
+            uint64_t mask = replay_mask;
             const uint32_t wave_s = __builtin_amdgcn_readfirstlane(wave);
             while (mask) {
                 const uint32_t l = (uint32_t)__builtin_ctzll(mask);
@@ -1047,20 +1107,21 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
                 uint32_t nd = __builtin_amdgcn_readlane(need, l);
                 const uint32_t jl = l & 31, hl = l >> 5;
                 while (nd) {
-                    const uint32_t it = (uint32_t)__builtin_ctz(nd);
+                    const uint32_t o = (uint32_t)__builtin_ctz(nd);
                     nd &= nd - 1;
-                    const uint32_t pl = it / TG, tg = it % TG;
-                    const uint32_t cbl = WIDE ? 2 * wave_s + pl : 2 * (2 * wave_s + pl) + hl;
+                    const uint32_t pl = o / TG, tg = o % TG;  // (WIDE: pl = 0)
+                    const uint32_t cbl = WIDE ? 2 * wave_s + hl : 2 * (2 * wave_s + pl) + hl;
                     uint32_t bi = 0;
                     if (tcb * RCB + cbl < CB) {
-                        const float* xo = tile + (tg * 32 + jl) * PITCH + (2 * wave_s + pl) * XSTEP + (WIDE ? 0 : V * hl);
+                        float xr[V];
+                        raw_x(xr, tg * 32 + jl, cbl);
                         const uint32_t cl = lane < C ? lane : C - 1;  // lanes past the last centroid repeat it; never read
                         const float* cp = cst + (cbl * C + cl) * V;
-                        float diff = __fsub_rn(xo[0], cp[0]);
+                        float diff = __fsub_rn(xr[0], cp[0]);
                         float d = __fmul_rn(diff, diff);
 #pragma unroll
                         for (int t = 1; t < V; ++t) {
-                            diff = __fsub_rn(xo[t], cp[t]);
+                            diff = __fsub_rn(xr[t], cp[t]);
                             d = __fadd_rn(d, __fmul_rn(diff, diff));
                         }
                         float best = 0.0f;
@@ -1071,8 +1132,7 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
                             bi = take ? c : bi;
                         }
                     }
-                    const uint32_t sh = WIDE ? 16 * (tg % 2) + 8 * pl : 16 * (tg % 2) + 8 * pl + 4 * hl;
-                    const uint32_t keep_mask = WIDE ? 255u : 15u;
+                    const uint32_t sh = 16 * (tg % 2) + (WIDE ? 0 : 8 * pl + 4 * hl);
                     const bool mine = lane == l;
 #pragma unroll
                     for (int i = 0; i < TG / 2; ++i)
@@ -1083,24 +1143,25 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
             // many lanes at once (ties: rows of zeros, repeated centroids): every lane replays its own items
             // kept rolled on purpose: the replay is rare and must not cost the fast path registers
 #pragma nounroll
-            for (int it = 0; it < ITEMS; ++it) {
-                if (!((need >> it) & 1u)) continue;
-                const int pl = it / TG, tg = it % TG;
-                const uint32_t cbl = WIDE ? 2 * wave + pl : 2 * (2 * wave + pl) + h;  // codebook within the tile
+            for (int o = 0; o < OWN; ++o) {
+                if (!((need >> o) & 1u)) continue;
+                const int pl = o / TG, tg = o % TG;  // (WIDE: pl = 0)
+                const uint32_t cbl = WIDE ? 2 * wave + h : 2 * (2 * wave + pl) + h;  // codebook within the tile
                 uint32_t bi = 0;
                 if (tcb * RCB + cbl < CB) {
-                    const float* xo = brow0 + tg * 32 * PITCH + pl * XSTEP + (WIDE ? 0 : V * h);
+                    float xr[V];
+                    raw_x(xr, tg * 32 + j, cbl);
                     const float* cp = cst + cbl * C * V;
                     float best = 0.0f;
                     // eight centroids per trip: their rows are read from LDS together, and the wave waits for
                     // LDS once per trip instead of once per centroid (rolled, a replay took 1.5 us)
 #pragma unroll 8
                     for (uint32_t c = 0; c < C; ++c) {
-                        float diff = __fsub_rn(xo[0], cp[c * V + 0]);
+                        float diff = __fsub_rn(xr[0], cp[c * V + 0]);
                         float d = __fmul_rn(diff, diff);
 #pragma unroll
                         for (int t = 1; t < V; ++t) {
-                            diff = __fsub_rn(xo[t], cp[c * V + t]);
+                            diff = __fsub_rn(xr[t], cp[c * V + t]);
                             d = __fadd_rn(d, __fmul_rn(diff, diff));
                         }
                         const bool take = (c == 0) || (__fsub_rn(best, d) > 1e-6f);
@@ -1108,10 +1169,7 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
                         bi = take ? c : bi;
                     }
                 }
-                // wide: both lanes of the pair replay all of the codebook's centroids; lane h = 0 keeps the byte
-                const uint32_t sh = WIDE ? 16 * (tg % 2) + 8 * pl : 16 * (tg % 2) + 8 * pl + 4 * h;
-                const uint32_t keep_mask = WIDE ? 255u : 15u;
-                if (WIDE && h != 0) bi = 0;
+                const uint32_t sh = 16 * (tg % 2) + (WIDE ? 0 : 8 * pl + 4 * h);
                 uint32_t w = words[0];
 #pragma unroll
                 for (int i = 1; i < TG / 2; ++i) w = (tg / 2 == i) ? words[i] : w;
@@ -1126,7 +1184,7 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
 #pragma unroll
         for (int i = 0; i < TG / 2; ++i) {  // lanes l and l + 32 exchange their words without going through LDS
             const auto sw = __builtin_amdgcn_permlane32_swap(words[i], words[i], false, false);
-            words[i] = sw[0] | sw[1];
+            words[i] = sw[0] | sw[1] << (WIDE ? 8 : 0);
         }
         if (h == 0) {
 #pragma unroll
@@ -1751,7 +1809,7 @@ int launch_ccs_mfma(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
 }
 
 template <int V, bool WIDE, int TTOK>
-int launch_ccs_bf16_tt(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent, uint8_t* d_idx, uint32_t n,
+int launch_ccs_f16_tt(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent, uint8_t* d_idx, uint32_t n,
                        uint32_t x_cols)
 {
     using S = CcsMfmaShape<V, WIDE, TTOK>;
@@ -1764,7 +1822,7 @@ int launch_ccs_bf16_tt(Ctx* ctx, const AmmGeom& g, const float* d_x, const float
     static int per_cu = 0;
     if (per_cu == 0) {
         int q = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, ccs_bf16_kernel<V, WIDE, TTOK>, CCS_THREADS, 0) != hipSuccess || q < 1) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&q, ccs_f16_kernel<V, WIDE, TTOK>, CCS_THREADS, 0) != hipSuccess || q < 1) {
             (void)hipGetLastError();
             q = 1;
         }
@@ -1782,18 +1840,19 @@ int launch_ccs_bf16_tt(Ctx* ctx, const AmmGeom& g, const float* d_x, const float
     const float* aux = d_cent + (size_t)g.CB * g.C * g.v;
     const float* cnmax = aux + ccs_aux_floats(g);
     const float* cnmax_pad = cnmax + g.CB + (size_t)(g.CB_pad / 2) * (g.v + 1) * 64;
-    const float* bf = d_cent + ccs_bf16_offset(g);
+    const float* bf = d_cent + ccs_f16_offset(g);
     const uint4* aux_b = reinterpret_cast<const uint4*>(bf);
-    const float* cn16 = bf + ccs_bf16_units(g) * ccs_bf16_nm(V) * 64 * 4;
-    hipLaunchKernelGGL((ccs_bf16_kernel<V, WIDE, TTOK>), grid, dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent, aux_b, cn16, cnmax_pad,
+    const float* cn16 = bf + ccs_f16_units(g) * ccs_f16_nm(V, WIDE) * 64 * 4;
+    const float* scale = cn16 + ccs_f16_units(g) * 2 * 16;
+    hipLaunchKernelGGL((ccs_f16_kernel<V, WIDE, TTOK>), grid, dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent, aux_b, cn16, scale, cnmax_pad,
                        d_idx, n, row, g.CB, g.C, g.idx_row_bytes, (int)g.idx_tiled, vec_ok, tiles_cb, total, tiles_x);
-    return hip_check(ctx, hipGetLastError(), "ccs_bf16_kernel launch");
+    return hip_check(ctx, hipGetLastError(), "ccs_f16_kernel launch");
 }
 
 // 128-token tiles amortise a tile's operand loads best, but a workgroup that gets only one or two of them
 // cannot overlap a tile's loads with the previous tile's arithmetic: small batches use 64-token tiles.
 template <int V, bool WIDE>
-int launch_ccs_bf16(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent, uint8_t* d_idx, uint32_t n,
+int launch_ccs_f16(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent, uint8_t* d_idx, uint32_t n,
                     uint32_t x_cols)
 {
     const uint64_t tiles128 = (uint64_t)((n + 127) / 128) * (g.CB_pad / CcsMfmaShape<V, WIDE>::RCB);
@@ -1807,8 +1866,8 @@ int launch_ccs_bf16(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     // tiles, 8.3 / 7.0 at 192, 15.1 / 9.7 at 512, 26 / 24.5 at 1536, 35.7 / 33.5 at 2376)
     const uint64_t few = (V == 8 && !WIDE) ? ctx->prop.multiProcessorCount / 2 : 6ull * ctx->prop.multiProcessorCount;
     const bool small_tiles = g.tune_search_tile ? g.tune_search_tile == 64 : tiles128 <= few;
-    if (small_tiles) return launch_ccs_bf16_tt<V, WIDE, 64>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
-    return launch_ccs_bf16_tt<V, WIDE, 128>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+    if (small_tiles) return launch_ccs_f16_tt<V, WIDE, 64>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+    return launch_ccs_f16_tt<V, WIDE, 128>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
 }
 
 template <int V, int IDX_BITS>
@@ -1820,7 +1879,7 @@ int launch_ccs_many(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     if (total > 0x7FFFFFFFull) return set_error(ctx, PIMDL_ERR_INVALID, "ccs: too many tiles");
     const int vec_ok = (g.K % 4 == 0) && ((reinterpret_cast<uintptr_t>(d_x) & 15) == 0);
     const float* cnmax = d_cent + (size_t)g.CB * g.C * g.v + ccs_aux_floats(g);
-    const float* many = d_cent + ccs_bf16_offset(g);
+    const float* many = d_cent + ccs_f16_offset(g);
     const float* cn32 = many + ccs_many_groups(g) * ccs_many_nm(V) * 64 * 4;
     hipLaunchKernelGGL((ccs_many_kernel<V, IDX_BITS>), dim3((uint32_t)total), dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent,
                        reinterpret_cast<const uint4*>(many), cn32, cnmax, d_idx, n, g.K, g.CB, g.C, g.idx_row_bytes,
@@ -1881,18 +1940,18 @@ int launch_ccs_bits(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     }
     if (IDX_BITS == 8 && g.C <= 32 && !exact && !f32) {
         switch (g.v) {
-            case 2: return launch_ccs_bf16<2, true>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
-            case 4: return launch_ccs_bf16<4, true>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
-            case 8: return launch_ccs_bf16<8, true>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+            case 2: return launch_ccs_f16<2, true>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+            case 4: return launch_ccs_f16<4, true>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+            case 8: return launch_ccs_f16<8, true>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
             default: break;
         }
     }
     if (IDX_BITS == 4 && !exact) {
         if (!f32) {
             switch (g.v) {
-                case 2: return launch_ccs_bf16<2, false>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
-                case 4: return launch_ccs_bf16<4, false>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
-                case 8: return launch_ccs_bf16<8, false>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+                case 2: return launch_ccs_f16<2, false>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+                case 4: return launch_ccs_f16<4, false>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
+                case 8: return launch_ccs_f16<8, false>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
                 default: break;
             }
         }
@@ -1958,10 +2017,10 @@ int launch_ccs_bits(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
 
 }  // namespace
 
-// Measures what the bf16-split search assumes about the matrix core: a chain of three
-// v_mfma_f32_32x32x16_bf16 (48 products + the initial accumulator) against the exact sum, over random
-// operands whose pieces differ in magnitude like xh/xm/xl do.  Reports max |D - exact| / (u * sum|terms|).
-// The search kernel's bound allows 2.02 (12 v + NM) u per partial sum, i.e. 51 in this unit for v = 4.
+// Measures what the matrix searches assume about the matrix core: a chain of three
+// v_mfma_f32_32x32x16_f16 (48 products + the initial accumulator) against the exact sum, over random
+// operands whose pieces differ in magnitude like xh/xm do, subnormal halves among them.  Reports max |D - exact| / (u * sum|terms|).
+// The searches' bounds allow one u per product and accumulator, i.e. 51 in this unit for such a chain.
 namespace {
 __global__ void mfma_error_kernel(const uint4* __restrict__ a, const uint4* __restrict__ b, const float* __restrict__ c,
                                   float* __restrict__ d, int chain)
@@ -1974,8 +2033,8 @@ __global__ void mfma_error_kernel(const uint4* __restrict__ a, const uint4* __re
     floatx16 acc;
     for (int r = 0; r < 16; ++r) acc[r] = c[(8 * (r / 4) + 4 * (l / 32) + r % 4) * 32 + (l % 32)];
     for (int m = 0; m < chain; ++m)
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[m * 64 + l]),
-                                                      __builtin_bit_cast(bf16x8, b[m * 64 + l]), acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a[m * 64 + l]),
+                                                     __builtin_bit_cast(f16x8, b[m * 64 + l]), acc, 0, 0, 0);
     for (int r = 0; r < 16; ++r) d[(8 * (r / 4) + 4 * (l / 32) + r % 4) * 32 + (l % 32)] = acc[r];
 }
 }  // namespace
@@ -1984,9 +2043,10 @@ __global__ void mfma_error_kernel(const uint4* __restrict__ a, const uint4* __re
 // accumulator of 1.0 that receives 48 equal products just below / just above a half, one and two units in its
 // last place (a sequential adder that rounds to nearest drops every product of the first kind, one that
 // truncates also drops the larger ones), of either sign, and products whose magnitudes fall by a factor of
-// four from slot to slot (bits shifted out when the terms of one instruction are aligned).  `trials` is
+// four from slot to slot (bits shifted out when the terms of one instruction are aligned); then sums of nothing but products with a
+// subnormal half on one side, which a matrix core that takes them for zero loses whole.  `trials` is
 // ignored then.
-constexpr uint32_t MFMA_CRAFTED_TRIALS = 14;
+constexpr uint32_t MFMA_CRAFTED_TRIALS = 18;
 int launch_diag_mfma_error(Ctx* ctx, uint32_t trials, bool crafted, float* max_err_u)
 {
     constexpr int CHAIN = 3;
@@ -2002,8 +2062,18 @@ int launch_diag_mfma_error(Ctx* ctx, uint32_t trials, bool crafted, float* max_e
         return z ^ (z >> 31);
     };
     auto unif = [&]() { return (float)((double)(next() >> 11) / 9007199254740992.0 * 2.0 - 1.0); };
-    auto to_bf16 = [](float f) { uint32_t u; memcpy(&u, &f, 4); return (uint16_t)(u >> 16); };
-    auto from_bf16 = [](uint16_t h) { uint32_t u = (uint32_t)h << 16; float f; memcpy(&f, &u, 4); return f; };
+    // halves, cut towards zero (magnitudes below 65536)
+    auto to_f16 = [](float f) {
+        const float a = fabsf(f);
+        const int e = a < 6.103515625e-5f ? -14 : ilogbf(a);  // (subnormal: the smallest exponent, no leading one)
+        const uint32_t m = (uint32_t)ldexpf(a, 10 - e);
+        return (uint16_t)((f < 0 ? 0x8000u : 0u) | (a < 6.103515625e-5f ? m : (uint32_t)(e + 14) * 1024 + m));
+    };
+    auto from_f16 = [](uint16_t h) {
+        const int e = h >> 10 & 31;
+        const float a = ldexpf((float)(e ? 1024 + (h & 1023) : h & 1023), (e ? e : 1) - 25);
+        return h & 0x8000 ? -a : a;
+    };
     for (uint32_t t = 0; crafted && t < trials; ++t) {
         static const float mags[6] = {0.4921875f, 0.5078125f, 0.9921875f, 1.0078125f, 1.984375f, 2.015625f};  // 8-bit significands
         const float sign = (t & 1) ? -1.0f : 1.0f;
@@ -2011,18 +2081,20 @@ int launch_diag_mfma_error(Ctx* ctx, uint32_t trials, bool crafted, float* max_e
             for (int r = 0; r < 32; ++r)
                 for (int kk = 0; kk < 16; ++kk) {
                     // A[r][kk] * B[kk][r]: 2^-12 * (sign * mag * 2^-12) = sign * mag * 2^-24, or the falling staircase
-                    const float a = t < 12 ? ldexpf(1.0f, -12) : 1.0f;
-                    const float b = t < 12 ? sign * ldexpf(mags[t / 2], -12) : sign * ldexpf(1.9921875f, -2 * kk - 1);
-                    A[((size_t)(t * CHAIN + m) * 32 + r) * 16 + kk] = to_bf16(a);
-                    B[((size_t)(t * CHAIN + m) * 16 + kk) * 32 + r] = to_bf16(b);
+                    // (of its products the later slots' are halves that are subnormal), or a subnormal half and a large one
+                    float a = t < 12 ? ldexpf(1.0f, -12) : t < 14 ? ldexpf(1.0f, -kk) : sign * ldexpf((float)(2 * kk + 1 + r), -24);
+                    float b = t < 12 ? sign * ldexpf(mags[t / 2], -12) : t < 14 ? sign * ldexpf(1.9921875f, -kk - 1) : (float)(1024 + 37 * kk + r);
+                    if (t >= 16) std::swap(a, b);
+                    A[((size_t)(t * CHAIN + m) * 32 + r) * 16 + kk] = to_f16(a);
+                    B[((size_t)(t * CHAIN + m) * 16 + kk) * 32 + r] = to_f16(b);
                 }
-        for (size_t i = 0; i < 1024; ++i) C[(size_t)t * 1024 + i] = 1.0f;
+        for (size_t i = 0; i < 1024; ++i) C[(size_t)t * 1024 + i] = t < 14 ? 1.0f : 0.0f;
     }
     for (uint32_t t = 0; !crafted && t < trials; ++t) {
         const float small = ldexpf(1.0f, (int)(t % 5) * 6 - 24);
         for (size_t i = 0; i < (size_t)CHAIN * 512; ++i) {
-            A[(size_t)t * CHAIN * 512 + i] = to_bf16(3.0f * unif() * ((next() & 1) ? 1.0f : small));
-            B[(size_t)t * CHAIN * 512 + i] = to_bf16(3.0f * unif() * ((next() & 3) ? 1.0f : small));
+            A[(size_t)t * CHAIN * 512 + i] = to_f16(3.0f * unif() * ((next() & 1) ? 1.0f : small));
+            B[(size_t)t * CHAIN * 512 + i] = to_f16(3.0f * unif() * ((next() & 3) ? 1.0f : small));
         }
         for (size_t i = 0; i < 1024; ++i) C[(size_t)t * 1024 + i] = 8.0f * unif();
     }
@@ -2066,12 +2138,12 @@ int launch_diag_mfma_error(Ctx* ctx, uint32_t trials, bool crafted, float* max_e
                 double ex = C[(size_t)t * 1024 + i * 32 + j], sabs = fabs(ex);
                 for (int m = 0; m < CHAIN; ++m)
                     for (int kk = 0; kk < 16; ++kk) {
-                        const double p = (double)from_bf16(A[((size_t)(t * CHAIN + m) * 32 + i) * 16 + kk]) *
-                                         (double)from_bf16(B[((size_t)(t * CHAIN + m) * 16 + kk) * 32 + j]);
+                        const double p = (double)from_f16(A[((size_t)(t * CHAIN + m) * 32 + i) * 16 + kk]) *
+                                         (double)from_f16(B[((size_t)(t * CHAIN + m) * 16 + kk) * 32 + j]);
                         ex += p;
                         sabs += fabs(p);
                     }
-                const double e = fabs((double)D[(size_t)t * 1024 + i * 32 + j] - ex) / (5.9604644775390625e-8 * sabs);
+                const double e = sabs == 0.0 ? 0.0 : fabs((double)D[(size_t)t * 1024 + i * 32 + j] - ex) / (5.9604644775390625e-8 * sabs);
                 if (e > worst) worst = e;
             }
     *max_err_u = (float)worst;
@@ -2101,7 +2173,7 @@ bool ccs_f32_only()
 
 size_t ccs_centroid_bytes(const AmmGeom& g)
 {
-    return (ccs_bf16_offset(g) + ccs_bf16_floats(g) + ccs_many_floats(g)) * sizeof(float);
+    return (ccs_f16_offset(g) + ccs_f16_floats(g) + ccs_many_floats(g)) * sizeof(float);
 }
 
 int launch_ccs_prep(Ctx* ctx, const AmmGeom& g, float* d_cent)
@@ -2117,29 +2189,30 @@ int launch_ccs_prep(Ctx* ctx, const AmmGeom& g, float* d_cent)
                        aux_a + (size_t)(g.CB_pad / 2) * (g.v + 1) * 64, g.CB, g.C, g.v);
     rc = hip_check(ctx, hipGetLastError(), "ccs_prep_mfma_kernel launch");
     if (!rc && ccs_has_many(g)) {
-        float* many = d_cent + ccs_bf16_offset(g);
+        float* many = d_cent + ccs_f16_offset(g);
         float* cn32 = many + ccs_many_groups(g) * ccs_many_nm(g.v) * 64 * 4;
         auto prep = g.v == 2 ? ccs_prep_many_kernel<2> : g.v == 4 ? ccs_prep_many_kernel<4> : g.v == 8 ? ccs_prep_many_kernel<8>
                   : g.v == 16 ? ccs_prep_many_kernel<16> : ccs_prep_many_kernel<32>;
         hipLaunchKernelGGL(prep, dim3(g.CB, (g.C + 31) / 32), dim3(64), 0, ctx->stream, d_cent, reinterpret_cast<uint4*>(many), cn32, g.C);
         rc = hip_check(ctx, hipGetLastError(), "ccs_prep_many_kernel launch");
     }
-    if (rc || !ccs_has_bf16(g)) return rc;
-    float* bf = d_cent + ccs_bf16_offset(g);
+    if (rc || !ccs_has_f16(g)) return rc;
+    float* bf = d_cent + ccs_f16_offset(g);
     uint4* aux_b = reinterpret_cast<uint4*>(bf);
-    float* cn16 = bf + ccs_bf16_units(g) * ccs_bf16_nm(g.v) * 64 * 4;
-    const dim3 pg((uint32_t)ccs_bf16_units(g)), pb(64);
-    const bool wide = ccs_bf16_wide(g);
-#define PIMDL_PREP_BF16(V_)                                                                                        \
-    if (wide) hipLaunchKernelGGL((ccs_prep_bf16_kernel<V_, true>), pg, pb, 0, ctx->stream, d_cent, aux_b, cn16, g.CB, g.C); \
-    else hipLaunchKernelGGL((ccs_prep_bf16_kernel<V_, false>), pg, pb, 0, ctx->stream, d_cent, aux_b, cn16, g.CB, g.C);
+    const bool wide = ccs_f16_wide(g);
+    float* cn16 = bf + ccs_f16_units(g) * ccs_f16_nm(g.v, wide) * 64 * 4;
+    float* scale = cn16 + ccs_f16_units(g) * 2 * 16;
+    const dim3 pg((uint32_t)ccs_f16_units(g)), pb(64);
+#define PIMDL_PREP_F16(V_)                                                                                        \
+    if (wide) hipLaunchKernelGGL((ccs_prep_f16_kernel<V_, true>), pg, pb, 0, ctx->stream, d_cent, cnmax, aux_b, cn16, scale, g.CB, g.C); \
+    else hipLaunchKernelGGL((ccs_prep_f16_kernel<V_, false>), pg, pb, 0, ctx->stream, d_cent, cnmax, aux_b, cn16, scale, g.CB, g.C);
     switch (g.v) {
-        case 2: PIMDL_PREP_BF16(2) break;
-        case 4: PIMDL_PREP_BF16(4) break;
-        default: PIMDL_PREP_BF16(8) break;
+        case 2: PIMDL_PREP_F16(2) break;
+        case 4: PIMDL_PREP_F16(4) break;
+        default: PIMDL_PREP_F16(8) break;
     }
-#undef PIMDL_PREP_BF16
-    return hip_check(ctx, hipGetLastError(), "ccs_prep_bf16_kernel launch");
+#undef PIMDL_PREP_F16
+    return hip_check(ctx, hipGetLastError(), "ccs_prep_f16_kernel launch");
 }
 
 uint32_t ccs_cb_per_wg(uint32_t v)
@@ -2168,9 +2241,9 @@ int launch_ccs(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_cent
 // matrix-core kernel and whole codebook tiles per operator.
 bool ccs_supports_shared_input(const AmmGeom& g, uint32_t x_cols)
 {
-    if (!ccs_has_bf16(g)) return false;
+    if (!ccs_has_f16(g)) return false;
     if (g.tune_search ? g.tune_search != PIMDL_SEARCH_MFMA_BF16 : (ccs_exact_only() || ccs_f32_only())) return false;
-    const uint32_t tf = (ccs_bf16_wide(g) ? 8 : 16) * g.v;
+    const uint32_t tf = (ccs_f16_wide(g) ? 8 : 16) * g.v;
     return x_cols % tf == 0;
 }
 

@@ -479,6 +479,31 @@ def test_search_with_a_few_near_ties_per_wave(ctx, v, C):
     amm.close()
 
 
+@pytest.mark.parametrize("v,C", [(2, 16), (4, 16), (8, 16), (4, 9), (2, 32), (4, 32), (8, 32), (4, 17)])
+@pytest.mark.parametrize("size", [1e-4, 0.03, 1.0, 900.0, 1100.0, 3e4, 1e9, 1e16])
+def test_search_over_the_range_of_halves(ctx, v, C, size):
+    """The matrix search works on halves, whose range ends at 65504 and 6e-8: centroids and activations of one size from far below
+    to far above it (tiles with centroids beyond 1024 are searched at a scale of their own), codebooks of another size beside them in
+    the same and in other tiles, activations that no half holds, an odd width; every index against the reference's scan."""
+    rng = np.random.default_rng(int(4000 + 10 * v + C))
+    N, CB = 210, 37
+    cent = rng.standard_normal((CB, C, v)).astype(np.float32)
+    x = rng.standard_normal((N, CB, v)).astype(np.float32)
+    cent[:20] *= np.float32(size)
+    x[:, :20] *= np.float32(size)
+    cent[3], x[:, 3] = cent[3] / np.float32(size), x[:, 3] / np.float32(size)
+    x[7::50] *= np.float32(7e4)
+    x[8, 30, 0], x[9, 5, v - 1] = 65504.0, -1e30
+    x = x.reshape(N, CB * v)
+    want = oracle.index_calculation(x, cent, v, threads=THREADS)
+    amm = ctx.amm(cent, np.zeros((CB, C, 4), np.int8), np.float32(1.0), None, max_n=N)
+    for tile in (64, 128):
+        amm.set_tuning(search_token_tile=tile)
+        got = amm.index_calculation(x)
+        assert np.array_equal(got, want), f"tile {tile}: {(got != want).sum()} of {got.size} differ"
+    amm.close()
+
+
 @pytest.mark.parametrize("v,C", [(4, 16), (2, 16), (8, 16), (4, 32)])
 def test_search_with_non_finite_values(ctx, v, C):
     """NaN / Inf / near-overflow values in activations and centroids take the exact path and match
@@ -506,9 +531,9 @@ def test_search_with_non_finite_values(ctx, v, C):
 
 
 def test_matrix_core_rounding_stays_inside_the_search_margin(ctx):
-    """The bf16-split search accepts a winner only outside an error margin that assumes every addition of
+    """The matrix search accepts a winner only outside an error margin that assumes every addition of
     the matrix core's chain (48 products + the initial accumulator) is within 2^-24 of the partial sum:
-    51 units of 2^-24 * sum|terms| for v = 4.  Measured on this device over 10^6 outputs with operand pieces
+    51 units of 2^-24 * sum|terms| for a chain of three.  Measured on this device over 10^6 outputs with operand pieces
     of mixed magnitude, the chain stays an order of magnitude inside that."""
     worst = ctx.diag_mfma_error(1024)
     assert 0.0 < worst < 12.0, worst
