@@ -99,16 +99,16 @@ inline size_t ccs_f16_floats(const AmmGeom& g)
 }
 
 // more than 32 centroids, or sub-vectors of 16 or 32 dimensions: the matrix search over groups of 32 centroids
-// (ccs_many_kernel).  Its operands stand where the bf16 ones of the shapes above would.
+// (ccs_many_kernel).  Its operands stand where those of the shapes above would.
 inline bool ccs_has_many(const AmmGeom& g)
 {
     return g.v == 16 || g.v == 32 || (g.C > 32 && (g.v == 2 || g.v == 4 || g.v == 8));
 }
 inline size_t ccs_many_groups(const AmmGeom& g) { return (size_t)g.CB * ((g.C + 31) / 32); }
-constexpr uint32_t ccs_many_nm(uint32_t v) { return v == 2 ? 1 : v == 4 ? 2 : 3 * (v / 8); }  // matrix instructions per group
+constexpr uint32_t ccs_many_nm(uint32_t v) { return (4 * v + 15) / 16; }  // matrix instructions per group: v dims x 4 cross products
 inline size_t ccs_many_floats(const AmmGeom& g)
 {
-    return ccs_has_many(g) ? ccs_many_groups(g) * (ccs_many_nm(g.v) * 64 * 4 + 32) : 0;
+    return ccs_has_many(g) ? ccs_many_groups(g) * (ccs_many_nm(g.v) * 64 * 4 + 32) + g.CB : 0;  // (and a scale per codebook)
 }
 
 template <int N, typename F>
@@ -679,7 +679,6 @@ __global__ __launch_bounds__(CCS_THREADS, V == 8 ? 2 : 4) void ccs_mfma_kernel(c
 //   cn16  [CB_pad][16] float          |c|^2 (r for padded codebooks, 3e38 for ids past C)
 //   scale [units / 8] float           what a tile's activations and centroids are multiplied with
 // =============================================================================================
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
@@ -1211,23 +1210,28 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
 // =============================================================================================
 // The matrix search for more than 32 centroids (v = 2, 4, 8) and for v = 16 and 32: one wave takes one codebook at a time
 // for 32 * TG tokens and goes through its centroids 32 by 32.  Scores, tags, tournament, margin test and exact replay are
-// those of the bf16 search above; a group's winner meets the smallest and second smallest so far.
+// those of ccs_f16_kernel; a group's winner meets the smallest and second smallest so far.
 // Operands of a group: lane (row i, half kh) supplies dims DL kh .. DL kh + DL - 1 (DL = v / 2) of centroid 32 grp + 16 h + r
 // (row i = (r & 3) + 8 (r >> 2) + 4 h, so that result register r of lane (token, h) is that centroid's score).  A register
-// holds a piece of dims d and d + 1; per two such pairs three instructions:
-//   [H0 M0 H1 M1] x [CH CH CH CH], the same x [CM CM CM CM], [H0 L0 H1 L1] x [CL CH CL CH]      (v >= 8)
-//   [H M H M] x [CH CH CM CM], [H L H L] x [CL CH 0 0]                                         (v = 4)
-//   [(xh|xh) (xm|xm) (xh|xl) 0] x [(ch|cm) (ch|cm) (cl|ch) 0]                                   (v = 2)
+// holds a piece of dims d and d + 1; per two such pairs two instructions:
+//   [xh(0) xm(0) xh(1) xm(1)] x [ch(0) ch(0) ch(1) ch(1)], the same x [cm ...]                  (v >= 8)
+//   [xh xm xh xm] x [ch ch cm cm]                                                               (v = 4)
+//   [(xh|xh) (xm|xm) 0 0] x [(ch|cm) (ch|cm) 0 0]                                               (v = 2)
 // The activations' pieces are made once per token and codebook, whatever the number of centroids.
 // Bound by the vector ALU: 16 tags, 20 operations of the tournament and 5 of the merge per 32 x 32 scores.
 // A lane per token and a scalar operand per centroid (ccs_kernel) spent v + 4 operations at half rate per score and
 // replayed 64 tokens for each near tie (us at N = 8192, before / now: v = 4, 64 centroids, K = 768 43 / 21, K = 3072 141 / 70; 128
 // centroids, K = 1024 97 / 42; 256 204 / 76; v = 16, K = 1024, 64 centroids 54 / 13; v = 32, K = 1280, 64 centroids 118 / 22,
 // K = 2048, 128 centroids 244 / 37, K = 1024, 16 centroids 24 / 9.3; N = 128: 21 / 8, 39 / 12, 22 / 7, 102 / 8).
+// Halves instead of three bf16 pieces, one of two token groups decided by each half of a wave, a codebook's first operands requested while
+// the codebook before it is searched; search and gather, us a pass at N = 8192, inputs and outputs in turn, before / now: 64 centroids, v = 4 K = 768
+// 102.4 / 95, K = 3072 168 / 147, v = 2 73.8 / 69.8, v = 8 31.2 / 28.5, v = 16 30.9 / 27.8, v = 32 37.5 / 32.6; 200 centroids 121.7 / 101;
+// 64 centroids, N = 1000 22.0 / 18.4.
 //   aux  [CB][groups][NM][64 lanes] uint4, then cn [CB][groups][2 h][16] |c|^2 (3e38 past the last centroid)
 // =============================================================================================
 template <uint32_t V>
-__global__ void ccs_prep_many_kernel(const float* __restrict__ cent, uint4* __restrict__ aux, float* __restrict__ cn32, uint32_t C)
+__global__ void ccs_prep_many_kernel(const float* __restrict__ cent, const float* __restrict__ cnmax, uint4* __restrict__ aux,
+                                     float* __restrict__ cn32, float* __restrict__ scale, uint32_t C)
 {
     constexpr uint32_t DL = V / 2, NM = ccs_many_nm(V);
     const uint32_t cb = blockIdx.x, grp = blockIdx.y, groups = gridDim.y, lane = threadIdx.x;
@@ -1235,34 +1239,28 @@ __global__ void ccs_prep_many_kernel(const float* __restrict__ cent, uint4* __re
     const uint32_t cid = 32 * grp + 16 * h + r;
     const bool real = cid < C;
     const float* cp = cent + ((size_t)cb * C + (real ? cid : 0)) * V;
-    uint32_t pc[DL][3];  // bf16 pieces of -2c
+    const float sc = half_scale(cnmax + cb, 1);
+    if (grp == 0 && lane == 0) scale[cb] = sc;
+    uint32_t pc[DL][2];  // pieces ch, cm of -2c
 #pragma unroll
     for (uint32_t d = 0; d < DL; ++d) {
-        const float a = real ? -2.0f * cp[DL * kh + d] : 0.0f;
-        const uint32_t au = __float_as_uint(a);
-        const float r1 = __fsub_rn(a, __uint_as_float(au & 0xffff0000u));
-        const uint32_t r1u = __float_as_uint(r1);
-        const float r2 = __fsub_rn(r1, __uint_as_float(r1u & 0xffff0000u));
-        pc[d][0] = au >> 16;
-        pc[d][1] = r1u >> 16;
-        pc[d][2] = __float_as_uint(r2) >> 16;
+        float a = real ? -2.0f * (cp[DL * kh + d] * sc) : 0.0f;
+        pc[d][0] = half_piece(a);
+        pc[d][1] = half_piece(a);
     }
     uint4* dst = aux + ((size_t)cb * groups + grp) * NM * 64 + lane;
     if constexpr (DL == 1) {
-        const uint32_t hm = pc[0][0] | pc[0][1] << 16, lh = pc[0][2] | pc[0][0] << 16;
-        dst[0] = make_uint4(hm, hm, lh, 0);
+        const uint32_t hm = pc[0][0] | pc[0][1] << 16;
+        dst[0] = make_uint4(hm, hm, 0, 0);
     } else {
         auto pair = [&](uint32_t d, uint32_t t) { return pc[d][t] | pc[d + 1][t] << 16; };
         if constexpr (DL == 2) {
             dst[0] = make_uint4(pair(0, 0), pair(0, 0), pair(0, 1), pair(0, 1));
-            dst[64] = make_uint4(pair(0, 2), pair(0, 0), 0, 0);
         } else {
 #pragma unroll
-            for (uint32_t q = 0; q < DL / 4; ++q) {
-                const uint32_t a = 4 * q, b = 4 * q + 2;
-                dst[(3 * q + 0) * 64] = make_uint4(pair(a, 0), pair(a, 0), pair(b, 0), pair(b, 0));
-                dst[(3 * q + 1) * 64] = make_uint4(pair(a, 1), pair(a, 1), pair(b, 1), pair(b, 1));
-                dst[(3 * q + 2) * 64] = make_uint4(pair(a, 2), pair(a, 0), pair(b, 2), pair(b, 0));
+            for (uint32_t m = 0; m < NM; ++m) {
+                const uint32_t a = 4 * (m / 2), b = a + 2, t = m % 2;
+                dst[m * 64] = make_uint4(pair(a, t), pair(a, t), pair(b, t), pair(b, t));
             }
         }
     }
@@ -1271,7 +1269,10 @@ __global__ void ccs_prep_many_kernel(const float* __restrict__ cent, uint4* __re
         if (real) {
             cn = 0.0f;
 #pragma unroll
-            for (uint32_t t = 0; t < V; ++t) cn = fmaf(cp[t], cp[t], cn);
+            for (uint32_t t = 0; t < V; ++t) {
+                const float c = cp[t] * sc;
+                cn = fmaf(c, c, cn);
+            }
         }
         cn32[((size_t)cb * groups + grp) * 32 + 16 * h + r] = cn;
     }
@@ -1340,20 +1341,35 @@ struct CcsManyShape {
 template <int V, int IDX_BITS>
 __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* __restrict__ x, const float* __restrict__ cent,
                                                                   const uint4* __restrict__ aux, const float* __restrict__ cn32,
-                                                                  const float* __restrict__ cnmax, uint8_t* __restrict__ idx,
+                                                                  const float* __restrict__ cnmax, const float* __restrict__ scale,
+                                                                  uint8_t* __restrict__ idx,
                                                                   uint32_t N, uint32_t K, uint32_t CB, uint32_t C,
                                                                   uint32_t idx_row_bytes, int idx_tiled, int vec_ok, uint32_t tiles_cb)
 {
     using S = CcsManyShape<V>;
     constexpr int TG = S::TG, TT = S::TT, P = S::P, CBW = S::CBW, TF = S::TF, PITCH = S::PITCH;
     constexpr int DL = V / 2, NM = (int)ccs_many_nm(V);
-    constexpr int NB = V == 2 ? 1 : V <= 8 ? 2 : V / 4;  // activation operands of a token group
+    constexpr int NB = V <= 8 ? 1 : V / 8;               // activation operands of a token group
     __shared__ __attribute__((aligned(16))) float tile[TT * PITCH];
     __shared__ __attribute__((aligned(16))) uint8_t ist[TT * CBW];
     const uint32_t lane = threadIdx.x & 63, j = lane & 31, h = lane >> 5;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t tcb = blockIdx.x % tiles_cb, tok0 = blockIdx.x / tiles_cb * TT;
     const uint32_t groups = (C + 31) / 32;
+
+    // Operands of the group after the one being searched, of this codebook or the next (they follow each other in memory).
+    const uint32_t group0 = (tcb * CBW + wave * P) * groups, last_group = CB * groups - 1;
+    uint4 an[NM];
+    float4 cnn[4];
+    auto load = [&](uint32_t g) {
+        g = g < last_group ? g : last_group;
+        const uint4* ap = aux + (size_t)g * NM * 64 + lane;
+        const float* cnp = cn32 + (size_t)g * 32 + 16 * h;
+#pragma unroll
+        for (int m = 0; m < NM; ++m) an[m] = ap[m * 64];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) cnn[q] = *reinterpret_cast<const float4*>(cnp + 4 * q);
+    };
 
     {
         constexpr int F4 = TF / 4, ROWS = CCS_THREADS / F4, PASSES = TT / ROWS;
@@ -1382,6 +1398,7 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
 #pragma unroll
         for (int i = 0; i < PASSES; ++i) *reinterpret_cast<float4*>(&tile[(fr + i * ROWS) * PITCH + 4 * fq]) = pf[i];
     }
+    load(group0);
     __syncthreads();
 
 #pragma nounroll
@@ -1392,10 +1409,11 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
             for (int tg = 0; tg < TG; ++tg) ist[(32 * tg + j) * CBW + cbl] = 0;
             continue;
         }
-        // pieces of the lane's activations, x = xh + xm + xl exactly, and |x|^2
+        // pieces of the lane's activations and |x|^2, at the codebook's scale
         v4u bop[TG][NB];
-        float mag[TG];
-        const float cmax = cnmax[cb];
+        float sqs[TG];
+        const float sc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(scale[cb]))), cmax = cnmax[cb] * sc * sc;
+        const float c0 = fmaf(1.001e-6f * sc, sc, 2.5f * V * 5.9604645e-8f);  // see ccs_f16_kernel
 #pragma unroll
         for (int tg = 0; tg < TG; ++tg) {
             const float* src = tile + (32 * tg + j) * PITCH + cbl * V + DL * h;
@@ -1415,34 +1433,28 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
                     xs[4 * q + 3] = t4.w;
                 }
             }
-            uint32_t u0[DL], u1[DL], u2[DL];
+            if (sc != 1.0f) {
+#pragma unroll
+                for (int d = 0; d < DL; ++d) xs[d] *= sc;
+            }
             float sq = 0.0f;
 #pragma unroll
-            for (int d = 0; d < DL; ++d) {
-                u0[d] = __float_as_uint(xs[d]);
-                const float r1 = xs[d] - __uint_as_float(u0[d] & 0xffff0000u);
-                u1[d] = __float_as_uint(r1);
-                u2[d] = __float_as_uint(r1 - __uint_as_float(u1[d] & 0xffff0000u));
-                sq = d == 0 ? xs[d] * xs[d] : fmaf(xs[d], xs[d], sq);
-            }
-            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(sq), __float_as_uint(sq), false, false);
-            mag[tg] = __uint_as_float(sw[0]) + __uint_as_float(sw[1]) + cmax;
-            // __builtin_amdgcn_perm(p, q, 0x07060302) = (bf16 of q | bf16 of p << 16)
-            auto both = [](uint32_t q, uint32_t p) { return __builtin_amdgcn_perm(p, q, 0x07060302u); };
-            if constexpr (DL == 1) {
-                bop[tg][0] = v4u{both(u0[0], u0[0]), both(u1[0], u1[0]), both(u0[0], u2[0]), 0};
-            } else if constexpr (DL == 2) {
-                const uint32_t H = both(u0[0], u0[1]), M = both(u1[0], u1[1]), L = both(u2[0], u2[1]);
-                bop[tg][0] = v4u{H, M, H, M};
-                bop[tg][1] = v4u{H, L, H, L};
-            } else {
+            for (int d = 0; d < DL; ++d) sq = d == 0 ? xs[d] * xs[d] : fmaf(xs[d], xs[d], sq);
+            sqs[tg] = sq;
+            constexpr int R = DL == 1 ? 1 : DL / 2;
+            uint32_t H[R], M[R];
 #pragma unroll
-                for (int q = 0; q < DL / 4; ++q) {
-                    const int a = 4 * q, b = 4 * q + 2;
-                    const uint32_t H0 = both(u0[a], u0[a + 1]), H1 = both(u0[b], u0[b + 1]);
-                    bop[tg][2 * q] = v4u{H0, both(u1[a], u1[a + 1]), H1, both(u1[b], u1[b + 1])};
-                    bop[tg][2 * q + 1] = v4u{H0, both(u2[a], u2[a + 1]), H1, both(u2[b], u2[b + 1])};
-                }
+            for (int q = 0; q < R; ++q) {
+                const float a = xs[2 * q], b = xs[DL == 1 ? 0 : 2 * q + 1];
+                H[q] = half_pair(a, b);
+                const float ra = half_rest<false>(H[q], a), rb = DL == 1 ? ra : half_rest<true>(H[q], b);
+                M[q] = half_pair(ra, rb);
+            }
+            if constexpr (DL == 1) bop[tg][0] = v4u{H[0], M[0], 0, 0};
+            else if constexpr (DL == 2) bop[tg][0] = v4u{H[0], M[0], H[0], M[0]};
+            else {
+#pragma unroll
+                for (int q = 0; q < DL / 4; ++q) bop[tg][q] = v4u{H[2 * q], M[2 * q], H[2 * q + 1], M[2 * q + 1]};
             }
         }
         // smallest and second smallest tagged score of the lane's half of every group so far, the group of the smallest
@@ -1453,24 +1465,15 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
             m1[tg] = m2[tg] = 3.2e38f;
             grp[tg] = 0;
         }
-        const uint4* ap = aux + (size_t)cb * groups * NM * 64 + lane;
-        const float* cnp = cn32 + (size_t)cb * groups * 32 + 16 * h;
-        uint4 aq[NM], an[NM];
-        float4 cn[4], cnn[4];
-        auto load = [&](uint32_t g) {
-#pragma unroll
-            for (int m = 0; m < NM; ++m) an[m] = ap[((size_t)g * NM + m) * 64];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) cnn[q] = *reinterpret_cast<const float4*>(cnp + g * 32 + 4 * q);
-        };
-        load(0);
+        uint4 aq[NM];
+        float4 cn[4];
 #pragma nounroll
         for (uint32_t g = 0; g < groups; ++g) {
 #pragma unroll
             for (int m = 0; m < NM; ++m) aq[m] = an[m];
 #pragma unroll
             for (int q = 0; q < 4; ++q) cn[q] = cnn[q];
-            load(g + 1 < groups ? g + 1 : g);
+            load(cb * groups + g + 1);
             floatx16 start;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -1484,8 +1487,7 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
                 floatx16 acc = start;
 #pragma unroll
                 for (int m = 0; m < NM; ++m) {
-                    const int b = V <= 4 ? m : 2 * (m / 3) + (m % 3 == 2);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, aq[m]), __builtin_bit_cast(bf16x8, bop[tg][b]), acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, aq[m]), __builtin_bit_cast(f16x8, bop[tg][m / 2]), acc, 0, 0, 0);
                 }
                 float key[16];
 #pragma unroll
@@ -1505,37 +1507,38 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
                 m1[tg] = vmin(m1[tg], g1);
             }
         }
-        uint32_t fail = 0, found = 0;  // found: one byte per token group
+        // Lanes l and l ^ 32 hold the two halves of every group's centroids: half h decides token groups 2 q + h.
+        bool fail[TG / 2];
+        uint32_t found[TG / 2];
 #pragma unroll
-        for (int tg = 0; tg < TG; ++tg) {
-            // lanes l and l ^ 32 hold the two halves of every group: both merge them.  Equal tagged minima give
-            // second == smallest, which fails the margin test.
-            const auto s1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m1[tg]), __float_as_uint(m1[tg]), false, false);
-            const auto s2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(m2[tg]), __float_as_uint(m2[tg]), false, false);
-            const auto sg = __builtin_amdgcn_permlane32_swap(grp[tg], grp[tg], false, false);
+        for (int q = 0; q < TG / 2; ++q) {
+            auto swap = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_permlane32_swap(a, b, false, false); };
+            const auto s1 = swap(__float_as_uint(m1[2 * q]), __float_as_uint(m1[2 * q + 1])), s2 = swap(__float_as_uint(m2[2 * q]), __float_as_uint(m2[2 * q + 1]));
+            const auto sg = swap(grp[2 * q], grp[2 * q + 1]), sx = swap(__float_as_uint(sqs[2 * q]), __float_as_uint(sqs[2 * q + 1]));
+            const float mag = __uint_as_float(sx[0]) + __uint_as_float(sx[1]) + cmax;
+            // (equal tagged minima give second == smallest, which fails the margin test)
             const float lo1 = __uint_as_float(s1[0]), hi1 = __uint_as_float(s1[1]);
             const float best = vmin(lo1, hi1), second = vmin3(vmax(lo1, hi1), __uint_as_float(s2[0]), __uint_as_float(s2[1]));
             const bool up = hi1 < lo1;
-            found |= ((__float_as_uint(best) & 15u) + (up ? 16u : 0u) + 32u * (up ? sg[1] : sg[0])) << (8 * tg);
-            // 2 * [ (v+1)u (|c|^2) + 16u (omitted products) + 2.02 (6v + NM + 1) u (that many additions, each within u of a
+            found[q] = (__float_as_uint(best) & 15u) + (up ? 16u : 0u) + 32u * (up ? sg[1] : sg[0]);
+            // 2 * [ (v+1)u (|c|^2) + 12u (what the pieces leave) + 2.02 * 17 NM u (16 NM products and NM accumulators, each within u of a
             //       partial sum below 2.02 mag) + 2(v+2)u (the reference's own chain) ], and the tags
             // (What this takes for granted of the matrix core, launch_diag_mfma_error measures on chains of three instructions that
-            // start from any accumulator: v = 16 and 32 are two and four of them one after the other, whose errors add up.  The
-            // device stays below 25.5 u per chain, which makes 51 and 102 of the 208 and 414 u allowed here.)
-            constexpr float A2 = 2.0f * ((V + 1) + 16.0f + 2.02f * (6 * V + NM + 1) + 2 * (V + 2)) * 5.9604645e-8f;
+            // start from any accumulator: v = 16 and 32 are chains of four and eight, which three in a row cover, whose errors add up.  The
+            // device stays below 25.5 u per chain of three, which makes 51 and 76.5 of the 137 and 275 u allowed here.)
+            constexpr float A2 = 2.0f * ((V + 1) + 12.0f + 2.02f * (17 * NM) + 2 * (V + 2)) * 5.9604645e-8f;
             constexpr float B2 = 2.0f * 16.0f * 2.3841858e-7f;  // 2 * 2^(4-22)
-            const float thr = fmaf(A2, mag[tg], fmaf(B2, fabsf(second), 1.001e-6f));
-            // NaN anywhere makes a compare false, which counts as "not safe"
-            const bool safe = ((second - best) > thr) && (mag[tg] < 1e36f);
-            fail |= (safe ? 0u : 1u) << tg;
+            const float thr = fmaf(A2, mag, fmaf(B2, fabsf(second), c0));
+            // NaN anywhere makes a compare false, which counts as "not safe"; beyond 1e9 a half may have run out
+            fail[q] = !((second - best) > thr && mag < 1e9f);
         }
         // ---- exact replay of the tokens that failed the margin test (rare) ----
-        if (__builtin_amdgcn_ballot_w64(fail != 0) != 0) {
+        {
             const float* cp = cent + (size_t)cb * C * V;
 #pragma unroll
             for (int q = 0; q < TG / 2; ++q) {  // token groups 2 q and 2 q + 1: a half of the wave each
-                auto set = [&](uint32_t k) { found = (found & ~(255u << (8 * (2 * q + h)))) | k << (8 * (2 * q + h)); };
-                const bool mine = (fail >> (2 * q + h)) & 1u;
+                auto set = [&](uint32_t k) { found[q] = k; };
+                const bool mine = fail[q];
                 uint64_t mask = __builtin_amdgcn_ballot_w64(mine);
                 if (mask == 0) continue;
                 const uint32_t row = 64 * q + lane;  // the lane's token in the tile
@@ -1585,7 +1588,7 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
             }
         }
 #pragma unroll
-        for (int q = 0; q < TG / 2; ++q) ist[(64 * q + lane) * CBW + cbl] = (uint8_t)(found >> (8 * (2 * q + h)));
+        for (int q = 0; q < TG / 2; ++q) ist[(64 * q + lane) * CBW + cbl] = (uint8_t)found[q];
     }
     __syncthreads();
     for (uint32_t e = threadIdx.x; e < (uint32_t)(TT * P); e += CCS_THREADS) {  // four codebooks of a token
@@ -1857,15 +1860,15 @@ int launch_ccs_f16(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_
 {
     const uint64_t tiles128 = (uint64_t)((n + 127) / 128) * (g.CB_pad / CcsMfmaShape<V, WIDE>::RCB);
     // 64-token tiles up to two 128-token tiles per resident workgroup: the grid fills more evenly, and since a
-    // workgroup keeps the operands of its codebooks from tile to tile the extra tiles cost little (asking the
-    // compiler for four workgroups per CU with them was measured slower: 10.9 against 10.1 us at K = 768)
-    // (measured 64 / 128-token tiles, us: 6.1 / 8.7 at 192 tiles; 11.0 / 11.9 at 768; 14.8 / 15.5 at 1188;
-    // 17.8 / 18.8 at 1536; 28.2 .. 31.5 / 28.2 .. 29.0 at 3072; 42.3 / 41.8 at 4752)
-    // v = 8 with up to 16 centroids: the 128-token kernel (two workgroups per CU: 237 registers, 76 KB of LDS) beats
-    // the 64-token one (three per CU, with spills) from half a tile per CU upwards (us, 64 / 128: 6.5 / 7.0 at 96
-    // tiles, 8.3 / 7.0 at 192, 15.1 / 9.7 at 512, 26 / 24.5 at 1536, 35.7 / 33.5 at 2376)
-    const uint64_t few = (V == 8 && !WIDE) ? ctx->prop.multiProcessorCount / 2 : 6ull * ctx->prop.multiProcessorCount;
-    const bool small_tiles = g.tune_search_tile ? g.tune_search_tile == 64 : tiles128 <= few;
+    // workgroup keeps the operands of its codebooks from tile to tile the extra tiles cost little.
+    // us, 64 / 128-token tiles, v = 4, 16 centroids (three workgroups of either per CU): 4.7 / 5.6 at 192 tiles of 128, 6.2 / 6.8 at 384, 7.7 / 7.8
+    // and 7.8 / 8.1 at 768, 13.0 / 13.8 at 1536, 20.9 / 21.1 at 3072, 89 / 87 at 12288; 32 centroids 8.5 / 8.4 at 768, 11.8 / 12.2 at 1536, 20.2 / 19.7 at
+    // 3072.  v = 2, whose tiles hold little, goes over sooner: 4.6 / 5.9 at 96, 5.0 / 5.5 at 256, 6.6 / 6.6 at 512, 7.5 / 7.3 at 768, 8.2 / 7.9 at
+    // 1024, 11.0 / 10.2 at 1536; 32 centroids 6.9 / 7.7 at 512, 9.0 / 8.4 at 768, 12.5 / 11.2 at 1536.  v = 8 with up to 16 centroids does not: its
+    // 128-token kernel has two workgroups per CU (220 registers, 76 KB of LDS), 6.1 / 6.5 at 192, 7.2 / 7.9 at 384, 13.3 / 15.5 at 768, 34.2 / 36.4 at
+    // 3072, 79 / 81 at 6144.
+    const uint64_t cus = ctx->prop.multiProcessorCount;
+    const bool small_tiles = g.tune_search_tile ? g.tune_search_tile == 64 : (V == 8 && !WIDE) || tiles128 <= (V == 2 ? 5 * cus / 2 : 6 * cus);
     if (small_tiles) return launch_ccs_f16_tt<V, WIDE, 64>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
     return launch_ccs_f16_tt<V, WIDE, 128>(ctx, g, d_x, d_cent, d_idx, n, x_cols);
 }
@@ -1881,8 +1884,9 @@ int launch_ccs_many(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     const float* cnmax = d_cent + (size_t)g.CB * g.C * g.v + ccs_aux_floats(g);
     const float* many = d_cent + ccs_f16_offset(g);
     const float* cn32 = many + ccs_many_groups(g) * ccs_many_nm(V) * 64 * 4;
+    const float* scale = cn32 + ccs_many_groups(g) * 32;
     hipLaunchKernelGGL((ccs_many_kernel<V, IDX_BITS>), dim3((uint32_t)total), dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent,
-                       reinterpret_cast<const uint4*>(many), cn32, cnmax, d_idx, n, g.K, g.CB, g.C, g.idx_row_bytes,
+                       reinterpret_cast<const uint4*>(many), cn32, cnmax, scale, d_idx, n, g.K, g.CB, g.C, g.idx_row_bytes,
                        (int)g.idx_tiled, vec_ok, tiles_cb);
     return hip_check(ctx, hipGetLastError(), "ccs_many_kernel launch");
 }
@@ -2193,7 +2197,8 @@ int launch_ccs_prep(Ctx* ctx, const AmmGeom& g, float* d_cent)
         float* cn32 = many + ccs_many_groups(g) * ccs_many_nm(g.v) * 64 * 4;
         auto prep = g.v == 2 ? ccs_prep_many_kernel<2> : g.v == 4 ? ccs_prep_many_kernel<4> : g.v == 8 ? ccs_prep_many_kernel<8>
                   : g.v == 16 ? ccs_prep_many_kernel<16> : ccs_prep_many_kernel<32>;
-        hipLaunchKernelGGL(prep, dim3(g.CB, (g.C + 31) / 32), dim3(64), 0, ctx->stream, d_cent, reinterpret_cast<uint4*>(many), cn32, g.C);
+        hipLaunchKernelGGL(prep, dim3(g.CB, (g.C + 31) / 32), dim3(64), 0, ctx->stream, d_cent, cnmax, reinterpret_cast<uint4*>(many), cn32,
+                           cn32 + ccs_many_groups(g) * 32, g.C);
         rc = hip_check(ctx, hipGetLastError(), "ccs_prep_many_kernel launch");
     }
     if (rc || !ccs_has_f16(g)) return rc;

@@ -479,14 +479,16 @@ def test_search_with_a_few_near_ties_per_wave(ctx, v, C):
     amm.close()
 
 
-@pytest.mark.parametrize("v,C", [(2, 16), (4, 16), (8, 16), (4, 9), (2, 32), (4, 32), (8, 32), (4, 17)])
+@pytest.mark.parametrize("v,C", [(2, 16), (4, 16), (8, 16), (4, 9), (2, 32), (4, 32), (8, 32), (4, 17),
+                                 (2, 64), (4, 33), (8, 130), (16, 16), (32, 40)])
 @pytest.mark.parametrize("size", [1e-4, 0.03, 1.0, 900.0, 1100.0, 3e4, 1e9, 1e16])
 def test_search_over_the_range_of_halves(ctx, v, C, size):
     """The matrix search works on halves, whose range ends at 65504 and 6e-8: centroids and activations of one size from far below
     to far above it (tiles with centroids beyond 1024 are searched at a scale of their own), codebooks of another size beside them in
     the same and in other tiles, activations that no half holds, an odd width; every index against the reference's scan."""
     rng = np.random.default_rng(int(4000 + 10 * v + C))
-    N, CB = 210, 37
+    many = C > 32 or v > 8                             # the search by groups of 32 centroids; fewer tokens take another
+    N, CB = 1500 if many else 210, 37
     cent = rng.standard_normal((CB, C, v)).astype(np.float32)
     x = rng.standard_normal((N, CB, v)).astype(np.float32)
     cent[:20] *= np.float32(size)
@@ -497,7 +499,7 @@ def test_search_over_the_range_of_halves(ctx, v, C, size):
     x = x.reshape(N, CB * v)
     want = oracle.index_calculation(x, cent, v, threads=THREADS)
     amm = ctx.amm(cent, np.zeros((CB, C, 4), np.int8), np.float32(1.0), None, max_n=N)
-    for tile in (64, 128):
+    for tile in (0,) if many else (64, 128):
         amm.set_tuning(search_token_tile=tile)
         got = amm.index_calculation(x)
         assert np.array_equal(got, want), f"tile {tile}: {(got != want).sum()} of {got.size} differ"
