@@ -7,10 +7,9 @@
 //
 // One wave computes a 16-centroid x 64-column tile of one codebook with v_mfma_f32_16x16x4_f32
 // (K = 4 matches sub_vec_len 4 in one step; other v loop/zero-pad).  The work is tiny
-// (2*C*K*M flop) and the kernel is bound by reading W and writing the LUT once.  Every workgroup leaves the largest
-// magnitude it has written beside the table, and the workgroups of the quantisation reduce those.  768 -> 3072, 16
-// centroids: 29 us for both kernels; 93 with a pass of its own over the table for the magnitudes (57 us, an atomic per
-// wave) and one entry per thread in the quantisation (21 us).
+// (2*C*K*M flop) and the kernels are bound by reading W and writing the table once: the entries of an int8 table are computed twice, for
+// their largest magnitude and again to be quantised, and never stored as floats -- a call needs a fifth of the device memory, and 768 ->
+// 3072, 16 centroids takes 21 us of kernels instead of 29 (and 93 with a pass of its own over the table for the magnitudes).
 #include "pimdl_internal.h"
 
 namespace pimdl {
@@ -32,17 +31,39 @@ __device__ __forceinline__ float block_max(float m)
     return fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
 }
 
-// part [codebook][workgroups of a codebook]: the largest magnitude each workgroup wrote (here and below)
-__global__ __launch_bounds__(LG_WAVES * 64) void lutgen_f32_kernel(const float* __restrict__ cent,
-                                                                  const float* __restrict__ W,
-                                                                  float* __restrict__ lut, float* __restrict__ part,
-                                                                  uint32_t CB, uint32_t C, uint32_t v, uint32_t M)
+__device__ __forceinline__ int8_t quantise(float x, float scale)
 {
+    float t = __fdiv_rn(x, scale);
+    t = fminf(fmaxf(t, -128.0f), 127.0f);
+    return (int8_t)rintf(t);  // round half to even
+}
+
+// What a pass does with the entries that it computes
+enum LutPass {
+    LUT_STORE,     // float *out
+    LUT_LARGEST,   // part [codebook][workgroups of a codebook]: the largest magnitude of each workgroup
+    LUT_QUANTISE,  // int8 *out, with the scale of the codebook's group
+};
+struct LutOut {
+    void* out;
+    float* part;
+    const float* scales;
+    uint32_t group_cbs;  // codebooks per scale
+};
+
+// Lane (j, k) of a wave holds columns 4 j .. 4 j + 3 of its 64 (one per matrix instruction) of four centroids: whole 16-byte loads of W and
+// 64 bytes of a table row per store and 16 lanes.
+template <LutPass PASS>
+__global__ __launch_bounds__(LG_WAVES * 64) void lutgen_kernel(const float* __restrict__ cent, const float* __restrict__ W, LutOut o,
+                                                               uint32_t CB, uint32_t C, uint32_t v, uint32_t M)
+{
+    static_assert(LG_FT == 4, "four columns per lane");
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint32_t j = lane & 15, k = lane >> 4;
     const uint32_t cb = blockIdx.z;
     const uint32_t c0 = blockIdx.y * 16;
-    const uint32_t f0 = (blockIdx.x * LG_WAVES + wave) * (16 * LG_FT);
+    const uint32_t f0 = (blockIdx.x * LG_WAVES + wave) * (16 * LG_FT), f = f0 + 4 * j;
+    const bool whole = M % 4 == 0;  // (uniform) else rows are not aligned to 16 bytes
 
     v4f acc[LG_FT];
 #pragma unroll
@@ -53,31 +74,52 @@ __global__ __launch_bounds__(LG_WAVES * 64) void lutgen_f32_kernel(const float* 
         // A[i = centroid c0 + j][k = t]
         float a = 0.0f;
         if (c0 + j < C && t < v) a = cent[((size_t)cb * C + c0 + j) * v + t];
+        v4f b = (v4f){0.f, 0.f, 0.f, 0.f};
+        const float* w = W + ((size_t)cb * v + t) * M + f;
+        if (whole) {
+            if (t < v && f < M) b = *reinterpret_cast<const v4f*>(w);
+        } else {
 #pragma unroll
-        for (int ft = 0; ft < LG_FT; ++ft) {
-            const uint32_t f = f0 + ft * 16 + j;
-            float b = 0.0f;
-            if (t < v && f < M) b = W[((size_t)cb * v + t) * M + f];
-            acc[ft] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[ft], 0, 0, 0);
+            for (int ft = 0; ft < LG_FT; ++ft)
+                if (t < v && f + ft < M) b[ft] = w[ft];
         }
-    }
-    // D[i = 4*k + r][j]: centroid c0 + 4k + r, column f0 + ft*16 + j
-    float m = 0.0f;
 #pragma unroll
-    for (int ft = 0; ft < LG_FT; ++ft) {
-        const uint32_t f = f0 + ft * 16 + j;
-        if (f >= M) continue;
+        for (int ft = 0; ft < LG_FT; ++ft) acc[ft] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b[ft], acc[ft], 0, 0, 0);
+    }
+    // D[i = 4*k + r][j]: centroid c0 + 4k + r, column f0 + 4 j + ft
+    if constexpr (PASS == LUT_LARGEST) {
+        // (rows past C and columns past M are sums of zeros)
+        float m = 0.0f;
+#pragma unroll
+        for (int ft = 0; ft < LG_FT; ++ft)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) m = fmaxf(m, fabsf(acc[ft][r]));
+        m = block_max(m);
+        if (threadIdx.x == 0) o.part[((size_t)cb * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = m;
+    } else {
+        const float scale = PASS == LUT_QUANTISE ? o.scales[cb / o.group_cbs] : 0.0f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const uint32_t c = c0 + 4 * k + r;
-            if (c < C) {
-                lut[((size_t)cb * C + c) * M + f] = acc[ft][r];
-                m = fmaxf(m, fabsf(acc[ft][r]));
+            if (c >= C || f >= M) continue;
+            const size_t at = ((size_t)cb * C + c) * M + f;
+            if constexpr (PASS == LUT_STORE) {
+                float* out = static_cast<float*>(o.out) + at;
+                if (whole) *reinterpret_cast<v4f*>(out) = (v4f){acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
+                else
+#pragma unroll
+                    for (int ft = 0; ft < LG_FT; ++ft)
+                        if (f + ft < M) out[ft] = acc[ft][r];
+            } else {
+                int8_t* out = static_cast<int8_t*>(o.out) + at;
+                if (whole) *reinterpret_cast<char4*>(out) = make_char4(quantise(acc[0][r], scale), quantise(acc[1][r], scale), quantise(acc[2][r], scale), quantise(acc[3][r], scale));
+                else
+#pragma unroll
+                    for (int ft = 0; ft < LG_FT; ++ft)
+                        if (f + ft < M) out[ft] = quantise(acc[ft][r], scale);
             }
         }
     }
-    m = block_max(m);
-    if (threadIdx.x == 0) part[((size_t)cb * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = m;
 }
 
 // The same product with the v terms of every entry added in ascending order, each multiplication and each
@@ -85,59 +127,64 @@ __global__ __launch_bounds__(LG_WAVES * 64) void lutgen_f32_kernel(const float* 
 // on a CPU.  torch.bmm fixes no order (pim_weight_converter.py:86-90 leaves it to the library), so neither
 // form is "the" reference result; this one makes a converter's output reproducible bit for bit by scalar code.
 // One thread = one output column of one codebook, all C centroids: W is read once, the LUT written once.
-__global__ __launch_bounds__(256) void lutgen_ordered_kernel(const float* __restrict__ cent, const float* __restrict__ W,
-                                                           float* __restrict__ lut, float* __restrict__ part, uint32_t C,
-                                                           uint32_t v, uint32_t M)
+template <LutPass PASS>
+__global__ __launch_bounds__(256) void lutgen_ordered_kernel(const float* __restrict__ cent, const float* __restrict__ W, LutOut o,
+                                                           uint32_t C, uint32_t v, uint32_t M)
 {
     const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x, cb = blockIdx.y;
     const float* w = W + (size_t)cb * v * M + f;
+    const float scale = PASS == LUT_QUANTISE ? o.scales[cb / o.group_cbs] : 0.0f;
     float m = 0.0f;
     for (uint32_t c = 0; c < C && f < M; ++c) {
         const float* a = cent + ((size_t)cb * C + c) * v;
         float acc = 0.0f;
         for (uint32_t t = 0; t < v; ++t) acc = __fadd_rn(acc, __fmul_rn(a[t], w[(size_t)t * M]));
-        lut[((size_t)cb * C + c) * M + f] = acc;
-        m = fmaxf(m, fabsf(acc));
+        const size_t at = ((size_t)cb * C + c) * M + f;
+        if constexpr (PASS == LUT_STORE) static_cast<float*>(o.out)[at] = acc;
+        else if constexpr (PASS == LUT_QUANTISE) static_cast<int8_t*>(o.out)[at] = quantise(acc, scale);
+        else m = fmaxf(m, fabsf(acc));
     }
-    m = block_max(m);
-    if (threadIdx.x == 0) part[(size_t)cb * gridDim.x + blockIdx.x] = m;
+    if constexpr (PASS == LUT_LARGEST) {
+        m = block_max(m);
+        if (threadIdx.x == 0) o.part[(size_t)cb * gridDim.x + blockIdx.x] = m;
+    }
 }
 
-__device__ __forceinline__ int8_t quantise(float x, float scale)
+// A workgroup per group: its scale from the magnitudes of its codebooks' workgroups (parts per codebook).
+__global__ __launch_bounds__(256) void lut_scale_kernel(const float* __restrict__ part, float* __restrict__ scales, uint32_t group_cbs,
+                                                        uint32_t parts, uint32_t CB)
 {
-    float t = __fdiv_rn(x, scale);
-    t = fminf(fmaxf(t, -128.0f), 127.0f);
-    return (int8_t)rintf(t);  // round half to even
-}
-
-// Workgroup (x, g): a share of group g's entries.  Every workgroup reduces the group's magnitudes for itself (a few KB
-// from L2).  group_cbs codebooks per group, parts workgroups per codebook in `part`.
-__global__ __launch_bounds__(256) void quant_kernel(const float* __restrict__ lut, int8_t* __restrict__ q, const float* __restrict__ part,
-                                                    float* __restrict__ scales, uint32_t group_cbs, uint32_t parts, uint32_t CB,
-                                                    uint64_t cb_elems)
-{
-    const uint32_t grp = blockIdx.y, cb0 = grp * group_cbs, cb1 = cb0 + group_cbs < CB ? cb0 + group_cbs : CB;
-    float m = 0.0f;
-    for (uint64_t i = (uint64_t)cb0 * parts + threadIdx.x; i < (uint64_t)cb1 * parts; i += 256) m = fmaxf(m, part[i]);
-    float scale = __fdiv_rn(block_max(m), 127.0f);
+    const uint32_t grp = blockIdx.x, cb0 = grp * group_cbs, cb1 = CB - cb0 < group_cbs ? CB : cb0 + group_cbs;
+    float m[8] = {};
+    const uint64_t end = (uint64_t)cb1 * parts;
+    for (uint64_t i = (uint64_t)cb0 * parts + threadIdx.x; i < end; i += 8 * 256)
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (i + 256 * u < end) m[u] = fmaxf(m[u], part[i + 256 * u]);
+#pragma unroll
+    for (int u = 1; u < 8; ++u) m[0] = fmaxf(m[0], m[u]);
+    float scale = __fdiv_rn(block_max(m[0]), 127.0f);
     if (!(scale > 0.0f)) scale = 1.0f;  // all-zero group: any scale represents it
-    if (blockIdx.x == 0 && threadIdx.x == 0) scales[grp] = scale;
-    const uint64_t beg = cb0 * cb_elems, end = cb1 * cb_elems;
-    const uint64_t step = (uint64_t)gridDim.x * 256, first = (uint64_t)blockIdx.x * 256 + threadIdx.x;
-    uint64_t done = beg;
-    if (beg % 4 == 0) {  // four entries per thread; the last ones of a ragged group below
-        done = beg + (end - beg) / 4 * 4;
-        for (uint64_t i = beg + 4 * first; i < done; i += 4 * step) {
-            const float4 x = *reinterpret_cast<const float4*>(lut + i);
-            char4 o;
-            o.x = quantise(x.x, scale);
-            o.y = quantise(x.y, scale);
-            o.z = quantise(x.z, scale);
-            o.w = quantise(x.w, scale);
-            *reinterpret_cast<char4*>(q + i) = o;
-        }
+    if (threadIdx.x == 0) scales[grp] = scale;
+}
+
+// Pinned host memory to device memory or back (either side aligned to 16 bytes): the transfers of the ring in pimdl_capi.hip.  Four pieces of 16 bytes
+// per thread are under way together, which the link's latency asks for.
+__global__ __launch_bounds__(256) void ring_copy_kernel(const unsigned char* __restrict__ src, unsigned char* __restrict__ dst, uint64_t bytes)
+{
+    const uint4* s = reinterpret_cast<const uint4*>(src);
+    uint4* d = reinterpret_cast<uint4*>(dst);
+    const uint64_t n = bytes / 16, step = (uint64_t)gridDim.x * 256, first = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    for (uint64_t i = first; i < n; i += 4 * step) {
+        uint4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u * step < n) v[u] = s[i + u * step];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (i + u * step < n) d[i + u * step] = v[u];
     }
-    for (uint64_t i = done + first; i < end; i += step) q[i] = quantise(lut[i], scale);
+    for (uint64_t i = n * 16 + first; i < bytes; i += step) dst[i] = src[i];
 }
 
 // ---- diagnostics: a plain copy (HBM) and a ds_read_b128 loop (LDS) ------------------------------
@@ -177,28 +224,41 @@ uint32_t lutgen_parts(uint32_t C, uint32_t M, bool ordered)
     return ordered ? (M + 255) / 256 : (M + LG_WAVES * 16 * LG_FT - 1) / (LG_WAVES * 16 * LG_FT) * ((C + 15) / 16);
 }
 
-int launch_lutgen_f32(Ctx* ctx, const float* d_cent, const float* d_w, float* d_lut, float* d_part, uint32_t CB, uint32_t C,
-                      uint32_t v, uint32_t M, bool ordered)
+template <LutPass PASS>
+static int launch_pass(Ctx* ctx, const float* d_cent, const float* d_w, const LutOut& o, uint32_t CB, uint32_t C, uint32_t v, uint32_t M, bool ordered)
 {
     if (ordered) {
-        hipLaunchKernelGGL(lutgen_ordered_kernel, dim3((M + 255) / 256, CB), dim3(256), 0, ctx->stream, d_cent, d_w, d_lut, d_part, C, v, M);
+        hipLaunchKernelGGL(lutgen_ordered_kernel<PASS>, dim3((M + 255) / 256, CB), dim3(256), 0, ctx->stream, d_cent, d_w, o, C, v, M);
         return hip_check(ctx, hipGetLastError(), "lutgen_ordered_kernel launch");
     }
     dim3 grid((M + LG_WAVES * 16 * LG_FT - 1) / (LG_WAVES * 16 * LG_FT), (C + 15) / 16, CB);
-    hipLaunchKernelGGL(lutgen_f32_kernel, grid, dim3(LG_WAVES * 64), 0, ctx->stream, d_cent, d_w, d_lut, d_part, CB, C, v, M);
-    return hip_check(ctx, hipGetLastError(), "lutgen_f32_kernel launch");
+    hipLaunchKernelGGL(lutgen_kernel<PASS>, grid, dim3(LG_WAVES * 64), 0, ctx->stream, d_cent, d_w, o, CB, C, v, M);
+    return hip_check(ctx, hipGetLastError(), "lutgen_kernel launch");
 }
 
-int launch_lut_quant(Ctx* ctx, const float* d_lut, const float* d_part, uint32_t parts, int8_t* d_q, float* d_scales, uint32_t CB,
-                     uint32_t C, uint32_t M, uint32_t scale_group)
+int launch_lutgen_f32(Ctx* ctx, const float* d_cent, const float* d_w, float* d_lut, uint32_t CB, uint32_t C, uint32_t v, uint32_t M, bool ordered)
+{
+    return launch_pass<LUT_STORE>(ctx, d_cent, d_w, LutOut{d_lut, nullptr, nullptr, 1}, CB, C, v, M, ordered);
+}
+
+int launch_lutgen_i8(Ctx* ctx, const float* d_cent, const float* d_w, float* d_part, int8_t* d_q, float* d_scales, uint32_t CB, uint32_t C,
+                     uint32_t v, uint32_t M, uint32_t scale_group, bool ordered)
 {
     const uint32_t cbs = scale_group && scale_group < CB ? scale_group : CB, ngroups = (CB + cbs - 1) / cbs;
-    const uint64_t cb_elems = (uint64_t)C * M;
-    uint64_t bx = (cbs * cb_elems + 256 * 16 - 1) / (256 * 16);
-    if (bx > 2048) bx = 2048;
-    hipLaunchKernelGGL(quant_kernel, dim3((uint32_t)bx, ngroups), dim3(256), 0, ctx->stream, d_lut, d_q, d_part, d_scales, cbs, parts,
-                       CB, cb_elems);
-    return hip_check(ctx, hipGetLastError(), "quant_kernel launch");
+    const LutOut o{d_q, d_part, d_scales, cbs};
+    int rc = launch_pass<LUT_LARGEST>(ctx, d_cent, d_w, o, CB, C, v, M, ordered);
+    if (rc) return rc;
+    hipLaunchKernelGGL(lut_scale_kernel, dim3(ngroups), dim3(256), 0, ctx->stream, d_part, d_scales, cbs, lutgen_parts(C, M, ordered), CB);
+    if ((rc = hip_check(ctx, hipGetLastError(), "lut_scale_kernel launch"))) return rc;
+    return launch_pass<LUT_QUANTISE>(ctx, d_cent, d_w, o, CB, C, v, M, ordered);
+}
+
+int launch_ring_copy(Ctx* ctx, const void* src, void* dst, size_t bytes)
+{
+    const uint64_t wgs = (bytes + 256 * 64 - 1) / (256 * 64);
+    hipLaunchKernelGGL(ring_copy_kernel, dim3((uint32_t)(wgs < 128 ? wgs : 128)), dim3(256), 0, ctx->stream, static_cast<const unsigned char*>(src),
+                       static_cast<unsigned char*>(dst), (uint64_t)bytes);
+    return hip_check(ctx, hipGetLastError(), "ring_copy_kernel launch");
 }
 
 int launch_diag(Ctx* ctx, uint64_t bytes, float* copy_gbps, float* lds_gbps)

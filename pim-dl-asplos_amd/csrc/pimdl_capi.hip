@@ -369,66 +369,74 @@ static int run_piped(Ctx* ctx, uint32_t K, uint32_t M, const float* in, bool in_
     return PIMDL_OK;
 }
 
-// One host buffer to device memory and back through the ring's pinned slots, 2 MiB at a time, so that the host's copy of one
-// piece overlaps the transfer of another (a pageable transfer of the runtime's takes about 25 GB/s, this the link's 57).
-// Ordered against the context's stream.  ring_to_device returns once `src` has been read, ring_to_host once `dst` is
-// complete.  Small buffers, and pointers the CPU cannot read, take the runtime's copy.
-constexpr size_t RING_PIECE = 2u << 20;
+// Host buffers to device memory and back through the ring's pinned slots, so that the host's copy of one piece overlaps the transfer of
+// another.  The transfers are kernels on the context's stream: a piece costs a launch and an event.  (As the runtime's copies on a stream of
+// their own, a transfer back took 140 us on top of the link's time once it had to wait for a slot -- 67 MB 5.2 ms, now 1.3 --, and a
+// pageable copy of a few KB waits for the device besides.)  Pieces of 4 MiB; the first ones in and the last ones out are smaller, so that the
+// link starts early and little is left to copy when it is done.  Table construction, us a call, table in a buffer used before / a fresh one,
+// pieces of 2 MiB down to 256 KiB: 768 -> 3072 576 / 573, 1024 -> 4096 with 32 centroids 1288 / 2334; 4 MiB, 256 KiB 587 / 586, 1241 / 1763; 4 MiB, 1 MiB
+// 550 / 548, 1200 / 1723; 6 MiB, 512 KiB 590 / 587, 1224 / 1638.  ring_to_device returns once `src` has been read, ring_to_host once
+// the destinations are complete.  Pointers that the CPU cannot read take the runtime's copy.
+constexpr size_t RING_PIECE = 4u << 20, RING_FIRST = 1u << 20;
 
 static int ring_to_device(Ctx* ctx, void* dst, const void* src, size_t bytes)
 {
-    if (bytes < RING_PIECE / 4 || is_device_ptr(src))
-        return hip_check(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream), "H2D");
+    if (is_device_ptr(src)) return hip_check(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, ctx->stream), "copy to the device");
     HostPipe* hp;
     int rc = pipe_get(ctx, &hp);
     if (rc) return rc;
     rc = pipe_reserve(ctx, hp, RING_PIECE, 0);
-    // the destination is free once what the context's stream has queued is done
-    if (!rc) rc = hip_check(ctx, hipEventRecord(ctx->ev[2], ctx->stream), "hipEventRecord");
-    if (!rc) rc = hip_check(ctx, hipStreamWaitEvent(hp->s_in, ctx->ev[2], 0), "hipStreamWaitEvent");
     int s = 0;
-    for (size_t at = 0; at < bytes && !rc; at += RING_PIECE, s = (s + 1) % HostPipe::SLOTS) {
-        const size_t len = std::min(RING_PIECE, bytes - at);
+    size_t piece = RING_FIRST;
+    for (size_t at = 0, len; at < bytes && !rc; at += len, s = (s + 1) % HostPipe::SLOTS, piece = std::min(2 * piece, RING_PIECE)) {
+        len = std::min(piece, bytes - at);
         if (hp->used_in[s] && (rc = hip_check(ctx, hipEventSynchronize(hp->ev_in[s]), "hipEventSynchronize(staging in)"))) break;
         parallel_copy(hp->pin_in[s], static_cast<const char*>(src) + at, len);
-        if ((rc = hip_check(ctx, hipMemcpyAsync(static_cast<char*>(dst) + at, hp->pin_in[s], len, hipMemcpyHostToDevice, hp->s_in), "H2D piece"))) break;
-        if ((rc = hip_check(ctx, hipEventRecord(hp->ev_in[s], hp->s_in), "hipEventRecord"))) break;
+        if ((rc = launch_ring_copy(ctx, hp->pin_in[s], static_cast<char*>(dst) + at, len))) break;
+        if ((rc = hip_check(ctx, hipEventRecord(hp->ev_in[s], ctx->stream), "hipEventRecord"))) break;
         hp->used_in[s] = true;
-        if (at + len == bytes) rc = hip_check(ctx, hipStreamWaitEvent(ctx->stream, hp->ev_in[s], 0), "hipStreamWaitEvent");
     }
-    if (rc) (void)hipStreamSynchronize(hp->s_in);
     return rc;
 }
 
-static int ring_to_host(Ctx* ctx, void* dst, const void* src, size_t bytes)
+// `bytes` from src to dst, and `more` from src + more_at (past them) to more_dst
+static int ring_to_host(Ctx* ctx, void* dst, const void* src, size_t bytes, void* more_dst = nullptr, size_t more_at = 0, size_t more = 0)
 {
-    if (bytes < RING_PIECE / 4 || is_device_ptr(dst)) {
-        const int r = hip_check(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream), "D2H");
+    if (is_device_ptr(dst) || (more && is_device_ptr(more_dst))) {
+        int r = hip_check(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, ctx->stream), "copy from the device");
+        if (!r && more) r = hip_check(ctx, hipMemcpyAsync(more_dst, static_cast<const char*>(src) + more_at, more, hipMemcpyDefault, ctx->stream), "copy from the device");
         return r ? r : hip_check(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     }
     HostPipe* hp;
     int rc = pipe_get(ctx, &hp);
     if (rc) return rc;
     if ((rc = pipe_reserve(ctx, hp, 0, RING_PIECE))) return rc;
-    rc = hip_check(ctx, hipEventRecord(ctx->ev[2], ctx->stream), "hipEventRecord");
-    if (!rc) rc = hip_check(ctx, hipStreamWaitEvent(hp->s_out, ctx->ev[2], 0), "hipStreamWaitEvent");
-    const size_t pieces = (bytes + RING_PIECE - 1) / RING_PIECE;
-    constexpr size_t LAG = HostPipe::SLOTS;
-    for (size_t p = 0; p < pieces + LAG && !rc; ++p) {
-        if (p >= LAG) {  // piece p - LAG is copied out before its slot is used again
-            const size_t r = p - LAG, at = r * RING_PIECE;
-            if (r >= pieces) break;
-            if ((rc = hip_check(ctx, hipEventSynchronize(hp->ev_out[r % LAG]), "hipEventSynchronize(staging out)"))) break;
-            parallel_copy(static_cast<char*>(dst) + at, hp->pin_out[r % LAG], std::min(RING_PIECE, bytes - at));
-        }
-        if (p < pieces) {
-            const size_t at = p * RING_PIECE, s = p % LAG;
-            if ((rc = hip_check(ctx, hipMemcpyAsync(hp->pin_out[s], static_cast<const char*>(src) + at, std::min(RING_PIECE, bytes - at), hipMemcpyDeviceToHost, hp->s_out), "D2H piece"))) break;
-            if ((rc = hip_check(ctx, hipEventRecord(hp->ev_out[s], hp->s_out), "hipEventRecord"))) break;
+    const size_t total = more ? more_at + more : bytes;
+    constexpr size_t SLOTS = HostPipe::SLOTS;
+    size_t first[SLOTS], len[SLOTS];  // the pieces under way
+    size_t queued = 0, taken = 0, at = 0;
+    while (!rc && (at < total || taken < queued)) {
+        if (at < total && queued - taken < SLOTS) {
+            const size_t s = queued % SLOTS, left = total - at;
+            // half of what is left once that is less than two pieces, whole 16 bytes
+            len[s] = left <= RING_FIRST ? left : std::min(RING_PIECE, std::max(RING_FIRST, (left / 2 + 15) / 16 * 16));
+            first[s] = at;
+            at += len[s];
+            if ((rc = launch_ring_copy(ctx, static_cast<const char*>(src) + first[s], hp->pin_out[s], len[s]))) break;
+            if ((rc = hip_check(ctx, hipEventRecord(hp->ev_out[s], ctx->stream), "hipEventRecord"))) break;
             hp->used_out[s] = true;
+            ++queued;
+            continue;
         }
+        const size_t s = taken++ % SLOTS;
+        if ((rc = hip_check(ctx, hipEventSynchronize(hp->ev_out[s]), "hipEventSynchronize(staging out)"))) break;
+        auto take = [&](void* to, size_t beg, size_t end) {  // the part of the piece that lies in beg .. end of the source
+            const size_t lo = std::max(beg, first[s]), hi = std::min(end, first[s] + len[s]);
+            if (lo < hi) parallel_copy(static_cast<char*>(to) + (lo - beg), static_cast<const char*>(hp->pin_out[s]) + (lo - first[s]), hi - lo);
+        };
+        take(dst, 0, bytes);
+        if (more) take(more_dst, more_at, more_at + more);
     }
-    if (rc) (void)hipStreamSynchronize(hp->s_out);
     return rc;
 }
 
@@ -1422,11 +1430,11 @@ int pimdl_lutgen_mode(pimdl_ctx* ctx, const float* centroids, const float* weigh
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(ctx->stream, &cap) != hipSuccess) (void)hipGetLastError();
     if (cap != hipStreamCaptureStatusNone) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_lutgen: the stream is being captured; the call copies from and to host memory");
-    // One block of device memory for the call: centroids, weight, fp32 table, magnitudes, int8 table, scales.  Up to 256 MiB
+    // One block of device memory for the call: centroids, weight, then the fp32 table, or magnitudes, int8 table and scales.  Up to 256 MiB
     // the context keeps it (an allocation and a release cost as much as the kernels); larger ones are given back.
     auto up = [](size_t b) { return (b + 255) / 256 * 256; };
-    const size_t o_w = up(cent_bytes), o_lut = o_w + up(w_bytes), o_part = o_lut + up(lut_elems * 4),
-                 o_q = o_part + up((size_t)CB * parts * 4), o_scales = o_q + (i8 ? up(lut_elems) : 0), need = o_scales + up((size_t)ngroups * 4);
+    const size_t o_w = up(cent_bytes), o_lut = o_w + up(w_bytes), o_q = o_lut + up((size_t)CB * parts * 4), q_bytes = up(lut_elems),
+                 need = i8 ? o_q + q_bytes + up((size_t)ngroups * 4) : o_lut + up(lut_elems * 4);
     const bool kept = need <= (256u << 20);
     std::lock_guard<std::mutex> lock(ctx->host_mutex);
     char* dev = ctx->d_lutgen;
@@ -1442,19 +1450,17 @@ int pimdl_lutgen_mode(pimdl_ctx* ctx, const float* centroids, const float* weigh
             ctx->lutgen_bytes = need;
         }
     }
-    float *d_cent = reinterpret_cast<float*>(dev), *d_w = reinterpret_cast<float*>(dev + o_w), *d_lut = reinterpret_cast<float*>(dev + o_lut),
-          *d_part = reinterpret_cast<float*>(dev + o_part), *d_scales = reinterpret_cast<float*>(dev + o_scales);
-    int8_t* d_q = reinterpret_cast<int8_t*>(dev + o_q);
-    rc = hip_check(ctx, hipMemcpyAsync(d_cent, centroids, cent_bytes, hipMemcpyHostToDevice, ctx->stream), "H2D centroids");
+    float *d_cent = reinterpret_cast<float*>(dev), *d_w = reinterpret_cast<float*>(dev + o_w), *d_lut = reinterpret_cast<float*>(dev + o_lut);
+    rc = ring_to_device(ctx, d_cent, centroids, cent_bytes);
     if (!rc) rc = ring_to_device(ctx, d_w, weight, w_bytes);
-    if (!rc) rc = launch_lutgen_f32(ctx, d_cent, d_w, d_lut, d_part, CB, C, v, M, ordered);
-    if (!rc && i8) {
-        rc = launch_lut_quant(ctx, d_lut, d_part, parts, d_q, d_scales, CB, C, M, scale_group);
-        if (!rc) rc = hip_check(ctx, hipMemcpyAsync(scales_out, d_scales, sizeof(float) * ngroups, hipMemcpyDeviceToHost, ctx->stream), "D2H scales");
+    if (i8) {
+        if (!rc) rc = launch_lutgen_i8(ctx, d_cent, d_w, d_lut, reinterpret_cast<int8_t*>(dev + o_q), reinterpret_cast<float*>(dev + o_q + q_bytes), CB, C, v, M, scale_group, ordered);
+        if (!rc) rc = ring_to_host(ctx, lut_out, dev + o_q, lut_elems, scales_out, q_bytes, sizeof(float) * ngroups);
+    } else {
+        if (!rc) rc = launch_lutgen_f32(ctx, d_cent, d_w, d_lut, CB, C, v, M, ordered);
+        if (!rc) rc = ring_to_host(ctx, lut_out, d_lut, lut_elems * 4);
     }
-    if (!rc) rc = ring_to_host(ctx, lut_out, i8 ? static_cast<void*>(d_q) : d_lut, lut_elems * (i8 ? 1 : 4));
-    if (!rc) rc = hip_check(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-    else (void)hipStreamSynchronize(ctx->stream);
+    if (rc) (void)hipStreamSynchronize(ctx->stream);  // (else ring_to_host has waited for all of it; a wait for nothing takes 28 us)
     if (!kept) (void)hipFree(dev);
     return rc;
 }

@@ -180,12 +180,13 @@ int launch_pack_idx(Ctx* ctx, const AmmGeom& g, const uint16_t* d_idx16, uint8_t
 int launch_tile_idx(Ctx* ctx, const uint8_t* d_rows, uint8_t* d_tiled, uint32_t n, uint32_t row_bytes);
 int launch_retile_output(Ctx* ctx, const float* d_rowmajor, float* d_tiled, uint32_t n, uint32_t M,
                          uint32_t n_stile, uint32_t f_stile, uint32_t f_mtile);
-// part: [CB][lutgen_parts()] floats, the largest magnitude that each workgroup wrote
+int launch_lutgen_f32(Ctx* ctx, const float* d_cent, const float* d_w, float* d_lut, uint32_t CB, uint32_t C, uint32_t v, uint32_t M, bool ordered);
+// d_part: [CB][lutgen_parts()] floats of scratch, the largest magnitude of every workgroup's entries
 uint32_t lutgen_parts(uint32_t C, uint32_t M, bool ordered);
-int launch_lutgen_f32(Ctx* ctx, const float* d_cent, const float* d_w, float* d_lut, float* d_part, uint32_t CB,
-                      uint32_t C, uint32_t v, uint32_t M, bool ordered);
-int launch_lut_quant(Ctx* ctx, const float* d_lut, const float* d_part, uint32_t parts, int8_t* d_q, float* d_scales,
-                     uint32_t CB, uint32_t C, uint32_t M, uint32_t scale_group);
+int launch_lutgen_i8(Ctx* ctx, const float* d_cent, const float* d_w, float* d_part, int8_t* d_q, float* d_scales, uint32_t CB, uint32_t C,
+                     uint32_t v, uint32_t M, uint32_t scale_group, bool ordered);
+// pinned host memory to device memory or back, both aligned to 16 bytes
+int launch_ring_copy(Ctx* ctx, const void* src, void* dst, size_t bytes);
 int launch_layer_norm(Ctx* ctx, const float* d_x, const float* d_w, const float* d_b, const float* d_residual,
                       float* d_out, uint32_t n, uint32_t d, float eps);
 int launch_attention_hd64(Ctx* ctx, const float* d_q, const float* d_k, const float* d_v, float* d_out, uint32_t batch,

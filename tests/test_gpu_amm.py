@@ -786,6 +786,27 @@ def test_lutgen_quantisation_of_any_group(ctx, CB, v, C, M, group, ordered):
         assert np.array_equal(table[g * cbs:(g + 1) * cbs], np.rint(np.clip(part / s, -128, 127)).astype(np.int8))
 
 
+@pytest.mark.parametrize("CB,v,C,M,group", [(1, 2, 2, 3, 0), (64, 4, 256, 1024, 0), (130, 2, 40, 3001, 1), (61, 8, 33, 2083, 7), (256, 4, 64, 1028, 0)])
+def test_lutgen_through_several_pieces_of_the_ring(ctx, CB, v, C, M, group):
+    """Weights and tables from less than a piece of the pinned ring to more than its slots hold, whole and ragged pieces, rows that are and
+    that are no multiple of 16 bytes: the float table is the matrix product's (1e-5 of the root mean square: v products of N(0, 1) x
+    N(0, 0.02) in fp32), the int8 table and the scales are that table's to the bit, twice in a row through the same slots."""
+    rng = np.random.default_rng(CB * M)
+    cent = rng.standard_normal((CB, C, v)).astype(np.float32)
+    weight = (rng.standard_normal((CB * v, M)) * 0.02).astype(np.float32)
+    cbs = group or CB
+    for _ in range(2):
+        full, _ = ctx.lutgen(cent, weight, lut_dtype=pimdl.LUT_F32)
+        want = np.matmul(cent, weight.reshape(CB, v, M))
+        assert np.abs(full - want).max() <= 1e-5 * np.sqrt(np.mean(np.square(want, dtype=np.float64)))
+        table, scales = ctx.lutgen(cent, weight, scale_group=group)
+        for g in range((CB + cbs - 1) // cbs):
+            part = full[g * cbs:(g + 1) * cbs]
+            assert scales[g] == np.abs(part).max() / np.float32(127)
+            assert np.array_equal(table[g * cbs:(g + 1) * cbs], np.rint(np.clip(part / scales[g], -128, 127)).astype(np.int8))
+        cent = cent[::-1].copy()
+
+
 @pytest.mark.parametrize("N,CB,v,C,lut", [(9000, 1, 2, 256, "f32"), (5000, 2, 8, 100, "f32"), (700, 31, 4, 65, "i8"), (900, 33, 2, 130, "f32"),
                                           (300, 33, 16, 64, "i8"), (8200, 1, 4, 200, "i8"), (3, 70, 2, 40, "f32")])
 def test_search_of_few_pairs_writes_the_padding_too(ctx, N, CB, v, C, lut):
