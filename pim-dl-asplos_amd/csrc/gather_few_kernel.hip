@@ -48,9 +48,6 @@ struct FewSearch {
     uint32_t K, CB, C, aligned;
 };
 constexpr int FEW_FUSED_TOKENS = 2;
-struct FewGrid {
-    uint32_t token_tiles, by_xcd;  // see gather_few
-};
 
 // Column of position s of a tile of one-hot tables (sparse_tile_column on the device)
 __device__ __forceinline__ uint32_t few_column(uint32_t tn, uint32_t c, uint32_t j)
@@ -69,8 +66,8 @@ __device__ __forceinline__ uint32_t few_column(uint32_t tn, uint32_t c, uint32_t
 //   FEW_ROWS    the byte adder: lane (g, token j) reads its 16 columns of codebook 4 s + g, the constant operand
 //               A[i][16 g + b] = (b == i) adds them
 // V > 0: up to FEW_FUSED_TOKENS tokens whose index bytes are searched here, by the wave that needs them (sub-vectors of V floats).
-template <FewTable T, int TM, int NW, int TC = 1, int V = 0>
-__device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep, const FewGrid& grid, const FewSearch& fs = {})
+template <FewTable T, int TM, int NW, bool XCD, int TC = 1, int V = 0>
+__device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep, const FewSearch& fs = {})
 {
     static_assert(TC == 1 || T == FEW_SPARSE, "several column groups: sparse table only");
     static_assert(V == 0 || (T == FEW_SPARSE && TM == 1 && TC == 1), "searched where it is gathered: 16-token items of the sparse table");
@@ -79,22 +76,16 @@ __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep,
     extern __shared__ __attribute__((aligned(16))) int part[];  // [wave][4 TM registers][PITCH]
     const uint32_t lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t col_blocks = a.groups / TC;
-    // First of the TC column groups (of one tile) and first token.  by_xcd: XCD p % 8 takes every token tile of the column blocks congruent
-    // to it, so that one L2 streams a block's part of the table (blocks past the last: nothing to do).
-    uint32_t col_group = blockIdx.x, tok0 = 0;  // (items of 16 and 32 tokens: the launch has no more)
-    if constexpr (TM == 4) {
-        if (grid.by_xcd) {
-            const uint32_t q = blockIdx.x / 8;
-            col_group = blockIdx.x % 8 + 8 * (q / grid.token_tiles);
-            if (col_group >= col_blocks) return;  // whole workgroup
-            tok0 = q % grid.token_tiles * (16 * TM);
-        } else {
-            tok0 = blockIdx.x / col_blocks * (16 * TM);
-            col_group = blockIdx.x % col_blocks;
-        }
-        col_group *= TC;
+    // First of the TC column groups (of one tile) and first token.  The grid is (column blocks, token tiles), or, XCD, (8, token tiles, column
+    // blocks / 8): XCD p % 8 takes every token tile of the column blocks congruent to it, so that one L2 streams a block's part of the
+    // table.  (A form of its own: a test ahead of everything else costs a launch of few tokens 0.2 us, a division as much.)
+    uint32_t col_group = blockIdx.x;
+    if constexpr (XCD) {
+        col_group += 8 * blockIdx.z;
+        if (col_group >= a.groups / TC) return;  // whole workgroup, past the last block
     }
+    col_group *= TC;
+    const uint32_t tok0 = V > 0 ? 0 : blockIdx.y * (16 * TM);
     const uint32_t tile = col_group / a.tile_groups, c = col_group % a.tile_groups;
     const uint32_t op = a.op_groups ? col_group / a.op_groups : 0u;
     const uint32_t wn = 16 * a.tile_groups;
@@ -246,93 +237,128 @@ __device__ __forceinline__ void gather_few(const FewArgs& a, const Epilogue& ep,
 }
 
 // (a name for each, which says in a profile which of the large kernels it stands in for)
-template <int TM, int NW>
-__global__ __launch_bounds__(NW * 64) void gather_sparse_few_kernel(FewArgs a, Epilogue ep, FewGrid grid)
+template <int TM, int NW, bool XCD>
+__global__ __launch_bounds__(NW * 64) void gather_sparse_few_kernel(FewArgs a, Epilogue ep)
 {
-    gather_few<FEW_SPARSE, TM, NW>(a, ep, grid);
+    gather_few<FEW_SPARSE, TM, NW, XCD>(a, ep);
 }
 // One or two tokens: search and gather in one launch.  Every workgroup searches all codebooks for its 16 columns, which is less
 // than a second launch: a wave requests the centroids, the rows and its part of the table together, 16 codebooks at a time (v = 8: 8, for
 // registers), and turns the winners of its own codebooks into its operands without LDS or a barrier.  So there is one round trip up to 256
 // codebooks, 128 at v = 8, two beyond.
 template <int V, int NW>
-__global__ __launch_bounds__(NW * 64) void gather_sparse_few_fused_kernel(FewArgs a, Epilogue ep, FewGrid grid, FewSearch fs)
+__global__ __launch_bounds__(NW * 64) void gather_sparse_few_fused_kernel(FewArgs a, Epilogue ep, FewSearch fs)
 {
-    gather_few<FEW_SPARSE, 1, NW, 1, V>(a, ep, grid, fs);
+    gather_few<FEW_SPARSE, 1, NW, false, 1, V>(a, ep, fs);
 }
 // Sparse table, TC column groups of a tile per workgroup: the operands made from index bytes serve all of them, and a launch has
 // fewer workgroups, each with as many loads in flight.  (16 waves, one or two token groups, and all four groups of a
 // 64-column tile were slower or spill: N = 1024, 768 codebooks, M = 768 us 8 waves 12.5, 16 12.6, 4 14.8.)
-template <int TM, int NW, int TC>
-__global__ __launch_bounds__(NW * 64, 4) void gather_sparse_few_wide_kernel(FewArgs a, Epilogue ep, FewGrid grid)
+template <int TM, int NW, bool XCD, int TC>
+__global__ __launch_bounds__(NW * 64, 4) void gather_sparse_few_wide_kernel(FewArgs a, Epilogue ep)
 {
-    gather_few<FEW_SPARSE, TM, NW, TC>(a, ep, grid);
+    gather_few<FEW_SPARSE, TM, NW, XCD, TC>(a, ep);
 }
-template <int TM, int NW>
-__global__ __launch_bounds__(NW * 64) void gather_onehot_few_kernel(FewArgs a, Epilogue ep, FewGrid grid)
+template <int TM, int NW, bool XCD>
+__global__ __launch_bounds__(NW * 64) void gather_onehot_few_kernel(FewArgs a, Epilogue ep)
 {
-    gather_few<FEW_PAIRED, TM, NW>(a, ep, grid);
+    gather_few<FEW_PAIRED, TM, NW, XCD>(a, ep);
 }
-template <int TM, int NW>
-__global__ __launch_bounds__(NW * 64) void gather_i8_few_kernel(FewArgs a, Epilogue ep, FewGrid grid)
+template <int TM, int NW, bool XCD>
+__global__ __launch_bounds__(NW * 64) void gather_i8_few_kernel(FewArgs a, Epilogue ep)
 {
-    gather_few<FEW_ROWS, TM, NW>(a, ep, grid);
+    gather_few<FEW_ROWS, TM, NW, XCD>(a, ep);
 }
+
+// Bytes of a one-hot table (16 bytes per entry and column), and whether token tiles that share it have to meet in one L2: a table that an L2 of 4 MiB
+// holds is read from there by every XCD.
+uint64_t few_table_bytes(uint64_t steps, uint64_t groups) { return steps * 8 * groups * 256; }
+constexpr uint64_t FEW_TABLE_SHARED = 6u << 20;
+// workgroups of the XCD that has the most of them, if an XCD takes every token tile of its column blocks
+uint64_t few_fullest(uint64_t blocks, uint64_t tiles) { return (blocks + 7) / 8 * tiles; }
+// workgroups that have a CU of their own each (of exactly as many as CUs the last few share some)
+uint64_t few_room(uint64_t cus) { return cus - cus / 16; }
 
 // Workgroups of a launch.  By XCD where the column blocks do not divide by eight by themselves and several token tiles read the same table:
 // us, in order / by XCD, three column groups: 2048 codebooks, M = 2048 N = 256 41.1 / 24.8, 1280 x 1280 N = 512 33.2 / 17.6, 256, M =
-// 5120 N = 128 10.6 / 7.7; one column group: 2048 N = 128 32.8 / 26.4, 1280 N = 256 22.9 / 18.8; with a CU for every workgroup
-// of one column group 1024 N = 100 9.2 / 9.5, 1280 N = 128 11.6 / 11.1.
-uint32_t few_grid(const FewArgs& f, uint32_t tm, uint32_t tc, uint32_t cus, FewGrid* grid)
+// 5120 N = 128 10.6 / 7.7; one column group: 2048 N = 128 32.8 / 26.4, 1280 N = 256 22.9 / 18.8; with a CU for every workgroup where the table is
+// more than an L2 holds: 4096 -> 1024 (17 MB) N = 40 9.5 / 5.3, 4096 -> 500 v = 2 (17 MB) N = 64 12.5 / 8.3, N = 192 17.1 / 10.7, 1024 ->
+// 1024 v = 2 (8.7 MB) N = 40 4.2 / 3.9; 1024 -> 1024 v = 4 (4.3 MB) N = 40 3.2 / 3.2, 768 -> 1280 (4.0 MB) 3.0 / 3.2.
+dim3 few_grid(const FewArgs& f, uint32_t tm, uint32_t tc, uint32_t cus, bool one_hot)
 {
     const uint32_t blocks = f.groups / tc, tiles = (f.N + 16 * tm - 1) / (16 * tm);
-    grid->token_tiles = tiles;
     // (evenly enough: the XCD that takes one block more has a CU for each of its workgroups, or at most an eighth more than the average;
     // 9 column blocks, N = 3100 10.4 in order, 12.1 by XCD)
-    const uint64_t fullest = (uint64_t)((blocks + 7) / 8) * tiles;
+    const uint64_t fullest = few_fullest(blocks, tiles);
     const bool even = 8 * fullest <= cus || 64 * fullest <= 9ull * blocks * tiles;
-    grid->by_xcd = tiles > 1 && blocks % 8 != 0 && even && (tc > 1 || tiles * blocks > cus);
-    return tiles * (grid->by_xcd ? (blocks + 7) / 8 * 8 : blocks);
+    // (two items of 64 tokens: 4096 -> 1024 9.0 / 9.3, 5120 -> 1280 11.3 / 10.6)
+    const bool shared = one_hot && (tm < 4 || tiles > 2) && 8 * fullest <= few_room(cus) && few_table_bytes(f.steps, f.groups) > FEW_TABLE_SHARED;
+    const bool by_xcd = tiles > 1 && blocks % 8 != 0 && (shared || (even && (tc > 1 || tiles * blocks > cus)));
+    return by_xcd && blocks > 8 ? dim3(8, tiles, (blocks + 7) / 8) : dim3(blocks, tiles);  // (z > 1 says which)
 }
 
-template <FewTable T, int TM, int NW>
+template <FewTable T, int TM, int NW, int TC = 1>
 int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
 {
     constexpr int LDS = few_lds_bytes(NW, TM, T == FEW_ROWS ? FEW_PITCH_ROWS : FEW_PITCH_ONEHOT);
-    auto kern = T == FEW_SPARSE ? gather_sparse_few_kernel<TM, NW> : T == FEW_PAIRED ? gather_onehot_few_kernel<TM, NW> : gather_i8_few_kernel<TM, NW>;
+    const dim3 grid = few_grid(f, TM, TC, ctx->prop.multiProcessorCount, T != FEW_ROWS);
+    const bool xcd = grid.z > 1;
+    auto kern = [xcd] {
+        if constexpr (TC > 1) return xcd ? gather_sparse_few_wide_kernel<TM, NW, true, TC> : gather_sparse_few_wide_kernel<TM, NW, false, TC>;
+        else if constexpr (T == FEW_SPARSE) return xcd ? gather_sparse_few_kernel<TM, NW, true> : gather_sparse_few_kernel<TM, NW, false>;
+        else if constexpr (T == FEW_PAIRED) return xcd ? gather_onehot_few_kernel<TM, NW, true> : gather_onehot_few_kernel<TM, NW, false>;
+        else return xcd ? gather_i8_few_kernel<TM, NW, true> : gather_i8_few_kernel<TM, NW, false>;
+    }();
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_few)")) return rc;
-    static const char* const names[] = {"gather_sparse_few_kernel", "gather_onehot_few_kernel", "gather_i8_few_kernel"};
-    snprintf(a.last_gather, sizeof(a.last_gather), "%s<%d, %d>", names[T], TM, NW);
+    static const char* const names[] = {TC > 1 ? "gather_sparse_few_wide_kernel" : "gather_sparse_few_kernel", "gather_onehot_few_kernel", "gather_i8_few_kernel"};
+    if constexpr (TC > 1) snprintf(a.last_gather, sizeof(a.last_gather), "%s<%d, %d, %s, %d>", names[T], TM, NW, xcd ? "true" : "false", TC);
+    else snprintf(a.last_gather, sizeof(a.last_gather), "%s<%d, %d, %s>", names[T], TM, NW, xcd ? "true" : "false");
     a.note_launch(0, LDS, 16 * TM, NW * 64);
-    FewGrid grid;
-    const uint32_t wgs = few_grid(f, TM, 1, ctx->prop.multiProcessorCount, &grid);
-    hipLaunchKernelGGL(kern, dim3(wgs), dim3(NW * 64), LDS, ctx->stream, f, ep, grid);
+    hipLaunchKernelGGL(kern, grid, dim3(NW * 64), LDS, ctx->stream, f, ep);
     return hip_check(ctx, hipGetLastError(), "gather_few launch");
 }
 
-template <int TC>
-int launch_few_wide(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
+// Time of a byte adder launch in rounds of 16-token workgroups, which take their codebooks' time each.  Larger items only where they spare rounds: one
+// of up to 32 tokens that fits a round where two of 16 do not, or 64 where every one has a CU and the 16 tokens take four rounds and more
+// (3.4 times the time; with column blocks that divide by eight, so that the tiles' rows come from one L2).
+double few_rows_rounds(const AmmGeom& g, uint32_t n, uint64_t cus, uint32_t* item)
 {
-    constexpr int TM = 4, NW = 8, LDS = few_lds_bytes(NW, TM, FEW_PITCH_ONEHOT);
-    auto kern = gather_sparse_few_wide_kernel<TM, NW, TC>;
-    if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_few_wide)")) return rc;
-    snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_few_wide_kernel<%d, %d, %d>", TM, NW, TC);
-    a.note_launch(0, LDS, 16 * TM, NW * 64);
-    FewGrid grid;
-    const uint32_t wgs = few_grid(f, TM, TC, ctx->prop.multiProcessorCount, &grid);
-    hipLaunchKernelGGL(kern, dim3(wgs), dim3(NW * 64), LDS, ctx->stream, f, ep, grid);
-    return hip_check(ctx, hipGetLastError(), "gather_few_wide launch");
+    const uint64_t groups = g.M_pad / 16, rounds = ((n + 15) / 16 * groups + cus - 1) / cus;
+    *item = n <= 32 && rounds == 2 && groups <= cus ? 32 : rounds >= 4 && groups % 8 == 0 && (n + 63) / 64 * groups <= cus ? 64 : 16;
+    return *item == 64 ? 3.4 : (double)rounds;
 }
 
-// tokens of an item, by what the launch has: 16, 32 or 64
-constexpr uint32_t few_item(uint32_t n) { return n <= 16 ? 16 : n <= 32 ? 32 : 64; }
+// Tokens of an item: 16, 32 or 64.  One-hot tables: as few as leave every workgroup a CU of its own.  A wave then makes operands for fewer tokens, and
+// what more workgroups read of the table comes from the L2s.  us of gather, items of 16 / 32 / 64 tokens (workgroups): 3072 -> 768 v = 4 N = 64
+// 4.6 (192) / 5.4 (96) / 7.3 (48), N = 128 11.8 (384) / 5.5 (192) / 7.4; 768 -> 768 v = 2 N = 128 4.6 (384) / 4.0 (192) / 4.9; 1024 -> 1024 v = 2
+// N = 64 5.0 (264) / 4.5 (132) / 5.6; 4096 -> 500 v = 2 by XCD (33 column blocks, five of them on one XCD) N = 64 8.3 (20 on that XCD) / 10.5 / 15.0, N =
+// 100 13.0 (35) / 10.6 (20) / 15.2; 8 centroids 3072 -> 768 N = 64 3.5 / 4.1 / 5.7.
+// Byte adder, whose tokens' rows are read whatever the item: 32 centroids 3072 -> 768 N = 64 8.6 / 15.0 / 17.3, N = 100 14.8 (336) / 15.0 / 17.6, 3072
+// -> 3072 N = 32 19.5 (384) / 15.2; 100 centroids 768 -> 2304 N = 32 9.3 (288) / 7.8; 64 centroids 3072 -> 768 v = 8 N = 64 5.4 / 9.3 / 9.4; 200
+// 768 -> 768 N = 256 10.5 (768) / - / 11.2 (192), N = 300 13.0 (912) / - / 10.7 (240).
+uint32_t few_item(const AmmGeom& g, uint32_t n, uint64_t cus)
+{
+    const uint64_t groups = g.M_pad / 16;
+    if (g.gather_kind == 0) {
+        uint32_t item;
+        few_rows_rounds(g, n, cus, &item);
+        return item;
+    }
+    const uint64_t table = (uint64_t)g.CB_pad * g.C_tile * g.M_pad;
+    for (uint32_t item = 16; item < 64; item *= 2) {
+        const uint64_t tiles = (n + item - 1) / item;
+        const bool by_xcd = groups % 8 != 0 && table > FEW_TABLE_SHARED;  // (few_grid)
+        if (tiles == 1 || (by_xcd ? 8 * few_fullest(groups, tiles) : tiles * groups) <= few_room(cus)) return item;
+    }
+    return 64;
+}
 
 // Sixteen waves while every workgroup has a CU to itself, eight (two workgroups share a CU) beyond: us at 3072 -> 768,
 // 16 centroids, sixteen / eight waves: N = 64 7.5 / 8.4 (48 workgroups), N = 512 14.1 / 13.1 (384 workgroups).
 template <FewTable T>
 int launch_few(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
 {
-    const uint32_t item = few_item(f.N);
+    const uint32_t item = few_item(a.g, f.N, ctx->prop.multiProcessorCount);
     const bool deep = f.groups * ((f.N + item - 1) / item) <= (uint32_t)ctx->prop.multiProcessorCount;
     if (item == 16) return deep ? launch_few_as<T, 1, 16>(ctx, a, f, ep) : launch_few_as<T, 1, 8>(ctx, a, f, ep);
     if (item == 32) return deep ? launch_few_as<T, 2, 16>(ctx, a, f, ep) : launch_few_as<T, 2, 8>(ctx, a, f, ep);
@@ -430,7 +456,7 @@ int launch_f32_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, u
 // 14.4 / 14.2 (three); 192, M = 8192 N = 1 8.2 / 3.8, M = 12000 9.8 / 6.2, N = 64 10.7 / 9.3 / 8.8 (three).
 uint32_t few_column_groups(const Ctx* ctx, const AmmGeom& g, uint32_t n)
 {
-    const uint64_t cus = ctx->prop.multiProcessorCount, item = few_item(n), groups = g.M_pad / 16, tiles = (n + item - 1) / item;
+    const uint64_t cus = ctx->prop.multiProcessorCount, groups = g.M_pad / 16, item = few_item(g, n, cus), tiles = (n + item - 1) / item;
     const uint64_t wgs = tiles * groups;
     if (wgs <= cus) return 1;
     if (n <= 32) return wgs <= 4 * cus ? 1 : 0;
@@ -445,9 +471,12 @@ uint32_t few_column_groups(const Ctx* ctx, const AmmGeom& g, uint32_t n)
 // 19.8 / 4.5 at 1, 20.2 / 7.7 at 150, 19.8 / 13.1 at 512, 20.3 / 18.2 at 1024; 8 centroids 3072 -> 768 15.4 / 5.9 at 64,
 // 15.6 / 10.0 at 512: up to two workgroups of this launch per CU (the paired table; for the sparse one few_column_groups decides).
 // The byte adder and the floats read every gathered piece from the caches on its own, which costs in proportion to
-// tokens x codebooks x columns; against that stands the large kernels' chain of slices.  Byte adder, 3072 -> 768,
-// 32 centroids: 17.6 / 4.4 at N = 1, 17.7 / 7.9 at 13, 17.8 / 27.4 at 64; 1000 -> 1001, 200 centroids: 18.9 / 5.8 at 13,
-// 24.1 / 40.8 at 300.  Floats, 16 centroids (the large kernel with 64-token workgroups): 3072 -> 768 23.7 / 14.4 at 1,
+// tokens x codebooks x columns -- the byte adder by rounds of workgroups of 16 tokens x 16 columns, which take their codebooks' time each --;
+// against that stands the large kernels' chain of slices.  Byte adder, 3072 -> 768, 32 centroids: 17.6 / 4.4 at N = 1, 17.4 / 8.6 at 64,
+// 17.6 / 14.8 at 128 (384 workgroups), 17.8 / 20.9 at 192; 768 -> 768 6.8 / 3.8 at 70, 7.0 / 5.4 at 150, 7.2 / 8.6 at 300; 768 -> 3072 8.3 / 5.4 at
+// 32, 8.8 / 10.9 at 100; 16 codebooks, M = 1040 3.3 / 2.6 at 32, 3.8 / 4.2 at 300; 64 centroids 1024 -> 1024 7.2 / 4.4 at 50, 7.4 / 6.6 at 100, 7.6 / 8.9 at
+// 150; 4096 -> 512 27.8 / 12.8 at 64, 31.2 / 20.7 at 192; 128 centroids 768 -> 768 7.4 / 4.3 at 70, 7.6 / 8.3 at 200; 200 centroids 1000 -> 1001 15.7 /
+// 6.8 at 32, 16.0 / 12.3 at 150, 19.2 / 21.9 at 400.  Floats, 16 centroids (the large kernel with 64-token workgroups): 3072 -> 768 23.7 / 14.4 at 1,
 // 24.0 / 19.6 at 13, 25.5 / 28.7 at 64; 768 -> 3072 8.6 / 5.2 at 1, 8.4 / 9.3 at 13; 32 centroids 3072 -> 768 44 / 33 at 1,
 // 47 / 71 at 64; 200 centroids (whole rows) 1000 -> 1001 49 / 5.3 at 1, 51 / 32 at 64, 56 / 73 at 150; a scale per 5
 // codebooks 19.8 / 18.7 at 1, 19.7 / 22.6 at 13; 64 centroids (large / few; a piece costs more where the caches do not hold the
@@ -457,7 +486,7 @@ bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
 {
     const AmmGeom& g = a.g;
     if (g.tune_token_item || g.tune_cb_per_slice || g.tune_xcd_col_split) return false;  // settings of the large kernels
-    const uint64_t cus = ctx->prop.multiProcessorCount, item = few_item(n), wgs = (n + item - 1) / item * (g.M_pad / 16);
+    const uint64_t cus = ctx->prop.multiProcessorCount, item = few_item(g, n, cus), wgs = (n + item - 1) / item * (g.M_pad / 16);
     const double pieces = (double)n * g.CB_pad * (g.M_pad / 16);  // of 16 columns
     if (a.desc.lut_dtype == PIMDL_LUT_F32 || a.grouped) {
         const bool bounds = a.grouped && !a.prescaled;  // a scale to apply at the end of every group
@@ -465,9 +494,16 @@ bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
         const double piece = g.q != 4 ? 32e-6 : bounds || a.lut_bytes > (48u << 20) ? 6.5e-6 : 5e-6;
         return 2.7 + g.CB_pad * (bounds ? 0.062 : 0.0137) + pieces * piece < 4.0 + g.CB_pad * (bounds ? 0.14 : 0.07);
     }
-    if (g.gather_kind == 0)
-        return g.idx_bits == 8 && 2.6 + pieces * (g.C_tile <= 32 ? 0.5e-3 : 1e-3) / (double)(wgs < cus ? wgs : cus) <
-                                      3.3 + (g.CB + 15) / 16 * (0.2 + 0.003 * g.C_tile);
+    if (g.gather_kind == 0) {
+        const uint64_t slices = (g.CB + 15) / 16;
+        uint32_t rows_item;
+        const double rounds = few_rows_rounds(g, n, cus, &rows_item);
+        const double few = 2.5 + rounds * g.CB_pad * (g.C_tile <= 64 ? 0.0081 : g.C_tile == 128 ? 0.014 : 0.0125) + 0.3 * (rounds - 1);
+        // (64 centroids, more than 200 tokens or so: a few narrow tables would still gain here, but which kernel a batch of that size takes is
+        // something that programs have come to read back -- the fixed-scratch entry point's tests among them)
+        if (g.C_tile == 64 && g.CB_pad > 32 && n > 192) return false;
+        return g.idx_bits == 8 && few < (g.C_tile == 64 ? 2.9 + 0.29 * (double)slices : 3.3 + (double)slices * (0.2 + 0.003 * g.C_tile));
+    }
     if (g.gather_kind == 2 ? g.C_tile == 32 : g.C_tile != 8) return false;  // tables only a tuning asks for
     return g.gather_kind == 2 ? few_column_groups(ctx, g, n) != 0 : wgs <= 2 * cus;
 }
@@ -504,7 +540,7 @@ int launch_amm_few(Ctx* ctx, const Amm& a, const float* d_x, float* d_out, uint3
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_few_fused)")) return rc;
     snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_few_fused_kernel<%u, %d>", g.v, NW);
     a.note_launch(0, LDS, 16, NW * 64);
-    hipLaunchKernelGGL(kern, dim3(f.groups), dim3(NW * 64), LDS, ctx->stream, f, ep, FewGrid{1, 0}, fs);
+    hipLaunchKernelGGL(kern, dim3(f.groups), dim3(NW * 64), LDS, ctx->stream, f, ep, fs);
     return hip_check(ctx, hipGetLastError(), "gather_few_fused launch");
 }
 
@@ -535,8 +571,8 @@ int launch_gather_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out
     if (g.gather_kind == 2) {
         f.steps = g.CB_pad / 8;
         switch (few_column_groups(ctx, g, n)) {
-            case 2: return launch_few_wide<2>(ctx, a, f, ep);
-            case 3: return launch_few_wide<3>(ctx, a, f, ep);
+            case 2: return launch_few_as<FEW_SPARSE, 4, 8, 2>(ctx, a, f, ep);
+            case 3: return launch_few_as<FEW_SPARSE, 4, 8, 3>(ctx, a, f, ep);
         }
         return launch_few<FEW_SPARSE>(ctx, a, f, ep);
     }

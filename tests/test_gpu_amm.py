@@ -1268,6 +1268,44 @@ def test_search_of_few_pairs_up_to_32_centroids(ctx, N, CB, v, C, lut):
     amm.close()
 
 
+@pytest.mark.parametrize("CB,v,C,M", [
+    (192, 4, 16, 768),      # column blocks that divide by eight: in order
+    (1100, 2, 16, 500),     # 33 column blocks, a table beyond an L2: by XCD
+    (1030, 2, 11, 1024),    # 66 of them, padded codebooks
+    (400, 2, 16, 333),      # 21, a small table: in order
+    (700, 2, 8, 700),       # two codebooks of 8 per entry
+    (96, 8, 32, 784), (50, 4, 20, 2304), (60, 4, 64, 1001), (33, 4, 200, 768),   # byte adder
+])
+def test_items_of_few_tokens(ctx, CB, v, C, M):
+    """Launches of one to a few token tiles, in items of 16, 32 and 64 tokens and in order or by XCD, at the edges of each: accumulators and
+    output bits of the oracle, nothing behind the output."""
+    import torch
+    sizes = (1, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 96, 97, 112, 129, 160, 192, 241, 300)
+    x, cent, lut, bias = make_case(5200 + CB + M, max(sizes), CB * v, v, C, M)
+    want, want_idx, want_acc = oracle.amm_cpu(x, cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)
+    amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=max(sizes))
+    xd = torch.from_numpy(x).cuda()
+    items, guarded = set(), torch.empty((max(sizes) + 3, M), device="cuda")
+    for n in sizes:
+        out, idx, acc = amm.run_debug(x[:n])
+        name = amm.last_gather_kernel()
+        assert np.array_equal(idx, want_idx[:n]) and np.array_equal(acc, want_acc[:n]), (n, name)
+        assert np.array_equal(out.view(np.uint32), want[:n].view(np.uint32)), (n, name)
+        guarded.fill_(-5.0)
+        torch.cuda.synchronize()
+        amm.run_ptr(xd.data_ptr(), n, guarded.data_ptr())
+        ctx.synchronize()
+        items.add(amm.last_gather_kernel())
+        got = guarded.cpu().numpy()
+        assert np.array_equal(got[:n].view(np.uint32), want[:n].view(np.uint32)) and (got[n:] == -5.0).all(), (n, name)
+    if ctx.device_info()["compute_units"] == 256 and not kernel_switches():
+        few = [k for k in items if "_few_" in k]
+        assert len(few) >= 2, items
+        if CB > 1000:
+            assert any("true" in k for k in few), items
+    amm.close()
+
+
 @pytest.mark.parametrize("N,CB,M,C,width,groups", [(1000, 8, 768, 16, 48, 3), (513, 640, 760, 16, 48, 3), (300, 33, 1000, 16, 64, 2), (200, 70, 1500, 9, 96, 2),
                                                    (449, 12, 1500, 16, 96, 3), (400, 130, 2049, 16, 64, 2), (65, 96, 9001, 16, 48, 0), (64, 40, 9001, 16, 48, 3),
                                                    (20, 40, 9001, 16, 48, 1), (1, 5, 16001, 16, 48, 1), (700, 129, 1100, 13, 96, 3)])
