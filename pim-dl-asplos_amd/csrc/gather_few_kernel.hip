@@ -6,6 +6,8 @@
 // on the tables of the large kernels, whatever their layout.  Those kernels give an item of 128 tokens or more and 16 to
 // 96 columns to a workgroup, which goes through all codebooks slice by slice; a launch with fewer items than CUs
 // then takes the time of that chain -- copy, barrier, operands, 32 codebooks further -- however few its tokens are.
+#include <string.h>
+
 #include "gather_common.h"
 #include "search_quad.h"
 
@@ -27,6 +29,14 @@ constexpr int FEW_PITCH_ONEHOT = 80, FEW_PITCH_ROWS = 68;
 constexpr int few_lds_bytes(int nw, int tm, int pitch) { return nw * tm * 4 * pitch * 4; }
 
 enum FewTable { FEW_SPARSE, FEW_PAIRED, FEW_ROWS };
+
+// What a launch leaves as Amm::last_gather, put together once: these launches are short enough for the host to feel a snprintf.
+struct KernelName {
+    char text[sizeof(Amm::last_gather)];
+    template <class... A>
+    explicit KernelName(const char* format, A... args) { snprintf(text, sizeof(text), format, args...); }
+    void to(char* last_gather) const { memcpy(last_gather, text, sizeof(text)); }
+};
 
 struct FewArgs {
     const uint8_t* idx;
@@ -311,8 +321,12 @@ int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
     }();
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_few)")) return rc;
     static const char* const names[] = {TC > 1 ? "gather_sparse_few_wide_kernel" : "gather_sparse_few_kernel", "gather_onehot_few_kernel", "gather_i8_few_kernel"};
-    if constexpr (TC > 1) snprintf(a.last_gather, sizeof(a.last_gather), "%s<%d, %d, %s, %d>", names[T], TM, NW, xcd ? "true" : "false", TC);
-    else snprintf(a.last_gather, sizeof(a.last_gather), "%s<%d, %d, %s>", names[T], TM, NW, xcd ? "true" : "false");
+    auto name = [](bool x) {
+        if constexpr (TC > 1) return KernelName("%s<%d, %d, %s, %d>", names[T], TM, NW, x ? "true" : "false", TC);
+        else return KernelName("%s<%d, %d, %s>", names[T], TM, NW, x ? "true" : "false");
+    };
+    static const KernelName name_of[2] = {name(false), name(true)};
+    name_of[xcd].to(a.last_gather);
     a.note_launch(0, LDS, 16 * TM, NW * 64);
     hipLaunchKernelGGL(kern, grid, dim3(NW * 64), LDS, ctx->stream, f, ep);
     return hip_check(ctx, hipGetLastError(), "gather_few launch");
@@ -437,7 +451,8 @@ int launch_f32_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out, u
 {
     const AmmGeom& g = a.g;
     const uint32_t colblocks = g.M_pad / FB, tok = 64 / FB;
-    snprintf(a.last_gather, sizeof(a.last_gather), "gather_f32_few_kernel<%d, %d, %s>", FB, IDX_BITS, GROUPED ? "true" : "false");
+    static const KernelName name("gather_f32_few_kernel<%d, %d, %s>", FB, IDX_BITS, GROUPED ? "true" : "false");
+    name.to(a.last_gather);
     a.note_launch(0, 0, tok, 64);
     hipLaunchKernelGGL((gather_f32_few_kernel<FB, IDX_BITS, GROUPED>), dim3(colblocks * ((n + tok - 1) / tok)), dim3(64), 0, ctx->stream,
                        d_idx, reinterpret_cast<const float*>(a.d_lut), d_out, n, g.M, g.CB_pad, g.idx_row_bytes, a.d_bias,
@@ -538,7 +553,9 @@ int launch_amm_few(Ctx* ctx, const Amm& a, const float* d_x, float* d_out, uint3
     const FewSearch fs = {d_x, a.d_centroids, g.K, g.CB, g.C, (reinterpret_cast<uintptr_t>(d_x) & 15) == 0};
     auto kern = g.v == 2 ? gather_sparse_few_fused_kernel<2, NW> : g.v == 4 ? gather_sparse_few_fused_kernel<4, NW> : gather_sparse_few_fused_kernel<8, NW>;
     if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_few_fused)")) return rc;
-    snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_few_fused_kernel<%u, %d>", g.v, NW);
+    static const KernelName names[] = {KernelName("gather_sparse_few_fused_kernel<2, %d>", NW), KernelName("gather_sparse_few_fused_kernel<4, %d>", NW),
+                                       KernelName("gather_sparse_few_fused_kernel<8, %d>", NW)};
+    names[g.v / 4].to(a.last_gather);
     a.note_launch(0, LDS, 16, NW * 64);
     hipLaunchKernelGGL(kern, dim3(f.groups), dim3(NW * 64), LDS, ctx->stream, f, ep, fs);
     return hip_check(ctx, hipGetLastError(), "gather_few_fused launch");
