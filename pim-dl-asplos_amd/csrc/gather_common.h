@@ -59,10 +59,12 @@ inline bool sparse_three_per_cu(uint64_t items256, uint32_t cb16, uint64_t cus) 
 
 // Time of that kernel's launch of n tokens x M columns, in rounds of 64-column 256-token items with two workgroups per CU, for the choice
 // of the column tile.  A round of three per CU takes 1.46 of one of two (which is half as many items again); of a partly filled one
-// the part counts 1.2-fold.  A 48-column item takes 0.85 of a 64-column one; eight waves and the split of the codebooks
+// the part counts 1.2-fold, but no less than 0.9 of the only round (some CU has three items) and a quarter of a last one (an item alone goes through its
+// chain of slices all the same).  A 48-column item takes 0.85 of a 64-column one; eight waves and the split of the codebooks
 // between the waves of a SIMD as in launch_sparse_tn.  What the figures give against passes timed with either tile, 48 / 64
-// columns: 3072 -> 768 N = 4096 39.9 / 44.9, N = 5000 58.0 / 51.6, N = 6000 58.8 / 63.0, N = 8192 68.3 / 72.6, N = 12608 115 / 105; 768 -> 768 N = 4096 19.6 / 20.1,
-// N = 16384 40.9 / 38.3; 768 -> 3072 N = 3072 26.5 / 28.8, N = 8192 54.3 / 50.7; 1024 -> 4096 N = 8192 84.7 / 76.3; 1280 -> 1280 N = 8192 52.3 / 46.0.
+// columns: 3072 -> 768 N = 4096 39.9 / 44.9, N = 5000 58.0 / 51.6, N = 6000 58.8 / 63.0, N = 8192 68.3 / 72.6; 768 -> 768 N = 4096 19.6 / 20.1,
+// N = 16384 40.9 / 38.3; items one round holds, or a few more: 3072 -> 768 N = 11000 (688 / 516) 94.7 / 100.1, N = 12608 (800 / 600) 118.6 / 111.6, N =
+// 14000 (880 / 660) 122.5 / 115.6, v = 2 N = 12608 195 / 179, 4096 -> 1024 N = 9000 (792 / 576) 137.7 / 124.9, N = 12608 (1100 / 800) 173 / 165; 768 -> 3072 N = 3072 26.5 / 28.8, N = 8192 54.3 / 50.7; 1024 -> 4096 N = 8192 84.7 / 76.3; 1280 -> 1280 N = 8192 52.3 / 46.0.
 // (96-column tiles, whose rows are pieces of 256 and 128 bytes, used to be the choice of most wide outputs; they are 0.5 to 25 % slower than
 // 64-column ones once outputs take turns instead of staying in the last cache: 768 -> 3072 N = 8192 66.6 / 57.1, N = 16384 119 / 104, 2048 -> 2048
 // N = 4096 60.5 / 47.5, before either had three workgroups per CU.)
@@ -74,9 +76,9 @@ inline double sparse_launch_cost(uint32_t tn, uint64_t n, uint64_t M, uint32_t c
     double t = grid_rounds(items, 2 * cus);
     if (grid_rounds(items_small, 2 * cus) * 0.62 < t) t = grid_rounds(items_small, 2 * cus) * 0.62;
     if (sparse_three_per_cu(items, cb16, cus)) {
-        const uint64_t rest = items % (3 * cus);
-        const double part = 1.2 * (double)rest / (double)(3 * cus);
-        const double t3 = 1.46 * ((double)(items / (3 * cus)) + (part < 1.0 ? part : 1.0));
+        const uint64_t full = items / (3 * cus), rest = items % (3 * cus);
+        const double least = rest == 0 ? 0.0 : full == 0 ? 0.9 : 0.25, filled = 1.2 * (double)rest / (double)(3 * cus);
+        const double t3 = 1.46 * ((double)full + (filled < least ? least : filled < 1.0 ? filled : 1.0));
         if (t3 < t) t = t3;
     }
     return t * item;
