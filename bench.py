@@ -30,18 +30,18 @@ MFMA_I8_PEAK_TOPS = 5000.0                 # MI355X dense int8 matrix peak
 # FETCH_SIZE is scaled by 2.0 and WRITE_SIZE by 1.0: what a streaming copy of known size reads for the same
 # counters in the same runs.
 MEASURED_GATHER_TRAFFIC = {
-    ("gather_sparse_kernel<6, 4, 16, 4, false>", 8192, 768, 3072): {"fetch_kib": 9830.5, "write_kib": 98317.1},
-    ("gather_sparse_kernel<3, 4, 64, 8, false>", 8192, 3072, 768): {"fetch_kib": 15643.5, "write_kib": 24948.0},
+    ("gather_sparse_blocks_kernel<4, 4, 16, 4>", 8192, 768, 3072): {"fetch_kib": 7843.1, "write_kib": 98306.1},
+    ("gather_sparse_blocks_kernel<3, 4, 64, 8>", 8192, 3072, 768): {"fetch_kib": 15618.5, "write_kib": 24987.1},
 }
 FETCH_SCALE, WRITE_SCALE = 2.0, 1.0
 # Busy fractions of the same kernels from a rocprofv3 --pmc run of this script (summary:
 # profiles/bench_ffn_pair_lds_mfma_counters.txt): matrix core (SQ_VALU_MFMA_BUSY_CYCLES / SQ_BUSY_CU_CYCLES), LDS
 # (SQ_LDS_IDX_ACTIVE / ...), LDS bank-conflict cycles over LDS-active cycles.  Reported only for the kernel they belong to.
 MEASURED_GATHER_COUNTERS = {
-    ("gather_sparse_kernel<6, 4, 16, 4, false>", 8192, 768, 3072): {
-        "matrix_core_busy_frac": 0.425, "lds_active_frac": 0.368, "lds_bank_conflict_frac_of_active": 0.225, "wave_cycles_waiting_to_issue_frac": 0.37},
-    ("gather_sparse_kernel<3, 4, 64, 8, false>", 8192, 3072, 768): {
-        "matrix_core_busy_frac": 0.440, "lds_active_frac": 0.501, "lds_bank_conflict_frac_of_active": 0.254, "wave_cycles_waiting_to_issue_frac": 0.37},
+    ("gather_sparse_blocks_kernel<4, 4, 16, 4>", 8192, 768, 3072): {
+        "matrix_core_busy_frac": 0.487, "lds_active_frac": 0.510, "lds_bank_conflict_frac_of_active": 0.279, "wave_cycles_waiting_to_issue_frac": 0.41},
+    ("gather_sparse_blocks_kernel<3, 4, 64, 8>", 8192, 3072, 768): {
+        "matrix_core_busy_frac": 0.462, "lds_active_frac": 0.525, "lds_bank_conflict_frac_of_active": 0.254, "wave_cycles_waiting_to_issue_frac": 0.38},
 }
 CLOCK_SETTLE_S = 0.08                      # untimed pre-heat: the engine clock needs ~20 ms of this load to ramp up
 
