@@ -220,7 +220,8 @@ static int pipe_get(Ctx* ctx, HostPipe** out)
     return PIMDL_OK;
 }
 
-// Per-slot buffers of at least the given sizes (0: that direction is not staged).  Only called while the ring is
+// Per-slot buffers of at least the given sizes (0: that direction is not staged).  The pinned ones are coherent: kernels read and write them too
+// (ring_to_device, ring_to_host).  Only called while the ring is
 // idle (every call that uses it drains it before it returns or before it touches a slot again).
 static int pipe_reserve(Ctx* ctx, HostPipe* hp, size_t in_bytes, size_t out_bytes)
 {
@@ -236,7 +237,7 @@ static int pipe_reserve(Ctx* ctx, HostPipe* hp, size_t in_bytes, size_t out_byte
         }
         hp->in_bytes = 0;
         for (int s = 0; s < HostPipe::SLOTS && !rc; ++s) {
-            rc = hip_check(ctx, hipHostMalloc(&hp->pin_in[s], in_bytes, hipHostMallocDefault), "hipHostMalloc(staging in)");
+            rc = hip_check(ctx, hipHostMalloc(&hp->pin_in[s], in_bytes, hipHostMallocCoherent), "hipHostMalloc(staging in)");
             if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&hp->d_in[s]), in_bytes), "hipMalloc(staging in)");
         }
         if (rc) return rc;
@@ -253,7 +254,7 @@ static int pipe_reserve(Ctx* ctx, HostPipe* hp, size_t in_bytes, size_t out_byte
         }
         hp->out_bytes = 0;
         for (int s = 0; s < HostPipe::SLOTS && !rc; ++s) {
-            rc = hip_check(ctx, hipHostMalloc(&hp->pin_out[s], out_bytes, hipHostMallocDefault), "hipHostMalloc(staging out)");
+            rc = hip_check(ctx, hipHostMalloc(&hp->pin_out[s], out_bytes, hipHostMallocCoherent), "hipHostMalloc(staging out)");
             if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&hp->d_out[s]), out_bytes), "hipMalloc(staging out)");
         }
         if (rc) return rc;
