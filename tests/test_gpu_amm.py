@@ -579,7 +579,7 @@ def _random_cases(count, seed):
 
 @pytest.mark.parametrize("case", _random_cases(48, 2024), ids=lambda c: "n%d_k%d_v%d_c%d_m%d_%s" % c[1:])
 def test_random_shapes_against_the_oracle(ctx, case):
-    """Seeded random shapes across every kernel variant (search: bf16 narrow / wide, exact, generic; gather:
+    """Seeded random shapes across every kernel variant (search: matrix narrow / wide, exact, generic; gather:
     one-hot, paired, byte adder, fp32 one and two tokens per lane, grouped), with a non-zero LUT bias in both
     bias modes for the int8 table."""
     i, N, K, v, C, M, kind = case
