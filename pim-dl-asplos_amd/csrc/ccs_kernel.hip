@@ -702,14 +702,16 @@ __device__ __forceinline__ uint32_t half_piece(float& a)
 }
 
 // The power of two that the activations and centroids of n codebooks are multiplied with: 1 unless one of their centroids is longer than
-// 1024, else what makes the longest one shorter than that.  (A codebook with a centroid that is not finite has no say: it is replayed.)
+// 1024, else what makes the longest one shorter than that, and never less than 2^-44: what a search accepts, |x|^2 + |c|^2 < 1e9 at this scale,
+// is then below 3.1e35 as it came, and no distance of the reference overflows (where one does, its scan stays where it is, and only a replay
+// says so).  Halves hold -2c of any centroid within that bound.  (A codebook with a centroid that is not finite has no say: it is replayed.)
 __device__ __forceinline__ float half_scale(const float* cnmax, uint32_t n)
 {
     float m = 0.0f;
     for (uint32_t i = 0; i < n; ++i) m = fmaxf(m, cnmax[i]);  // (a NaN gives way)
     if (!(m > 1048576.0f)) return 1.0f;
     const int e = ilogbf(m) - 20;  // m < 2^(21 + e), e >= 0
-    return ldexpf(1.0f, -(e / 2 + 1));
+    return ldexpf(1.0f, e / 2 + 1 < 44 ? -(e / 2 + 1) : -44);
 }
 
 // K-slot registers (two half K-slots each, four registers per MFMA) of lane (row i, half kh).  The lane
@@ -1064,7 +1066,7 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
                 constexpr float A2 = 2.0f * ((V + 1) + 12.0f + 2.02f * (17 * NM) + 2 * (V + 2)) * 5.9604645e-8f;
                 constexpr float B2 = 2.0f * 16.0f * 2.3841858e-7f;               // 2 * 2^(4-22)
                 const float thr = fmaf(A2, mag, fmaf(B2, fabsf(m2), c0));
-                // NaN anywhere makes a compare false, which counts as "not safe"; beyond 1e9 a half may have run out
+                // NaN anywhere makes a compare false, which counts as "not safe"; beyond 1e9 a half may have run out (and see half_scale)
                 const bool safe = ((m2 - m1) > thr) && (mag < 1e9f);
                 need |= (safe ? 0u : 1u) << (WIDE ? tg : it);
                 words[tg / 2] |= bi << (16 * (tg % 2) + (WIDE ? 0 : 8 * pl + 4 * h));
@@ -1529,7 +1531,7 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
             constexpr float A2 = 2.0f * ((V + 1) + 12.0f + 2.02f * (17 * NM) + 2 * (V + 2)) * 5.9604645e-8f;
             constexpr float B2 = 2.0f * 16.0f * 2.3841858e-7f;  // 2 * 2^(4-22)
             const float thr = fmaf(A2, mag, fmaf(B2, fabsf(second), c0));
-            // NaN anywhere makes a compare false, which counts as "not safe"; beyond 1e9 a half may have run out
+            // NaN anywhere makes a compare false, which counts as "not safe"; beyond 1e9 a half may have run out (and see half_scale)
             fail[q] = !((second - best) > thr && mag < 1e9f);
         }
         // ---- exact replay of the tokens that failed the margin test (rare) ----

@@ -506,6 +506,29 @@ def test_search_over_the_range_of_halves(ctx, v, C, size):
     amm.close()
 
 
+@pytest.mark.parametrize("v,C", [(4, 16), (2, 16), (8, 16), (4, 9), (2, 32), (4, 20), (8, 32), (2, 64), (4, 33), (8, 130), (16, 16), (32, 40)])
+@pytest.mark.parametrize("length", [1e15, 1e17, 9.5e17])
+def test_search_where_distances_overflow(ctx, v, C, length):
+    """Finite centroids up to the longest that the matrix search takes (|c|^2 < 1e36), and rows from that length to lengths whose squared
+    distances are beyond FLT_MAX for some or for all of the centroids: the reference's distances are infinite there, and its scan stays
+    where it is.  Every index against that scan."""
+    rng = np.random.default_rng(6000 + 10 * v + C)
+    many = C > 32 or v > 8
+    N, CB = 1500 if many else 330, 37
+    unit = lambda a: a / np.linalg.norm(a, axis=-1, keepdims=True)
+    cent = (unit(rng.standard_normal((CB, C, v))) * length * rng.uniform(0.9, 1.0, (CB, C, 1))).astype(np.float32)
+    x = unit(rng.standard_normal((N, CB, v))) * rng.choice([length, 30 * length, 1.5e19, 1.8e19, 1.9e19, 2.2e19, 3.5e19], (N, CB, 1))
+    x = x.astype(np.float32).reshape(N, CB * v)
+    with np.errstate(all="ignore"):
+        want = oracle.index_calculation(x, cent, v, threads=THREADS)
+    amm = ctx.amm(cent, np.zeros((CB, C, 4), np.int8), np.float32(1.0), None, max_n=N)
+    for tile in (0,) if many else (64, 128):
+        amm.set_tuning(search_token_tile=tile)
+        got = amm.index_calculation(x)
+        assert np.array_equal(got, want), f"tile {tile}: {(got != want).sum()} of {got.size} differ"
+    amm.close()
+
+
 @pytest.mark.parametrize("v,C", [(4, 16), (2, 16), (8, 16), (4, 32)])
 def test_search_with_non_finite_values(ctx, v, C):
     """NaN / Inf / near-overflow values in activations and centroids take the exact path and match
