@@ -892,7 +892,7 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
             return pick;
         };
         // Sparse kernel, up to 16 centroids: 64 or 48 columns (96 on request).  An output of a multiple of 48 columns that 64 does not
-        // divide takes 48, which lets operators of such outputs share a gather launch.
+        // divide takes 48, which operators of such outputs share in a gather launch (plan_side_by_side).
         auto pick_sparse = [&] {
             if (col_block_hint) return col_block_hint / 16;
             if (M % 48 == 0 && M % 64 != 0) return 3u;
@@ -915,6 +915,7 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
             return false;
         }
         g->q = g->gather_kind == 2 && C <= 16 ? pick_sparse() : pick_dense(paired);
+        g->cols_named = col_block_hint != 0 || tune.gather_kernel == PIMDL_GATHER_ONEHOT;
         g->gq = 4;
         g->cb_per_slice = 16;
         g->col_block = 16 * g->q;
@@ -969,6 +970,25 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
     g->ccs_lds_bytes = g->ccs_cb_per_wg ? 64 * (g->ccs_row_floats + 4) * 4 : 0;
     if (col_block_hint && !i8) { *why = "fp32 tables have one column block width"; return false; }
     return apply_runtime_tuning(g, tune, why);
+}
+
+bool plan_side_by_side(const Amm& first, uint32_t count, uint32_t max_n, uint32_t num_cus, AmmGeom* g)
+{
+    const uint64_t cus = num_cus ? num_cus : 256, cols = (uint64_t)count * first.g.M;
+    uint32_t tn = 0;
+    for (uint32_t t : {4u, 3u})
+        if (first.g.M % (16 * t) == 0 &&
+            (tn == 0 || sparse_launch_cost(t, max_n, cols, first.g.CB_pad, cus) < sparse_launch_cost(tn, max_n, cols, first.g.CB_pad, cus) - 1e-9))
+            tn = t;
+    if (tn == 0) return false;
+    pimdl_amm_tuning t = {16 * tn, PIMDL_GATHER_SPARSE, first.g.tune_token_item, first.g.tune_cb_per_slice, first.g.tune_xcd_col_split,
+                          first.g.tune_search, first.g.tune_search_tile};
+    std::string why;
+    *g = AmmGeom{};
+    if (plan_geometry(first.desc, num_cus, g, &why, &t)) return true;
+    t.token_item = t.cb_per_slice = 0;  // (a setting that this tile does not have)
+    *g = AmmGeom{};
+    return plan_geometry(first.desc, num_cus, g, &why, &t);
 }
 
 int launch_amm(Ctx* ctx, const Amm& a, const float* d_x, uint8_t* d_idx, float* d_out, uint32_t n)

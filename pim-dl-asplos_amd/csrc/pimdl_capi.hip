@@ -526,6 +526,25 @@ static void retile_lut_onehot(const int8_t* lut, int8_t* tiled, const AmmGeom& g
         }
 }
 
+// a table of either one-hot kernel, up to 16 centroids, as the sparse kernel has it with the column tile of `b`
+static void move_lut_onehot(const int8_t* from, const AmmGeom& a, int8_t* to, const AmmGeom& b)
+{
+    auto places = [](const AmmGeom& g) {
+        std::vector<uint32_t> where(g.col_block);
+        for (uint32_t s = 0; s < g.col_block; ++s) where[g.gather_kind == 2 ? sparse_tile_column(g.col_block / 16, s) : s] = s;
+        return where;
+    };
+    const std::vector<uint32_t> at = places(a), bt = places(b);
+    const bool paired = a.C_tile == 8;
+    const uint32_t entries = paired ? a.CB_pad / 2 : a.CB_pad;
+    for (uint32_t cb = 0; cb < a.CB; ++cb)
+        for (uint32_t f = 0; f < a.M; ++f) {
+            const size_t entry = ((size_t)(f / a.col_block) * entries + (paired ? cb / 2 : cb)) * a.col_block + at[f % a.col_block];
+            int8_t* dst = to + (((size_t)(f / b.col_block) * b.CB_pad + cb) * b.col_block + bt[f % b.col_block]) * 16;
+            memcpy(dst, from + entry * 16 + (paired ? 8 * (cb & 1) : 0), paired ? 8 : 16);
+        }
+}
+
 }  // namespace pimdl
 
 using namespace pimdl;
@@ -1003,6 +1022,22 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
                a->desc.activation == first->desc.activation && lbt == lbt0;
     }
     for (uint32_t i = 0; i < count && same && !rc; ++i) rc = table_as(amms[i], mg[i], &mtab[i]);
+    // Members whose tables are of different column tiles, or of one that does not divide their width, as the library has chosen for each
+    // alone: the group's copy is laid out in a tile of its own.
+    bool moved = false;
+    if (!rc && !same) {
+        moved = true;
+        bool sparse = false;
+        for (uint32_t i = 0; i < count && moved; ++i) {
+            const Amm* a = amms[i];
+            const float lbt = a->desc.bias_mode == PIMDL_BIAS_TIMES_CB ? a->desc.lut_bias * (float)a->g.CB : a->desc.lut_bias;
+            moved = a->desc.lut_dtype == PIMDL_LUT_I8 && !a->grouped && a->g.gather_kind != 0 && a->g.C <= 16 && !a->g.cols_named &&
+                    a->g.M == first->g.M && a->desc.activation == first->desc.activation && lbt == lbt0;
+            sparse |= a->g.gather_kind == 2;
+        }
+        moved = moved && sparse && plan_side_by_side(*first, count, max_n, ctx->prop.multiProcessorCount, &mg[0]);
+        same = moved;
+    }
     if (!rc && same) {
         Amm& m = grp->merged;
         m = *first;  // epilogue constants; geometry and pointers below are the group's own
@@ -1026,9 +1061,23 @@ int pimdl_amm_group_create(pimdl_ctx* ctx, pimdl_amm* const* amms, uint32_t coun
         rc = hip_check(ctx, hipMalloc(&m.d_lut, m.lut_bytes), "hipMalloc(group lut)");
         if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&m.d_bias), (size_t)m.g.M * sizeof(float)), "hipMalloc(group bias)");
         if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&m.d_op_scales), count * sizeof(float)), "hipMalloc(group scales)");
+        std::vector<int8_t> have, want;
         for (uint32_t i = 0; i < count && !rc; ++i) {
-            rc = hip_check(ctx, hipMemcpyAsync(static_cast<char*>(m.d_lut) + (size_t)i * one_table, mtab[i],
-                                               one_table, hipMemcpyDeviceToDevice, ctx->stream), "D2D lut");
+            char* dst = static_cast<char*>(m.d_lut) + (size_t)i * one_table;
+            if (moved) {
+                try {
+                    have.resize(amms[i]->lut_bytes);
+                    want.assign(one_table, 0);
+                } catch (...) {
+                    rc = set_error(ctx, PIMDL_ERR_NOMEM, "pimdl_amm_group_create: host staging of a table of %zu bytes failed", one_table);
+                    break;
+                }
+                if ((rc = hip_check(ctx, hipMemcpy(have.data(), amms[i]->d_lut, have.size(), hipMemcpyDeviceToHost), "D2H lut"))) break;
+                move_lut_onehot(have.data(), amms[i]->g, want.data(), mg[0]);
+                rc = hip_check(ctx, hipMemcpy(dst, want.data(), one_table, hipMemcpyHostToDevice), "H2D group lut");
+            } else {
+                rc = hip_check(ctx, hipMemcpyAsync(dst, mtab[i], one_table, hipMemcpyDeviceToDevice, ctx->stream), "D2D lut");
+            }
             if (!rc) rc = hip_check(ctx, hipMemcpyAsync(m.d_bias + (size_t)i * first->g.M, amms[i]->d_bias,
                                                         (size_t)first->g.M * sizeof(float), hipMemcpyDeviceToDevice, ctx->stream), "D2D bias");
         }

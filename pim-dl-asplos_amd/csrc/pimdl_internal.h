@@ -42,7 +42,7 @@ struct AmmGeom {
     uint32_t q;             // 16-byte chunks per LUT row in LDS
     uint32_t col_block;     // columns per workgroup (int8: 16*q -- the byte adder picks its own at launch, see cols --, fp32: 4*q)
     uint32_t cols;          // byte adder of up to 64 centroids: columns per item that the caller has named (0: the launch picks)
-    uint32_t cols_named;    // ... at creation
+    uint32_t cols_named;    // ... at creation; one-hot kernels: the caller has named the column tile, or the dense kernel
     uint32_t row_pitch;     // bytes between LUT rows in LDS
     uint32_t gq;            // int8: codebooks per lane group per slice
     uint32_t cb_per_slice;
@@ -225,6 +225,9 @@ bool gather_rows_only();
 // tuning: choices taken over by the caller (nullptr: none); an error if the shape has no kernel for one
 bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::string* why,
                    const pimdl_amm_tuning* tuning = nullptr);
+// The sparse gather of one of `count` operators of first's shape (up to 16 centroids) side by side in one launch: the column tile is
+// the launch's, not what each operator would take alone, and divides its width.  False if none does.
+bool plan_side_by_side(const Amm& first, uint32_t count, uint32_t max_n, uint32_t num_cus, AmmGeom* g);
 // checks the run-time fields of a tuning against a planned geometry and stores them in it
 bool apply_runtime_tuning(AmmGeom* g, const pimdl_amm_tuning& t, std::string* why);
 

@@ -331,6 +331,63 @@ def test_operators_sharing_an_input_are_searched_by_one_launch(ctx, N, K, v, C, 
         a.close()
 
 
+@pytest.mark.parametrize("CB,v,C,M,max_n,named", [
+    (128, 2, 16, 1280, (9856, 9856, 9856), None),       # alone each takes 48 columns, which do not divide its width
+    (128, 2, 16, 1216, (10400, 10400), None),
+    (128, 2, 16, 1024, (1024, 1024, 1024), None), (32, 4, 12, 1024, (4608, 4608), None),
+    (128, 2, 16, 768, (11008, 12608), None),            # 48 columns and 64
+    (128, 2, 8, 1280, (9856, 10048, 4096), None),       # up to 8 centroids: tables of both one-hot kernels, two column tiles
+    (128, 2, 16, 1280, (9856, 9856), {"col_block": 48}),   # a tile that the caller has named stays
+    (128, 2, 16, 1280, (9856, 9856), {"token_item": 128}), (128, 2, 16, 1280, (9856, 9856), {"token_item": 256, "cb_per_slice": 64}),
+    (32, 2, 16, 1000, (700, 700), None),                # no tile divides the width
+])
+def test_operators_side_by_side_take_a_column_tile_of_their_own(ctx, CB, v, C, M, max_n, named):
+    """Whether operators share one gather launch depends on their width, not on the column tile that suits each of them alone at its
+    largest batch: every column bit for bit that of the operator alone, at few tokens and many."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    import torch
+    amms = []
+    for i, n in enumerate(max_n):
+        _, cent, lut, bias = make_case(5600 + i, 1, CB * v, v, C, M)
+        amms.append(ctx.amm(cent, lut, np.float32(0.01 * (i + 1)), bias, max_n=n, tuning=named or {}))
+    group = ctx.amm_group(amms)
+    tiles = {a.geometry()["col_block"] for a in amms}
+    fused = M % 64 == 0 or M % 48 == 0
+    if named and "col_block" in named:
+        fused = M % named["col_block"] == 0
+    elif not named and fused and ctx.device_info()["compute_units"] == 256:
+        assert len(tiles) > 1 or M % min(tiles), tiles   # (what the case is about)
+    assert group.fused_cols == (len(amms) * M if fused else 0)
+    x = torch.randn((min(max_n), CB * v), device="cuda", generator=torch.Generator(device="cuda").manual_seed(M))
+    for n in (min(max_n), 700, 33, 1) if fused else (33,):
+        want = torch.empty((n, len(amms), M), device="cuda")
+        part = torch.empty((n, M), device="cuda")
+        for i, a in enumerate(amms):
+            torch.cuda.synchronize()
+            a.run_ptr(x.data_ptr(), n, part.data_ptr())
+            ctx.synchronize()
+            want[:, i] = part
+        if fused:
+            out = torch.full((n + 1, len(amms) * M), -5.0, device="cuda")
+            torch.cuda.synchronize()
+            group.run_fused_ptr(x.data_ptr(), n, out.data_ptr())
+            ctx.synchronize()
+            assert torch.equal(out[:n], want.view(n, -1)) and bool((out[n:] == -5.0).all()), n
+        else:
+            with pytest.raises(pimdl.PimdlError) as e:
+                group.run_fused(x[:n].cpu().numpy())
+            assert e.value.code == pimdl.ERR_UNSUPPORTED
+        outs = [torch.empty((n, M), device="cuda") for _ in amms]
+        torch.cuda.synchronize()
+        group.run_ptr(x.data_ptr(), n, [o.data_ptr() for o in outs])
+        ctx.synchronize()
+        assert all(torch.equal(o, want[:, i]) for i, o in enumerate(outs)), n
+    group.close()
+    for a in amms:
+        a.close()
+
+
 def test_group_conditions(ctx):
     if kernel_switches():
         pytest.skip("a kernel this test is about is switched off by the environment")
