@@ -702,16 +702,17 @@ __device__ __forceinline__ uint32_t half_piece(float& a)
 }
 
 // The power of two that the activations and centroids of n codebooks are multiplied with: 1 unless one of their centroids is longer than
-// 1024, else what makes the longest one shorter than that, and never less than 2^-44: what a search accepts, |x|^2 + |c|^2 < 1e9 at this scale,
-// is then below 3.1e35 as it came, and no distance of the reference overflows (where one does, its scan stays where it is, and only a replay
-// says so).  Halves hold -2c of any centroid within that bound.  (A codebook with a centroid that is not finite has no say: it is replayed.)
+// 1024, else what makes the longest one shorter than that, and never less than 2^-48: what a search accepts, |x|^2 + |c|^2 < 1e9 at this scale,
+// is then below 8e37 as it came, and no distance of the reference overflows (where one does, its scan stays where it is, and only a replay
+// says so).  The longest centroids of a codebook that is not replayed anyway, of 1e18, are 3553 at that scale.  (A codebook with a centroid that
+// is not finite has no say: it is replayed.)
 __device__ __forceinline__ float half_scale(const float* cnmax, uint32_t n)
 {
     float m = 0.0f;
     for (uint32_t i = 0; i < n; ++i) m = fmaxf(m, cnmax[i]);  // (a NaN gives way)
     if (!(m > 1048576.0f)) return 1.0f;
     const int e = ilogbf(m) - 20;  // m < 2^(21 + e), e >= 0
-    return ldexpf(1.0f, e / 2 + 1 < 44 ? -(e / 2 + 1) : -44);
+    return ldexpf(1.0f, e / 2 + 1 < 48 ? -(e / 2 + 1) : -48);
 }
 
 // K-slot registers (two half K-slots each, four registers per MFMA) of lane (row i, half kh).  The lane
