@@ -94,8 +94,8 @@ inline size_t ccs_f16_offset(const AmmGeom& g)
 }
 inline size_t ccs_f16_floats(const AmmGeom& g)
 {
-    // (and a scale for every 8 units, CB_pad being a multiple of 32; see half_scale)
-    return ccs_has_f16(g) ? ccs_f16_units(g) * ccs_f16_nm(g.v, ccs_f16_wide(g)) * 64 * 4 + ccs_f16_units(g) * 2 * 16 + ccs_f16_units(g) / 8 : 0;
+    // (then what ccs_f16_kernel lists: a flag for every 8 units, CB_pad being a multiple of 32, a scale and a margin per codebook)
+    return ccs_has_f16(g) ? ccs_f16_units(g) * ccs_f16_nm(g.v, ccs_f16_wide(g)) * 64 * 4 + ccs_f16_units(g) * 2 * 16 + ccs_f16_units(g) / 8 + 2 * g.CB_pad : 0;
 }
 
 // more than 32 centroids, or sub-vectors of 16 or 32 dimensions: the matrix search over groups of 32 centroids
@@ -108,7 +108,7 @@ inline size_t ccs_many_groups(const AmmGeom& g) { return (size_t)g.CB * ((g.C + 
 constexpr uint32_t ccs_many_nm(uint32_t v) { return (4 * v + 15) / 16; }  // matrix instructions per group: v dims x 4 cross products
 inline size_t ccs_many_floats(const AmmGeom& g)
 {
-    return ccs_has_many(g) ? ccs_many_groups(g) * (ccs_many_nm(g.v) * 64 * 4 + 32) + g.CB : 0;  // (and a scale per codebook)
+    return ccs_has_many(g) ? ccs_many_groups(g) * (ccs_many_nm(g.v) * 64 * 4 + 32) + 2 * g.CB : 0;  // (and a scale and a margin per codebook)
 }
 
 template <int N, typename F>
@@ -672,12 +672,14 @@ __global__ __launch_bounds__(CCS_THREADS, V == 8 ? 2 : 4) void ccs_mfma_kernel(c
 // a pass, inputs and outputs in turn, before / now: v = 4 N = 8192 K = 3072 66.1 / 62.6, N = 4096 38.4 / 37.6, K = 768 18.5 / 18.1; v = 8 N =
 // 8192 K = 3072 50.5 / 46.9, v = 2 105.7 / 101.1; beyond 16 centroids, where it also counts that a lane decides a codebook instead of both lanes of
 // a token the same one, N = 12608 K = 3072 160 / 140.7, N = 8192 v = 8 72.8 / 65.0, v = 2 188 / 178.)
-// Halves end at 65504: a tile with a centroid longer than 1024 is searched at a power-of-two scale, and
+// Halves end at 65504: a codebook with a centroid longer than 1024 is searched at a power of two of its own, and
 // sub-vectors longer than 31623 of that scale are replayed exactly.
 // Operands:
 //   aux_b [units][NM][64 lanes] uint4 A-operand images (pieces of -2c, by K-slot); a unit is two codebooks, or one (wide)
 //   cn16  [CB_pad][16] float          |c|^2 (r for padded codebooks, 3e38 for ids past C)
-//   scale [units / 8] float           what a tile's activations and centroids are multiplied with
+//   plain [units / 8] float           the smallest scale of a tile
+//   scale [CB_pad] float              what a codebook's activations and centroids are multiplied with
+//   fixed [CB_pad] float              what its margin has beside |x|^2 (see half_fixed)
 // =============================================================================================
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
@@ -701,18 +703,31 @@ __device__ __forceinline__ uint32_t half_piece(float& a)
     return __builtin_bit_cast(uint16_t, p);
 }
 
-// The power of two that the activations and centroids of n codebooks are multiplied with: 1 unless one of their centroids is longer than
-// 1024, else what makes the longest one shorter than that, and never less than 2^-48: what a search accepts, |x|^2 + |c|^2 < 1e9 at this scale,
-// is then below 8e37 as it came, and no distance of the reference overflows (where one does, its scan stays where it is, and only a replay
-// says so).  The longest centroids of a codebook that is not replayed anyway, of 1e18, are 3553 at that scale.  (A codebook with a centroid that
-// is not finite has no say: it is replayed.)
-__device__ __forceinline__ float half_scale(const float* cnmax, uint32_t n)
+// The power of two that a codebook's activations and centroids are multiplied with (m: the largest |c|^2): 1 unless one of the centroids is longer
+// than 1024, else what makes the longest one shorter than 1, and never less than 2^-48: what a search accepts, |x|^2 < 1e9 at this
+// scale, is then below 8e37 as it came, and no distance of the reference overflows (where one does, its scan stays where it is, and only a
+// replay says so).  The longest centroids of a codebook that is not replayed anyway, of 1e18, are 3553 at that scale.  (NaN, of a codebook that
+// is: 1.)  Length 1 leaves activations all of the range of halves and costs nothing: A m, which the margin has of centroids of length 1, is 20 times what
+// it has of subnormal pieces.  And a scale of the codebook's own: one for a tile left small codebooks beside a large one few bits, and
+// replayed them.  us of search, N = 8192, K = 3072, v = 4, with a scale for 16 codebooks that makes them shorter than 1024 / as it is: one codebook in
+// 16 1e4 times as large as the others 30.4 / 23.9, a million times 59.2 / 23.2; centroids of 1000, every hundredth row of 3e5 36.0 / 23.0.
+__device__ __forceinline__ float half_scale(float m)
 {
-    float m = 0.0f;
-    for (uint32_t i = 0; i < n; ++i) m = fmaxf(m, cnmax[i]);  // (a NaN gives way)
     if (!(m > 1048576.0f)) return 1.0f;
-    const int e = ilogbf(m) - 20;  // m < 2^(21 + e), e >= 0
-    return ldexpf(1.0f, e / 2 + 1 < 48 ? -(e / 2 + 1) : -48);
+    const int e = ilogbf(m) / 2 + 1;  // m < 2^(2 e)
+    return ldexpf(1.0f, e < 48 ? -e : -48);
+}
+
+// The margin of a search is A (|x|^2 + fixed) + B |second smallest score|, with fixed = m and, over A, what the hysteresis is at scale sc and
+// 2 * 1.25 v u for pieces below the smallest half (u = 2^-24);
+//   A = 2 * [ (v+1)u (|c|^2) + 12u (what the pieces leave: 8u of x, 2u of c, where subnormal u) + 2.02 * 17 NM u (16 NM products
+//       and NM accumulators, each within u of a partial sum below 2.02 (|x|^2 + m)) + 2(v+2)u (the reference's own chain) ]
+//     = 2 * {57, 98, 178} u  for v = {2, 4, 8}; 17 centroids and more {57, 63, 109}
+constexpr float half_margin(int v, int nm) { return 2.0f * ((v + 1) + 12.0f + 2.02f * (17 * nm) + 2 * (v + 2)) * 5.9604645e-8f; }
+template <uint32_t V, uint32_t NM>
+__device__ __forceinline__ float half_fixed(float m, float sc)
+{
+    return fmaf(1.0f / half_margin(V, NM), fmaf(1.001e-6f * sc, sc, 2.5f * V * 5.9604645e-8f), m * sc * sc);
 }
 
 // K-slot registers (two half K-slots each, four registers per MFMA) of lane (row i, half kh).  The lane
@@ -727,7 +742,8 @@ __device__ __forceinline__ float half_scale(const float* cnmax, uint32_t n)
 //     DL == 4     xh(0,1) xh(2,3) xm(0,1) xm(2,3)          twice    ch(0,1) ch(2,3) ch(0,1) ch(2,3), the same of cm
 template <uint32_t V, bool WIDE>
 __global__ void ccs_prep_f16_kernel(const float* __restrict__ cent, const float* __restrict__ cnmax, uint4* __restrict__ aux_b,
-                                    float* __restrict__ cn16, float* __restrict__ scale, uint32_t CB, uint32_t C)
+                                    float* __restrict__ cn16, float* __restrict__ plain, float* __restrict__ scale,
+                                    float* __restrict__ fixed, uint32_t CB, uint32_t C)
 {
     constexpr uint32_t DL = V / 2, NM = ccs_f16_nm(V, WIDE);
     const uint32_t pair = blockIdx.x, lane = threadIdx.x;
@@ -738,9 +754,16 @@ __global__ void ccs_prep_f16_kernel(const float* __restrict__ cent, const float*
     const bool real = (cb < CB) && (cid < C);
     const float* cp = cent + ((size_t)cb * C + cid) * V;
     constexpr uint32_t PER_TILE = WIDE ? 8 : 16;
-    const uint32_t first = pair / 8 * PER_TILE;
-    const float sc = half_scale(cnmax + first, first >= CB ? 0u : CB - first < PER_TILE ? CB - first : PER_TILE);
-    if (pair % 8 == 0 && lane == 0) scale[pair / 8] = sc;
+    const float m = cb < CB ? cnmax[cb] : 0.0f, sc = half_scale(m);
+    if (kh == 0 && r == 0 && (!WIDE || h == 0)) {
+        scale[cb] = sc;
+        fixed[cb] = half_fixed<V, NM>(m, sc);
+    }
+    if (pair % 8 == 0 && lane == 0) {
+        float all = 1.0f;
+        for (uint32_t c = pair / 8 * PER_TILE; c < CB && c < (pair / 8 + 1) * PER_TILE; ++c) all = fminf(all, half_scale(cnmax[c]));
+        plain[pair / 8] = all;
+    }
     uint32_t pc[DL][2];  // pieces ch, cm of -2c for the lane's dims
     for (uint32_t d = 0; d < DL; ++d) {
         float a = real ? -2.0f * (cp[DL * kh + d] * sc) : 0.0f;
@@ -778,15 +801,15 @@ __global__ void ccs_prep_f16_kernel(const float* __restrict__ cent, const float*
 }
 
 // Register budget: three waves per SIMD (168 registers) but for v = 8 with 128-token tiles and up to 16 centroids,
-// whose 64 prefetch registers do not fit: asked for three the compiler gives up and takes 288 (one workgroup per
-// CU); asked for two it takes 237 without spills, and the 76 KB of LDS allow no more than two anyway.
+// whose 64 prefetch registers do not fit: asked for two it takes 221 without spills, and the 76 KB of LDS allow no more than two anyway.
 template <int V, bool WIDE, int TTOK>
 __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 : 3) void ccs_f16_kernel(const float* __restrict__ x,
                                                                  const float* __restrict__ cent,
                                                                  const uint4* __restrict__ aux_b,
                                                                  const float* __restrict__ cn16,
+                                                                 const float* __restrict__ tile_plain,
                                                                  const float* __restrict__ scale,
-                                                                 const float* __restrict__ cnmax_pad,
+                                                                 const float* __restrict__ fixed,
                                                                  uint8_t* __restrict__ idx, uint32_t N,
                                                                  uint32_t K, uint32_t CB, uint32_t C,
                                                                  uint32_t idx_row_bytes, int idx_tiled, int vec_ok,
@@ -856,9 +879,8 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
     uint32_t tiles_done = 0;
     uint32_t tcb_loaded = 0xFFFFFFFFu;  // codebook tile whose operands are resident (registers and LDS)
     uint4 aq[2][NM];
-    float cmax[NCB];
-    float sc = 1.0f;                        // the tile's scale (uniform)
-    bool plain = true;
+    float fix[NCB];
+    bool plain = true;                      // no codebook of the tile has a scale (uniform)
     for (uint32_t tile_id = blockIdx.x; tile_id < total_tiles; tile_id += gridDim.x) {
         switch (4 * tiles_done / my_tiles) {
             case 0: __builtin_amdgcn_s_setprio(3); break;
@@ -876,8 +898,7 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
         const bool new_cb = tcb != tcb_loaded;  // workgroup-uniform
         tcb_loaded = tcb;
         if (new_cb) {
-            sc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(scale[tcb])));
-            plain = sc == 1.0f;
+            plain = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(tile_plain[tcb]))) == 1.0f;
 #pragma unroll
             for (int pl = 0; pl < 2; ++pl)
 #pragma unroll
@@ -885,15 +906,17 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
             // every global load the search needs is issued here, ahead of the next tile's prefetch:
             // loads complete in order, so a later load would have to wait for the prefetch from HBM
 #pragma unroll
-            for (int o = 0; o < NCB; ++o) cmax[o] = cnmax_pad[WIDE ? pair0 + h : 2 * (pair0 + o) + h] * sc * sc;
+            for (int o = 0; o < NCB; ++o) fix[o] = fixed[WIDE ? pair0 + h : 2 * (pair0 + o) + h];
         }
         if (!plain) {
+            const float* sp = scale + tcb * RCB + 4 * fq / V;  // the thread's columns: one codebook, two of 2 floats
+            const float s0 = sp[0], s1 = V == 2 ? sp[1] : s0;
 #pragma unroll
             for (int i = 0; i < PASSES; ++i) {
-                pf[i].x *= sc;
-                pf[i].y *= sc;
-                pf[i].z *= sc;
-                pf[i].w *= sc;
+                pf[i].x *= s0;
+                pf[i].y *= s0;
+                pf[i].z *= s1;
+                pf[i].w *= s1;
             }
         }
 #pragma unroll
@@ -912,9 +935,6 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
         }
         __syncthreads();
         if (tile_id + gridDim.x < total_tiles) fetch(pf, tile_id + gridDim.x);
-
-        // what the hysteresis is at this scale, and 2 * 1.25 v u for pieces below the smallest half
-        const float c0 = fmaf(1.001e-6f * sc, sc, 2.5f * V * 5.9604645e-8f);
 
         // Scores of item `it` (unit pl, token group tg) for this lane's token: this lane (half h) holds
         // dims DL*h .. DL*h + DL-1 of the unit's codebooks, cut into two halves each; the accumulators start from |c|^2.
@@ -1060,13 +1080,9 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
                 } else {
                     bi = __float_as_uint(m1) & 15u;
                 }
-                const float mag = xx + cmax[WIDE ? 0 : pl];
-                // 2 * [ (v+1)u (|c|^2) + 12u (what the pieces leave: 8u of x, 2u of c, where subnormal u) + 2.02 * 17 NM u (16 NM products
-                //       and NM accumulators, each within u of a partial sum below 2.02 mag) + 2(v+2)u (the reference's own chain) ]
-                //       = 2 * {57, 98, 178} u  for v = {2, 4, 8}; WIDE {57, 63, 109}
-                constexpr float A2 = 2.0f * ((V + 1) + 12.0f + 2.02f * (17 * NM) + 2 * (V + 2)) * 5.9604645e-8f;
                 constexpr float B2 = 2.0f * 16.0f * 2.3841858e-7f;               // 2 * 2^(4-22)
-                const float thr = fmaf(A2, mag, fmaf(B2, fabsf(m2), c0));
+                const float mag = xx + fix[WIDE ? 0 : pl];
+                const float thr = fmaf(half_margin(V, NM), mag, B2 * fabsf(m2));
                 // NaN anywhere makes a compare false, which counts as "not safe"; beyond 1e9 a half may have run out (and see half_scale)
                 const bool safe = ((m2 - m1) > thr) && (mag < 1e9f);
                 need |= (safe ? 0u : 1u) << (WIDE ? tg : it);
@@ -1230,11 +1246,11 @@ __global__ __launch_bounds__(CCS_THREADS, (V == 8 && !WIDE && TTOK == 128) ? 2 :
 // the codebook before it is searched; search and gather, us a pass at N = 8192, inputs and outputs in turn, before / now: 64 centroids, v = 4 K = 768
 // 102.4 / 95, K = 3072 168 / 147, v = 2 73.8 / 69.8, v = 8 31.2 / 28.5, v = 16 30.9 / 27.8, v = 32 37.5 / 32.6; 200 centroids 121.7 / 101;
 // 64 centroids, N = 1000 22.0 / 18.4.
-//   aux  [CB][groups][NM][64 lanes] uint4, then cn [CB][groups][2 h][16] |c|^2 (3e38 past the last centroid)
+//   aux  [CB][groups][NM][64 lanes] uint4, then cn [CB][groups][2 h][16] |c|^2 (3e38 past the last centroid), scale [CB], fixed [CB]
 // =============================================================================================
 template <uint32_t V>
 __global__ void ccs_prep_many_kernel(const float* __restrict__ cent, const float* __restrict__ cnmax, uint4* __restrict__ aux,
-                                     float* __restrict__ cn32, float* __restrict__ scale, uint32_t C)
+                                     float* __restrict__ cn32, float* __restrict__ scale, float* __restrict__ fixed, uint32_t C)
 {
     constexpr uint32_t DL = V / 2, NM = ccs_many_nm(V);
     const uint32_t cb = blockIdx.x, grp = blockIdx.y, groups = gridDim.y, lane = threadIdx.x;
@@ -1242,8 +1258,11 @@ __global__ void ccs_prep_many_kernel(const float* __restrict__ cent, const float
     const uint32_t cid = 32 * grp + 16 * h + r;
     const bool real = cid < C;
     const float* cp = cent + ((size_t)cb * C + (real ? cid : 0)) * V;
-    const float sc = half_scale(cnmax + cb, 1);
-    if (grp == 0 && lane == 0) scale[cb] = sc;
+    const float sc = half_scale(cnmax[cb]);
+    if (grp == 0 && lane == 0) {
+        scale[cb] = sc;
+        fixed[cb] = half_fixed<V, NM>(cnmax[cb], sc);
+    }
     uint32_t pc[DL][2];  // pieces ch, cm of -2c
 #pragma unroll
     for (uint32_t d = 0; d < DL; ++d) {
@@ -1344,7 +1363,7 @@ struct CcsManyShape {
 template <int V, int IDX_BITS>
 __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* __restrict__ x, const float* __restrict__ cent,
                                                                   const uint4* __restrict__ aux, const float* __restrict__ cn32,
-                                                                  const float* __restrict__ cnmax, const float* __restrict__ scale,
+                                                                  const float* __restrict__ scale, const float* __restrict__ fixed,
                                                                   uint8_t* __restrict__ idx,
                                                                   uint32_t N, uint32_t K, uint32_t CB, uint32_t C,
                                                                   uint32_t idx_row_bytes, int idx_tiled, int vec_ok, uint32_t tiles_cb)
@@ -1415,8 +1434,7 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
         // pieces of the lane's activations and |x|^2, at the codebook's scale
         v4u bop[TG][NB];
         float sqs[TG];
-        const float sc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(scale[cb]))), cmax = cnmax[cb] * sc * sc;
-        const float c0 = fmaf(1.001e-6f * sc, sc, 2.5f * V * 5.9604645e-8f);  // see ccs_f16_kernel
+        const float sc = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(scale[cb]))), fix = fixed[cb];
 #pragma unroll
         for (int tg = 0; tg < TG; ++tg) {
             const float* src = tile + (32 * tg + j) * PITCH + cbl * V + DL * h;
@@ -1518,20 +1536,17 @@ __global__ __launch_bounds__(CCS_THREADS, 2) void ccs_many_kernel(const float* _
             auto swap = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_permlane32_swap(a, b, false, false); };
             const auto s1 = swap(__float_as_uint(m1[2 * q]), __float_as_uint(m1[2 * q + 1])), s2 = swap(__float_as_uint(m2[2 * q]), __float_as_uint(m2[2 * q + 1]));
             const auto sg = swap(grp[2 * q], grp[2 * q + 1]), sx = swap(__float_as_uint(sqs[2 * q]), __float_as_uint(sqs[2 * q + 1]));
-            const float mag = __uint_as_float(sx[0]) + __uint_as_float(sx[1]) + cmax;
+            const float mag = __uint_as_float(sx[0]) + __uint_as_float(sx[1]) + fix;
             // (equal tagged minima give second == smallest, which fails the margin test)
             const float lo1 = __uint_as_float(s1[0]), hi1 = __uint_as_float(s1[1]);
             const float best = vmin(lo1, hi1), second = vmin3(vmax(lo1, hi1), __uint_as_float(s2[0]), __uint_as_float(s2[1]));
             const bool up = hi1 < lo1;
             found[q] = (__float_as_uint(best) & 15u) + (up ? 16u : 0u) + 32u * (up ? sg[1] : sg[0]);
-            // 2 * [ (v+1)u (|c|^2) + 12u (what the pieces leave) + 2.02 * 17 NM u (16 NM products and NM accumulators, each within u of a
-            //       partial sum below 2.02 mag) + 2(v+2)u (the reference's own chain) ], and the tags
             // (What this takes for granted of the matrix core, launch_diag_mfma_error measures on chains of three instructions that
             // start from any accumulator: v = 16 and 32 are chains of four and eight, which three in a row cover, whose errors add up.  The
             // device stays below 25.5 u per chain of three, which makes 51 and 76.5 of the 137 and 275 u allowed here.)
-            constexpr float A2 = 2.0f * ((V + 1) + 12.0f + 2.02f * (17 * NM) + 2 * (V + 2)) * 5.9604645e-8f;
             constexpr float B2 = 2.0f * 16.0f * 2.3841858e-7f;  // 2 * 2^(4-22)
-            const float thr = fmaf(A2, mag, fmaf(B2, fabsf(second), c0));
+            const float thr = fmaf(half_margin(V, NM), mag, B2 * fabsf(second));
             // NaN anywhere makes a compare false, which counts as "not safe"; beyond 1e9 a half may have run out (and see half_scale)
             fail[q] = !((second - best) > thr && mag < 1e9f);
         }
@@ -1843,14 +1858,12 @@ int launch_ccs_f16_tt(Ctx* ctx, const AmmGeom& g, const float* d_x, const float*
     const uint32_t row = x_cols ? x_cols : g.K;  // floats per activation row
     const uint32_t tiles_x = x_cols ? x_cols / S::TF : tiles_cb;
     const int vec_ok = (row % 4 == 0) && ((reinterpret_cast<uintptr_t>(d_x) & 15) == 0);
-    const float* aux = d_cent + (size_t)g.CB * g.C * g.v;
-    const float* cnmax = aux + ccs_aux_floats(g);
-    const float* cnmax_pad = cnmax + g.CB + (size_t)(g.CB_pad / 2) * (g.v + 1) * 64;
     const float* bf = d_cent + ccs_f16_offset(g);
     const uint4* aux_b = reinterpret_cast<const uint4*>(bf);
     const float* cn16 = bf + ccs_f16_units(g) * ccs_f16_nm(V, WIDE) * 64 * 4;
-    const float* scale = cn16 + ccs_f16_units(g) * 2 * 16;
-    hipLaunchKernelGGL((ccs_f16_kernel<V, WIDE, TTOK>), grid, dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent, aux_b, cn16, scale, cnmax_pad,
+    const float* plain = cn16 + ccs_f16_units(g) * 2 * 16;
+    const float* scale = plain + ccs_f16_units(g) / 8;
+    hipLaunchKernelGGL((ccs_f16_kernel<V, WIDE, TTOK>), grid, dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent, aux_b, cn16, plain, scale, scale + g.CB_pad,
                        d_idx, n, row, g.CB, g.C, g.idx_row_bytes, (int)g.idx_tiled, vec_ok, tiles_cb, total, tiles_x);
     return hip_check(ctx, hipGetLastError(), "ccs_f16_kernel launch");
 }
@@ -1884,12 +1897,11 @@ int launch_ccs_many(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d
     const uint64_t total = (uint64_t)((n + S::TT - 1) / S::TT) * tiles_cb;
     if (total > 0x7FFFFFFFull) return set_error(ctx, PIMDL_ERR_INVALID, "ccs: too many tiles");
     const int vec_ok = (g.K % 4 == 0) && ((reinterpret_cast<uintptr_t>(d_x) & 15) == 0);
-    const float* cnmax = d_cent + (size_t)g.CB * g.C * g.v + ccs_aux_floats(g);
     const float* many = d_cent + ccs_f16_offset(g);
     const float* cn32 = many + ccs_many_groups(g) * ccs_many_nm(V) * 64 * 4;
     const float* scale = cn32 + ccs_many_groups(g) * 32;
     hipLaunchKernelGGL((ccs_many_kernel<V, IDX_BITS>), dim3((uint32_t)total), dim3(CCS_THREADS), 0, ctx->stream, d_x, d_cent,
-                       reinterpret_cast<const uint4*>(many), cn32, cnmax, scale, d_idx, n, g.K, g.CB, g.C, g.idx_row_bytes,
+                       reinterpret_cast<const uint4*>(many), cn32, scale, scale + g.CB, d_idx, n, g.K, g.CB, g.C, g.idx_row_bytes,
                        (int)g.idx_tiled, vec_ok, tiles_cb);
     return hip_check(ctx, hipGetLastError(), "ccs_many_kernel launch");
 }
@@ -2201,7 +2213,7 @@ int launch_ccs_prep(Ctx* ctx, const AmmGeom& g, float* d_cent)
         auto prep = g.v == 2 ? ccs_prep_many_kernel<2> : g.v == 4 ? ccs_prep_many_kernel<4> : g.v == 8 ? ccs_prep_many_kernel<8>
                   : g.v == 16 ? ccs_prep_many_kernel<16> : ccs_prep_many_kernel<32>;
         hipLaunchKernelGGL(prep, dim3(g.CB, (g.C + 31) / 32), dim3(64), 0, ctx->stream, d_cent, cnmax, reinterpret_cast<uint4*>(many), cn32,
-                           cn32 + ccs_many_groups(g) * 32, g.C);
+                           cn32 + ccs_many_groups(g) * 32, cn32 + ccs_many_groups(g) * 32 + g.CB, g.C);
         rc = hip_check(ctx, hipGetLastError(), "ccs_prep_many_kernel launch");
     }
     if (rc || !ccs_has_f16(g)) return rc;
@@ -2209,11 +2221,12 @@ int launch_ccs_prep(Ctx* ctx, const AmmGeom& g, float* d_cent)
     uint4* aux_b = reinterpret_cast<uint4*>(bf);
     const bool wide = ccs_f16_wide(g);
     float* cn16 = bf + ccs_f16_units(g) * ccs_f16_nm(g.v, wide) * 64 * 4;
-    float* scale = cn16 + ccs_f16_units(g) * 2 * 16;
+    float* plain = cn16 + ccs_f16_units(g) * 2 * 16;
+    float* scale = plain + ccs_f16_units(g) / 8;
     const dim3 pg((uint32_t)ccs_f16_units(g)), pb(64);
 #define PIMDL_PREP_F16(V_)                                                                                        \
-    if (wide) hipLaunchKernelGGL((ccs_prep_f16_kernel<V_, true>), pg, pb, 0, ctx->stream, d_cent, cnmax, aux_b, cn16, scale, g.CB, g.C); \
-    else hipLaunchKernelGGL((ccs_prep_f16_kernel<V_, false>), pg, pb, 0, ctx->stream, d_cent, cnmax, aux_b, cn16, scale, g.CB, g.C);
+    if (wide) hipLaunchKernelGGL((ccs_prep_f16_kernel<V_, true>), pg, pb, 0, ctx->stream, d_cent, cnmax, aux_b, cn16, plain, scale, scale + g.CB_pad, g.CB, g.C); \
+    else hipLaunchKernelGGL((ccs_prep_f16_kernel<V_, false>), pg, pb, 0, ctx->stream, d_cent, cnmax, aux_b, cn16, plain, scale, scale + g.CB_pad, g.CB, g.C);
     switch (g.v) {
         case 2: PIMDL_PREP_F16(2) break;
         case 4: PIMDL_PREP_F16(4) break;

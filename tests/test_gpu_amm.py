@@ -586,6 +586,60 @@ def test_search_where_distances_overflow(ctx, v, C, length):
     amm.close()
 
 
+def _search_us(ctx, cent, x):
+    """Shortest of several timings of the search alone."""
+    import torch
+    CB, C, v = cent.shape
+    n = x.shape[0]
+    amm = ctx.amm(cent, np.zeros((CB, C, 16), np.int8), np.float32(1.0), None, max_n=n)
+    xd, out = torch.from_numpy(x).cuda(), torch.empty((n, 16), device="cuda")
+    torch.cuda.synchronize()
+    us = min(amm.profile(xd.data_ptr(), n, out.data_ptr(), warmup=20, iters=20)["ccs_ms"] for _ in range(5)) * 1e3
+    amm.close()
+    return us
+
+
+@pytest.mark.parametrize("v,C", [(2, 16), (4, 16), (8, 16), (4, 32)])
+def test_search_of_small_codebooks_beside_a_large_one(ctx, v, C):
+    """One codebook in 16 a million times as large as the others: its neighbours are searched as they would be without it, not replayed.  The
+    time of a launch in which one in 16 may be, against the same launch without a large codebook; replays of the whole tile take 2.3 to 2.8 times."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    rng = np.random.default_rng(6200 + v + C)
+    N, CB = 8192, 3072 // v
+    cent = rng.standard_normal((CB, C, v), dtype=np.float32)
+    x = rng.standard_normal((N, CB, v), dtype=np.float32)
+    plain = _search_us(ctx, cent, x.reshape(N, -1))
+    cent[5::16] *= np.float32(1e6)
+    x[:, 5::16] *= np.float32(1e6)
+    beside = _search_us(ctx, cent, x.reshape(N, -1))
+    print(f"v {v}, {C} centroids: {plain:.1f} us, beside large codebooks {beside:.1f}")
+    assert beside < 1.5 * plain, (plain, beside)
+    rows = np.arange(0, N, 64)
+    amm = ctx.amm(cent, np.zeros((CB, C, 4), np.int8), np.float32(1.0), None, max_n=N)
+    got = amm.index_calculation(x.reshape(N, -1))[rows]
+    assert np.array_equal(got, oracle.index_calculation(x.reshape(N, -1)[rows], cent, v, threads=THREADS))
+    amm.close()
+
+
+@pytest.mark.parametrize("v,C", [(2, 16), (4, 16), (8, 16), (4, 32)])
+def test_search_of_rows_longer_than_large_centroids(ctx, v, C):
+    """Centroids of about 3000, every hundredth row of 3e5 in each dimension: far enough from a tie in every codebook but a few, and inside the range
+    that halves have at the codebooks' scale.  The time against the same launch without such rows; with their replays it is 1.5 to 1.8
+    times."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    rng = np.random.default_rng(6300 + v + C)
+    N, CB = 8192, 3072 // v
+    cent = rng.standard_normal((CB, C, v), dtype=np.float32) * np.float32(3000)
+    x = rng.standard_normal((N, CB * v), dtype=np.float32) * np.float32(3000)
+    plain = _search_us(ctx, cent, x)
+    x[::100] = np.sign(x[::100]) * np.float32(3e5)
+    beyond = _search_us(ctx, cent, x)
+    print(f"v {v}, {C} centroids: {plain:.1f} us, with long rows {beyond:.1f}")
+    assert beyond < 1.25 * plain, (plain, beyond)
+
+
 @pytest.mark.parametrize("v,C", [(4, 16), (2, 16), (8, 16), (4, 32)])
 def test_search_with_non_finite_values(ctx, v, C):
     """NaN / Inf / near-overflow values in activations and centroids take the exact path and match
