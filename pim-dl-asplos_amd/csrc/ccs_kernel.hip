@@ -707,8 +707,8 @@ __device__ __forceinline__ uint32_t half_piece(float& a)
 // than 1024, else what makes the longest one shorter than 1, and never less than 2^-48: what a search accepts, |x|^2 < 1e9 at this
 // scale, is then below 8e37 as it came, and no distance of the reference overflows (where one does, its scan stays where it is, and only a
 // replay says so).  The longest centroids of a codebook that is not replayed anyway, of 1e18, are 3553 at that scale.  (NaN, of a codebook that
-// is: 1.)  Length 1 leaves activations all of the range of halves and costs nothing: A m, which the margin has of centroids of length 1, is 20 times what
-// it has of subnormal pieces.  And a scale of the codebook's own: one for a tile left small codebooks beside a large one few bits, and
+// is: 1.)  Length 1 leaves activations all of the range of halves and costs little: A m, which the margin has of centroids that long, is ten
+// times what it has of subnormal pieces and more.  And a scale of the codebook's own: one for a tile left small codebooks beside a large one few bits, and
 // replayed them.  us of search, N = 8192, K = 3072, v = 4, with a scale for 16 codebooks that makes them shorter than 1024 / as it is: one codebook in
 // 16 1e4 times as large as the others 30.4 / 23.9, a million times 59.2 / 23.2; centroids of 1000, every hundredth row of 3e5 36.0 / 23.0.
 __device__ __forceinline__ float half_scale(float m)
@@ -719,15 +719,20 @@ __device__ __forceinline__ float half_scale(float m)
 }
 
 // The margin of a search is A (|x|^2 + fixed) + B |second smallest score|, with fixed = m and, over A, what the hysteresis is at scale sc and
-// 2 * 1.25 v u for pieces below the smallest half (u = 2^-24);
-//   A = 2 * [ (v+1)u (|c|^2) + 12u (what the pieces leave: 8u of x, 2u of c, where subnormal u) + 2.02 * 17 NM u (16 NM products
+// S = 2 u min(1.25 v, 2 sqrt(v m) + v / 32) for pieces below the smallest half (u = 2^-24);
+//   A = 2 * [ (v+1)u (|c|^2) + 12u (what the pieces leave: 8u of x, 2u of c, where subnormal 2u) + 2.02 * 17 NM u (16 NM products
 //       and NM accumulators, each within u of a partial sum below 2.02 (|x|^2 + m)) + 2(v+2)u (the reference's own chain) ]
 //     = 2 * {57, 98, 178} u  for v = {2, 4, 8}; 17 centroids and more {57, 63, 109}
+// A subnormal piece leaves up to u of x_i, which meets 2 c_i, and u / 2 of 2 c_i, which meets x_i: u sum (2 |c_i| + |x_i| / 2).  With 2 |c_i| <= 1 + c_i^2
+// and |x_i| / 2 <= (1 + x_i^2) / 4 that is 1.25 v u + u (|c|^2 + |x|^2 / 4); with sum |c_i| <= sqrt(v m) and |x_i| / 2 <= 1 / 32 + 2 x_i^2 it is u (2 sqrt(v m) +
+// v / 32) + 2u |x|^2, which is less for small centroids: of 0.01 with activations to match, search as above, 45.7 / 41.5
+// us, v = 8 41.5 / 29.7.
 constexpr float half_margin(int v, int nm) { return 2.0f * ((v + 1) + 12.0f + 2.02f * (17 * nm) + 2 * (v + 2)) * 5.9604645e-8f; }
 template <uint32_t V, uint32_t NM>
 __device__ __forceinline__ float half_fixed(float m, float sc)
 {
-    return fmaf(1.0f / half_margin(V, NM), fmaf(1.001e-6f * sc, sc, 2.5f * V * 5.9604645e-8f), m * sc * sc);
+    const float ms = m * sc * sc, pieces = fminf(1.25f * V, fmaf(2.001f, sqrtf((float)V * ms), V / 32.0f));
+    return fmaf(1.0f / half_margin(V, NM), fmaf(1.001e-6f * sc, sc, 2.0f * 5.9604645e-8f * pieces), ms);
 }
 
 // K-slot registers (two half K-slots each, four registers per MFMA) of lane (row i, half kh).  The lane

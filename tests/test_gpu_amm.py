@@ -599,6 +599,47 @@ def _search_us(ctx, cent, x):
     return us
 
 
+@pytest.mark.parametrize("v,C", [(2, 16), (4, 16), (8, 16), (2, 32), (4, 20), (8, 32), (2, 64), (4, 33), (16, 16), (32, 40)])
+@pytest.mark.parametrize("size", [2e-4, 2e-3, 0.01, 0.05, 0.3])
+def test_search_of_small_centroids(ctx, v, C, size):
+    """Centroids and activations whose pieces are subnormal halves, one in 100 sub-vectors close to the middle of two centroids (off it by
+    up to three times the hysteresis), activations from a hundredth to a hundred times the centroids' size: every index against the reference's
+    scan."""
+    rng = np.random.default_rng(int(1e6 * size) + 10 * v + C)
+    N, CB = 1500, 37
+    cent = (rng.standard_normal((CB, C, v)) * size).astype(np.float32)
+    x = (rng.standard_normal((N, CB, v)) * size).astype(np.float32)
+    x[::9] *= np.float32(100)
+    x[4::9] *= np.float32(0.01)
+    on = rng.random((N, CB)) < 0.01
+    cbi, a = np.nonzero(on)[1], rng.integers(0, C, on.sum())
+    b = (a + 1 + rng.integers(0, C - 1, on.sum())) % C
+    between = (cent[cbi, b] - cent[cbi, a]).astype(np.float64)
+    gap = rng.uniform(-3e-6, 3e-6, (on.sum(), 1))      # of the two squared distances
+    x[on] = cent[cbi, a] + between * (0.5 + gap / (2 * (between ** 2).sum(-1, keepdims=True)))
+    x = x.reshape(N, CB * v)
+    want = oracle.index_calculation(x, cent, v, threads=THREADS)
+    amm = ctx.amm(cent, np.zeros((CB, C, 4), np.int8), np.float32(1.0), None, max_n=N)
+    for tile in (0,) if C > 32 or v > 8 else (64, 128):
+        amm.set_tuning(search_token_tile=tile)
+        got = amm.index_calculation(x)
+        assert np.array_equal(got, want), f"tile {tile}: {(got != want).sum()} of {got.size} differ"
+    amm.close()
+
+
+def test_search_of_small_centroids_is_not_all_replays(ctx):
+    """Centroids of 0.01 in 8 dimensions: nearest and second nearest are as often within the hysteresis as they are, but what the margin
+    allows for subnormal halves is in proportion to the centroids.  1.5 times the time of a launch with centroids of 1, and 1.9 to 2.1 times with an
+    allowance of its own for any size."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    rng = np.random.default_rng(6100)
+    cent, x = rng.standard_normal((384, 16, 8), dtype=np.float32), rng.standard_normal((8192, 3072), dtype=np.float32)
+    usual, small = _search_us(ctx, cent, x), _search_us(ctx, cent * np.float32(0.01), x * np.float32(0.01))
+    print(f"centroids of 1 {usual:.1f} us, of 0.01 {small:.1f}")
+    assert small < 1.7 * usual, (usual, small)
+
+
 @pytest.mark.parametrize("v,C", [(2, 16), (4, 16), (8, 16), (4, 32)])
 def test_search_of_small_codebooks_beside_a_large_one(ctx, v, C):
     """One codebook in 16 a million times as large as the others: its neighbours are searched as they would be without it, not replayed.  The
