@@ -175,8 +175,9 @@ PIMDL_API int pimdl_amm_create_with(pimdl_ctx* ctx, const pimdl_amm_desc* desc, 
  * centroids that was created without one: also 48 or 64, 0 = the launch picks).  An int8 operator of 17..32 centroids
  * created without any of the gather's settings runs on the byte adder until settings of the sparse kernel are named here
  * (gather_kernel, its token_item, cb_per_slice, xcd_col_split or col_block), and again when none is: the choice
- * pimdl_amm_create_with makes.  The first such change lays out a second table, which cannot happen while the context's
- * stream is being captured.  pimdl_amm_get_tuning reports the operator's current settings (0 where the library still
+ * pimdl_amm_create_with makes.  An int8 operator of up to 16 centroids on the sparse kernel that was created without col_block takes
+ * the column tile, 48 or 64, that has the settings named here, for as long as they are.  The first such change lays out a second table, which
+ * cannot happen while the context's stream is being captured.  pimdl_amm_get_tuning reports the operator's current settings (0 where the library still
  * chooses per launch); creating an operator with them gives the same choices. */
 PIMDL_API int pimdl_amm_set_tuning(pimdl_amm* amm, const pimdl_amm_tuning* tuning);
 PIMDL_API int pimdl_amm_get_tuning(const pimdl_amm* amm, pimdl_amm_tuning* tuning);

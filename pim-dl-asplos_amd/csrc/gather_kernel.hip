@@ -895,6 +895,9 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
         // divide takes 48, which operators of such outputs share in a gather launch (plan_side_by_side).
         auto pick_sparse = [&] {
             if (col_block_hint) return col_block_hint / 16;
+            // (settings of the caller that only one of the two has: see apply_runtime_tuning)
+            if (tune.cb_per_slice == 64) return 3u;
+            if (tune.cb_per_slice == 16 && tune.token_item == 512) return 4u;
             if (M % 48 == 0 && M % 64 != 0) return 3u;
             return sparse_launch_cost(3, d.max_n, M, g->CB_pad, cus) < sparse_launch_cost(4, d.max_n, M, g->CB_pad, cus) - 1e-9 ? 3u : 4u;
         };
@@ -918,7 +921,7 @@ bool plan_geometry(const pimdl_amm_desc& d, uint32_t num_cus, AmmGeom* g, std::s
         g->cols_named = col_block_hint != 0 || tune.gather_kernel == PIMDL_GATHER_ONEHOT;
         g->gq = 4;
         g->cb_per_slice = 16;
-        g->col_block = 16 * g->q;
+        g->col_block = g->home_block = 16 * g->q;
         g->gather_threads = 256;
         g->tokens_per_wg = 256;
         g->row_pitch = 16;

@@ -600,14 +600,33 @@ static int geometry_as(const Amm* a, uint32_t kind, AmmGeom* g)
     return PIMDL_OK;
 }
 
-// The operator's table as geometry_as(kind) = g has it.  The second one is laid out from the first when it is first asked for and
+// The geometry of an operator whose tile of the sparse kernel (up to 16 centroids) the library has chosen, with the settings of t: in the tile
+// that it was created with, or in the other where only that one has them.
+static bool geometry_with(const Amm* a, const pimdl_amm_tuning& t, AmmGeom* g, std::string* why)
+{
+    for (uint32_t block : {a->g.home_block, a->g.home_block == 48 ? 64u : 48u}) {
+        pimdl_amm_tuning s = t;
+        s.gather_kernel = PIMDL_GATHER_SPARSE;
+        s.col_block = block;
+        std::string other;
+        memset(g, 0, sizeof(*g));
+        if (plan_geometry(a->desc, a->ctx->prop.multiProcessorCount, g, block == a->g.home_block ? why : &other, &s)) {
+            g->cols_named = 0;
+            g->home_block = a->g.home_block;
+            return true;
+        }
+    }
+    return false;
+}
+
+// The operator's table as g has it, one of geometry_as or geometry_with.  The second one is laid out from the first when it is first asked for and
 // kept until the operator is destroyed: graphs captured before hold the other's address.
 static int table_as(Amm* a, const AmmGeom& g, void** table)
 {
     Ctx* ctx = a->ctx;
-    *table = a->g.gather_kind == g.gather_kind ? a->d_lut : a->d_lut_other;
+    *table = a->g.gather_kind == g.gather_kind && (g.gather_kind == 0 || a->g.col_block == g.col_block) ? a->d_lut : a->d_lut_other;
     if (*table) return PIMDL_OK;
-    // (what the operator has is the byte adder's, which it was created with)
+    // (what the operator has is what it was created with: the byte adder's, or the sparse kernel's)
     int rc = activate(ctx);
     if (rc) return rc;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -619,11 +638,15 @@ static int table_as(Amm* a, const AmmGeom& g, void** table)
     std::vector<int8_t> have, canonical, want;
     try {
         have.resize(a->lut_bytes);
-        canonical.resize((size_t)g.CB * g.C * g.M);
+        if (a->g.gather_kind == 0) canonical.resize((size_t)g.CB * g.C * g.M);
         want.assign(bytes, 0);
         if ((rc = hip_check(ctx, hipMemcpy(have.data(), a->d_lut, a->lut_bytes, hipMemcpyDeviceToHost), "D2H lut"))) return rc;
-        untile_lut_rows(have.data(), canonical.data(), a->g);
-        retile_lut_onehot(canonical.data(), want.data(), g);
+        if (a->g.gather_kind == 0) {
+            untile_lut_rows(have.data(), canonical.data(), a->g);
+            retile_lut_onehot(canonical.data(), want.data(), g);
+        } else {
+            move_lut_onehot(have.data(), a->g, want.data(), g);
+        }
     } catch (...) {
         return set_error(ctx, PIMDL_ERR_NOMEM, "host staging of a table of %zu bytes failed", bytes);
     }
@@ -776,7 +799,9 @@ int pimdl_amm_set_tuning(pimdl_amm* a, const pimdl_amm_tuning* t)
         return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_set_tuning: col_block and gather_kernel fix the resident table; "
                                                  "create the operator with them (pimdl_amm_create_with)");
     std::string why;
-    if (!apply_runtime_tuning(&g, *t, &why)) return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_set_tuning: %s", why.c_str());
+    const bool any_tile = g.gather_kind == 2 && g.C <= 16 && !g.cols_named && !t->col_block;
+    if (!(any_tile ? geometry_with(a, *t, &g, &why) : apply_runtime_tuning(&g, *t, &why)))
+        return set_error(ctx, PIMDL_ERR_INVALID, "pimdl_amm_set_tuning: %s", why.c_str());
     void* table;
     if (int rc = table_as(a, g, &table)) return rc;
     if (table != a->d_lut) std::swap(a->d_lut, a->d_lut_other);

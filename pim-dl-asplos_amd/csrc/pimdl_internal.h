@@ -43,6 +43,7 @@ struct AmmGeom {
     uint32_t col_block;     // columns per workgroup (int8: 16*q -- the byte adder picks its own at launch, see cols --, fp32: 4*q)
     uint32_t cols;          // byte adder of up to 64 centroids: columns per item that the caller has named (0: the launch picks)
     uint32_t cols_named;    // ... at creation; one-hot kernels: the caller has named the column tile, or the dense kernel
+    uint32_t home_block;    // one-hot kernels: col_block at creation
     uint32_t row_pitch;     // bytes between LUT rows in LDS
     uint32_t gq;            // int8: codebooks per lane group per slice
     uint32_t cb_per_slice;
@@ -83,7 +84,8 @@ struct Amm {
     float* d_centroids;  // [CB][C][v], then the derived search data (ccs_centroid_bytes)
     void* d_lut;         // tiled
     size_t lut_bytes;
-    void* d_lut_other;   // auto_rows: the table as the kernel that is not in use reads it, once it has been needed (else null)
+    void* d_lut_other;   // the table as the kernel that is not in use reads it (auto_rows), or in the sparse kernel's other column tile, once it
+                         // has been needed (else null)
     float* d_scales;     // int8: scales
     uint32_t nscales;
     float* d_bias;       // [M]

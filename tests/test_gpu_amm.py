@@ -1067,6 +1067,75 @@ def test_tuning_of_an_operator_the_library_gave_to_the_byte_adder(ctx):
     amm.close()
 
 
+@pytest.mark.parametrize("N,C,M,home", [(9856, 16, 1280, 48), (2304, 16, 768, 64), (8200, 8, 1001, 48), (600, 11, 128, 48)])
+def test_settings_that_one_column_tile_has(ctx, N, C, M, home):
+    """Slices of 64 codebooks are the 48-column tile's, and eight waves with slices of 16 the 64-column one's: an operator whose tile the library
+    chooses has either, whichever tile suits it alone, when it is created and afterwards; a tile that the caller names does not change."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the library's choice")
+    import torch
+    CB, v = 128, 2
+    x, cent, lut, bias = make_case(6400 + M, 300, CB * v, v, C, M)
+    want = oracle.amm_cpu(x, cent, lut, bias, v, 0.01, 0.0, threads=THREADS)[0]
+    local = pimdl.Context(0)
+
+    def make(**tuning):
+        return local.amm(cent, lut, np.float32(0.01), bias, max_n=N, tuning=tuning)
+
+    def check(op, block, slices=0):
+        assert op.geometry()["col_block"] == block == op.tuning()["col_block"]
+        assert np.array_equal(op.run(x).view(np.uint32), want.view(np.uint32))
+        if slices:
+            assert "<%d, 4, %d, 8" % (block // 16, slices) in op.last_gather_kernel(), op.last_gather_kernel()
+
+    amm = make(**({"gather_kernel": pimdl.GATHER_SPARSE} if C == 8 else {}))
+    if local.device_info()["compute_units"] == 256:
+        check(amm, home)
+    home = amm.geometry()["col_block"]
+    stream = torch.cuda.Stream()
+    xd, out = torch.from_numpy(x).cuda(), torch.empty(300, M, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        local.set_stream(stream.cuda_stream)
+        amm.run_ptr(xd.data_ptr(), 300, out.data_ptr())
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+            amm.run_ptr(xd.data_ptr(), 300, out.data_ptr())
+            with pytest.raises(pimdl.PimdlError):   # the other table cannot be laid out here
+                amm.set_tuning(**({"token_item": 512, "cb_per_slice": 16} if home == 48 else {"token_item": 256, "cb_per_slice": 64}))
+            assert amm.geometry()["col_block"] == home
+    local.set_stream(None)
+    for _ in range(2):
+        for token_item, slices, block in ((512, 16, 64), (512, 64, 48), (512, 32, home), (256, 64, 48), (128, 32, home), (0, 0, home)):
+            amm.set_tuning(token_item=token_item, cb_per_slice=slices)
+            assert amm.tuning()["token_item"] == token_item and amm.tuning()["cb_per_slice"] == slices
+            check(amm, block, slices if token_item == 512 else 0)
+            tuned = amm.tuning()
+            amm.set_tuning(**tuned)
+            assert amm.tuning() == tuned
+            out.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(out.cpu().numpy(), want), (token_item, slices)
+    for bad in ({"token_item": 512, "cb_per_slice": 48}, {"token_item": 128, "cb_per_slice": 64}, {"col_block": 112 - home}):
+        with pytest.raises(pimdl.PimdlError) as e:
+            amm.set_tuning(**bad)
+        assert e.value.code == pimdl.ERR_INVALID and amm.geometry()["col_block"] == home
+    amm.close()
+    kernel = {"gather_kernel": pimdl.GATHER_SPARSE} if C == 8 else {}
+    for token_item, slices, block in ((512, 16, 64), (512, 64, 48), (256, 64, 48), (512, 32, home)):
+        amm = make(token_item=token_item, cb_per_slice=slices, **kernel)
+        check(amm, block, slices if token_item == 512 else 0)
+        amm.close()
+    for token_item, slices, block in ((512, 16, 48), (512, 64, 64), (256, 64, 64)):
+        with pytest.raises(pimdl.PimdlError) as e:
+            make(token_item=token_item, cb_per_slice=slices, col_block=block, **kernel)
+        assert e.value.code == pimdl.ERR_INVALID
+    local.close()
+
+
 def test_a_graph_captured_before_a_change_of_tables_replays(ctx):
     """A captured run holds the address of the table it was captured with."""
     if kernel_switches():
