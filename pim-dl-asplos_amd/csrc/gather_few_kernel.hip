@@ -8,6 +8,8 @@
 // then takes the time of that chain -- copy, barrier, operands, 32 codebooks further -- however few its tokens are.
 #include <string.h>
 
+#include <algorithm>
+
 #include "gather_common.h"
 #include "search_quad.h"
 
@@ -286,6 +288,12 @@ uint64_t few_table_bytes(uint64_t steps, uint64_t groups) { return steps * 8 * g
 constexpr uint64_t FEW_TABLE_SHARED = 6u << 20;
 // workgroups of the XCD that has the most of them, if an XCD takes every token tile of its column blocks
 uint64_t few_fullest(uint64_t blocks, uint64_t tiles) { return (blocks + 7) / 8 * tiles; }
+// (evenly enough: the XCD that takes one block more has a CU for each of its workgroups, or at most an eighth more than the average;
+// 9 column blocks, N = 3100 10.4 in order, 12.1 by XCD)
+bool few_even(uint64_t blocks, uint64_t tiles, uint64_t cus)
+{
+    return 8 * few_fullest(blocks, tiles) <= cus || 64 * few_fullest(blocks, tiles) <= 9 * blocks * tiles;
+}
 // workgroups that have a CU of their own each (of exactly as many as CUs the last few share some)
 uint64_t few_room(uint64_t cus) { return cus - cus / 16; }
 
@@ -297,10 +305,8 @@ uint64_t few_room(uint64_t cus) { return cus - cus / 16; }
 dim3 few_grid(const FewArgs& f, uint32_t tm, uint32_t tc, uint32_t cus, bool one_hot)
 {
     const uint32_t blocks = f.groups / tc, tiles = (f.N + 16 * tm - 1) / (16 * tm);
-    // (evenly enough: the XCD that takes one block more has a CU for each of its workgroups, or at most an eighth more than the average;
-    // 9 column blocks, N = 3100 10.4 in order, 12.1 by XCD)
     const uint64_t fullest = few_fullest(blocks, tiles);
-    const bool even = 8 * fullest <= cus || 64 * fullest <= 9ull * blocks * tiles;
+    const bool even = few_even(blocks, tiles, cus);
     // (two items of 64 tokens: 4096 -> 1024 9.0 / 9.3, 5120 -> 1280 11.3 / 10.6)
     const bool shared = one_hot && (tm < 4 || tiles > 2) && 8 * fullest <= few_room(cus) && few_table_bytes(f.steps, f.groups) > FEW_TABLE_SHARED;
     const bool by_xcd = tiles > 1 && blocks % 8 != 0 && (shared || (even && (tc > 1 || tiles * blocks > cus)));
@@ -340,6 +346,31 @@ double few_rows_rounds(const AmmGeom& g, uint32_t n, uint64_t cus, uint32_t* ite
     const uint64_t groups = g.M_pad / 16, rounds = ((n + 15) / 16 * groups + cus - 1) / cus;
     *item = n <= 32 && rounds == 2 && groups <= cus ? 32 : rounds >= 4 && groups % 8 == 0 && (n + 63) / 64 * groups <= cus ? 64 : 16;
     return *item == 64 ? 3.4 : (double)rounds;
+}
+
+// Whether a byte adder launch of 33..64 centroids is shorter here than on the large kernel, by the prices of gather_few_wanted and, where the
+// column blocks do not divide by eight, by what one XCD has to do: by XCD the fullest one has the rounds of its own 1/8 of the
+// CUs, and in order the blocks of `tiles` token tiles meet on an XCD, of whose tables what goes beyond 2.5 MB of its L2 takes 0.5 us per MB; the
+// large kernel, in tiles of 128 tokens, takes a fifth longer once its part is more than the L2 of 4 MiB.  us of gather, few / large, blocks x
+// codebooks: 8 x 192 N = 512 4.1 / 6.5, N = 1024 5.7 / 6.5; 5 x 768 N = 816 11.5 / 24.6; 31 x 768 (by XCD, two rounds) N = 256 16.4 / 25.8; 26 x 768
+// N = 160 21.3 / 25.5; not 38 x 192 (by XCD, three rounds) N = 208 7.4 / 6.3; 33 x 192 (in order) N = 128 10.0 / 6.2; 17 x 384 N = 256 13.4 / 9.6; 33 x
+// 384 N = 128 17.3 / 9.6.  Of 1179 launches of 1 .. 75 blocks, 16 .. 1024 codebooks and 16 .. 8192 tokens the kernel that this takes is the shorter one, or
+// less than 4 % longer, in 1082 (853 with one price for all and no more than 192 tokens).
+bool few_rows64_wanted(const AmmGeom& g, uint32_t n, uint64_t cus)
+{
+    uint32_t item;
+    double rounds = few_rows_rounds(g, n, cus, &item), streamed = 0.0;
+    const uint64_t blocks = g.M_pad / 16, tiles = (n + item - 1) / item;
+    const double eighth_mb = (double)g.CB_pad * 64 * 16 * 1e-6 * (double)blocks / 8;
+    // eighths of the table that an XCD reads of so many token tiles in order
+    auto meet = [&](uint64_t t) { return std::min<uint64_t>(t, blocks % 8 == 0 ? 1 : blocks % 4 == 0 ? 2 : blocks % 2 == 0 ? 4 : 8); };
+    if (blocks % 8 != 0) {
+        if (item == 16 && blocks > 8 && tiles > 1 && tiles * blocks > cus && few_even(blocks, tiles, cus))
+            rounds = (double)((8 * few_fullest(blocks, tiles) + cus - 1) / cus);
+        else streamed = 0.5 * std::max(0.0, (double)meet(tiles) * eighth_mb - std::max(2.5, eighth_mb));
+    }
+    const double few = 2.5 + rounds * g.CB_pad * 0.0081 + 0.3 * (rounds - 1) + streamed, large = 2.9 + (g.CB + 15) / 16 * 0.29;
+    return few < ((double)meet((n + 127) / 128) * eighth_mb > 4.2 ? 1.2 * large : large);
 }
 
 // Tokens of an item: 16, 32 or 64.  One-hot tables: as few as leave every workgroup a CU of its own.  A wave then makes operands for fewer tokens, and
@@ -510,14 +541,12 @@ bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
         return 2.7 + g.CB_pad * (bounds ? 0.062 : 0.0137) + pieces * piece < 4.0 + g.CB_pad * (bounds ? 0.14 : 0.07);
     }
     if (g.gather_kind == 0) {
+        if (g.C_tile == 64) return g.idx_bits == 8 && few_rows64_wanted(g, n, cus);
         const uint64_t slices = (g.CB + 15) / 16;
         uint32_t rows_item;
         const double rounds = few_rows_rounds(g, n, cus, &rows_item);
-        const double few = 2.5 + rounds * g.CB_pad * (g.C_tile <= 64 ? 0.0081 : g.C_tile == 128 ? 0.014 : 0.0125) + 0.3 * (rounds - 1);
-        // (64 centroids, more than 200 tokens or so: a few narrow tables would still gain here, but which kernel a batch of that size takes is
-        // something that programs have come to read back -- the fixed-scratch entry point's tests among them)
-        if (g.C_tile == 64 && g.CB_pad > 32 && n > 192) return false;
-        return g.idx_bits == 8 && few < (g.C_tile == 64 ? 2.9 + 0.29 * (double)slices : 3.3 + (double)slices * (0.2 + 0.003 * g.C_tile));
+        const double few = 2.5 + rounds * g.CB_pad * (g.C_tile < 64 ? 0.0081 : g.C_tile == 128 ? 0.014 : 0.0125) + 0.3 * (rounds - 1);
+        return g.idx_bits == 8 && few < 3.3 + (double)slices * (0.2 + 0.003 * g.C_tile);
     }
     if (g.gather_kind == 2 ? g.C_tile == 32 : g.C_tile != 8) return false;  // tables only a tuning asks for
     return g.gather_kind == 2 ? few_column_groups(ctx, g, n) != 0 : wgs <= 2 * cus;

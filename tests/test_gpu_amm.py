@@ -1849,6 +1849,34 @@ def test_float_gathers_take_whole_workgroups_where_the_copies_are_the_chain(ctx)
     assert a < 1.2 * b, (a, b)
 
 
+@pytest.mark.parametrize("CB,M,N,kernel", [
+    (64, 128, 500, "gather_i8_few_kernel<"), (192, 128, 512, "gather_i8_few_kernel<"), (192, 128, 1024, "gather_i8_few_kernel<"),
+    (192, 128, 1040, "gather_i8_kernel<"), (768, 80, 816, "gather_i8_few_kernel<"),     # column blocks that divide by eight, few of them
+    (768, 496, 256, "gather_i8_few_kernel<"),                                           # 31 blocks by XCD, two rounds
+    (192, 600, 208, "gather_i8_kernel<"),                                               # 38 of them, three rounds of an XCD
+    (192, 528, 128, "gather_i8_kernel<"), (384, 265, 250, "gather_i8_kernel<"),         # in order, tables beyond an L2
+])
+def test_gather_of_64_centroids_by_what_an_xcd_has_to_do(ctx, CB, M, N, kernel):
+    """Which of the byte adder's kernels a launch takes, whatever its batch: the rounds of the fullest XCD, and what an XCD reads of the
+    table.  Accumulators and output bits of the oracle with either, nothing behind the output."""
+    import torch
+    v, C = 1, 64
+    x, cent, lut, bias = make_case(6700 + M + N, N, CB * v, v, C, M)
+    want, _, want_acc = oracle.amm_cpu(x, cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)
+    amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=N)
+    _, _, acc = amm.run_debug(x)
+    assert np.array_equal(acc, want_acc)
+    xd, out = torch.from_numpy(x).cuda(), torch.full((N + 2, M), -5.0, device="cuda")
+    torch.cuda.synchronize()
+    amm.run_ptr(xd.data_ptr(), N, out.data_ptr())
+    ctx.synchronize()
+    if ctx.device_info()["compute_units"] == 256 and not kernel_switches():
+        assert amm.last_gather_kernel().startswith(kernel), amm.last_gather_kernel()
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:N].view(np.uint32), want.view(np.uint32)) and (got[N:] == -5.0).all()
+    amm.close()
+
+
 @pytest.mark.parametrize("CB,lut,group,M", [(96, "f32", 0, 2441), (768, "f32", 0, 2441), (96, "i8", 8, 3692)])
 def test_few_tokens_of_64_centroids_take_the_large_gather_where_it_is_shorter(ctx, CB, lut, group, M):
     """93 tokens, gathered piece by piece, took 1.4 to 1.7 times as long as 150 on the large kernel."""

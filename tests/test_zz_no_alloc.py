@@ -86,13 +86,14 @@ def test_noalloc_matches_run_on_two_calls_in_a_row(ctx):
     amm3.close()
 
 
-def test_noalloc_first_call_on_a_fresh_context_allocates_nothing():
+@pytest.mark.parametrize("M,kernel", [(128, "gather_i8_few_kernel<"), (768, "gather_i8_kernel<64,")])
+def test_noalloc_first_call_on_a_fresh_context_allocates_nothing(M, kernel):
     """The entry point on a context and operator that have never seen pimdl_amm_run (nothing has sized the
-    context's scratch buffers for it), with 64 centroids: row-major index rows of one byte per codebook and the
-    byte-adder gather go through the fixed array.  Device memory in use must not change across the calls."""
+    context's scratch buffers for it), with 64 centroids: index rows of one byte per codebook and both of the
+    byte adder's gathers go through the fixed array.  Device memory in use must not change across the calls."""
     import torch
 
-    N, K, v, C, M = 500, 256, 4, 64, 128
+    N, K, v, C = 500, 256, 4, 64
     x, cent, lut, bias = _case(15, N, K, v, C, M)
     idx = oracle.index_calculation(x, cent, v, threads=THREADS)
     want = oracle.dequant(oracle.gather_i8(idx, lut, threads=THREADS), bias, K // v, 0.25, 0.0, 0, threads=THREADS)
@@ -119,7 +120,7 @@ def test_noalloc_first_call_on_a_fresh_context_allocates_nothing():
     fresh.synchronize()
     free2 = torch.cuda.mem_get_info()[0]
     assert free0 == free1 == free2, (free0, free1, free2)
-    assert amm.last_gather_kernel().startswith("gather_i8_kernel<64,")
+    assert amm.last_gather_kernel().startswith(kernel), amm.last_gather_kernel()
     assert np.array_equal(got1.cpu().numpy().view(np.uint32), want.view(np.uint32))
     assert np.array_equal(got2.cpu().numpy().view(np.uint32), want[:200].view(np.uint32))
     # and the existing entry point gives the same bits
