@@ -220,47 +220,41 @@ static int pipe_get(Ctx* ctx, HostPipe** out)
     return PIMDL_OK;
 }
 
-// Per-slot buffers of at least the given sizes (0: that direction is not staged).  The pinned ones are coherent: kernels read and write them too
-// (ring_to_device, ring_to_host).  Only called while the ring is
-// idle (every call that uses it drains it before it returns or before it touches a slot again).
-static int pipe_reserve(Ctx* ctx, HostPipe* hp, size_t in_bytes, size_t out_bytes)
+// Pinned buffers of one direction with at least `bytes` per slot, and device buffers to go with them (`device`; the transfers of table construction
+// have their own device memory).  The pinned ones are coherent: kernels read and write them too (ring_to_device, ring_to_host).  Only called while
+// the ring is idle (every call that uses it drains it before it returns or before it touches a slot again).
+static int pipe_grow(Ctx* ctx, hipStream_t transfers, void** pin, size_t* pin_bytes, float** dev, size_t* dev_bytes, size_t bytes, bool device)
 {
-    int rc = PIMDL_OK;
-    if (in_bytes > hp->in_bytes) {
-        if ((rc = hip_check(ctx, hipStreamSynchronize(hp->s_in), "hipStreamSynchronize(staging in)"))) return rc;
-        if ((rc = hip_check(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize"))) return rc;
+    if (bytes <= *pin_bytes && (!device || bytes <= *dev_bytes)) return PIMDL_OK;
+    int rc = hip_check(ctx, hipStreamSynchronize(transfers), "hipStreamSynchronize(staging)");
+    if (!rc) rc = hip_check(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    if (!rc && bytes > *pin_bytes) {
         for (int s = 0; s < HostPipe::SLOTS; ++s) {
-            if (hp->pin_in[s]) (void)hipHostFree(hp->pin_in[s]);
-            (void)hipFree(hp->d_in[s]);
-            hp->pin_in[s] = nullptr;
-            hp->d_in[s] = nullptr;
+            if (pin[s]) (void)hipHostFree(pin[s]);
+            pin[s] = nullptr;
         }
-        hp->in_bytes = 0;
-        for (int s = 0; s < HostPipe::SLOTS && !rc; ++s) {
-            rc = hip_check(ctx, hipHostMalloc(&hp->pin_in[s], in_bytes, hipHostMallocCoherent), "hipHostMalloc(staging in)");
-            if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&hp->d_in[s]), in_bytes), "hipMalloc(staging in)");
-        }
-        if (rc) return rc;
-        hp->in_bytes = in_bytes;
+        *pin_bytes = 0;
+        for (int s = 0; s < HostPipe::SLOTS && !rc; ++s) rc = hip_check(ctx, hipHostMalloc(&pin[s], bytes, hipHostMallocCoherent), "hipHostMalloc(staging)");
+        if (!rc) *pin_bytes = bytes;
     }
-    if (out_bytes > hp->out_bytes) {
-        if ((rc = hip_check(ctx, hipStreamSynchronize(hp->s_out), "hipStreamSynchronize(staging out)"))) return rc;
-        if ((rc = hip_check(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize"))) return rc;
+    if (!rc && device && bytes > *dev_bytes) {
         for (int s = 0; s < HostPipe::SLOTS; ++s) {
-            if (hp->pin_out[s]) (void)hipHostFree(hp->pin_out[s]);
-            (void)hipFree(hp->d_out[s]);
-            hp->pin_out[s] = nullptr;
-            hp->d_out[s] = nullptr;
+            (void)hipFree(dev[s]);
+            dev[s] = nullptr;
         }
-        hp->out_bytes = 0;
-        for (int s = 0; s < HostPipe::SLOTS && !rc; ++s) {
-            rc = hip_check(ctx, hipHostMalloc(&hp->pin_out[s], out_bytes, hipHostMallocCoherent), "hipHostMalloc(staging out)");
-            if (!rc) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&hp->d_out[s]), out_bytes), "hipMalloc(staging out)");
-        }
-        if (rc) return rc;
-        hp->out_bytes = out_bytes;
+        *dev_bytes = 0;
+        for (int s = 0; s < HostPipe::SLOTS && !rc; ++s) rc = hip_check(ctx, hipMalloc(reinterpret_cast<void**>(&dev[s]), bytes), "hipMalloc(staging)");
+        if (!rc) *dev_bytes = bytes;
     }
-    return PIMDL_OK;
+    return rc;
+}
+static int pipe_reserve_in(Ctx* ctx, HostPipe* hp, size_t bytes, bool device)
+{
+    return pipe_grow(ctx, hp->s_in, hp->pin_in, &hp->pin_in_bytes, hp->d_in, &hp->d_in_bytes, bytes, device);
+}
+static int pipe_reserve_out(Ctx* ctx, HostPipe* hp, size_t bytes, bool device)
+{
+    return pipe_grow(ctx, hp->s_out, hp->pin_out, &hp->pin_out_bytes, hp->d_out, &hp->d_out_bytes, bytes, device);
 }
 
 // Chunk boundaries (first token of each chunk, then n).  Chunks hold about 12 MiB of the wider staged side, in
@@ -318,7 +312,8 @@ static int run_piped(Ctx* ctx, uint32_t K, uint32_t M, const float* in, bool in_
     const uint32_t nchunks = (uint32_t)first.size() - 1;
     uint32_t chunk = 0;  // the largest
     for (uint32_t c = 0; c < nchunks; ++c) chunk = std::max(chunk, first[c + 1] - first[c]);
-    if ((rc = pipe_reserve(ctx, hp, in_host ? chunk * in_row : 0, out_host ? chunk * out_row : 0))) return rc;
+    if (in_host && (rc = pipe_reserve_in(ctx, hp, chunk * in_row, true))) return rc;
+    if (out_host && (rc = pipe_reserve_out(ctx, hp, chunk * out_row, true))) return rc;
 
     auto fail = [&](int code) {  // nothing may stay in flight towards buffers the caller owns
         (void)hipStreamSynchronize(hp->s_in);
@@ -377,16 +372,25 @@ static int run_piped(Ctx* ctx, uint32_t K, uint32_t M, const float* in, bool in_
 // link starts early and little is left to copy when it is done.  Table construction, us a call, table in a buffer used before / a fresh one,
 // pieces of 2 MiB down to 256 KiB: 768 -> 3072 576 / 573, 1024 -> 4096 with 32 centroids 1288 / 2334; 4 MiB, 256 KiB 587 / 586, 1241 / 1763; 4 MiB, 1 MiB
 // 550 / 548, 1200 / 1723; 6 MiB, 512 KiB 590 / 587, 1224 / 1638.  ring_to_device returns once `src` has been read, ring_to_host once
-// the destinations are complete.  Pointers that the CPU cannot read take the runtime's copy.
+// the destinations are complete.  Pointers that the CPU cannot read take the runtime's copy.  So does what goes to the device and is smaller than
+// the first piece: from pageable memory such a copy returns before the device has it, and no launch waits for another one (buffers in turn, as kernels /
+// as copies: 64 -> 64 55 / 41, 512 KiB of weight 130 / 99, 1 MiB 164 / 140, of which 20 are the centroids; weights of 4 MiB and more 355 / 380, 9 MiB
+// 615 / 705).  A slot is as large as the largest call has needed, in powers of two up to a piece.
 constexpr size_t RING_PIECE = 4u << 20, RING_FIRST = 1u << 20;
+static size_t ring_slot(size_t bytes)
+{
+    size_t slot = 64u << 10;
+    while (slot < bytes && slot < RING_PIECE) slot *= 2;
+    return slot;
+}
 
 static int ring_to_device(Ctx* ctx, void* dst, const void* src, size_t bytes)
 {
-    if (is_device_ptr(src)) return hip_check(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, ctx->stream), "copy to the device");
+    if (bytes < RING_FIRST || is_device_ptr(src)) return hip_check(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, ctx->stream), "copy to the device");
     HostPipe* hp;
     int rc = pipe_get(ctx, &hp);
     if (rc) return rc;
-    rc = pipe_reserve(ctx, hp, RING_PIECE, 0);
+    rc = pipe_reserve_in(ctx, hp, ring_slot(bytes), false);
     int s = 0;
     size_t piece = RING_FIRST;
     for (size_t at = 0, len; at < bytes && !rc; at += len, s = (s + 1) % HostPipe::SLOTS, piece = std::min(2 * piece, RING_PIECE)) {
@@ -411,8 +415,8 @@ static int ring_to_host(Ctx* ctx, void* dst, const void* src, size_t bytes, void
     HostPipe* hp;
     int rc = pipe_get(ctx, &hp);
     if (rc) return rc;
-    if ((rc = pipe_reserve(ctx, hp, 0, RING_PIECE))) return rc;
     const size_t total = more ? more_at + more : bytes;
+    if ((rc = pipe_reserve_out(ctx, hp, ring_slot(total), false))) return rc;
     constexpr size_t SLOTS = HostPipe::SLOTS;
     size_t first[SLOTS], len[SLOTS];  // the pieces under way
     size_t queued = 0, taken = 0, at = 0;

@@ -122,7 +122,7 @@ struct HostPipe {
     void* pin_out[SLOTS] = {};
     float* d_in[SLOTS] = {};
     float* d_out[SLOTS] = {};
-    size_t in_bytes = 0, out_bytes = 0;                // per slot
+    size_t pin_in_bytes = 0, pin_out_bytes = 0, d_in_bytes = 0, d_out_bytes = 0;  // per slot
 };
 
 struct Ctx {

@@ -982,6 +982,32 @@ def test_lutgen_through_several_pieces_of_the_ring(ctx, CB, v, C, M, group):
         cent = cent[::-1].copy()
 
 
+def test_lutgen_takes_device_memory_for_its_own_scratch_only(ctx):
+    """A context's first table construction, of a few KB and of 12 MB of weight: device memory for centroids, weight, table and magnitudes, and
+    none for the pinned ring's chunks of a batch (32 MB that no table construction reads)."""
+    import torch
+    rng = np.random.default_rng(31)
+    for K, M, v, C in ((64, 64, 4, 16), (1024, 3072, 4, 16)):
+        cent, weight = rng.standard_normal((K // v, C, v), dtype=np.float32), rng.standard_normal((K, M), dtype=np.float32)
+        want = ctx.lutgen(cent, weight)          # (the kernels' code objects are on the device)
+        fresh = pimdl.Context(0)
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        got = fresh.lutgen(cent, weight)
+        used = before - torch.cuda.mem_get_info()[0]
+        scratch = 4 * (cent.size + weight.size + K // v * ((M + 255) // 256)) + want[0].size
+        assert used <= scratch + (4 << 20), (used, scratch)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        x = rng.standard_normal((3000, K), dtype=np.float32)   # a batch from host buffers has them, after table construction too
+        amm = fresh.amm(cent, got[0], got[1], None, max_n=3000)
+        idx = oracle.index_calculation(x[:50], cent, v, threads=THREADS)
+        out = amm.run(x)
+        assert np.array_equal(out[:50], oracle.dequant(oracle.gather_i8(idx, got[0], threads=THREADS), np.zeros(M, np.float32), K // v, float(got[1][0]), 0.0, 0, threads=THREADS))
+        assert np.array_equal(fresh.lutgen(cent[::-1].copy(), weight)[0], ctx.lutgen(cent[::-1].copy(), weight)[0])
+        amm.close()
+        fresh.close()
+
+
 @pytest.mark.parametrize("N,CB,v,C,lut", [(9000, 1, 2, 256, "f32"), (5000, 2, 8, 100, "f32"), (700, 31, 4, 65, "i8"), (900, 33, 2, 130, "f32"),
                                           (300, 33, 16, 64, "i8"), (8200, 1, 4, 200, "i8"), (3, 70, 2, 40, "f32")])
 def test_search_of_few_pairs_writes_the_padding_too(ctx, N, CB, v, C, lut):
