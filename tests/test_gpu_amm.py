@@ -664,6 +664,44 @@ def test_search_of_small_codebooks_beside_a_large_one(ctx, v, C):
 
 
 @pytest.mark.parametrize("v,C", [(2, 16), (4, 16), (8, 16), (4, 32)])
+def test_search_of_a_group_with_codebooks_of_any_size(ctx, v, C):
+    """Operators that share a search read the same columns with codebooks of their own: some of each beyond 1024, others small or tiny, ties and long
+    rows among the activations, so that replays read the row from memory.  Every output as of the operator alone and of the reference's scan."""
+    rng = np.random.default_rng(6350 + v + C)
+    N, CB, M = 700, 64, 48
+    x = rng.standard_normal((N, CB, v), dtype=np.float32)
+    x[::7] = 0.0
+    x[3::11] *= np.float32(7e4)
+    sizes = np.float32([1.0, 3e4, 1.0, 1e-3, 1e7, 30.0])
+    amms, want = [], []
+    for i in range(3):
+        _, cent, lut, bias = make_case(6360 + i, 1, CB * v, v, C, M)
+        size = sizes[rng.integers(0, len(sizes), CB)]
+        cent = cent.reshape(CB, C, v) * size[:, None, None]
+        cent[::5, C // 2] = cent[::5, 0]
+        if i == 0:
+            x *= size[:, None]
+        amms.append(ctx.amm(cent, lut, np.float32(0.01), bias, max_n=N))
+        want.append((cent, lut, bias))
+    x = x.reshape(N, CB * v)
+    group = ctx.amm_group(amms)
+    for tile in (64, 128):
+        for a in amms:
+            a.set_tuning(search_token_tile=tile)
+        tiled = ctx.amm_group(amms)              # (a group keeps the search settings that its first member has when it is created)
+        for g in (group, tiled):
+            for a, out, (cent, lut, bias) in zip(amms, g.run(x), want):
+                idx = oracle.index_calculation(x, cent, v, threads=THREADS)
+                acc = oracle.gather_i8(idx, lut, threads=THREADS)
+                assert np.array_equal(out.view(np.uint32), oracle.dequant(acc, bias, CB, 0.01, 0.0, 0, threads=THREADS).view(np.uint32)), tile
+                assert np.array_equal(a.index_calculation(x), idx)
+        tiled.close()
+    group.close()
+    for a in amms:
+        a.close()
+
+
+@pytest.mark.parametrize("v,C", [(2, 16), (4, 16), (8, 16), (4, 32)])
 def test_search_of_rows_longer_than_large_centroids(ctx, v, C):
     """Centroids of about 3000, every hundredth row of 3e5 in each dimension: far enough from a tie in every codebook but a few, and inside the range
     that halves have at the codebooks' scale.  The time against the same launch without such rows; with their replays it is 1.5 to 1.8
