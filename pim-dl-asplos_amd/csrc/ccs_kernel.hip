@@ -664,7 +664,7 @@ __global__ __launch_bounds__(CCS_THREADS, V == 8 ? 2 : 4) void ccs_mfma_kernel(c
 // the top-two search (100 ns).  v_mfma_f32_32x32x16_f16 is twice as fast per K-slot and runs beside
 // VALU work.  A half has 11 significand bits, so two pieces (x = xh + xm) hold a float up to 2^-21 of it, or up to 2^-24 where
 // the second one is subnormal; all four cross products with the pieces of -2c are taken.  The score then carries a known error
-// bound like the fp32 form's, only larger (A2, E2 below), and everything after the scores -- tagged
+// bound like the fp32 form's, only larger (half_margin below), and everything after the scores -- tagged
 // keys, tournament, margin test, exact replay -- is the same.
 // Bound by the vector ALU, of which the pieces are what a form can choose: cut in one v_cvt_pkrtz_f16_f32 per two values and piece, the
 // remainder by one v_fma_mix_f32, they are 8 operations per 64 pairs at v = 4, and two matrix instructions.  (Three bf16 pieces by
@@ -1886,7 +1886,7 @@ int launch_ccs_f16(Ctx* ctx, const AmmGeom& g, const float* d_x, const float* d_
     // and 7.8 / 8.1 at 768, 13.0 / 13.8 at 1536, 20.9 / 21.1 at 3072, 89 / 87 at 12288; 32 centroids 8.5 / 8.4 at 768, 11.8 / 12.2 at 1536, 20.2 / 19.7 at
     // 3072.  v = 2, whose tiles hold little, goes over sooner: 4.6 / 5.9 at 96, 5.0 / 5.5 at 256, 6.6 / 6.6 at 512, 7.5 / 7.3 at 768, 8.2 / 7.9 at
     // 1024, 11.0 / 10.2 at 1536; 32 centroids 6.9 / 7.7 at 512, 9.0 / 8.4 at 768, 12.5 / 11.2 at 1536.  v = 8 with up to 16 centroids does not: its
-    // 128-token kernel has two workgroups per CU (220 registers, 76 KB of LDS), 6.1 / 6.5 at 192, 7.2 / 7.9 at 384, 13.3 / 15.5 at 768, 34.2 / 36.4 at
+    // 128-token kernel has two workgroups per CU (221 registers, 76 KB of LDS), 6.1 / 6.5 at 192, 7.2 / 7.9 at 384, 13.3 / 15.5 at 768, 34.2 / 36.4 at
     // 3072, 79 / 81 at 6144.
     const uint64_t cus = ctx->prop.multiProcessorCount;
     const bool small_tiles = g.tune_search_tile ? g.tune_search_tile == 64 : (V == 8 && !WIDE) || tiles128 <= (V == 2 ? 5 * cus / 2 : 6 * cus);

@@ -801,7 +801,7 @@ bool apply_runtime_tuning(AmmGeom* g, const pimdl_amm_tuning& t, std::string* wh
         return false;
     }
     if (t.search_kernel == PIMDL_SEARCH_MFMA_BF16 && !(g->C <= 32 && v248)) {
-        *why = "the bf16 matrix-core search needs up to 32 centroids and sub_vec_len 2, 4 or 8";
+        *why = "the matrix-core search on 16-bit pieces needs up to 32 centroids and sub_vec_len 2, 4 or 8";
         return false;
     }
     if (t.search_token_tile && t.search_token_tile != 64 && t.search_token_tile != 128) {

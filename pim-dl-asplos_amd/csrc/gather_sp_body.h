@@ -218,9 +218,9 @@
                     if (full) {  // workgroup-uniform: every token and column of the tile exists
                         if constexpr (W == 4) {
                             typedef float v4f __attribute__((ext_vector_type(4)));
-                            // 96-column tiles (the widest outputs): plain stores, which the caches may hold for the
-                            // operator that reads the output next; measured 0.7 us faster at 768 -> 3072, N = 8192
-                            // (100 MB), while the 25 MB of 3072 -> 768 are 1.4 us faster with streaming stores
+                            // Streaming stores; 96-column tiles, which only a caller that names them takes, plain ones.  (Measured over
+                            // one output written again and again, when 96 columns were the choice at 768 -> 3072: 0.7 us faster there, N =
+                            // 8192, 100 MB, and 1.4 us slower in the 48 columns of 3072 -> 768, 25 MB.)
                             if constexpr (TN == 6) *reinterpret_cast<v4f*>(dst) = (v4f){o[0], o[1], o[2], o[3]};
                             else __builtin_nontemporal_store((v4f){o[0], o[1], o[2], o[3]}, reinterpret_cast<v4f*>(dst));
                         } else if constexpr (W == 2) {

@@ -541,7 +541,7 @@ def test_search_with_a_few_near_ties_per_wave(ctx, v, C):
 @pytest.mark.parametrize("size", [1e-4, 0.03, 1.0, 900.0, 1100.0, 3e4, 1e9, 1e16])
 def test_search_over_the_range_of_halves(ctx, v, C, size):
     """The matrix search works on halves, whose range ends at 65504 and 6e-8: centroids and activations of one size from far below
-    to far above it (tiles with centroids beyond 1024 are searched at a scale of their own), codebooks of another size beside them in
+    to far above it (codebooks with centroids beyond 1024 are searched at a scale of their own), codebooks of another size beside them in
     the same and in other tiles, activations that no half holds, an odd width; every index against the reference's scan."""
     rng = np.random.default_rng(int(4000 + 10 * v + C))
     many = C > 32 or v > 8                             # the search by groups of 32 centroids; fewer tokens take another
