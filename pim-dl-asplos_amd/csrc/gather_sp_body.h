@@ -194,8 +194,7 @@
         if (ep.op_col_tiles) epl.scale = scalar_load1(ep.op_scales + colblk / ep.op_col_tiles);
         const uint32_t tile_tok0 = tok_tile_of(item) * TOK_ITEM;
         const uint32_t tok0 = tile_tok0 + tw * (TM * 16) + 4 * ge;
-        const bool vec_ok = (M % 4 == 0);
-        const bool full = vec_ok && !acc_out && tile_tok0 + TOK_ITEM <= N && (colblk + 1) * WN <= M;
+        const bool full = !acc_out && tile_tok0 + TOK_ITEM <= N && (colblk + 1) * WN <= M;
         auto piece = [&](auto c0c, auto wc) __attribute__((always_inline)) {
             constexpr int c0 = decltype(c0c)::value, W = decltype(wc)::value;
             const uint32_t f = colblk * WN + 16 * c0 + W * je;  // first of this lane's W columns
@@ -216,7 +215,13 @@
                     }
                     float* dst = out + (size_t)tok * M + f;
                     if (full) {  // workgroup-uniform: every token and column of the tile exists
-                        if constexpr (W == 4) {
+                        if constexpr (!STREAM) {  // (see streaming_stores)
+                            typedef float vf __attribute__((ext_vector_type(W), aligned(4)));  // columns of a row of any width: dword alignment only
+                            vf v;
+#pragma unroll
+                            for (int e = 0; e < W; ++e) v[e] = o[e];
+                            *reinterpret_cast<vf*>(dst) = v;
+                        } else if constexpr (W == 4) {
                             typedef float v4f __attribute__((ext_vector_type(4)));
                             // Streaming stores; 96-column tiles, which only a caller that names them takes, plain ones.  (Measured over
                             // one output written again and again, when 96 columns were the choice at 768 -> 3072: 0.7 us faster there, N =

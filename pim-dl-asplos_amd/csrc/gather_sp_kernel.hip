@@ -127,6 +127,7 @@ __global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TN, TM, GS, NW, WIDE) * NW /
     int32_t* __restrict__ acc_out, uint32_t N, uint32_t M, uint32_t CB_pad, uint32_t idx_row_bytes,
     uint32_t n_token_tiles, uint32_t n_items, Epilogue ep, XcdMap xmap)
 {
+    constexpr bool STREAM = true;
 #include "gather_sp_body.h"
 }
 // the launch deals its items in blocks of token tiles
@@ -138,7 +139,45 @@ __global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TN, TM, GS, NW, false) * NW 
 {
     constexpr bool WIDE = false;
     constexpr int KS = 1;
+    constexpr bool STREAM = true;
 #include "gather_sp_body.h"
+}
+// The same two for rows that are written with plain stores (see streaming_stores): another type of the last argument, so that
+// the code of the others stays what it is without a second epilogue (which cost a forward of 48-column tiles 0.6 %).
+template <class Map>
+struct PlainStores : Map {};
+template <int TN, int TM, int GS, int NW, bool WIDE, int KS = 1>
+__global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TN, TM, GS, NW, WIDE) * NW / 4 /* waves per SIMD */) void gather_sparse_kernel(
+    const uint8_t* __restrict__ idx, const int8_t* __restrict__ lut, float* __restrict__ out,
+    int32_t* __restrict__ acc_out, uint32_t N, uint32_t M, uint32_t CB_pad, uint32_t idx_row_bytes,
+    uint32_t n_token_tiles, uint32_t n_items, Epilogue ep, PlainStores<XcdMap> xmap)
+{
+    constexpr bool STREAM = false;
+#include "gather_sp_body.h"
+}
+template <int TN, int TM, int GS, int NW>
+__global__ __launch_bounds__(NW * 64, sp_wgs_per_cu(TN, TM, GS, NW, false) * NW / 4) void gather_sparse_blocks_kernel(
+    const uint8_t* __restrict__ idx, const int8_t* __restrict__ lut, float* __restrict__ out,
+    int32_t* __restrict__ acc_out, uint32_t N, uint32_t M, uint32_t CB_pad, uint32_t idx_row_bytes,
+    uint32_t n_token_tiles, uint32_t n_items, Epilogue ep, PlainStores<XcdBlocks> xmap)
+{
+    constexpr bool WIDE = false;
+    constexpr int KS = 1;
+    constexpr bool STREAM = false;
+#include "gather_sp_body.h"
+}
+
+// Streaming stores where rows are whole half lines of 64 bytes.  Where they are not, a row's part of a tile ends inside one that the neighbour
+// tile writes the rest of: streamed, the two parts go to memory one by one; plain stores meet in L2.  They also push the table out of it, so
+// that one of about an L2 of 4 MiB, or an output that shows nothing of all this, is better off streamed.  Widths that four does not
+// divide (16 bytes at any multiple of four bytes, where they used to be four stores of one column each) are plain always.  us a pass,
+// inputs and outputs in turn, streamed / plain: 11 codebooks, M = 1112 N = 16034 47.2 / 25.4, 64 N = 13893 38.1 / 27.3, 256 (4.5 MB) N = 10225 52.3 /
+// 58.2; 192 codebooks, M = 1244 N = 7696 41.6 / 34.6, 2340 (7.2 MB) N = 19245 106.8 / 113.0; 326, 744 (4.2 MB) N = 20054 113.3 / 117.8; 64, M = 828 N =
+// 3989 (13 MB of output) 13.2 / 14.2; half lines, 20 codebooks, M = 624 N = 15729 20.5 / 21.3; whole lines, 247 launches, 1.06 times as long plain;
+// one column each / four: 17 codebooks, M = 2890 N = 8936 53.8 / 35.8, 96, 2091 N = 10864 65.1 / 51.3, 640, 1754 N = 9000 123 / 118.
+bool streaming_stores(uint32_t n, uint32_t M, uint32_t cb16)
+{
+    return M % 4 == 0 && (M % 16 == 0 || (uint64_t)n * M * 4 < SP_BLOCK_OUTPUT || (uint64_t)cb16 * 16 * M > 4000000);
 }
 
 template <int TN, int TM, int GS, int NW, bool WIDE, int KS, bool BLOCKS>
@@ -149,12 +188,17 @@ int launch_sparse_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out,
     constexpr int PER_CU = sp_wgs_per_cu(TN, TM, GS, NW, WIDE);
     static_assert(PER_CU * LDS <= 160 * 1024, "the CU's LDS holds the workgroups that its registers hold");
     constexpr int TOK_ITEM = sp_tok_item(TM, NW / KS);
-    auto kern = [] {
-        if constexpr (BLOCKS) return gather_sparse_blocks_kernel<TN, TM, GS, NW>;
-        else return gather_sparse_kernel<TN, TM, GS, NW, WIDE, KS>;
-    }();
+    using Map = std::conditional_t<BLOCKS, XcdBlocks, XcdMap>;
+    auto kernel_for = [](auto map) {
+        using K = void (*)(const uint8_t*, const int8_t*, float*, int32_t*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, Epilogue, decltype(map));
+        if constexpr (BLOCKS) return static_cast<K>(gather_sparse_blocks_kernel<TN, TM, GS, NW>);
+        else return static_cast<K>(gather_sparse_kernel<TN, TM, GS, NW, WIDE, KS>);
+    };
+    const auto streamed = kernel_for(Map{});
+    const auto plain = kernel_for(PlainStores<Map>{});
     const uint32_t cb16 = sparse_codebooks(a.g);  // codebooks of 16 centroids in the tiled table
-    if (int rc = allow_dynamic_lds(ctx, reinterpret_cast<const void*>(kern), LDS, "hipFuncSetAttribute(gather_sparse)")) return rc;
+    const bool stream = streaming_stores(n, a.g.M, cb16);
+    if (int rc = allow_dynamic_lds(ctx, stream ? reinterpret_cast<const void*>(streamed) : reinterpret_cast<const void*>(plain), LDS, "hipFuncSetAttribute(gather_sparse)")) return rc;
     const uint32_t n_token_tiles = (n + TOK_ITEM - 1) / TOK_ITEM;
     const uint32_t n_items = n_token_tiles * (a.g.M_pad / (16 * TN));
     uint32_t grid = ctx->prop.multiProcessorCount * PER_CU;
@@ -179,8 +223,12 @@ int launch_sparse_as(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out,
     else if (KS == 1) snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_kernel<%d, %d, %d, %d, %s>", TN, TM, GS, NW, WIDE ? "true" : "false");
     else snprintf(a.last_gather, sizeof(a.last_gather), "gather_sparse_kernel<%d, %d, %d, %d, %s, %d>", TN, TM, GS, NW, WIDE ? "true" : "false", KS);
     a.note_launch(GS, LDS, TOK_ITEM, NW * 64);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), LDS, ctx->stream, d_idx, reinterpret_cast<const int8_t*>(a.d_lut),
-                       d_out, d_acc, n, a.g.M, cb16, a.g.idx_row_bytes, n_token_tiles, n_items, ep, xmap);
+    auto launch = [&](auto kern, const auto& map) {
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), LDS, ctx->stream, d_idx, reinterpret_cast<const int8_t*>(a.d_lut),
+                           d_out, d_acc, n, a.g.M, cb16, a.g.idx_row_bytes, n_token_tiles, n_items, ep, map);
+    };
+    if (stream) launch(streamed, xmap);
+    else launch(plain, PlainStores<Map>{xmap});
     return hip_check(ctx, hipGetLastError(), "gather_sparse_kernel launch");
 }
 

@@ -1719,6 +1719,44 @@ def test_forms_of_the_sparse_gather_of_large_outputs(ctx, N, CB, M, act, tuning,
     amm.close()
 
 
+@pytest.mark.parametrize("act", [pimdl.ACT_NONE, pimdl.ACT_GELU_TANH])
+@pytest.mark.parametrize("N,CB,M", [
+    (16500, 16, 260),   # rows of no whole half lines, 16 MiB and more: plain stores
+    (16100, 16, 260),   # below: streamed
+    (16500, 16, 261), (16500, 16, 262), (16300, 8, 259),  # widths that 16 bytes do not divide, either side of 16 MiB
+    (4200, 260, 1028),  # a table of more than 4 MiB: streamed
+    (4200, 260, 1027), (4200, 240, 1084),
+])
+def test_sparse_gather_of_rows_that_end_within_lines(ctx, N, CB, M, act):
+    """Both kinds of stores in every tile width, the oracle's bits without an activation and otherwise the same as 4-byte stores give."""
+    if kernel_switches():
+        pytest.skip("the environment keeps one kernel for every shape; this test is about the sparse gather")
+    import torch
+    v, C = 2, 16
+    x, cent, lut, bias = make_case(88 + M + CB, N, CB * v, v, C, M)
+    xd = torch.from_numpy(x).cuda()
+    want = oracle.amm_cpu(x, cent, lut, bias, v, 0.0123, 0.0, threads=THREADS)[0] if act == pimdl.ACT_NONE else None
+    for tuning in ({"col_block": 48}, {"col_block": 64}, {"col_block": 96}, {"col_block": 64, "token_item": 128}, {"col_block": 48, "cb_per_slice": 16}):
+        amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=N, activation=act, tuning=dict(tuning, gather_kernel=pimdl.GATHER_SPARSE))
+        out = torch.full((N + 2, M), -5.0, device="cuda")
+        torch.cuda.synchronize()
+        amm.run_ptr(xd.data_ptr(), N, out.data_ptr())
+        ctx.synchronize()
+        assert amm.last_gather_kernel().startswith("gather_sparse_"), amm.last_gather_kernel()
+        if want is None:
+            want = amm.run_debug(x)[0]  # (with the sums, which takes every column's store by itself)
+        assert bool((out[N:] == -5.0).all())
+        assert np.array_equal(out[:N].cpu().numpy().view(np.uint32), want.view(np.uint32)), tuning
+        amm.close()
+
+
+def test_sparse_gather_of_rows_that_end_within_lines_takes_no_longer(ctx):
+    """11 codebooks, 1112 columns, 16034 tokens took 2.1 times as long as 1120 columns, whose rows are 35 lines; 17 codebooks, 2890 columns 1.5 times as 2912."""
+    for n, cb, ragged, whole in ((16034, 11, 1112, 1120), (8936, 17, 2890, 2912)):
+        a, b = (gather_us(ctx, n, cb, 16, m) for m in (ragged, whole))
+        assert a < 1.35 * b, (n, cb, ragged, a, b)
+
+
 @pytest.mark.parametrize("N,CB,M,form", [
     (8300, 97, 1100, "blocks_kernel<4, 4, 16, 4>"),        # three workgroups per CU: just beyond two of them, ragged tokens and columns
     (7700, 128, 1088, "blocks_kernel<4, 4, 16, 4>"),
