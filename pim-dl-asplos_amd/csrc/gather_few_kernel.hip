@@ -6,6 +6,7 @@
 // on the tables of the large kernels, whatever their layout.  Those kernels give an item of 128 tokens or more and 16 to
 // 96 columns to a workgroup, which goes through all codebooks slice by slice; a launch with fewer items than CUs
 // then takes the time of that chain -- copy, barrier, operands, 32 codebooks further -- however few its tokens are.
+#include <math.h>
 #include <string.h>
 
 #include <algorithm>
@@ -297,28 +298,27 @@ bool few_even(uint64_t blocks, uint64_t tiles, uint64_t cus)
 // workgroups that have a CU of their own each (of exactly as many as CUs the last few share some)
 uint64_t few_room(uint64_t cus) { return cus - cus / 16; }
 
-// Workgroups of a launch.  By XCD where the column blocks do not divide by eight by themselves and several token tiles read the same table:
+// By XCD where the column blocks do not divide by eight by themselves and several token tiles read the same table:
 // us, in order / by XCD, three column groups: 2048 codebooks, M = 2048 N = 256 41.1 / 24.8, 1280 x 1280 N = 512 33.2 / 17.6, 256, M =
 // 5120 N = 128 10.6 / 7.7; one column group: 2048 N = 128 32.8 / 26.4, 1280 N = 256 22.9 / 18.8; with a CU for every workgroup where the table is
 // more than an L2 holds: 4096 -> 1024 (17 MB) N = 40 9.5 / 5.3, 4096 -> 500 v = 2 (17 MB) N = 64 12.5 / 8.3, N = 192 17.1 / 10.7, 1024 ->
 // 1024 v = 2 (8.7 MB) N = 40 4.2 / 3.9; 1024 -> 1024 v = 4 (4.3 MB) N = 40 3.2 / 3.2, 768 -> 1280 (4.0 MB) 3.0 / 3.2.
-dim3 few_grid(const FewArgs& f, uint32_t tm, uint32_t tc, uint32_t cus, bool one_hot)
+bool few_by_xcd(const FewArgs& f, uint32_t tm, uint32_t tc, uint32_t cus, bool one_hot)
 {
     const uint32_t blocks = f.groups / tc, tiles = (f.N + 16 * tm - 1) / (16 * tm);
     const uint64_t fullest = few_fullest(blocks, tiles);
     const bool even = few_even(blocks, tiles, cus);
     // (two items of 64 tokens: 4096 -> 1024 9.0 / 9.3, 5120 -> 1280 11.3 / 10.6)
     const bool shared = one_hot && (tm < 4 || tiles > 2) && 8 * fullest <= few_room(cus) && few_table_bytes(f.steps, f.groups) > FEW_TABLE_SHARED;
-    const bool by_xcd = tiles > 1 && blocks % 8 != 0 && (shared || (even && (tc > 1 || tiles * blocks > cus)));
-    return by_xcd && blocks > 8 ? dim3(8, tiles, (blocks + 7) / 8) : dim3(blocks, tiles);  // (z > 1 says which)
+    return tiles > 1 && blocks > 8 && blocks % 8 != 0 && (shared || (even && (tc > 1 || tiles * blocks > cus)));
 }
 
 template <FewTable T, int TM, int NW, int TC = 1>
-int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
+int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep, bool xcd)
 {
     constexpr int LDS = few_lds_bytes(NW, TM, T == FEW_ROWS ? FEW_PITCH_ROWS : FEW_PITCH_ONEHOT);
-    const dim3 grid = few_grid(f, TM, TC, ctx->prop.multiProcessorCount, T != FEW_ROWS);
-    const bool xcd = grid.z > 1;
+    const uint32_t blocks = f.groups / TC, tiles = (f.N + 16 * TM - 1) / (16 * TM);
+    const dim3 grid = xcd ? dim3(8, tiles, (blocks + 7) / 8) : dim3(blocks, tiles);
     auto kern = [xcd] {
         if constexpr (TC > 1) return xcd ? gather_sparse_few_wide_kernel<TM, NW, true, TC> : gather_sparse_few_wide_kernel<TM, NW, false, TC>;
         else if constexpr (T == FEW_SPARSE) return xcd ? gather_sparse_few_kernel<TM, NW, true> : gather_sparse_few_kernel<TM, NW, false>;
@@ -338,7 +338,8 @@ int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
     return hip_check(ctx, hipGetLastError(), "gather_few launch");
 }
 
-// Time of a byte adder launch in rounds of 16-token workgroups, which take their codebooks' time each.  Larger items only where they spare rounds: one
+constexpr uint32_t FEW_ROWS_BLOCKS = 75;  // column blocks up to which the byte adder's launches are priced by their rounds alone (see few_rows)
+// Time of such a launch in rounds of 16-token workgroups, which take their codebooks' time each.  Larger items only where they spare rounds: one
 // of up to 32 tokens that fits a round where two of 16 do not, or 64 where every one has a CU and the 16 tokens take four rounds and more
 // (3.4 times the time; with column blocks that divide by eight, so that the tiles' rows come from one L2).
 double few_rows_rounds(const AmmGeom& g, uint32_t n, uint64_t cus, uint32_t* item)
@@ -373,12 +374,63 @@ bool few_rows64_wanted(const AmmGeom& g, uint32_t n, uint64_t cus)
     return few < ((double)meet((n + 127) / 128) * eighth_mb > 4.2 ? 1.2 * large : large);
 }
 
+// Beyond, where rounds overlap (a CU has two workgroups of eight waves) and tables no L2 holds are what a launch waits for: us on items of 16, 32 or
+// 64 tokens x 16 columns, each of which takes its codebooks' time a round and its token tile's part of the table from memory.  Such a table is
+// read again for every token tile of a column block that comes a round later, or on another XCD: by XCD the tiles run together, and it is
+// read once.  (Up to 32 centroids, whose rows any 16 tokens read nearly all of, only where the blocks meet on several XCDs.)
+// us of gather, blocks x codebooks, items of 16 in order / by XCD / 32 / 64 / the large kernel: 200 centroids 192 x 256 N = 76 45.0 / 24.7 / 37.1 /
+// 30.1 / 29.4, 80 x 320 N = 144 29.2 / 19.5 / 26.4 / 24.4 / 23.8; 128 centroids 192 x 128 N = 43 10.3 / 10.2 / 9.3 / 9.9 / 10.8; 64 centroids 192 x
+// 48 N = 17 3.0 / 3.4 / 3.1 / - / 3.8, 475 x 11 N = 8 2.7 (large 3.8); 24 centroids 512 x 512 N = 17 23.4 / 23.5 / 19.5 / - / 22.8, 320 x 320 N = 18 9.7 /
+// 11.0 / 11.2 / - / 13.0.  Of 533 launches of 1 .. 475 blocks, 8 .. 1536 codebooks and 2 .. 600 tokens the form that is taken is within 5 % of the shortest
+// in 480 (444 by rounds alone at any width; 353 with items by the number of tokens, which 26 of those 444 took longer than).
+struct FewRows {
+    uint32_t item;
+    bool by_xcd;
+    double us;
+};
+FewRows few_rows(const AmmGeom& g, uint32_t n, uint64_t cus)
+{
+    constexpr double L2_MB = 3.5;  // of a table, beside what else there is
+    const struct { uint32_t item; double base, step, step_mem; } forms[] = {{16, 2.4, 6.2e-3, 9.2e-3}, {32, 2.6, 14.8e-3, 17.2e-3}, {64, 2.95, 28.5e-3, 31e-3}};
+    const uint64_t blocks = g.M_pad / 16;
+    // MB that the tokens read of the table: lines of eight codebooks' pieces of a row
+    const double read = (double)g.CB_pad * g.C_tile * g.M_pad * 1e-6 * (1.0 - exp(-8.0 * n / g.C_tile));
+    const double us_per_mb = g.C_tile > 32 ? 0.08 : 0.025;
+    FewRows best{0, false, 1e300};
+    for (const auto& f : forms) {
+        if (f.item > 16 && 2 * n <= f.item) break;
+        const uint64_t tiles = (n + f.item - 1) / f.item;
+        // XCDs on which the token tiles of a column block meet
+        const uint64_t meet = std::min<uint64_t>(tiles, blocks % 8 == 0 ? 1 : blocks % 4 == 0 ? 2 : blocks % 2 == 0 ? 4 : 8);
+        const bool streams = read / 8 * (double)meet > L2_MB;
+        const bool by_xcd = streams && tiles > 1 && blocks > 8 && (blocks % 8 != 0 || (tiles * blocks > cus && g.C_tile > 32));
+        const double rounds = (double)(((by_xcd ? 8 * few_fullest(blocks, tiles) : tiles * blocks) + cus - 1) / cus);
+        const double once = g.C_tile > 32 && !by_xcd ? (double)meet : 1.0;
+        const double us = f.base + g.CB_pad * rounds * (streams ? f.step_mem : f.step) +
+                          (streams ? us_per_mb * std::max(0.0, read * once - 16.0) : 0.1 * (rounds - 1));
+        if (us < best.us) best = {f.item, by_xcd, us};
+    }
+    return best;
+}
+// ... and on the large kernel (gather_rows_kernel.hip), whose workgroups go through their slices of 16 codebooks: alone on a CU, two to a CU, and in
+// further rounds; its smallest items, which launches that are in question take.
+double large_rows_us(const AmmGeom& g, uint32_t n, uint64_t cus)
+{
+    const bool one_per_cu = g.C_tile == 256;
+    const uint64_t blocks = g.M_pad / 16, items = one_per_cu ? (n + 255) / 256 * blocks : (n + 127) / 128 * (g.C_tile <= 32 ? (blocks + 1) / 2 : blocks);
+    const double load = (double)items / (double)(one_per_cu ? cus : 2 * cus);
+    const double slice = g.C_tile <= 32 ? 0.3 : g.C_tile == 64 ? 0.305 : g.C_tile == 128 ? 0.39 : 0.72;
+    const double second = g.C_tile <= 32 ? 1.1 : g.C_tile == 64 ? 0.42 : g.C_tile == 128 ? 0.355 : 0.86, further = g.C_tile <= 32 ? 0.2 : one_per_cu ? 1.2 : 0.0;
+    const double table = (double)g.CB_pad * g.C_tile * g.M_pad * 1e-6;
+    return 3.3 + (g.CB + 15) / 16 * (slice + second * std::min(std::max(load - 0.5, 0.0), 0.5) + further * std::max(0.0, load - 1.0)) + 0.09 * std::max(0.0, table - 20.0);
+}
+
 // Tokens of an item: 16, 32 or 64.  One-hot tables: as few as leave every workgroup a CU of its own.  A wave then makes operands for fewer tokens, and
 // what more workgroups read of the table comes from the L2s.  us of gather, items of 16 / 32 / 64 tokens (workgroups): 3072 -> 768 v = 4 N = 64
 // 4.6 (192) / 5.4 (96) / 7.3 (48), N = 128 11.8 (384) / 5.5 (192) / 7.4; 768 -> 768 v = 2 N = 128 4.6 (384) / 4.0 (192) / 4.9; 1024 -> 1024 v = 2
 // N = 64 5.0 (264) / 4.5 (132) / 5.6; 4096 -> 500 v = 2 by XCD (33 column blocks, five of them on one XCD) N = 64 8.3 (20 on that XCD) / 10.5 / 15.0, N =
 // 100 13.0 (35) / 10.6 (20) / 15.2; 8 centroids 3072 -> 768 N = 64 3.5 / 4.1 / 5.7.
-// Byte adder, whose tokens' rows are read whatever the item: 32 centroids 3072 -> 768 N = 64 8.6 / 15.0 / 17.3, N = 100 14.8 (336) / 15.0 / 17.6, 3072
+// Byte adder (up to FEW_ROWS_BLOCKS), whose tokens' rows are read whatever the item: 32 centroids 3072 -> 768 N = 64 8.6 / 15.0 / 17.3, N = 100 14.8 (336) / 15.0 / 17.6, 3072
 // -> 3072 N = 32 19.5 (384) / 15.2; 100 centroids 768 -> 2304 N = 32 9.3 (288) / 7.8; 64 centroids 3072 -> 768 v = 8 N = 64 5.4 / 9.3 / 9.4; 200
 // 768 -> 768 N = 256 10.5 (768) / - / 11.2 (192), N = 300 13.0 (912) / - / 10.7 (240).
 uint32_t few_item(const AmmGeom& g, uint32_t n, uint64_t cus)
@@ -392,7 +444,7 @@ uint32_t few_item(const AmmGeom& g, uint32_t n, uint64_t cus)
     const uint64_t table = (uint64_t)g.CB_pad * g.C_tile * g.M_pad;
     for (uint32_t item = 16; item < 64; item *= 2) {
         const uint64_t tiles = (n + item - 1) / item;
-        const bool by_xcd = groups % 8 != 0 && table > FEW_TABLE_SHARED;  // (few_grid)
+        const bool by_xcd = groups % 8 != 0 && table > FEW_TABLE_SHARED;  // (few_by_xcd)
         if (tiles == 1 || (by_xcd ? 8 * few_fullest(groups, tiles) : tiles * groups) <= few_room(cus)) return item;
     }
     return 64;
@@ -403,11 +455,21 @@ uint32_t few_item(const AmmGeom& g, uint32_t n, uint64_t cus)
 template <FewTable T>
 int launch_few(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
 {
-    const uint32_t item = few_item(a.g, f.N, ctx->prop.multiProcessorCount);
-    const bool deep = f.groups * ((f.N + item - 1) / item) <= (uint32_t)ctx->prop.multiProcessorCount;
-    if (item == 16) return deep ? launch_few_as<T, 1, 16>(ctx, a, f, ep) : launch_few_as<T, 1, 8>(ctx, a, f, ep);
-    if (item == 32) return deep ? launch_few_as<T, 2, 16>(ctx, a, f, ep) : launch_few_as<T, 2, 8>(ctx, a, f, ep);
-    return deep ? launch_few_as<T, 4, 16>(ctx, a, f, ep) : launch_few_as<T, 4, 8>(ctx, a, f, ep);
+    const uint32_t cus = ctx->prop.multiProcessorCount;
+    uint32_t item;
+    bool xcd;
+    if (T == FEW_ROWS && a.g.M_pad / 16 > FEW_ROWS_BLOCKS) {
+        const FewRows r = few_rows(a.g, f.N, cus);
+        item = r.item;
+        xcd = r.by_xcd;
+    } else {
+        item = few_item(a.g, f.N, cus);
+        xcd = few_by_xcd(f, item / 16, 1, cus, T != FEW_ROWS);
+    }
+    const bool deep = f.groups * ((f.N + item - 1) / item) <= cus;
+    if (item == 16) return deep ? launch_few_as<T, 1, 16>(ctx, a, f, ep, xcd) : launch_few_as<T, 1, 8>(ctx, a, f, ep, xcd);
+    if (item == 32) return deep ? launch_few_as<T, 2, 16>(ctx, a, f, ep, xcd) : launch_few_as<T, 2, 8>(ctx, a, f, ep, xcd);
+    return deep ? launch_few_as<T, 4, 16>(ctx, a, f, ep, xcd) : launch_few_as<T, 4, 8>(ctx, a, f, ep, xcd);
 }
 
 // fp32 tables (and int8 ones with a scale per group of codebooks, resident as floats): a lane is one column of one
@@ -541,6 +603,7 @@ bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
         return 2.7 + g.CB_pad * (bounds ? 0.062 : 0.0137) + pieces * piece < 4.0 + g.CB_pad * (bounds ? 0.14 : 0.07);
     }
     if (g.gather_kind == 0) {
+        if (g.M_pad / 16 > FEW_ROWS_BLOCKS) return g.idx_bits == 8 && few_rows(g, n, cus).us < large_rows_us(g, n, cus);
         if (g.C_tile == 64) return g.idx_bits == 8 && few_rows64_wanted(g, n, cus);
         const uint64_t slices = (g.CB + 15) / 16;
         uint32_t rows_item;
@@ -617,8 +680,8 @@ int launch_gather_few(Ctx* ctx, const Amm& a, const uint8_t* d_idx, float* d_out
     if (g.gather_kind == 2) {
         f.steps = g.CB_pad / 8;
         switch (few_column_groups(ctx, g, n)) {
-            case 2: return launch_few_as<FEW_SPARSE, 4, 8, 2>(ctx, a, f, ep);
-            case 3: return launch_few_as<FEW_SPARSE, 4, 8, 3>(ctx, a, f, ep);
+            case 2: return launch_few_as<FEW_SPARSE, 4, 8, 2>(ctx, a, f, ep, few_by_xcd(f, 4, 2, ctx->prop.multiProcessorCount, true));
+            case 3: return launch_few_as<FEW_SPARSE, 4, 8, 3>(ctx, a, f, ep, few_by_xcd(f, 4, 3, ctx->prop.multiProcessorCount, true));
         }
         return launch_few<FEW_SPARSE>(ctx, a, f, ep);
     }

@@ -1979,6 +1979,40 @@ def test_gather_of_64_centroids_by_what_an_xcd_has_to_do(ctx, CB, M, N, kernel):
     amm.close()
 
 
+@pytest.mark.parametrize("N,CB,C,M,kernel", [
+    (17, 48, 64, 3072, "gather_i8_few_kernel<1, 8, false>"),    # rounds that overlap
+    (5, 8, 64, 5120, "gather_i8_few_kernel<1, 8, false>"), (25, 11, 200, 6144, "gather_i8_few_kernel<1, 8, false>"),
+    (300, 48, 64, 3072, "gather_i8_kernel<"),
+    (76, 100, 200, 2048, "gather_i8_few_kernel<1, 8, true>"),   # a table no L2 holds: its token tiles together, also of blocks that eight divides
+    (33, 300, 128, 2441, "gather_i8_few_kernel<1, 8, true>"),   # 153 blocks: seven of the grid's past the last
+    (40, 20, 64, 1216, "gather_i8_few_kernel<1, 16, false>"), (40, 20, 64, 1200, "gather_i8_few_kernel<1, 16, false>"),  # 76 and 75 blocks
+    (17, 512, 24, 8192, "gather_i8_few_kernel<2, 8, false>"),
+])
+def test_byte_adder_of_few_tokens_and_many_column_blocks(ctx, N, CB, C, M, kernel):
+    """The items that the launch takes by its prices: accumulators and output bits of the oracle, nothing behind the output."""
+    import torch
+    x, cent, lut, bias = make_case(9100 + M + N, N, CB, 1, C, M)
+    want, _, want_acc = oracle.amm_cpu(x, cent, lut, bias, 1, 0.0123, 0.0, threads=THREADS)
+    amm = ctx.amm(cent, lut, np.float32(0.0123), bias, max_n=N)
+    _, _, acc = amm.run_debug(x)
+    assert np.array_equal(acc, want_acc)
+    xd, out = torch.from_numpy(x).cuda(), torch.full((N + 2, M), -5.0, device="cuda")
+    torch.cuda.synchronize()
+    amm.run_ptr(xd.data_ptr(), N, out.data_ptr())
+    ctx.synchronize()
+    if ctx.device_info()["compute_units"] == 256 and not kernel_switches():
+        assert amm.last_gather_kernel().startswith(kernel), amm.last_gather_kernel()
+    got = out.cpu().numpy()
+    assert np.array_equal(got[:N].view(np.uint32), want.view(np.uint32)) and (got[N:] == -5.0).all()
+    amm.close()
+
+
+def test_byte_adder_of_large_tables_reads_them_once(ctx):
+    """76 tokens, five tiles of 16, read 200 MB five times over: 45 us, where 300 tokens on the large kernel take 31 (25 by XCD)."""
+    a, b = (gather_us(ctx, n, 256, 200, 3072, v=1) for n in (76, 300))
+    assert a < 0.95 * b, (a, b)
+
+
 @pytest.mark.parametrize("CB,lut,group,M", [(96, "f32", 0, 2441), (768, "f32", 0, 2441), (96, "i8", 8, 3692)])
 def test_few_tokens_of_64_centroids_take_the_large_gather_where_it_is_shorter(ctx, CB, lut, group, M):
     """93 tokens, gathered piece by piece, took 1.4 to 1.7 times as long as 150 on the large kernel."""
