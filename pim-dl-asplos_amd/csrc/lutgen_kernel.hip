@@ -20,6 +20,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 
 constexpr int LG_WAVES = 4;
 constexpr int LG_FT = 4;  // 16-column tiles per wave
+constexpr uint32_t LG_ORDERED = 8;  // centroids per thread of the ordered form
 
 // largest value of a workgroup of four waves, in thread 0 (m >= 0; NaN is passed over)
 __device__ __forceinline__ float block_max(float m)
@@ -126,16 +127,20 @@ __global__ __launch_bounds__(LG_WAVES * 64) void lutgen_kernel(const float* __re
 // addition rounded on its own, starting from 0.0f: the order in which a plain loop over the sub-vector runs
 // on a CPU.  torch.bmm fixes no order (pim_weight_converter.py:86-90 leaves it to the library), so neither
 // form is "the" reference result; this one makes a converter's output reproducible bit for bit by scalar code.
-// One thread = one output column of one codebook, all C centroids: W is read once, the LUT written once.
+// One thread = one output column of one codebook, LG_ORDERED centroids one after the other: a small table is as long as this chain, and an int8
+// one goes through it twice.  us a call, all centroids by one thread, from a table of floats that was kept / twice without it / by eights: 64 ->
+// 64 v = 16, 64 centroids 142 / 206 / 65, v = 4 73 / 102 / 40; 256 -> 512 v = 16, 64 centroids 260 / 274 / 108; 768 -> 3072 v = 4, 16 centroids 637 / 545 / 522.
 template <LutPass PASS>
 __global__ __launch_bounds__(256) void lutgen_ordered_kernel(const float* __restrict__ cent, const float* __restrict__ W, LutOut o,
                                                            uint32_t C, uint32_t v, uint32_t M)
 {
-    const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x, cb = blockIdx.y;
+    const uint32_t groups = (C + LG_ORDERED - 1) / LG_ORDERED;  // workgroup x: centroid group x % groups of column tile x / groups
+    const uint32_t f = blockIdx.x / groups * blockDim.x + threadIdx.x, cb = blockIdx.y, c0 = blockIdx.x % groups * LG_ORDERED;
+    const uint32_t c1 = C - c0 < LG_ORDERED ? C : c0 + LG_ORDERED;
     const float* w = W + (size_t)cb * v * M + f;
     const float scale = PASS == LUT_QUANTISE ? o.scales[cb / o.group_cbs] : 0.0f;
     float m = 0.0f;
-    for (uint32_t c = 0; c < C && f < M; ++c) {
+    for (uint32_t c = c0; c < c1 && f < M; ++c) {
         const float* a = cent + ((size_t)cb * C + c) * v;
         float acc = 0.0f;
         for (uint32_t t = 0; t < v; ++t) acc = __fadd_rn(acc, __fmul_rn(a[t], w[(size_t)t * M]));
@@ -221,14 +226,14 @@ __global__ __launch_bounds__(1024) void lds_read_kernel(int* __restrict__ sink, 
 // workgroups per codebook, each of which leaves its largest magnitude
 uint32_t lutgen_parts(uint32_t C, uint32_t M, bool ordered)
 {
-    return ordered ? (M + 255) / 256 : (M + LG_WAVES * 16 * LG_FT - 1) / (LG_WAVES * 16 * LG_FT) * ((C + 15) / 16);
+    return ordered ? (M + 255) / 256 * ((C + LG_ORDERED - 1) / LG_ORDERED) : (M + LG_WAVES * 16 * LG_FT - 1) / (LG_WAVES * 16 * LG_FT) * ((C + 15) / 16);
 }
 
 template <LutPass PASS>
 static int launch_pass(Ctx* ctx, const float* d_cent, const float* d_w, const LutOut& o, uint32_t CB, uint32_t C, uint32_t v, uint32_t M, bool ordered)
 {
     if (ordered) {
-        hipLaunchKernelGGL(lutgen_ordered_kernel<PASS>, dim3((M + 255) / 256, CB), dim3(256), 0, ctx->stream, d_cent, d_w, o, C, v, M);
+        hipLaunchKernelGGL(lutgen_ordered_kernel<PASS>, dim3(lutgen_parts(C, M, true), CB), dim3(256), 0, ctx->stream, d_cent, d_w, o, C, v, M);
         return hip_check(ctx, hipGetLastError(), "lutgen_ordered_kernel launch");
     }
     dim3 grid((M + LG_WAVES * 16 * LG_FT - 1) / (LG_WAVES * 16 * LG_FT), (C + 15) / 16, CB);

@@ -60,6 +60,38 @@ def test_ordered_lutgen_is_bit_identical_to_the_scalar_loop(ctx, CB, C, v, M):
         assert np.array_equal(got_q, want_q)
 
 
+@pytest.mark.parametrize("CB,C,v,M", [(3, 8, 4, 257), (2, 9, 16, 256), (1, 7, 1, 255), (2, 200, 3, 300), (65, 64, 16, 64)])
+def test_ordered_lutgen_of_any_number_of_centroids(ctx, CB, C, v, M):
+    """Eight centroids to a thread: the edges of such a group and of a column tile, bit for bit."""
+    rng = np.random.default_rng(CB * 7 + C + v + M)
+    cent = rng.standard_normal((CB, C, v)).astype(np.float32)
+    W = (rng.standard_normal((CB * v, M)) * 0.02).astype(np.float32)
+    want_f = oracle.lutgen_f32(cent, W, threads=8)
+    got_f, _ = ctx.lutgen(cent, W, pimdl.LUT_F32, 0, ordered=True)
+    assert np.array_equal(got_f.view(np.uint32), want_f.view(np.uint32))
+    for group in (0, 1):
+        want_q, want_s = oracle.lut_quant(want_f, group)
+        got_q, got_s = ctx.lutgen(cent, W, pimdl.LUT_I8, group, ordered=True)
+        assert np.array_equal(got_s.view(np.uint32), np.asarray(want_s, np.float32).view(np.uint32)) and np.array_equal(got_q, want_q)
+
+
+def test_ordered_lutgen_of_many_centroids_is_no_longer_chain(ctx):
+    """64 -> 64, sub-vectors of 16: 64 centroids took 2.5 times as long as 8, one after the other and twice over."""
+    import time
+    rng = np.random.default_rng(5)
+    W = (rng.standard_normal((64, 64)) * 0.02).astype(np.float32)
+    us = {}
+    for C in (8, 64):
+        cent = rng.standard_normal((4, C, 16)).astype(np.float32)
+        best = 1e9
+        for _ in range(40):
+            t = time.perf_counter()
+            ctx.lutgen(cent, W, pimdl.LUT_I8, 0, ordered=True)
+            best = min(best, time.perf_counter() - t)
+        us[C] = best * 1e6
+    assert us[64] < 1.6 * us[8], us
+
+
 def test_converter_writes_the_engine_format_and_the_model_runs_from_it(ctx, tmp_path):
     """A synthetic 'calibrated checkpoint' in the reference's input naming (safetensors, HF BERT encoder keys)
     goes through the converter; the result loads into the model wrapper and runs."""
