@@ -338,7 +338,7 @@ int launch_few_as(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep, 
     return hip_check(ctx, hipGetLastError(), "gather_few launch");
 }
 
-constexpr uint32_t FEW_ROWS_BLOCKS = 75;  // column blocks up to which the byte adder's launches are priced by their rounds alone (see few_rows)
+constexpr uint32_t FEW_ROWS_BLOCKS = 75;  // column blocks up to which a byte adder launch is priced by its rounds alone if the L2s hold its table (see few_rows)
 // Time of such a launch in rounds of 16-token workgroups, which take their codebooks' time each.  Larger items only where they spare rounds: one
 // of up to 32 tokens that fits a round where two of 16 do not, or 64 where every one has a CU and the 16 tokens take four rounds and more
 // (3.4 times the time; with column blocks that divide by eight, so that the tiles' rows come from one L2).
@@ -374,40 +374,53 @@ bool few_rows64_wanted(const AmmGeom& g, uint32_t n, uint64_t cus)
     return few < ((double)meet((n + 127) / 128) * eighth_mb > 4.2 ? 1.2 * large : large);
 }
 
-// Beyond, where rounds overlap (a CU has two workgroups of eight waves) and tables no L2 holds are what a launch waits for: us on items of 16, 32 or
-// 64 tokens x 16 columns, each of which takes its codebooks' time a round and its token tile's part of the table from memory.  Such a table is
-// read again for every token tile of a column block that comes a round later, or on another XCD: by XCD the tiles run together, and it is
-// read once.  (Up to 32 centroids, whose rows any 16 tokens read nearly all of, only where the blocks meet on several XCDs.)
+// Beyond, and with tables of more than 64 centroids that no L2 holds, rounds overlap, a CU having two workgroups of eight waves, and
+// the table is what a launch waits for: us on items of 16, 32 or 64 tokens x 16 columns, each of which takes its codebooks' time a round (less where
+// its last tokens are missing) and its token tile's part of the table from memory.  Such a table is read again for every token tile of a column
+// block that comes a round later, or on another XCD: by XCD the tiles run together, and it is read once.  (Up to 32 centroids, whose rows any 16
+// tokens read nearly all of, only where the blocks meet on several XCDs.)
 // us of gather, blocks x codebooks, items of 16 in order / by XCD / 32 / 64 / the large kernel: 200 centroids 192 x 256 N = 76 45.0 / 24.7 / 37.1 /
-// 30.1 / 29.4, 80 x 320 N = 144 29.2 / 19.5 / 26.4 / 24.4 / 23.8; 128 centroids 192 x 128 N = 43 10.3 / 10.2 / 9.3 / 9.9 / 10.8; 64 centroids 192 x
-// 48 N = 17 3.0 / 3.4 / 3.1 / - / 3.8, 475 x 11 N = 8 2.7 (large 3.8); 24 centroids 512 x 512 N = 17 23.4 / 23.5 / 19.5 / - / 22.8, 320 x 320 N = 18 9.7 /
-// 11.0 / 11.2 / - / 13.0.  Of 533 launches of 1 .. 475 blocks, 8 .. 1536 codebooks and 2 .. 600 tokens the form that is taken is within 5 % of the shortest
-// in 480 (444 by rounds alone at any width; 353 with items by the number of tokens, which 26 of those 444 took longer than).
+// 30.1 / 29.4, 80 x 320 N = 144 29.2 / 19.5 / 26.4 / 24.4 / 23.8, 41 x 1536 N = 148 120 / 57 / 99 / 105 / 100, 134 x 421 N = 52 42.1 / 32.6 / 41.3 / 28.2 / 36.3;
+// 128 centroids 17 x 746 N = 409 47.7 / 26.1 / 30.4 / 43.4 / 33.9, 192 x 128 N = 43 10.3 / 10.2 / 9.3 / 9.9 / 10.8; 64 centroids 192 x 48 N = 17 3.0 / 3.4 / 3.1 / - /
+// 3.8, 475 x 11 N = 8 2.7 (large 3.8), 334 x 340 N = 20 23.6 / 22.0 / 19.3 / - / 19.5; 24 centroids 512 x 512 N = 17 23.4 / 23.5 / 19.5 / - / 22.8, 320 x 320 N =
+// 18 9.7 / 11.0 / 11.2 / - / 13.0.  Of 681 launches of 2 .. 600 tokens that these prices decide (four fifths of them went into the figures) the form that
+// is taken is within 5 % of the shortest in 635 and beyond 10 % in 25; by rounds alone 160 are beyond 5 %.
 struct FewRows {
     uint32_t item;
     bool by_xcd;
     double us;
 };
+constexpr double FEW_ROWS_L2 = 3.0;  // MB of a table that an L2 holds beside what else there is
+// MB that n tokens read of the table: lines of eight codebooks' pieces of a row
+double few_rows_read(const AmmGeom& g, uint32_t n) { return (double)g.CB * g.C * g.M_pad * 1e-6 * (1.0 - exp(-8.0 * n / g.C)); }
+// XCDs on which the token tiles of a column block meet in order
+uint64_t few_rows_meet(uint64_t blocks, uint64_t tiles)
+{
+    return std::min<uint64_t>(tiles, blocks % 8 == 0 ? 1 : blocks % 4 == 0 ? 2 : blocks % 2 == 0 ? 4 : 8);
+}
+bool few_rows_priced(const AmmGeom& g, uint32_t n)
+{
+    const uint64_t blocks = g.M_pad / 16;
+    return blocks > FEW_ROWS_BLOCKS || (g.C_tile > 64 && few_rows_read(g, n) / 8 * (double)few_rows_meet(blocks, (n + 15) / 16) > FEW_ROWS_L2);
+}
 FewRows few_rows(const AmmGeom& g, uint32_t n, uint64_t cus)
 {
-    constexpr double L2_MB = 3.5;  // of a table, beside what else there is
-    const struct { uint32_t item; double base, step, step_mem; } forms[] = {{16, 2.4, 6.2e-3, 9.2e-3}, {32, 2.6, 14.8e-3, 17.2e-3}, {64, 2.95, 28.5e-3, 31e-3}};
+    // us of a launch; of a codebook and round with a table that the L2s hold, with one that they don't, and of that by XCD
+    const struct { uint32_t item; double base, step, step_mem, step_xcd; } forms[] = {
+        {16, 2.4, 6.1e-3, 9.2e-3, 9.2e-3}, {32, 3.0, 21.4e-3, 15.6e-3, 14.3e-3}, {64, 3.5, 29.1e-3, 28.7e-3, 37.3e-3}};
     const uint64_t blocks = g.M_pad / 16;
-    // MB that the tokens read of the table: lines of eight codebooks' pieces of a row
-    const double read = (double)g.CB_pad * g.C_tile * g.M_pad * 1e-6 * (1.0 - exp(-8.0 * n / g.C_tile));
-    const double us_per_mb = g.C_tile > 32 ? 0.08 : 0.025;
+    const double read = few_rows_read(g, n);
     FewRows best{0, false, 1e300};
     for (const auto& f : forms) {
         if (f.item > 16 && 2 * n <= f.item) break;
-        const uint64_t tiles = (n + f.item - 1) / f.item;
-        // XCDs on which the token tiles of a column block meet
-        const uint64_t meet = std::min<uint64_t>(tiles, blocks % 8 == 0 ? 1 : blocks % 4 == 0 ? 2 : blocks % 2 == 0 ? 4 : 8);
-        const bool streams = read / 8 * (double)meet > L2_MB;
+        const uint64_t tiles = (n + f.item - 1) / f.item, meet = few_rows_meet(blocks, tiles);
+        const bool streams = read / 8 * (double)meet > FEW_ROWS_L2;
         const bool by_xcd = streams && tiles > 1 && blocks > 8 && (blocks % 8 != 0 || (tiles * blocks > cus && g.C_tile > 32));
         const double rounds = (double)(((by_xcd ? 8 * few_fullest(blocks, tiles) : tiles * blocks) + cus - 1) / cus);
         const double once = g.C_tile > 32 && !by_xcd ? (double)meet : 1.0;
-        const double us = f.base + g.CB_pad * rounds * (streams ? f.step_mem : f.step) +
-                          (streams ? us_per_mb * std::max(0.0, read * once - 16.0) : 0.1 * (rounds - 1));
+        const double filled = (0.66 + 0.34 * n / (double)(tiles * f.item)) * (tiles == 1 && f.item > 16 ? 0.83 : 1.0);
+        const double us = f.base + (by_xcd ? 0.55 : 0.0) + g.CB_pad * rounds * (by_xcd ? f.step_xcd : streams ? f.step_mem : f.step) * filled +
+                          (streams ? (g.C_tile > 32 ? 0.091 : 0.039) * std::max(0.0, read * once - 20.5) : 0.1 * (rounds - 1));
         if (us < best.us) best = {f.item, by_xcd, us};
     }
     return best;
@@ -419,10 +432,10 @@ double large_rows_us(const AmmGeom& g, uint32_t n, uint64_t cus)
     const bool one_per_cu = g.C_tile == 256;
     const uint64_t blocks = g.M_pad / 16, items = one_per_cu ? (n + 255) / 256 * blocks : (n + 127) / 128 * (g.C_tile <= 32 ? (blocks + 1) / 2 : blocks);
     const double load = (double)items / (double)(one_per_cu ? cus : 2 * cus);
-    const double slice = g.C_tile <= 32 ? 0.3 : g.C_tile == 64 ? 0.305 : g.C_tile == 128 ? 0.39 : 0.72;
-    const double second = g.C_tile <= 32 ? 1.1 : g.C_tile == 64 ? 0.42 : g.C_tile == 128 ? 0.355 : 0.86, further = g.C_tile <= 32 ? 0.2 : one_per_cu ? 1.2 : 0.0;
-    const double table = (double)g.CB_pad * g.C_tile * g.M_pad * 1e-6;
-    return 3.3 + (g.CB + 15) / 16 * (slice + second * std::min(std::max(load - 0.5, 0.0), 0.5) + further * std::max(0.0, load - 1.0)) + 0.09 * std::max(0.0, table - 20.0);
+    const double slice = g.C_tile <= 32 ? 0.255 : g.C_tile == 64 ? 0.26 : g.C_tile == 128 ? 0.332 : 0.613;
+    const double second = g.C_tile <= 32 ? 1.35 : g.C_tile == 64 ? 0.52 : g.C_tile == 128 ? 0.436 : 1.06, further = g.C_tile <= 32 ? 0.17 : one_per_cu ? 1.02 : 0.0;
+    const double table = (double)g.CB * g.C * g.M_pad * 1e-6;
+    return 3.65 + (g.CB + 15) / 16 * (slice + second * std::min(std::max(load - 0.5, 0.0), 0.5) + further * std::max(0.0, load - 1.0)) + 0.084 * std::max(0.0, table - 14.0);
 }
 
 // Tokens of an item: 16, 32 or 64.  One-hot tables: as few as leave every workgroup a CU of its own.  A wave then makes operands for fewer tokens, and
@@ -458,7 +471,7 @@ int launch_few(Ctx* ctx, const Amm& a, const FewArgs& f, const Epilogue& ep)
     const uint32_t cus = ctx->prop.multiProcessorCount;
     uint32_t item;
     bool xcd;
-    if (T == FEW_ROWS && a.g.M_pad / 16 > FEW_ROWS_BLOCKS) {
+    if (T == FEW_ROWS && few_rows_priced(a.g, f.N)) {
         const FewRows r = few_rows(a.g, f.N, cus);
         item = r.item;
         xcd = r.by_xcd;
@@ -579,7 +592,7 @@ uint32_t few_column_groups(const Ctx* ctx, const AmmGeom& g, uint32_t n)
 // 19.8 / 4.5 at 1, 20.2 / 7.7 at 150, 19.8 / 13.1 at 512, 20.3 / 18.2 at 1024; 8 centroids 3072 -> 768 15.4 / 5.9 at 64,
 // 15.6 / 10.0 at 512: up to two workgroups of this launch per CU (the paired table; for the sparse one few_column_groups decides).
 // The byte adder and the floats read every gathered piece from the caches on its own, which costs in proportion to
-// tokens x codebooks x columns -- the byte adder by rounds of workgroups of 16 tokens x 16 columns, which take their codebooks' time each --;
+// tokens x codebooks x columns -- the byte adder by rounds of workgroups of 16 tokens x 16 columns, which take their codebooks' time each (see few_rows) --;
 // against that stands the large kernels' chain of slices.  Byte adder, 3072 -> 768, 32 centroids: 17.6 / 4.4 at N = 1, 17.4 / 8.6 at 64,
 // 17.6 / 14.8 at 128 (384 workgroups), 17.8 / 20.9 at 192; 768 -> 768 6.8 / 3.8 at 70, 7.0 / 5.4 at 150, 7.2 / 8.6 at 300; 768 -> 3072 8.3 / 5.4 at
 // 32, 8.8 / 10.9 at 100; 16 codebooks, M = 1040 3.3 / 2.6 at 32, 3.8 / 4.2 at 300; 64 centroids 1024 -> 1024 7.2 / 4.4 at 50, 7.4 / 6.6 at 100, 7.6 / 8.9 at
@@ -603,7 +616,7 @@ bool gather_few_wanted(const Ctx* ctx, const Amm& a, uint32_t n)
         return 2.7 + g.CB_pad * (bounds ? 0.062 : 0.0137) + pieces * piece < 4.0 + g.CB_pad * (bounds ? 0.14 : 0.07);
     }
     if (g.gather_kind == 0) {
-        if (g.M_pad / 16 > FEW_ROWS_BLOCKS) return g.idx_bits == 8 && few_rows(g, n, cus).us < large_rows_us(g, n, cus);
+        if (few_rows_priced(g, n)) return g.idx_bits == 8 && few_rows(g, n, cus).us < large_rows_us(g, n, cus);
         if (g.C_tile == 64) return g.idx_bits == 8 && few_rows64_wanted(g, n, cus);
         const uint64_t slices = (g.CB + 15) / 16;
         uint32_t rows_item;

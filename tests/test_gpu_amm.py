@@ -1987,6 +1987,8 @@ def test_gather_of_64_centroids_by_what_an_xcd_has_to_do(ctx, CB, M, N, kernel):
     (33, 300, 128, 2441, "gather_i8_few_kernel<1, 8, true>"),   # 153 blocks: seven of the grid's past the last
     (40, 20, 64, 1216, "gather_i8_few_kernel<1, 16, false>"), (40, 20, 64, 1200, "gather_i8_few_kernel<1, 16, false>"),  # 76 and 75 blocks
     (17, 512, 24, 8192, "gather_i8_few_kernel<2, 8, false>"),
+    (50, 300, 200, 520, "gather_i8_few_kernel<1, 16, true>"),   # 33 blocks, by XCD for the size of the table
+    (409, 300, 128, 266, "gather_i8_kernel<"),
 ])
 def test_byte_adder_of_few_tokens_and_many_column_blocks(ctx, N, CB, C, M, kernel):
     """The items that the launch takes by its prices: accumulators and output bits of the oracle, nothing behind the output."""
